@@ -6,83 +6,27 @@
 // [tile_begin_p, tile_begin_{p+1}).  A problem sums several K-segments, each
 // an (optionally transposed) A x B product with its own alpha, so the whole
 // sum_k L_k x_k or sum_r U_r R_r^T of one local step is one accumulation in
-// registers.  Workgroup: 256 lanes = 4 wavefronts of 64, each wavefront owns
-// a 32x32 quarter of the tile as 2x2 MFMA 16x16 blocks.
-//   f64 : v_mfma_f64_16x16x4_f64   (K step 4,  LDS chunk 32, two LDS stages)
-//   f32 : v_mfma_f32_16x16x4_f32   (K step 4,  LDS chunk 64, one stage)
-//   bf16: v_mfma_f32_16x16x32_bf16 (K step 32, LDS chunk 128, one stage, f32
-//         accumulate)
-// The K chunks of all segments form one stream; the global loads of the next
-// chunk are in flight in registers during the MFMAs of the current one, and
-// runs of 16 bytes are loaded as one vector when they are in bounds and
-// aligned.
+// registers.
+//   f64 : v_mfma_f64_16x16x4_f64    f32: v_mfma_f32_16x16x4_f32
+//   bf16: v_mfma_f32_16x16x32_bf16 (f32 accumulate)
 #include <type_traits>
 
 #include "tnx_common.h"
 
 namespace {
 
-// A configuration (kernel template argument CFG) fixes the GEMM mode, the K
-// depth KB of one staged chunk, NE (elements of A and of B each lane fetches
-// per chunk; 256 x NE = 64 x KB) and DB (LDS double buffering).
-// - f64 is MFMA bound at these shapes. Two variants, both with two LDS stages
-//   (one barrier per chunk, the commit of chunk c+1 overlapping the MFMAs of
-//   chunk c); they differ in depth and occupancy, and neither wins
-//   everywhere.  Mid-chain matvec, 64 solves:
-//     variant 0, 32-deep chunks, 69.6 KB, 2 workgroups per CU:
-//       GEMM 1 (2048 tiles, K 128) 69 us, GEMM 2 (512 tiles, K 512) 64 us;
-//     variant 1, 16-deep chunks, 34.8 KB, 4 workgroups per CU:
-//       GEMM 1 59 us, GEMM 2 75 us.
-//   (One stage of 64: 75 / 69 us.)  The caller picks the variant per launch
-//   (the mode's second byte); the engine times both on first use.
-// - f32 / bf16 are latency bound at these shapes: one stage of a deep chunk
-//   (34.8 KB, four workgroups per CU), two barriers per chunk; a second stage
-//   measured slower (f32 GEMM 2: 38 -> 42 us; bf16 GEMM 1: 16 -> 22 us).
-// All variants of a mode issue the same MFMAs in the same k order, so they
-// give the same bits.
-// NT lanes per workgroup as WR x WC wavefronts, each owning a
-// (64 / WR) x (64 / WC) part of the tile as 16x16 MFMA blocks.  The 8-wave
-// bf16 variants (16x32 per wave) double the waves per workgroup for
-// launches of few tiles: mid-chain GEMM 2 (K 512), 16 solves 12.7 -> 11.0
-// us, 64 solves 19.9 -> 17.8 us; each output block still sees the same
-// MFMAs in the same k order.  Measured and not kept: the same 8-wave split
-// for f32 (25.0 -> 25.2 us), 128-deep f32 chunks (25.0 -> 27.7 us) and
-// 64-deep f64 chunks with one workgroup per CU (43.1 -> 45.0 us).
-template <int CFG> struct Cfg;
-template <> struct Cfg<0> {
-  typedef double TI; typedef double TC; typedef double ACC; typedef double CT;
-  static constexpr int MODE = TNX_GEMM_F64, KB = 32, NE = 8, NT = 256, WR = 2, WC = 2;
-  static constexpr bool DB = true;
+template <int MODE> struct Tr;
+template <> struct Tr<TNX_GEMM_F64> {
+  typedef double TI; typedef double TC; typedef tnx_d4 V4;
 };
-template <> struct Cfg<1> {
-  typedef float TI; typedef float TC; typedef float ACC; typedef float CT;
-  static constexpr int MODE = TNX_GEMM_F32, KB = 64, NE = 16, NT = 256, WR = 2, WC = 2;
-  static constexpr bool DB = false;
+template <> struct Tr<TNX_GEMM_F32> {
+  typedef float TI; typedef float TC; typedef tnx_f4 V4;
 };
-template <> struct Cfg<2> {
-  typedef __bf16 TI; typedef float TC; typedef float ACC; typedef __bf16 CT;
-  static constexpr int MODE = TNX_GEMM_BF16_F32, KB = 128, NE = 32, NT = 256, WR = 2, WC = 2;
-  static constexpr bool DB = false;
+template <> struct Tr<TNX_GEMM_BF16_F32> {
+  typedef __bf16 TI; typedef float TC; typedef tnx_f4 V4;
 };
-template <> struct Cfg<3> {
-  typedef __bf16 TI; typedef __bf16 TC; typedef float ACC; typedef __bf16 CT;
-  static constexpr int MODE = TNX_GEMM_BF16_BF16, KB = 128, NE = 32, NT = 256, WR = 2, WC = 2;
-  static constexpr bool DB = false;
-};
-template <> struct Cfg<4> {   // f64, variant 1
-  typedef double TI; typedef double TC; typedef double ACC; typedef double CT;
-  static constexpr int MODE = TNX_GEMM_F64, KB = 16, NE = 4, NT = 256, WR = 2, WC = 2;
-  static constexpr bool DB = true;
-};
-template <> struct Cfg<6> {   // bf16 -> f32, variant 1: 8 waves
-  typedef __bf16 TI; typedef float TC; typedef float ACC; typedef __bf16 CT;
-  static constexpr int MODE = TNX_GEMM_BF16_F32, KB = 128, NE = 16, NT = 512, WR = 4, WC = 2;
-  static constexpr bool DB = false;
-};
-template <> struct Cfg<7> {   // bf16 -> bf16, variant 1: 8 waves
-  typedef __bf16 TI; typedef __bf16 TC; typedef float ACC; typedef __bf16 CT;
-  static constexpr int MODE = TNX_GEMM_BF16_BF16, KB = 128, NE = 16, NT = 512, WR = 4, WC = 2;
-  static constexpr bool DB = false;
+template <> struct Tr<TNX_GEMM_BF16_BF16> {
+  typedef __bf16 TI; typedef __bf16 TC; typedef tnx_f4 V4;
 };
 
 template <typename T> __device__ __forceinline__ double to_d(T v) { return (double)v; }
@@ -90,297 +34,477 @@ template <> __device__ __forceinline__ double to_d<__bf16>(__bf16 v) { return (d
 template <typename T> __device__ __forceinline__ T from_d(double v) { return (T)v; }
 template <> __device__ __forceinline__ __bf16 from_d<__bf16>(double v) { return (__bf16)(float)v; }
 
-constexpr int TM = 64, TN = 64;
+// Pointers of the global address space (the records carry plain integers: a
+// generic pointer made from one would be accessed with flat loads, which
+// wait on the LDS counter too).
+#define TNX_GLOBAL __attribute__((address_space(1)))
+template <typename T> __device__ __forceinline__ T TNX_GLOBAL* as_global(uint64_t p) {
+  return (T TNX_GLOBAL*)p;
+}
 
-// NE contiguous elements starting at p, of which the first `valid` are in
-// bounds; out-of-bounds ones read as zero.  Loaded as 16-byte vectors when
-// every element is valid and p is 16-byte aligned.
-template <typename TI, int NE>
-__device__ __forceinline__ void load_run(const TI* p, int valid, TI (&v)[NE]) {
-  constexpr int VB = 16 / sizeof(TI);  // elements per 16-byte vector
-  if (valid >= NE && (((uintptr_t)p) & 15) == 0) {
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+// A K chunk is 128 bytes deep (KB = 16, 32 or 64 elements) and is staged
+// through LDS in the layout of its source, 16 bytes at a time:
+// - an operand contiguous in k as rows of 128 bytes, [row][k], the 16-byte
+//   pieces of a row permuted by (row / MB) % 8 so that the 16 rows an MFMA
+//   reads at one k lie in distinct banks;
+// - an operand contiguous along its rows (A) or columns (B) as [k][row].
+// Lane group g = lane / 16 holds k = KL g .. KL g + KL - 1 of each half
+// chunk (KL elements are 16 bytes) and MFMA t takes element t of every
+// group; block i of a wave has rows MB m + i.  So every access to LDS and
+// to global memory, the stores of C included, is as wide as the layout lets
+// it be, and the k order of an element is the same for every tile shape:
+// the shape never changes the bits.
+template <typename TI, int TT, int MB> struct Operand {
+  static constexpr int E = 16 / (int)sizeof(TI);      // elements per piece
+  static constexpr int KL = E;
+  static constexpr int KB = 128 / (int)sizeof(TI);
+  static constexpr int NP = TT * 8 / 256;             // pieces per lane and chunk
+  static constexpr int PR = TT / E;                   // pieces per k row of the [k][row] layout
+  static constexpr bool HALF = sizeof(TI) == 2;
+
+  // The lane's pieces of the chunk at k0, without a branch (the waits then
+  // count loads and leave the later ones in flight).  Rows past `lim` repeat
+  // earlier ones (their products are not stored) and k past K earlier k,
+  // which clear() zeroes when the chunk is staged.  WIDE: one 16-byte load a
+  // piece, for sizes that pieces divide (wide_ok); otherwise by elements.
+  template <bool KC> static __device__ __forceinline__ bool wide_ok(int lim, int K) {
+    return ((KC ? K : lim) % E) == 0;
+  }
+  template <bool KC, bool WIDE>
+  static __device__ __forceinline__ void fetch(u4 (&r)[NP], uint64_t b, int64_t ld, int row0,
+                                               int lim, int k0, int K) {
+    typedef TI V __attribute__((ext_vector_type(E), aligned(sizeof(TI))));
+    const TI TNX_GLOBAL* base = as_global<const TI>(b);
 #pragma unroll
-    for (int q = 0; q < NE / VB; ++q) {
-      const uint4 w = *(const uint4*)(p + q * VB);
-      TI e[VB];
-      __builtin_memcpy(e, &w, 16);
+    for (int q = 0; q < NP; ++q) {
+      const int c = threadIdx.x + 256 * q;
+      const int row = row0 + (KC ? c >> 3 : (c % PR) * E);
+      const int k = k0 + (KC ? (c & 7) * E : c / PR);
+      if constexpr (WIDE) {
+        const int64_t off = KC ? min(row, lim - 1) * ld + min(k, K - E)
+                               : min(k, K - 1) * ld + min(row, lim - E);
+        r[q] = __builtin_bit_cast(u4, *(const V TNX_GLOBAL*)(base + off));
+      } else {
+        TI e[E];
 #pragma unroll
-      for (int t = 0; t < VB; ++t) v[q * VB + t] = e[t];
+        for (int x = 0; x < E; ++x)
+          e[x] = KC ? base[min(row, lim - 1) * ld + min(k + x, K - 1)]
+                    : base[min(k, K - 1) * ld + min(row + x, lim - 1)];
+        __builtin_memcpy(&r[q], e, 16);
+        // piece by piece: the addresses of all of them would cost occupancy
+        if constexpr (HALF) __builtin_amdgcn_sched_barrier(0);
+      }
     }
-  } else {
-#pragma unroll
-    for (int e = 0; e < NE; ++e) v[e] = (e < valid) ? p[e] : (TI)0.0f;
   }
-}
 
-// Per-thread fragment of one K chunk: NE elements of the A tile and NE of the
-// B tile, with the addressing mode they were fetched in.
-template <int CFG> struct Frag {
-  typename Cfg<CFG>::TI a[Cfg<CFG>::NE];
-  typename Cfg<CFG>::TI b[Cfg<CFG>::NE];
-  double alpha;
-  int ta, tb;
-};
+  static __device__ __forceinline__ int swz(int row) { return (row / MB) & 7; }
 
-// Thread t's share of a 64 x KB A tile / KB x 64 B tile (NT threads x NE =
-// 64 x KB).
-//   transA = 0 (k contiguous): row t/(KB/NE), k = (t%(KB/NE))*NE .. +NE
-//   transA = 1 (i contiguous): k  t/(64/NE), i = (t%(64/NE))*NE .. +NE
-template <int CFG>
-__device__ __forceinline__ void fetch(Frag<CFG>& f, const tnx_gemm_seg& S, int M, int N, int row0,
-                                      int col0, int k0) {
-  typedef typename Cfg<CFG>::TI TI;
-  constexpr int KB = Cfg<CFG>::KB, NE = Cfg<CFG>::NE;
-  const int t = threadIdx.x;
-  const TI* A = (const TI*)S.a;
-  const TI* B = (const TI*)S.b;
-  f.alpha = S.alpha;
-  f.ta = S.transA;
-  f.tb = S.transB;
-  if (!S.transA) {
-    const int i = t / (KB / NE), kq = (t % (KB / NE)) * NE;
-    const int gi = row0 + i, gk = k0 + kq;
-    const int valid = (gi < M) ? min(NE, S.K - gk) : 0;
-    load_run<TI, NE>(A + (int64_t)(gi < M ? gi : 0) * S.lda + gk, valid, f.a);
-  } else {
-    const int k = t / (TM / NE), iq = (t % (TM / NE)) * NE;
-    const int gi = row0 + iq, gk = k0 + k;
-    const int valid = (gk < S.K) ? min(NE, M - gi) : 0;
-    load_run<TI, NE>(A + (int64_t)(gk < S.K ? gk : 0) * S.lda + gi, valid, f.a);
-  }
-  if (!S.transB) {
-    const int k = t / (TN / NE), jq = (t % (TN / NE)) * NE;
-    const int gj = col0 + jq, gk = k0 + k;
-    const int valid = (gk < S.K) ? min(NE, N - gj) : 0;
-    load_run<TI, NE>(B + (int64_t)(gk < S.K ? gk : 0) * S.ldb + gj, valid, f.b);
-  } else {
-    const int j = t / (KB / NE), kq = (t % (KB / NE)) * NE;
-    const int gj = col0 + j, gk = k0 + kq;
-    const int valid = (gj < N) ? min(NE, S.K - gk) : 0;
-    load_run<TI, NE>(B + (int64_t)(gj < N ? gj : 0) * S.ldb + gk, valid, f.b);
-  }
-}
-
-// f64/f32: LDS tiles k-major, As[k][i], Bs[k][j] (conflict-free MFMA reads)
-template <int CFG>
-__device__ __forceinline__ void commit_k4(const Frag<CFG>& f, typename Cfg<CFG>::CT (*As)[TM + 4],
-                                          typename Cfg<CFG>::CT (*Bs)[TN + 4]) {
-  typedef typename Cfg<CFG>::CT CT;
-  constexpr int KB = Cfg<CFG>::KB, NE = Cfg<CFG>::NE;
-  const int t = threadIdx.x;
-  if (!f.ta) {
-    const int i = t / (KB / NE), kq = (t % (KB / NE)) * NE;
+  template <bool KC> static __device__ __forceinline__ void commit(const u4 (&r)[NP], u4* lds) {
+    const int t = threadIdx.x;
 #pragma unroll
-    for (int e = 0; e < NE; ++e) As[kq + e][i] = (CT)(f.alpha * to_d(f.a[e]));
-  } else {
-    const int k = t / (TM / NE), iq = (t % (TM / NE)) * NE;
-#pragma unroll
-    for (int e = 0; e < NE; ++e) As[k][iq + e] = (CT)(f.alpha * to_d(f.a[e]));
-  }
-  if (!f.tb) {
-    const int k = t / (TN / NE), jq = (t % (TN / NE)) * NE;
-#pragma unroll
-    for (int e = 0; e < NE; ++e) Bs[k][jq + e] = (CT)to_d(f.b[e]);
-  } else {
-    const int j = t / (KB / NE), kq = (t % (KB / NE)) * NE;
-#pragma unroll
-    for (int e = 0; e < NE; ++e) Bs[kq + e][j] = (CT)to_d(f.b[e]);
-  }
-}
-
-// bf16: LDS tiles row-major in k, As[i][k], Bs[j][k] (8 consecutive k per lane)
-template <int CFG>
-__device__ __forceinline__ void commit_bf16(const Frag<CFG>& f, __bf16 (*As)[Cfg<CFG>::KB + 8],
-                                            __bf16 (*Bs)[Cfg<CFG>::KB + 8]) {
-  constexpr int KB = Cfg<CFG>::KB, NE = Cfg<CFG>::NE;
-  const int t = threadIdx.x;
-  const float alpha = (float)f.alpha;
-  if (!f.ta) {
-    const int i = t / (KB / NE), kq = (t % (KB / NE)) * NE;
-    if (alpha == 1.0f) {
-#pragma unroll
-      for (int e = 0; e < NE; ++e) As[i][kq + e] = f.a[e];
-    } else {
-#pragma unroll
-      for (int e = 0; e < NE; ++e) As[i][kq + e] = (__bf16)(alpha * (float)f.a[e]);
+    for (int q = 0; q < NP; ++q) {
+      const int c = t + 256 * q;
+      lds[KC ? (c & ~7) | ((c & 7) ^ swz(c >> 3)) : c] = r[q];
     }
-  } else {
-    const int k = t / (TM / NE), iq = (t % (TM / NE)) * NE;
-#pragma unroll
-    for (int e = 0; e < NE; ++e) As[iq + e][k] = (__bf16)(alpha * (float)f.a[e]);
   }
-  if (!f.tb) {
-    const int k = t / (TN / NE), jq = (t % (TN / NE)) * NE;
+
+  // zero the pieces' elements from k index `valid` of the chunk on
+  template <bool KC> static __device__ __forceinline__ void clear(u4 (&r)[NP], int valid) {
 #pragma unroll
-    for (int e = 0; e < NE; ++e) Bs[jq + e][k] = f.b[e];
-  } else {
-    const int j = t / (KB / NE), kq = (t % (KB / NE)) * NE;
+    for (int q = 0; q < NP; ++q) {
+      const int c = threadIdx.x + 256 * q;
+      TI e[E];
+      __builtin_memcpy(e, &r[q], 16);
 #pragma unroll
-    for (int e = 0; e < NE; ++e) Bs[j][kq + e] = f.b[e];
-  }
-}
-
-template <int CFG>
-__global__ __launch_bounds__(Cfg<CFG>::NT) void gemm_grouped_kernel(const tnx_gemm_problem* __restrict__ probs,
-                                                          int nprob,
-                                                          const tnx_gemm_seg* __restrict__ segs,
-                                                          const int32_t* __restrict__ active,
-                                                          unsigned long long* ts) {
-  tnx_stamp_begin(ts);
-  typedef Cfg<CFG> C;
-  constexpr int MODE = C::MODE;
-  typedef typename C::ACC ACC;
-  typedef typename C::TC TC;
-  constexpr int KB = C::KB;
-  const int bid = tnx_xcd_remap(blockIdx.x, gridDim.x);
-  const int pi = tnx_find_owner(probs, sizeof(tnx_gemm_problem),
-                                offsetof(tnx_gemm_problem, tile_begin), nprob, bid);
-  const tnx_gemm_problem P = probs[pi];
-  if (P.active >= 0 && active != nullptr && active[P.active] == 0) return;
-  const int tiles_n = (P.N + TN - 1) / TN;
-  const int t_local = bid - P.tile_begin;
-  const int row0 = (t_local / tiles_n) * TM, col0 = (t_local % tiles_n) * TN;
-  if (row0 >= P.M) return;  // cannot happen with exact prefix sums
-
-  static_assert(C::NT * C::NE == TM * KB && C::WR * C::WC * 64 == C::NT, "tile split");
-  constexpr int MB = TM / C::WR / 16, NB = TN / C::WC / 16;   // MFMA blocks per wave
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wr = (wave / C::WC) * (TM / C::WR), wc = (wave % C::WC) * (TN / C::WC);
-
-  typedef typename std::conditional<sizeof(ACC) == 8, tnx_d4, tnx_f4>::type V4;
-  V4 acc[MB][NB];
-#pragma unroll
-  for (int a = 0; a < MB; ++a)
-#pragma unroll
-    for (int b = 0; b < NB; ++b) acc[a][b] = V4{0, 0, 0, 0};
-
-  typedef typename std::conditional<(MODE == TNX_GEMM_F64 || MODE == TNX_GEMM_F32),
-                                    typename C::CT, __bf16>::type CT;
-  constexpr bool K4 = (MODE == TNX_GEMM_F64 || MODE == TNX_GEMM_F32);
-  constexpr int AR = K4 ? KB : TM, AC = K4 ? TM + 4 : KB + 8;
-  constexpr int BR = K4 ? KB : TN, BC = K4 ? TN + 4 : KB + 8;
-  constexpr bool DB = C::DB;
-  __shared__ __attribute__((aligned(16))) CT As[DB ? 2 : 1][AR][AC];
-  __shared__ __attribute__((aligned(16))) CT Bs[DB ? 2 : 1][BR][BC];
-
-  // Flattened stream of (segment, k0) chunks; (s, k0) is the next chunk to
-  // fetch.  Pipeline: chunk c+1 is in registers while chunk c is in LDS;
-  // each step runs chunk c's MFMAs, commits chunk c+1 (double buffered: to
-  // the other stage, which the barrier of the previous step guarantees every
-  // wave has finished reading; single stage: after a barrier), one barrier,
-  // then fetches chunk c+2, whose loads fly during the next MFMAs.
-  int s = P.seg_begin, k0 = 0;
-  const int s_end = P.seg_begin + P.seg_count;
-  while (s < s_end && segs[s].K <= 0) ++s;
-  Frag<CFG> f;
-  tnx_gemm_seg S;
-  if (s < s_end) S = segs[s];
-  auto advance = [&]() {
-    k0 += KB;
-    if (k0 >= S.K) {
-      k0 = 0;
-      ++s;
-      while (s < s_end && segs[s].K <= 0) ++s;
-      if (s < s_end) S = segs[s];
+      for (int x = 0; x < E; ++x)
+        if ((KC ? (c & 7) * E + x : c / PR) >= valid) e[x] = (TI)0.0f;
+      __builtin_memcpy(&r[q], e, 16);
     }
-  };
-  bool staged = false;  // chunk c is in LDS
-  if (s < s_end) {
-    fetch<CFG>(f, S, P.M, P.N, row0, col0, k0);
-    advance();
-    if constexpr (K4) commit_k4<CFG>(f, As[0], Bs[0]);
-    else commit_bf16<CFG>(f, As[0], Bs[0]);
-    staged = true;
   }
-  __syncthreads();
-  bool held = false;  // chunk c+1 is in registers
-  if (s < s_end) {
-    fetch<CFG>(f, S, P.M, P.N, row0, col0, k0);
-    advance();
-    held = true;
+
+  static __device__ __forceinline__ void scale(u4 (&r)[NP], double alpha) {
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      TI e[E];
+      __builtin_memcpy(e, &r[q], 16);
+#pragma unroll
+      for (int x = 0; x < E; ++x) {
+        if constexpr (HALF) e[x] = (TI)((float)alpha * (float)e[x]);
+        else e[x] = (TI)(alpha * (double)e[x]);
+      }
+      __builtin_memcpy(&r[q], e, 16);
+    }
   }
-  int stage = 0;
-  while (staged) {
-    if constexpr (K4) {
+
+  // Half chunk h of the wave's rows from `row` (within the tile)
+  template <bool KC> struct Raw {
+    // [k][row]: KL loads of MB elements (16-bit ones as whole words)
+    static constexpr int W = KC ? 4 : (MB * (int)sizeof(TI) + 3) / 4;
+    uint32_t w[KC ? MB : KL][W];
+
+    __device__ __forceinline__ void read(const u4* lds, int row, int h) {
+      const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+      if constexpr (KC) {
 #pragma unroll
-      for (int kk = 0; kk < KB; kk += 4) {
-        CT a[MB], b[NB];
+        for (int i = 0; i < MB; ++i) {
+          const int rr = row + MB * m + i;
+          const u4 v = lds[rr * 8 + ((4 * h + g) ^ swz(rr))];
 #pragma unroll
-        for (int mi = 0; mi < MB; ++mi) a[mi] = As[stage][kk + (lane >> 4)][wr + 16 * mi + (lane & 15)];
+          for (int x = 0; x < 4; ++x) w[i][x] = v[x];
+        }
+      } else {
+        const char* p = (const char*)lds + ((h * (KB / 2) + KL * g) * TT + row + MB * m) * (int)sizeof(TI);
 #pragma unroll
-        for (int nj = 0; nj < NB; ++nj) b[nj] = Bs[stage][kk + (lane >> 4)][wc + 16 * nj + (lane & 15)];
+        for (int s = 0; s < KL; ++s) {
+          const char* q = p + s * TT * (int)sizeof(TI);
+          if constexpr (MB * sizeof(TI) == 2) w[s][0] = *(const uint16_t*)q;
+          else {
+            typedef uint32_t V __attribute__((ext_vector_type(W)));
+            const V v = *(const V*)q;
 #pragma unroll
-        for (int mi = 0; mi < MB; ++mi)
-#pragma unroll
-          for (int nj = 0; nj < NB; ++nj) {
-            if constexpr (MODE == TNX_GEMM_F64)
-              acc[mi][nj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mi], b[nj], acc[mi][nj], 0, 0, 0);
-            else
-              acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[mi], b[nj], acc[mi][nj], 0, 0, 0);
+            for (int x = 0; x < W; ++x) w[s][x] = v[x];
           }
-      }
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < KB; kk += 32) {
-        const int kq = kk + (lane >> 4) * 8;
-        tnx_bf8 a[MB], b[NB];
-#pragma unroll
-        for (int mi = 0; mi < MB; ++mi) a[mi] = *(const tnx_bf8*)&As[stage][wr + 16 * mi + (lane & 15)][kq];
-#pragma unroll
-        for (int nj = 0; nj < NB; ++nj) b[nj] = *(const tnx_bf8*)&Bs[stage][wc + 16 * nj + (lane & 15)][kq];
-#pragma unroll
-        for (int mi = 0; mi < MB; ++mi)
-#pragma unroll
-          for (int nj = 0; nj < NB; ++nj)
-            acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mi], b[nj], acc[mi][nj], 0, 0, 0);
-      }
-    }
-    staged = held;
-    if constexpr (!DB) __syncthreads();  // every wave has read the single stage
-    const int next = DB ? stage ^ 1 : 0;
-    if (held) {
-      if constexpr (K4) commit_k4<CFG>(f, As[next], Bs[next]);
-      else commit_bf16<CFG>(f, As[next], Bs[next]);
-    }
-    __syncthreads();
-    held = false;
-    if (staged && s < s_end) {
-      fetch<CFG>(f, S, P.M, P.N, row0, col0, k0);
-      advance();
-      held = true;
-    }
-    stage = next;
-  }
-
-  // epilogue: column lane%16 of each 16x16 block; the row of accumulator
-  // element r is 4*(lane/16)+r for the f32-output MFMAs and (lane/16)+4*r for
-  // v_mfma_f64_16x16x4_f64 (measured on gfx950)
-  TC* Cp = (TC*)P.c;
-  const TC* C0 = (const TC*)P.c0;
-#pragma unroll
-  for (int mi = 0; mi < MB; ++mi)
-#pragma unroll
-    for (int nj = 0; nj < NB; ++nj)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
-        const int gi = row0 + wr + mi * 16 + rr;
-        const int gj = col0 + wc + nj * 16 + (lane & 15);
-        if (gi < P.M && gj < P.N) {
-          double v = (double)acc[mi][nj][r];
-          if (C0 != nullptr) v += P.beta * to_d(C0[(int64_t)gi * P.ldc0 + gj]);
-          Cp[(int64_t)gi * P.ldc + gj] = from_d<TC>(v);
         }
       }
-  tnx_stamp_end(ts);
+    }
+    // element s of block i (f64, f32)
+    __device__ __forceinline__ TI get(int i, int s) const {
+      TI v;
+      constexpr int WE = sizeof(TI) >= 4 ? (int)sizeof(TI) / 4 : 1;
+      __builtin_memcpy(&v, KC ? &w[KC ? i : 0][WE * s] : &w[KC ? 0 : s][KC ? 0 : WE * i], sizeof(TI));
+      return v;
+    }
+    // the 8 k of block i (bf16)
+    __device__ __forceinline__ tnx_bf8 get8(int i) const {
+      uint32_t x[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if constexpr (KC) x[t] = w[i][t];
+        else x[t] = __builtin_amdgcn_perm(w[2 * t + 1][i / 2], w[2 * t][i / 2],
+                                          (i & 1) ? 0x07060302u : 0x05040100u);
+      }
+      tnx_bf8 v;
+      __builtin_memcpy(&v, x, 16);
+      return v;
+    }
+  };
+};
+
+// acc += the staged chunk's A B, the wave's rows from wr and columns from wc
+template <int MODE, int TT, int MB, bool KA, bool KBc>
+__device__ __forceinline__ void mma_chunk(typename Tr<MODE>::V4 (&acc)[MB][MB], const u4* As,
+                                          const u4* Bs, int wr, int wc) {
+  typedef typename Tr<MODE>::TI TI;
+  typedef Operand<TI, TT, MB> O;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    typename O::template Raw<KA> a;
+    typename O::template Raw<KBc> b;
+    a.read(As, wr, h);
+    b.read(Bs, wc, h);
+    if constexpr (O::HALF) {
+      tnx_bf8 av[MB], bv[MB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) av[i] = a.get8(i);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) bv[i] = b.get8(i);
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < MB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < O::KL; ++t)
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int j = 0; j < MB; ++j) {
+            if constexpr (MODE == TNX_GEMM_F64)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.get(i, t), b.get(j, t), acc[i][j], 0, 0, 0);
+            else
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.get(i, t), b.get(j, t), acc[i][j], 0, 0, 0);
+          }
+    }
+  }
+}
+
+// The problem that owns 64x64 tile `bid`: problems of a launch are mostly of
+// one size, so the record at its share of the range is tried first (one
+// round of loads), then the search.
+__device__ __forceinline__ int find_problem(const tnx_gemm_problem* __restrict__ probs, int nprob,
+                                            int bid, int ntiles) {
+  const int guess = (int)((int64_t)bid * nprob / ntiles);
+  const int lo = probs[guess].tile_begin;
+  const int hi = guess + 1 < nprob ? probs[guess + 1].tile_begin : ntiles;
+  if (bid >= lo && bid < hi) return guess;
+  return tnx_find_owner(probs, sizeof(tnx_gemm_problem), offsetof(tnx_gemm_problem, tile_begin),
+                        nprob, bid);
+}
+
+// Barrier of the LDS stages: LDS accesses only are ordered (the loads from
+// global memory of the chunks ahead stay in flight across it).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Descriptor records are read through the scalar cache: they do not change
+// during the launch, and the vector counter then counts operand loads only.
+#define TNX_CONST __attribute__((address_space(4)))
+
+// whether a segment's operands can be fetched by 16-byte pieces
+template <typename O, bool KA, bool KBc>
+__device__ __forceinline__ bool wide(int M, int N, int K) {
+  return O::template wide_ok<KA>(M, K) && O::template wide_ok<KBc>(N, K);
+}
+
+// acc += the products of the segments [s, ...) with the same layouts as
+// segment s (KA: A contiguous in k, KBc: B) and the same WIDE; returns the
+// first segment after them.  Their chunks form one stream: PD chunks are in flight in registers
+// ahead of the staged one, across the segments; past the last chunk it is
+// fetched again, unused (no branch around the loads, so that the waits count
+// them and never drain them).
+template <int MODE, int TT, int PD, bool KA, bool KBc, bool WIDE>
+__device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][TT / 32],
+                                          const tnx_gemm_seg TNX_CONST* segs, int s, int s_end,
+                                          int M, int N, int row0, int col0, int wr, int wc,
+                                          u4 (*As)[TT * 8], u4 (*Bs)[TT * 8]) {
+  constexpr int MB = TT / 32;
+  typedef Operand<typename Tr<MODE>::TI, TT, MB> O;
+  u4 ra[PD][O::NP], rb[PD][O::NP];
+  double al[PD];
+  int kv[PD];           // k of the chunk that exist
+  // the stream's extent: its segments and chunks
+  int chunks = 0, end = s;
+  for (; end < s_end; ++end) {
+    const int K = segs[end].K;
+    if (K <= 0) continue;
+    if ((segs[end].transA == 0) != KA || (segs[end].transB != 0) != KBc ||
+        wide<O, KA, KBc>(M, N, K) != WIDE)
+      break;
+    chunks += (K + O::KB - 1) / O::KB;
+  }
+  uint64_t A = segs[s].a, B = segs[s].b;
+  int lda = segs[s].lda, ldb = segs[s].ldb, K = segs[s].K, k0 = 0;
+  double alpha = segs[s].alpha;
+  auto fetch = [&](int d) {
+    O::template fetch<KA, WIDE>(ra[d], A, lda, row0, M, k0, K);
+    O::template fetch<KBc, WIDE>(rb[d], B, ldb, col0, N, k0, K);
+    al[d] = alpha;
+    kv[d] = K - k0;
+    if (k0 + O::KB < K) {
+      k0 += O::KB;
+    } else {
+      int n = s + 1;
+      while (n < end && segs[n].K <= 0) ++n;
+      if (n < end) {
+        s = n;
+        A = segs[n].a;
+        B = segs[n].b;
+        lda = segs[n].lda;
+        ldb = segs[n].ldb;
+        K = segs[n].K;
+        alpha = segs[n].alpha;
+        k0 = 0;
+      }
+    }
+  };
+  auto commit = [&](int d, int stage) {
+    if (kv[d] < O::KB) {
+      asm volatile("");   // a branch, not selects on every chunk
+      O::template clear<KA>(ra[d], kv[d]);
+      O::template clear<KBc>(rb[d], kv[d]);
+    }
+    if (__double_as_longlong(al[d]) != 0x3FF0000000000000ll) {
+      asm volatile("");
+      O::scale(ra[d], al[d]);
+    }
+    O::template commit<KA>(ra[d], As[stage]);
+    O::template commit<KBc>(rb[d], Bs[stage]);
+  };
+#pragma unroll
+  for (int d = 0; d < PD; ++d) fetch(d);
+  commit(0, 0);
+  fetch(0);
+  lds_barrier();
+  // each step: the MFMAs of the staged chunk, then the next one into the
+  // other stage (read by all before the last barrier) and its registers
+  // refilled
+  auto step = [&](int u) {
+    const int d = (u + 1) % PD, stage = u & 1;
+    mma_chunk<MODE, TT, MB, KA, KBc>(acc, As[stage], Bs[stage], wr, wc);
+    commit(d, stage ^ 1);
+    fetch(d);
+    lds_barrier();
+  };
+  for (int t = chunks / (2 * PD); t > 0; --t) {
+#pragma unroll
+    for (int u = 0; u < 2 * PD; ++u) step(u);
+  }
+  const int rest = chunks % (2 * PD);
+#pragma unroll
+  for (int u = 0; u < 2 * PD - 1; ++u)
+    if (u < rest) step(u);
+  return end;
+}
+
+// Workgroup of 4 wavefronts (2 x 2) over a TT x TT part of the problem: a
+// quarter of a 64x64 tile (TT = 32) or one tile (64).  Two LDS stages (16 or
+// 32 KB), W waves per SIMD at least.
+// Bound: the f64 and f32 MFMA rate where the chip is full (28 problems of
+// 1024 x 2048 x 1024: f64 64 of the 73 TFLOP/s a library product reaches,
+// f32 117 of 153; 53 and 92 with scalar LDS accesses, flat loads and the
+// loads drained at every barrier), latency for the K of 64 to 512 and the few
+// tiles of a chain's step: there a workgroup lives for a handful of chunks
+// and descriptor, first loads and barriers are most of it (64 products of
+// 256 x 128 x 512 f64 64 -> 45 us; 16 of 128 x 64 x 256 21 -> 8.4 us; bf16 15
+// -> 11 us).  PD: three (32) f64 chunks in flight hide a cold load behind
+// MFMAs of 256 cycles; one is enough behind the 1024 of the 64x64 shape.
+// Tried and not kept: operands straight from global memory to the MFMA
+// registers (an operand contiguous in k then touches 16 lines per load: f64
+// 58 of 73 and 42 where both are), 128 x 128 workgroups (f64 32, f32 63).
+template <int MODE, int TT, int PD, int W>
+__global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_problem* __restrict__ probs,
+                                                           int nprob,
+                                                           const tnx_gemm_seg* __restrict__ segs,
+                                                           int ntiles,
+                                                           const int32_t* __restrict__ active,
+                                                           unsigned long long* ts) {
+  tnx_stamp_begin(ts);
+  constexpr int MB = TT / 32, NB = MB;
+  typedef Tr<MODE> T;
+  typedef typename T::TC TC;
+  typedef typename T::V4 V4;
+  __shared__ u4 As[2][TT * 8], Bs[2][TT * 8];
+  int bid = tnx_xcd_remap(blockIdx.x, gridDim.x), sub = 0;
+  if constexpr (TT == 32) {
+    sub = bid & 3;
+    bid >>= 2;
+  }
+  const int pi = __builtin_amdgcn_readfirstlane(find_problem(probs, nprob, bid, ntiles));
+  const tnx_gemm_problem TNX_CONST* cp = (const tnx_gemm_problem TNX_CONST*)(uint64_t)probs + pi;
+  const tnx_gemm_seg TNX_CONST* cs = (const tnx_gemm_seg TNX_CONST*)(uint64_t)segs;
+  const tnx_gemm_problem TNX_CONST& P = *cp;
+  if (P.active >= 0 && active != nullptr && active[P.active] == 0) return;
+  const int tiles_n = (P.N + 63) / 64;
+  const int t_local = bid - P.tile_begin;
+  const int tr = t_local / tiles_n, tc = t_local - tr * tiles_n;
+  const int row0 = tr * 64 + (TT == 32 ? 32 * (sub >> 1) : 0);
+  const int col0 = tc * 64 + (TT == 32 ? 32 * (sub & 1) : 0);
+  if (row0 >= P.M || col0 >= P.N) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = (wave >> 1) * 16 * MB, wc = (wave & 1) * 16 * NB;
+  V4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = V4{0, 0, 0, 0};
+
+  int s = P.seg_begin;
+  const int s_end = s + P.seg_count;
+  while (s < s_end) {
+    if (cs[s].K <= 0) {
+      ++s;
+      continue;
+    }
+    const bool ta = cs[s].transA != 0, tb = cs[s].transB != 0;
+    const int K = cs[s].K;
+    typedef Operand<typename T::TI, TT, MB> O;
+#define TNX_STREAM(KA, KBc)                                                                 \
+  s = wide<O, KA, KBc>(P.M, P.N, K)                                                         \
+          ? run_stream<MODE, TT, PD, KA, KBc, true>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
+                                                    wc, As, Bs)                             \
+          : run_stream<MODE, TT, PD, KA, KBc, false>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
+                                                     wc, As, Bs)
+    if (!ta && tb) TNX_STREAM(true, true);
+    else if (!ta) TNX_STREAM(true, false);
+    else if (tb) TNX_STREAM(false, true);
+    else TNX_STREAM(false, false);
+#undef TNX_STREAM
+  }
+
+  // C: lane % 16 is the column index of a block; the row index of
+  // accumulator element r is 4 (lane / 16) + r for the f32-output MFMAs
+  // and lane / 16 + 4 r for v_mfma_f64_16x16x4_f64 (measured on gfx950)
+  TC TNX_GLOBAL* Cp = as_global<TC>(P.c);
+  const TC TNX_GLOBAL* C0 = as_global<const TC>(P.c0);
+  const int gj = col0 + wc + NB * (lane & 15);
+  const bool wide = gj + NB <= P.N;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
+      const int gi = row0 + wr + MB * rr + i;
+      if (gi >= P.M) continue;
+      typedef TC VC __attribute__((ext_vector_type(NB), aligned(sizeof(TC))));
+      if (wide) {
+        double v[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) v[j] = (double)acc[i][j][r];
+        if (C0 != nullptr) {
+          TC c0[NB];
+          if constexpr (NB == 1) c0[0] = C0[(int64_t)gi * P.ldc0 + gj];
+          else {
+            const VC c = *(const VC TNX_GLOBAL*)(C0 + (int64_t)gi * P.ldc0 + gj);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) c0[j] = c[j];
+          }
+#pragma unroll
+          for (int j = 0; j < NB; ++j) v[j] += P.beta * to_d(c0[j]);
+        }
+        if constexpr (NB == 1) Cp[(int64_t)gi * P.ldc + gj] = from_d<TC>(v[0]);
+        else {
+          VC c;
+#pragma unroll
+          for (int j = 0; j < NB; ++j) c[j] = from_d<TC>(v[j]);
+          *(VC TNX_GLOBAL*)(Cp + (int64_t)gi * P.ldc + gj) = c;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          if (gj + j < P.N) {
+            double v = (double)acc[i][j][r];
+            if (C0 != nullptr) v += P.beta * to_d(C0[(int64_t)gi * P.ldc0 + gj + j]);
+            Cp[(int64_t)gi * P.ldc + gj + j] = from_d<TC>(v);
+          }
+      }
+    }
+  if (ts != nullptr) {
+    __syncthreads();
+    tnx_stamp_end(ts);
+  }
 }
 
 }  // namespace
 
+// Both shapes give the same bits; which is faster depends on whether the 64x64
+// tiles fill the 256 CUs: a tile's MFMAs take their time on the one CU that
+// holds it, so below one tile per CU the 32x32 shape spreads a tile over four,
+// above it the larger shape reads its operands half as often (f64, us, 32x32
+// against 64x64: 128 tiles of K = 512 18 / 27, 256 tiles 28 / 29, 512 tiles
+// 52 / 46, 2048 tiles of K = 128 67 / 51; f32 11 / 16, 17 / 17, 33 / 28, 48 /
+// 32).  The bf16 MFMAs are fast enough for the line to lie at half that (128
+// tiles of K = 512 7.4 / 7.8 and of K = 3584 21 / 26, 192 tiles 8.6 / 8.0,
+// 256 tiles 12.5 / 8.3).
+static int gemm_small_tiles(int mode) { return mode <= TNX_GEMM_F32 ? 256 : 128; }
+
+template <int MODE, int TT, int PD, int W>
+static void launch_gemm(const tnx_gemm_problem* prob, int nprob, const tnx_gemm_seg* seg, int ntiles,
+                        const int32_t* active, hipStream_t s, unsigned long long* ts) {
+  hipLaunchKernelGGL((gemm_grouped_kernel<MODE, TT, PD, W>), dim3(TT == 32 ? 4 * ntiles : ntiles),
+                     dim3(256), 0, s, prob, nprob, seg, ntiles, active, ts);
+}
+
 extern "C" int tnx_gemm_variants(int mode) {
   switch (mode) {
-    case TNX_GEMM_F64: return 2;
-    case TNX_GEMM_F32: return 1;
+    case TNX_GEMM_F64:
+    case TNX_GEMM_F32:
     case TNX_GEMM_BF16_F32:
     case TNX_GEMM_BF16_BF16: return 2;
     default:
@@ -411,26 +535,17 @@ int tnx_gemm_grouped_ts(int mode, const tnx_gemm_problem* prob, int nprob,
   }
   if (ntiles == 0) return TNX_OK;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(ntiles);
-#define TNX_GEMM_LAUNCH(CFG)                                                       \
-  hipLaunchKernelGGL(gemm_grouped_kernel<CFG>, grid, dim3(Cfg<CFG>::NT), 0, s, prob, nprob, \
-                     seg, active, ts)
+  // variant 0 takes the shape of the rule, variant 1 the other one; the 32x32
+  // grid has four workgroups a tile, which a launch's x extent must hold
+  const bool small = ((ntiles <= gemm_small_tiles(base)) != (var == 1)) && ntiles < (1 << 29);
+#define TNX_GEMM_LAUNCH(MODE, PDS, WS, PDL, WL)                                           \
+  if (small) launch_gemm<MODE, 32, PDS, WS>(prob, nprob, seg, ntiles, active, s, ts);     \
+  else launch_gemm<MODE, 64, PDL, WL>(prob, nprob, seg, ntiles, active, s, ts)
   switch (base) {
-    case TNX_GEMM_F64:
-      if (var == 0) TNX_GEMM_LAUNCH(0);
-      else TNX_GEMM_LAUNCH(4);
-      break;
-    case TNX_GEMM_F32:
-      TNX_GEMM_LAUNCH(1);
-      break;
-    case TNX_GEMM_BF16_F32:
-      if (var == 0) TNX_GEMM_LAUNCH(2);
-      else TNX_GEMM_LAUNCH(6);
-      break;
-    default:
-      if (var == 0) TNX_GEMM_LAUNCH(3);
-      else TNX_GEMM_LAUNCH(7);
-      break;
+    case TNX_GEMM_F64: TNX_GEMM_LAUNCH(TNX_GEMM_F64, 3, 4, 1, 3); break;
+    case TNX_GEMM_F32: TNX_GEMM_LAUNCH(TNX_GEMM_F32, 3, 4, 1, 3); break;
+    case TNX_GEMM_BF16_F32: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_F32, 4, 3, 1, 2); break;
+    default: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_BF16, 4, 3, 1, 2); break;
   }
 #undef TNX_GEMM_LAUNCH
   TNX_CHECK_LAUNCH();

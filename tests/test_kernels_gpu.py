@@ -143,6 +143,80 @@ def test_gemm_variants_agree(gpu, mode_name):
     assert rc == L.EINVAL
 
 
+@pytest.mark.parametrize('mode_name', ['f64', 'f32', 'bf16_f32', 'bf16_bf16'])
+@pytest.mark.parametrize('ta,tb', [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_tile_edges(gpu, mode_name, ta, tb):
+    """Every tile shape at the edges of tiles, K chunks and 16-byte pieces:
+    sizes one below, at and above them, odd leading dimensions, operands that
+    start one element past an aligned address, segments of different K in one
+    sum, an empty one, a scaled one.  Elementwise against f64 products: the
+    sum of K products and alpha a carries at most (K + 2) unit roundoffs of
+    the accumulator per |a| |b|, the result one of its own type (alpha = 0.5
+    is exact)."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    mode, tin, tout, acc = {'f64': (L.GEMM_F64, torch.float64, torch.float64, 2.0 ** -53),
+                            'f32': (L.GEMM_F32, torch.float32, torch.float32, 2.0 ** -24),
+                            'bf16_f32': (L.GEMM_BF16_F32, torch.bfloat16, torch.float32, 2.0 ** -24),
+                            'bf16_bf16': (L.GEMM_BF16_BF16, torch.bfloat16, torch.bfloat16,
+                                          2.0 ** -24)}[mode_name]
+    out_eps = {torch.float64: 2.0 ** -53, torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8}[tout]
+    rng = np.random.RandomState(21)
+    g = R.GemmList()
+    keep, outs, want, bound = [], [], [], []
+    shapes = [(31, 33, [15]), (32, 64, [16, 16]), (65, 63, [1, 0, 17]), (64, 129, [31, 64, 2]),
+              (1, 65, [128]), (97, 1, [63, 65]), (96, 96, [130])]
+    for M, N, Ks in shapes:
+        segs, ref, mag = [], np.zeros((M, N)), np.zeros((M, N))
+        for q, K in enumerate(Ks):
+            pad = q % 2      # odd leading dimension and start
+            A = rng.randn(*((max(K, 1), M + pad) if ta else (M, max(K, 1) + pad)))
+            B = rng.randn(*((N, max(K, 1) + pad) if tb else (max(K, 1), N + pad)))
+            alpha = 0.5 if q == 1 else 1.0
+            bufs = []
+            for X in (A, B):
+                t = torch.zeros(X.size + pad, dtype=tin, device='cuda')
+                t[pad:] = _dev(X).to(tin).reshape(-1)
+                bufs.append(t)
+            keep += bufs
+            qa, qb = [b[pad:].to(torch.float64).cpu().numpy().reshape(X.shape)
+                      for b, X in zip(bufs, (A, B))]
+            a = (qa[:K, :M].T if ta else qa[:M, :K])
+            b = (qb[:N, :K].T if tb else qb[:K, :N])
+            ref += alpha * (a @ b)
+            mag += (sum(Ks) + 2) * (np.abs(alpha * a) @ np.abs(b))
+            es = bufs[0].element_size()
+            segs.append((bufs[0].data_ptr() + pad * es, A.shape[1], ta,
+                         bufs[1].data_ptr() + pad * es, B.shape[1], tb, K, alpha))
+        C = torch.full((M, N + 1), 7.0, dtype=tout, device='cuda')
+        outs.append(C)
+        g.add(C.data_ptr(), M, N, N + 1, segs)
+        want.append(ref)
+        bound.append(acc * mag + out_eps * (np.abs(ref) + acc * mag) + 1e-300)
+    p, s = g.arrays()
+    # the list drops empty segments: one back in, in the middle of the sum
+    k = int(p[2]['seg_begin'])
+    hole = s[k:k + 1].copy()
+    hole['K'] = 0
+    s = np.concatenate([s[:k + 1], hole, s[k + 1:]])
+    p['seg_count'][2] += 1
+    p['seg_begin'][3:] += 1
+    dp, ds = _upload([p, s])
+    for v in range(lib.tnx_gemm_variants(mode)):
+        print('gemm edges', mode_name, ta, tb, 'variant', v, flush=True)
+        for C in outs:
+            C.fill_(7.0)
+        L.check(lib.tnx_gemm_grouped(mode | (v << 8), _vp(dp.data_ptr()), len(p),
+                                     _vp(ds.data_ptr()), R.gemm_tiles(p), None, _stream()), 'gemm')
+        torch.cuda.synchronize()
+        for C, ref, bd, sh in zip(outs, want, bound, shapes):
+            got = C.to(torch.float64).cpu().numpy()
+            assert np.all(got[:, -1] == 7.0), sh          # nothing past the columns
+            assert np.all(np.abs(got[:, :-1] - ref) <= bd), (sh, np.abs(got[:, :-1] - ref).max())
+
+
 def test_gemm_active_mask_skips_problems(gpu):
     import torch
     from tnalg_amd import _lib as L
