@@ -297,13 +297,15 @@ int tnx_svd_jacobi_f64(const tnx_svd_job* jobs, int njob, int max_sweeps, tnx_st
  * Outputs (row-major n x n): row k of u is the k-th left singular vector of
  * R, row k of v is s_k times the k-th right singular vector, so R = u^T v;
  * s holds the singular values in descending order.  The columns of R^T are
- * rotated in blocks of bw (a power of two, 4 <= bw <= 32, bw * n <= 4096);
- * one launch per round of the round-robin over block pairs, sweeps until
- * none rotates (flag: one device int32 shared by the call).  Returns
- * TNX_ENOCONV after max_sweeps sweeps that still rotated.
+ * taken in blocks of bw (a power of two, 4 <= bw <= 64; blocks of more than
+ * 16 are worked off 16 columns at a time, so 16 is the width to use); one
+ * launch per round of the round-robin over block pairs, sweeps until none
+ * rotates (flag: one device int32 shared by the call; a sweep's flag is read
+ * while the next sweep runs).  Returns TNX_ENOCONV after max_sweeps sweeps
+ * that still rotated.
  * A job with u == 0 computes the singular values only (work: n^2 + n + 1
- * doubles; bw * n <= 8192; r may equal work with ld_r == n), the
- * entanglement spectrum of a bond whose gauge move was a QR.              */
+ * doubles; r may equal work with ld_r == n), the entanglement spectrum of a
+ * bond whose gauge move was a QR.                                           */
 typedef struct tnx_svdj_job {
   uint64_t r;          /* R, row-major n x n, leading dimension ld_r (read)   */
   uint64_t work;       /* scratch: 2 n^2 + n + 1 doubles                      */

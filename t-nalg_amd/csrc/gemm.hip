@@ -34,14 +34,6 @@ template <> __device__ __forceinline__ double to_d<__bf16>(__bf16 v) { return (d
 template <typename T> __device__ __forceinline__ T from_d(double v) { return (T)v; }
 template <> __device__ __forceinline__ __bf16 from_d<__bf16>(double v) { return (__bf16)(float)v; }
 
-// Pointers of the global address space (the records carry plain integers: a
-// generic pointer made from one would be accessed with flat loads, which
-// wait on the LDS counter too).
-#define TNX_GLOBAL __attribute__((address_space(1)))
-template <typename T> __device__ __forceinline__ T TNX_GLOBAL* as_global(uint64_t p) {
-  return (T TNX_GLOBAL*)p;
-}
-
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 // A K chunk is 128 bytes deep (KB = 16, 32 or 64 elements) and is staged

@@ -10,30 +10,50 @@
 // A = Q R then keeps A_new = Q u^T (an isometry even when R is rank
 // deficient) and hands v to the neighbour.
 //
-// Columns are grouped into blocks of bw (a power of two, bw * n <= 4096, so
-// two blocks of B and of W fill at most 128 KiB of LDS).  One launch is one
-// round of the round-robin over block pairs: a workgroup loads its pair into
-// LDS, runs one round-robin sweep of plane rotations over the 2 bw columns
-// (bw disjoint column pairs at a time, 256 / bw lanes each) and writes the
-// columns back.  Rounds repeat until a sweep rotates nothing.  A column
-// whose norm is at most n eps ||R||_F is numerical zero (rounding residue of
-// a rank-deficient R) and takes part in no rotation: rotating pairs of such
-// columns never settles, and leaving them alone keeps R = u^T v exact and u
-// orthogonal.
+// Columns are grouped into blocks of bw; one launch is one round of the
+// round-robin over block pairs, rounds repeat until a sweep rotates nothing.
+// A workgroup takes its pair in panels of 16 + 16 columns (all of it for
+// bw <= 16): the 32 x 32 Gram matrix of the columns by f64 MFMA, one sweep of
+// plane rotations on that matrix (16 disjoint ones at a time, from both
+// sides) accumulated into an orthogonal Q, and B and W times Q by MFMA.  The
+// columns cross the memory once per round instead of LDS once per rotation,
+// and a panel whose Gram matrix needs no rotation is not written.  What ends
+// the sweeps is decided on Gram matrices formed anew from B.
+// A rotation puts the larger column first, which sorts the columns as they
+// converge, and is applied as x - s (y + t x), whose rounding errors are
+// those of the small numbers s and t: relative error of the singular values
+// 1.5e-15 (n = 128, 200) where c x - s y on the columns had 1.5e-14 to 4e-14.
+// ms (MI355X), rotations of columns in LDS -> this: one matrix of order 64 1.8
+// -> 0.8, 128 6.5 -> 1.8, 256 21.8 -> 5.6, 1024 195 -> 61; 16 of order 256
+// 23.1 -> 6.5, with singular values over 10 decades in rows of any size 75.6
+// -> 17.0; values only, 500 of order 128 15.8 -> 10.2.
+// Bound: latency.  A round (n = 128 about 25 us) is 31 steps of one barrier,
+// each a chain of some 40 dependent f64 operations for the angles; Gram matrix
+// and products are the rest.  Tried and not kept: two sweeps over a Gram
+// matrix (fewer rounds, more steps: 128 2.7 ms), two for panels whose column
+// norms differ by 1e4 (10 decades 5.4 -> 8.9 ms), angles in f32 (no gain), 256
+// lanes for both G and Q (10% slower; faster only for many values-only jobs).
+// A column whose norm is at most n eps ||R||_F is numerical zero (rounding
+// residue of a rank-deficient R) and takes part in no rotation: rotating
+// pairs of such columns never settles, and leaving them alone keeps
+// R = u^T v exact and u orthogonal.
 //
 // A job with u == 0 asks for the singular values only (the entanglement
 // spectrum of a bond whose gauge move was a QR): W is neither formed nor
-// rotated, the work area is n^2 + n + 1 doubles (B, column norms, scale),
-// and with one block of B per pair there is room for twice the block width
-// (bw n <= 8192).  R may then be the work area itself (r == work, ld_r == n):
-// forming B is a copy onto itself.
+// rotated, and the work area is n^2 + n + 1 doubles (B, column norms, scale).
+// R may then be the work area itself (r == work, ld_r == n): forming B is a
+// copy onto itself.
 #include "tnx_common.h"
 
 namespace {
 
 constexpr int NT = 256;
 constexpr int SJ_NMAX = 1024;
-constexpr size_t SJ_LDS = sizeof(double) * 4 * 4096;  // 2 (B, W) x 2 bw x n, bw n <= 4096
+constexpr int SB = 16;         // columns of a sub-block; a panel is two
+constexpr int PW = 2 * SB;
+constexpr int GLD = PW + 2;    // LDS row stride of G and Q (with 33 the pairs of a round, u + v
+                               // constant, would share a bank)
+constexpr int RT = 512;        // lanes of a round's workgroup
 
 // values-only job: no W (see the header)
 __device__ __forceinline__ bool values_only(const tnx_svdj_job& J) { return J.u == 0; }
@@ -42,14 +62,14 @@ __device__ __forceinline__ double* norms_of(const tnx_svdj_job& J) {
   return (double*)J.work + (values_only(J) ? 1 : 2) * (int64_t)J.n * J.n;
 }
 
+// pair p of round `round` (< players - 1) of the round-robin, a < b
 __device__ __forceinline__ void pair_of(int players, int round, int p, int& a, int& b) {
-  if (p == 0) {
-    a = players - 1;
-    b = round;
-  } else {
-    a = (round + p) % (players - 1);
-    b = (round + players - 1 - p) % (players - 1);
-  }
+  const int last = players - 1;
+  const int x = round + p, y = round + last - p;
+  const int u = p == 0 ? last : (x >= last ? x - last : x);
+  const int v = p == 0 ? round : (y >= last ? y - last : y);
+  a = min(u, v);
+  b = max(u, v);
 }
 
 // B (column j = row j of R) and W = I, both column-major n x n in the work area.
@@ -89,87 +109,242 @@ __global__ void k_svdj_clear(int32_t* flag) {
   if (threadIdx.x == 0) *flag = 0;
 }
 
-__global__ __launch_bounds__(NT) void k_svdj_round(const tnx_svdj_job* __restrict__ jobs, int njob,
+// The rotation of the pair (x, y) with Gram entries a, c and g: x' = x - s (y +
+// tau x), y' = y + s (x - tau y), tau = s / (1 + cos); swap: the results
+// change places (x'' = y', y'' = -x'), so that the larger column comes first.
+// The tangent needs no more than the hardware's reciprocal and root (any
+// angle is a rotation; an approximate one leaves 1e-7 of g), the cosine and
+// tau are refined to working accuracy, so the transformation is orthogonal.
+struct Rot { double s, tau; bool rot, swap; };
+__device__ __forceinline__ Rot rot_of(double a, double c, double g, double eps2, double zero2) {
+  Rot r;
+  r.rot = g != 0.0 && a > zero2 && c > zero2 && g * g > eps2 * (a * c);
+  r.swap = c > a && a > zero2;   // never with a zero column (the padding of a panel among them)
+  const double h = c - a, g2 = r.rot ? 2.0 * g : 1.0;
+  const double w = fma(h, h, g2 * g2);
+  const double den = fabs(h) + w * __builtin_amdgcn_rsq(w);
+  const double t = (h >= 0.0 ? g2 : -g2) * __builtin_amdgcn_rcp(den);   // |t| <= 1
+  const double x = fma(t, t, 1.0);
+  double y = __builtin_amdgcn_rsq(x);              // cos = 1 / sqrt(1 + t^2)
+  const double e = fma(-x * y, y, 1.0);            // third order: e^3 of the root's 2^-20 or less
+  y = fma(y * e, fma(0.375, e, 0.5), y);
+  const double d = 1.0 + y;
+  double q = __builtin_amdgcn_rcp(d);
+  const double f = fma(-d, q, 1.0);
+  q = fma(q, fma(f, f, f), q);
+  r.s = r.rot ? y * t : 0.0;
+  r.tau = r.s * q;
+  return r;
+}
+__device__ __forceinline__ void rotate(const Rot& r, double& x, double& y) {
+  const double xn = fma(-r.s, fma(r.tau, x, y), x), yn = fma(r.s, fma(-r.tau, y, x), y);
+  x = r.swap ? yn : xn;
+  y = r.swap ? -xn : yn;
+}
+
+// Column c (0..31) of a panel: sub-blocks starting at columns ca and cb, cnt
+// columns each; -1 past them or past n.
+__device__ __forceinline__ int panel_col(int c, int ca, int cb, int cnt, int n) {
+  const int l = c & (SB - 1), g = (c < SB ? ca : cb) + l;
+  return l < cnt && g < n ? g : -1;
+}
+
+// P <- Q^T P for the panel's columns of the column-major n x n matrix P: wave
+// `wave` of `waves` takes 32 rows at a time, reads them whole and writes them
+// back.
+__device__ __forceinline__ void apply_q(double TNX_GLOBAL* P, const double (*Q)[GLD], int n, int ca,
+                                        int cb, int cnt, int wave, int waves) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+#pragma unroll 1
+  for (int r0 = 32 * wave; r0 < n; r0 += 32 * waves) {
+    const int row = r0 + 2 * m;
+    const bool ok0 = row < n, ok1 = row + 1 < n;
+    double b[8][2];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int col = panel_col(4 * s + g, ca, cb, cnt, n);
+      const int off = max(col, 0) * n + row;
+      b[s][0] = (col >= 0 && ok0) ? P[off] : 0.0;
+      b[s][1] = (col >= 0 && ok1) ? P[off + 1] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      tnx_d4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const double qa = Q[4 * s + g][16 * i + m];
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(qa, b[s][0], acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(qa, b[s][1], acc[1], 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = panel_col(16 * i + g + 4 * r, ca, cb, cnt, n);
+        const int off = col * n + row;
+        if (col >= 0 && ok0) P[off] = acc[0][r];
+        if (col >= 0 && ok1) P[off + 1] = acc[1][r];
+      }
+      __builtin_amdgcn_sched_barrier(0);   // one half of the columns at a time: registers
+    }
+  }
+}
+
+// One round: block pair p of every job that has that many rounds.  Of the 512
+// lanes, the first half owns the 2 x 2 blocks of the Gram matrix, the second
+// half those of Q, so that the two updates of a step run side by side.
+__global__ __launch_bounds__(RT, 4) void k_svdj_round(const tnx_svdj_job* __restrict__ jobs, int njob,
                                                    int round, int32_t* flag) {
-  extern __shared__ double lds[];
+  // the partial Gram matrices of the waves, then G and Q, two copies of each
+  // (a step reads one and writes the other)
+  __shared__ union {
+    double part[RT / 64][3][256];
+    struct { double G[2][PW][GLD], Q[2][PW][GLD]; } m;
+  } L;
+  __shared__ int turned;
   const int ji = tnx_find_owner(jobs, sizeof(tnx_svdj_job), offsetof(tnx_svdj_job, pair_begin),
                                 njob, blockIdx.x);
   const tnx_svdj_job J = jobs[ji];
-  const int nb = J.nblk, n = J.n, bw = J.bw, w2 = 2 * J.bw;
+  const int nb = J.nblk, n = J.n, bw = J.bw;
   if (round >= nb - 1) return;  // this job has fewer blocks than the largest one
-  const int p = blockIdx.x - J.pair_begin;
   int ba, bb;
-  pair_of(nb, round, p, ba, bb);
-  double* B = (double*)J.work;
-  double* W = B + (int64_t)n * n;
+  pair_of(nb, round, blockIdx.x - J.pair_begin, ba, bb);
+  double TNX_GLOBAL* B = as_global<double>(J.work);
+  double TNX_GLOBAL* W = B + (int64_t)n * n;
   const bool vo = values_only(J);
-  double* Bs = lds;
-  double* Ws = lds + (int64_t)w2 * n;
-  // local column c: block ba for c < bw, block bb after; columns >= n are zero
-  for (int c = 0; c < w2; ++c) {
-    const int g = (c < bw ? ba * bw + c : bb * bw + (c - bw));
-    for (int i = threadIdx.x; i < n; i += NT) {
-      Bs[c * n + i] = (g < n) ? B[(int64_t)g * n + i] : 0.0;
-      if (!vo) Ws[c * n + i] = (g < n) ? W[(int64_t)g * n + i] : 0.0;
-    }
-  }
-  __shared__ int rotated;
-  if (threadIdx.x == 0) rotated = 0;
-  __syncthreads();
-  const int T = NT / bw;  // lanes per column pair: 8 .. 64, aligned groups of one wavefront
-  const int k = threadIdx.x / T, l = threadIdx.x % T;
-  const double eps = 2.220446049250313e-16 * (double)(n > 8 ? n : 8);
-  const double zero2 = eps * eps * norms_of(J)[n];  // column norm^2 of numerical zero
-  for (int ir = 0; ir < w2 - 1; ++ir) {
-    int u, v;
-    pair_of(w2, ir, k, u, v);
-    double* x = Bs + u * n;
-    double* y = Bs + v * n;
-    double a = 0.0, c = 0.0, g = 0.0;
-    // loops unrolled so that several LDS loads are in flight (same operations
-    // in the same order per element)
-#pragma unroll 4
-    for (int i = l; i < n; i += T) {
-      const double xi = x[i], yi = y[i];
-      a += xi * xi;
-      c += yi * yi;
-      g += xi * yi;
-    }
-    for (int o = T >> 1; o > 0; o >>= 1) {
-      a += __shfl_xor(a, o, 64);
-      c += __shfl_xor(c, o, 64);
-      g += __shfl_xor(g, o, 64);
-    }
-    if (g != 0.0 && fabs(g) > eps * sqrt(a * c) && a > zero2 && c > zero2) {
-      const double zeta = (c - a) / (2.0 * g);
-      const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-      const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
-      double* wx = Ws + u * n;
-      double* wy = Ws + v * n;
-#pragma unroll 4
-      for (int i = l; i < n; i += T) {
-        const double xi = x[i], yi = y[i];
-        x[i] = cs * xi - sn * yi;
-        y[i] = sn * xi + cs * yi;
-        if (!vo) {
-          const double pi = wx[i], qi = wy[i];
-          wx[i] = cs * pi - sn * qi;
-          wy[i] = sn * pi + cs * qi;
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool q_half = wave >= RT / 128;
+  const int t = threadIdx.x & (RT / 2 - 1);
+  const int pi = t >> 4, qi = t & 15;   // the lane's 2 x 2 block: rotations pi (rows), qi (columns)
+  // Gram entries are scaled by a power of two near 1 / ||R||_F^2, so that
+  // products of them neither over- nor underflow
+  const double fro2 = norms_of(J)[n];
+  const double scale = (fro2 > 1e-300 && fro2 < 1e300) ? ldexp(1.0, -ilogb(fro2)) : 1.0;
+  const double eps = 2.220446049250313e-16 * (double)(n > 8 ? n : 8), eps2 = eps * eps;
+  const double zero2 = eps2 * fro2 * scale;  // column norm^2 of numerical zero
+  const int cnt = bw < SB ? bw : SB, nsub = bw < SB ? 1 : bw / SB;
+  int any = 0;
+  // the pair's sub-blocks (one per block for bw <= 16), every two of them
+  for (int sr = 0; sr < 2 * nsub - 1; ++sr)
+    for (int sp = 0; sp < nsub; ++sp) {
+      int sa, sb;
+      pair_of(2 * nsub, sr, sp, sa, sb);
+      const int ca = (sa < nsub ? ba : bb) * bw + (sa % nsub) * SB;
+      const int cb = (sb < nsub ? ba : bb) * bw + (sb % nsub) * SB;
+      if (ca >= n) continue;
+      if (sr + sp > 0) __syncthreads();   // the last panel is written
+      // Gram matrix: blocks (0, 0), (0, 1), (1, 1), each wave every eighth
+      // 8 rows; lane group g holds rows 2 g, 2 g + 1 of them
+      {
+        const int c0 = panel_col(m, ca, cb, cnt, n), c1 = panel_col(16 + m, ca, cb, cnt, n);
+        const double TNX_GLOBAL* p0 = B + (int64_t)max(c0, 0) * n;
+        const double TNX_GLOBAL* p1 = B + (int64_t)max(c1, 0) * n;
+        tnx_d4 g00 = {0, 0, 0, 0}, g01 = {0, 0, 0, 0}, g11 = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int r0 = 8 * wave; r0 < n; r0 += 8 * (RT / 64)) {
+          const int r = r0 + 2 * g;
+          double x[2], y[2];
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const int rr = min(r + k, n - 1);
+            const double xv = p0[rr], yv = p1[rr];
+            x[k] = (c0 >= 0 && r + k < n) ? xv : 0.0;
+            y[k] = (c1 >= 0 && r + k < n) ? yv : 0.0;
+          }
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            g00 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], x[k], g00, 0, 0, 0);
+            g01 = __builtin_amdgcn_mfma_f64_16x16x4f64(x[k], y[k], g01, 0, 0, 0);
+            g11 = __builtin_amdgcn_mfma_f64_16x16x4f64(y[k], y[k], g11, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          L.part[wave][0][(g + 4 * r) * 16 + m] = g00[r];
+          L.part[wave][1][(g + 4 * r) * 16 + m] = g01[r];
+          L.part[wave][2][(g + 4 * r) * 16 + m] = g11[r];
         }
       }
-      if (l == 0) rotated = 1;
-    }
-    __syncthreads();
-  }
-  for (int c = 0; c < w2; ++c) {
-    const int g = (c < bw ? ba * bw + c : bb * bw + (c - bw));
-    if (g < n)
-      for (int i = threadIdx.x; i < n; i += NT) {
-        B[(int64_t)g * n + i] = Bs[c * n + i];
-        if (!vo) W[(int64_t)g * n + i] = Ws[c * n + i];
+      if (threadIdx.x == 0) turned = 0;
+      __syncthreads();
+      double v[3];
+      if (!q_half) {
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+          v[x] = 0.0;
+#pragma unroll
+          for (int w = 0; w < RT / 64; ++w) v[x] += L.part[w][x][t];
+          v[x] *= scale;
+        }
       }
-  }
-  if (threadIdx.x == 0 && rotated) atomicOr(flag, 1);
+      __syncthreads();
+      if (!q_half) {
+        L.m.G[0][pi][qi] = v[0];
+        L.m.G[0][pi][16 + qi] = v[1];
+        L.m.G[0][16 + qi][pi] = v[1];
+        L.m.G[0][16 + pi][16 + qi] = v[2];
+      } else {
+        L.m.Q[0][pi][qi] = pi == qi ? 1.0 : 0.0;
+        L.m.Q[0][pi][16 + qi] = 0.0;
+        L.m.Q[0][16 + pi][qi] = 0.0;
+        L.m.Q[0][16 + pi][16 + qi] = pi == qi ? 1.0 : 0.0;
+      }
+      __syncthreads();
+      // a pair that the Gram matrix has to rotate?
+      if (!q_half) {
+        bool need = false;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int i = pi + 16 * (x >> 1), j = qi + 16 * (x & 1);
+          if (i < j) {
+            const double a = L.m.G[0][i][i], c = L.m.G[0][j][j], gg = L.m.G[0][i][j];
+            need = need || (gg != 0.0 && a > zero2 && c > zero2 && gg * gg > eps2 * (a * c));
+          }
+        }
+        if (need) turned = 1;
+      }
+      __syncthreads();
+      if (turned == 0) continue;
+      any = 1;
+#pragma unroll 1
+      for (int ir = 0; ir < PW - 1; ++ir) {
+        const int cur = ir & 1;
+        const double (*G)[GLD] = L.m.G[cur];
+        int up, vp, uq, vq;
+        pair_of(PW, ir, qi, uq, vq);
+        const Rot rq = rot_of(G[uq][uq], G[vq][vq], G[uq][vq], eps2, zero2);
+        if (!q_half) {
+          pair_of(PW, ir, pi, up, vp);
+          const Rot rp = rot_of(G[up][up], G[vp][vp], G[up][vp], eps2, zero2);
+          double g11 = G[up][uq], g12 = G[up][vq], g21 = G[vp][uq], g22 = G[vp][vq];
+          rotate(rq, g11, g12);
+          rotate(rq, g21, g22);
+          rotate(rp, g11, g21);
+          rotate(rp, g12, g22);
+          double (*H)[GLD] = L.m.G[cur ^ 1];
+          H[up][uq] = g11;
+          H[up][vq] = g12;
+          H[vp][uq] = g21;
+          H[vp][vq] = g22;
+        } else {
+          const double (*Q)[GLD] = L.m.Q[cur];
+          double q11 = Q[2 * pi][uq], q12 = Q[2 * pi][vq];
+          double q21 = Q[2 * pi + 1][uq], q22 = Q[2 * pi + 1][vq];
+          rotate(rq, q11, q12);
+          rotate(rq, q21, q22);
+          double (*H)[GLD] = L.m.Q[cur ^ 1];
+          H[2 * pi][uq] = q11;
+          H[2 * pi][vq] = q12;
+          H[2 * pi + 1][uq] = q21;
+          H[2 * pi + 1][vq] = q22;
+        }
+        __syncthreads();
+      }
+      const double (*Q)[GLD] = L.m.Q[(PW - 1) & 1];
+      const bool w_half = q_half && !vo;
+      const int waves = vo ? RT / 64 : RT / 128;
+      apply_q(w_half ? W : B, Q, n, ca, cb, cnt, w_half ? wave - RT / 128 : wave, waves);
+    }
+  if (any && threadIdx.x == 0) atomicOr(flag, 1);
 }
 
 // su[j] = ||B_j|| (one wavefront per column)
@@ -220,7 +395,7 @@ __global__ __launch_bounds__(NT) void k_svdj_sort(const tnx_svdj_job* __restrict
   if (threadIdx.x == 0) ((double*)J.s)[rank] = sj;
 }
 
-thread_local int32_t* g_flag_pin = nullptr;
+thread_local int32_t* g_flag_pin = nullptr;   // two slots: sweeps alternate
 
 }  // namespace
 
@@ -235,26 +410,43 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
     return TNX_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
-  static bool attr_set = false;
-  if (!attr_set) {
-    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)k_svdj_round,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)SJ_LDS));
-    attr_set = true;
-  }
   if (g_flag_pin == nullptr)
     TNX_CHECK_HIP(hipHostMalloc((void**)&g_flag_pin, 64, hipHostMallocDefault));
   hipLaunchKernelGGL(k_svdj_init, dim3(max_n < 1024 ? max_n : 1024, njob), dim3(NT), 0, s, jobs);
   hipLaunchKernelGGL(k_svdj_scale, dim3(njob), dim3(NT), 0, s, jobs);
   TNX_CHECK_LAUNCH();
+  // The flag of a sweep is read while the next one runs: a sweep after the
+  // last is a Gram matrix per panel and nothing else (n = 128: 30 us for one
+  // job), less than the stop after every sweep that it saves.
+  hipEvent_t ev[2];
+  TNX_CHECK_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
+  if (hipEventCreateWithFlags(&ev[1], hipEventDisableTiming) != hipSuccess) {
+    (void)hipEventDestroy(ev[0]);
+    tnx_set_error("tnx_svd_block_jacobi: no event");
+    return TNX_EHIP;
+  }
   bool converged = false;
-  for (int sweep = 0; sweep < max_sweeps && !converged; ++sweep) {
+  hipError_t err = hipSuccess;
+  for (int sweep = 0; sweep < max_sweeps && !converged && err == hipSuccess; ++sweep) {
     hipLaunchKernelGGL(k_svdj_clear, dim3(1), dim3(64), 0, s, flag);
     for (int r = 0; r < max_nblk - 1; ++r)
-      hipLaunchKernelGGL(k_svdj_round, dim3(npairs), dim3(NT), SJ_LDS, s, jobs, njob, r, flag);
-    TNX_CHECK_LAUNCH();
-    TNX_CHECK_HIP(hipMemcpyAsync(g_flag_pin, flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-    TNX_CHECK_HIP(hipStreamSynchronize(s));
-    converged = (*(volatile int32_t*)g_flag_pin == 0);
+      hipLaunchKernelGGL(k_svdj_round, dim3(npairs), dim3(RT), 0, s, jobs, njob, r, flag);
+    err = hipGetLastError();
+    if (err == hipSuccess)
+      err = hipMemcpyAsync(g_flag_pin + (sweep & 1), flag, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+    if (err == hipSuccess) err = hipEventRecord(ev[sweep & 1], s);
+    // the previous sweep's flag, or after the last allowed sweep its own too
+    for (int k = sweep > 0 ? sweep - 1 : 0; err == hipSuccess && !converged && k <= sweep; ++k) {
+      if (k == sweep && sweep + 1 < max_sweeps) break;
+      err = hipEventSynchronize(ev[k & 1]);
+      converged = err == hipSuccess && ((volatile int32_t*)g_flag_pin)[k & 1] == 0;
+    }
+  }
+  (void)hipEventDestroy(ev[0]);
+  (void)hipEventDestroy(ev[1]);
+  if (err != hipSuccess) {
+    tnx_set_error("tnx_svd_block_jacobi: %s", hipGetErrorString(err));
+    return TNX_EHIP;
   }
   hipLaunchKernelGGL(k_svdj_norms, dim3((max_n + 3) / 4, njob), dim3(NT), 0, s, jobs);
   hipLaunchKernelGGL(k_svdj_sort, dim3(max_n, njob), dim3(NT), 0, s, jobs);

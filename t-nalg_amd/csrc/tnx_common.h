@@ -73,6 +73,14 @@ typedef double tnx_d4 __attribute__((ext_vector_type(4)));
 typedef float tnx_f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 tnx_bf8 __attribute__((ext_vector_type(8)));
 
+// Pointers of the global address space (the records carry plain integers: a
+// generic pointer made from one would be accessed with flat loads, which
+// wait on the LDS counter too).
+#define TNX_GLOBAL __attribute__((address_space(1)))
+template <typename T> __device__ __forceinline__ T TNX_GLOBAL* as_global(uint64_t p) {
+  return (T TNX_GLOBAL*)p;
+}
+
 // Load element idx of a buffer of runtime dtype as double.
 __device__ __forceinline__ double tnx_load(const void* p, int dtype, int64_t idx) {
   if (dtype == TNX_F64) return ((const double*)p)[idx];

@@ -70,19 +70,11 @@ SVDJ_NMAX = 1024
 OK, EINVAL, ENOCONV = 0, -1, -3   # tnx_status values
 
 
-def svdj_blocking(n, values_only=False):
-    """(bw, nblk) of tnx_svd_block_jacobi for order n: bw the largest power of
-    two <= min(32, 4096 / n) (at least 4), nblk = ceil(n / bw) rounded up to
-    even.  Values-only jobs (no W in LDS): bw <= min(64, 8192 / n) and at most
-    n / 2, so an order up to 128 is one block pair."""
-    if values_only:
-        bw = 64
-        while bw > 4 and (bw * n > 8192 or 2 * bw > max(n, 8)):
-            bw //= 2
-    else:
-        bw = 32
-        while bw > 4 and bw * n > 4096:
-            bw //= 2
+def svdj_blocking(n):
+    """(bw, nblk) of tnx_svd_block_jacobi for order n: blocks of the 16
+    columns a panel's Gram matrix takes from each side, nblk = ceil(n / 16)
+    rounded up to even."""
+    bw = 16
     nblk = -(-n // bw)
     return bw, nblk + (nblk % 2)
 CHOL_NMAX = 128

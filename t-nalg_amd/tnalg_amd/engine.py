@@ -1362,7 +1362,7 @@ class Solve:
         jobs = []
         for b in range(b0, b1 + 1):
             n = self.dims[b + 1]
-            bw, nblk = L.svdj_blocking(n, values_only=True)
+            bw, nblk = L.svdj_blocking(n)
             slot = self._rsv_slot(b)
             jobs.append((slot, slot, 0, 0, _p(self.lmv, b * self.dmax_max), n, n, bw, nblk, 0, 0))
         ph['svdj'] = np.array(jobs, dtype=L.SVDJ_JOB)

@@ -540,6 +540,60 @@ def test_svd_block_jacobi(gpu):
         assert np.allclose(np.linalg.norm(Vs, axis=1), sv, rtol=1e-12, atol=1e-14), n
 
 
+@pytest.mark.parametrize('bw', [4, 16, 32, 64])
+@pytest.mark.parametrize('vectors', [True, False])
+def test_svd_block_jacobi_panels(gpu, bw, vectors):
+    """Orders at the edges of the 16-column panels, every block width the
+    call takes, column norms over many decades in any order, exact zero
+    columns, entries of 1e-120, and values-only jobs in place: the same
+    bounds as test_svd_block_jacobi (1e-12 n for the products of rotations,
+    1e-13 n for the values)."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(17)
+    Rs = [rng.randn(n, n) for n in (8, 15, 16, 17, 31, 33, 65)]
+    Rs.append(rng.randn(40, 40) * 10.0 ** rng.uniform(-8, 0, 40)[:, None])
+    z = rng.randn(34, 34)
+    z[[0, 5, 16, 33]] = 0.0
+    Rs.append(z)
+    Rs.append(rng.randn(20, 20) * 1e-120)
+    bufs, recs = [], []
+    for R in Rs:
+        n = R.shape[0]
+        nblk = -(-n // bw)
+        nblk = max(2, nblk + nblk % 2)
+        work = torch.zeros(2 * n * n + n + 1, dtype=torch.float64, device='cuda')
+        r = _dev(R) if vectors else work
+        if not vectors:
+            work[:n * n] = _dev(R).reshape(-1)
+        u = torch.zeros(n * n, dtype=torch.float64, device='cuda')
+        v = torch.zeros(n * n, dtype=torch.float64, device='cuda')
+        s = torch.zeros(n, dtype=torch.float64, device='cuda')
+        bufs.append((r, work, u, v, s))
+        recs.append((r.data_ptr(), work.data_ptr(), u.data_ptr() if vectors else 0,
+                     v.data_ptr() if vectors else 0, s.data_ptr(), n, n, bw, nblk, 0, 0))
+    jobs = np.array(recs, dtype=L.SVDJ_JOB)
+    jobs['pair_begin'] = np.concatenate([[0], np.cumsum(jobs['nblk'] // 2)[:-1]])
+    (dj,) = _upload([jobs])
+    flag = torch.zeros(4, dtype=torch.int32, device='cuda')
+    print('svd_block_jacobi panels bw', bw, 'vectors', vectors, flush=True)
+    L.check(lib.tnx_svd_block_jacobi(_vp(dj.data_ptr()), len(jobs), int((jobs['nblk'] // 2).sum()),
+                                     int(jobs['nblk'].max()), int(jobs['n'].max()),
+                                     _vp(flag.data_ptr()), 60, _stream()), 'svd_block_jacobi')
+    torch.cuda.synchronize()
+    for R, (_, _, u, v, s) in zip(Rs, bufs):
+        n = R.shape[0]
+        sv = s.cpu().numpy()
+        ref = np.linalg.svd(R, compute_uv=False)
+        assert np.all(np.diff(sv) <= 0), n
+        assert np.abs(sv - ref).max() < 1e-13 * ref[0] * n, n
+        if vectors:
+            U, Vs = (x.cpu().numpy().reshape(n, n) for x in (u, v))
+            assert np.abs(U.T @ Vs - R).max() < 1e-12 * np.abs(R).max() * n, n
+            assert np.abs(U @ U.T - np.eye(n)).max() < 1e-12 * n, n
+
+
 def test_trace_dot(gpu):
     import torch
     from tnalg_amd import _lib as L
