@@ -105,9 +105,43 @@ __device__ __forceinline__ int tnx_xcd_remap(int bid, int nblocks) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// One step of the butterfly below: v plus the value `DPP` (a row rotation of
+// the data-parallel primitives) brings from another lane of the 16-lane row.
+template <int DPP> __device__ __forceinline__ double tnx_row_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)x, DPP, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), DPP, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// x[lane] + x[lane ^ 32] (HALF) or x[lane] + x[lane ^ 16], by the swap of the
+// odd rows of one register with the even rows of another.
+template <bool HALF> __device__ __forceinline__ double tnx_swap_add(double v) {
+  const long long x = __double_as_longlong(v);
+  const unsigned l = (unsigned)x, h = (unsigned)(x >> 32);
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  u2 lo, hi;
+  if constexpr (HALF) {
+    lo = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+    hi = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+  } else {
+    lo = __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    hi = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+  }
+  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+         __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+// Sum over the wavefront, the same bits in every lane: the butterfly over lane
+// ^ 32, 16, 8, 4, 2, 1.  Within a 16-lane row a rotation by d = 8, 4, 2, 1
+// brings lane ^ d's value, as the values repeat with period 2 d by then.  All
+// steps are VALU operations: through the LDS crossbar (__shfl_xor) each of the
+// six took about 120 cycles on the path of every reduction.
 __device__ __forceinline__ double tnx_wave_sum(double v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = tnx_swap_add<true>(v);
+  v = tnx_swap_add<false>(v);
+  v = tnx_row_add<0x128>(v);
+  v = tnx_row_add<0x124>(v);
+  v = tnx_row_add<0x122>(v);
+  return tnx_row_add<0x121>(v);
 }
 
 // Largest index i in [0, n) whose 32-bit field at byte offset `off` of the
