@@ -1,68 +1,310 @@
-// f64 orthogonalisations of MPS tensors: Householder QR (gauge moves) and
-// one-sided Jacobi (Hestenes) SVD (entanglement spectrum moves).
-//
-// One workgroup (256 lanes) per matrix; the working copy lives column-major
-// in the job's work buffer so every reflector / rotation touches contiguous
-// columns.  Columns are distributed over the 4 wavefronts, rows over the 64
-// lanes of a wavefront, and column dot products are wavefront reductions.
+// f64 orthogonalisations of MPS tensors: Householder QR (gauge moves), the
+// Cholesky factor of CholeskyQR3 and one-sided Jacobi (Hestenes) SVD
+// (entanglement spectrum moves).  One workgroup per matrix.
 #include "tnx_common.h"
 
 namespace {
 
 constexpr int NT = 256;
+constexpr int NQ = 1024;    // lanes of the QR kernel
 constexpr int KMAX = 4096;  // max columns of a gauge-move matrix
 
-__device__ __forceinline__ double src_at(const double* src, int ld, int trans, int r, int c) {
+__device__ __forceinline__ double src_at(const double TNX_GLOBAL* src, int ld, int trans, int r, int c) {
   return trans ? src[(int64_t)c * ld + r] : src[(int64_t)r * ld + c];
 }
 
-// column-major m x n work matrix W (ld = m); Q scratch m x k after it.
-__global__ __launch_bounds__(NT) void qr_kernel(const tnx_qr_job* __restrict__ jobs) {
-  const tnx_qr_job J = jobs[blockIdx.x];
-  const int m = J.m, n = J.n, k = m < n ? m : n;
-  if (k > KMAX || m <= 0 || n <= 0) return;  // rejected on the host
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double* W = (double*)J.work;
-  double* Q = W + (int64_t)m * n;
-  const double* src = (const double*)J.src;
-  __shared__ double tau[KMAX];
-  __shared__ double bcast[2];
+// ------------------------------------------------------ Householder QR
+// Three ways, by the number of rows:
+// - m <= 16 (chain ends): a lane holds a column in registers; the reflectors
+//   of the first columns are formed one after the other, every lane applies
+//   them to its own column.
+// - m <= 512 with at least 16 reflectors (the wide panels of a random MPS
+//   that is brought into canonical form: 32 x chi .. chi/2 x chi): blocks of
+//   16 columns, factored in LDS with one barrier per column, then applied to
+//   the columns right of them as I - V T V^T on f64 MFMA; Q the same way in
+//   reverse.
+// - otherwise (tall panels of less than 8 columns, where CholeskyQR3 is not
+//   used) column by column in global memory.
+// Bound: a serial chain of reflectors (about 700 cycles each) in the panels,
+// the f64 MFMA rate of the one CU in the products.  us (MI355X), one wave per
+// column in global memory -> this: 16 matrices of 4 x 128 74 -> 8, of 16 x 128
+// 327 -> 24, of 64 x 128 1387 -> 167; one of 32 x 512 2440 -> 106, of 256 x
+// 512 37200 -> 2040.
+constexpr int QS = 16;       // rows of the small path, columns of a block
+constexpr int QB_MAX = 512;  // rows of the blocked path
 
-  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NT) {
-    int r, c;
-    if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }   // src[c*ld+r] contiguous in r
-    else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }           // src[r*ld+c] contiguous in c
-    W[(int64_t)c * m + r] = src_at(src, J.ld, J.trans, r, c);
+struct QrLds {
+  double tau[KMAX];
+  double P[QS * (QB_MAX + 1)];   // the block's columns, then its V, stride m + 1
+  double S[QS][QS + 1], T[QS][QS + 1];
+  double beta[QS], scal[QS];
+};
+
+// Reflector of (x0, x) with s = |x|^2: beta, tau and the scale of x
+__device__ __forceinline__ void reflector(double x0, double s, double& beta, double& tau, double& scal) {
+  if (s == 0.0) {
+    beta = x0;
+    tau = 0.0;
+    scal = 0.0;
+  } else {
+    const double nrm = sqrt(x0 * x0 + s);
+    beta = x0 >= 0.0 ? -nrm : nrm;
+    tau = (beta - x0) / beta;
+    scal = 1.0 / (x0 - beta);
   }
-  __syncthreads();
+}
 
+template <int MR>   // m <= MR
+__device__ __forceinline__ void qr_small(const tnx_qr_job& J, QrLds& L) {
+  const int m = J.m, n = J.n, k = m < n ? m : n, t = threadIdx.x;
+  const int w0 = t & ~63;   // first column of the wave: waves without columns only keep the barriers
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
+  double TNX_GLOBAL* R = as_global<double>(J.r);
+  double TNX_GLOBAL* q = as_global<double>(J.q);
+  double (*V)[QS + 1] = L.S;   // V[j]: zeros, V[j][j] = 1, the reflector, zeros past m
+  double x[MR];
+  auto load = [&](int c) {
+#pragma unroll
+    for (int r = 0; r < MR; ++r) x[r] = (r < m && c < n) ? src_at(src, J.ld, J.trans, r, c) : 0.0;
+  };
+  auto apply = [&](int j) {   // (I - tau v v^T) x
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int r = 0; r < MR; ++r) s[r & 1] += V[j][r] * x[r];
+    const double f = (s[0] + s[1]) * L.tau[j];
+#pragma unroll
+    for (int r = 0; r < MR; ++r) x[r] -= f * V[j][r];
+  };
+  auto store_r = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < MR; ++i)
+      if (i < k && c < n) R[(int64_t)i * n + c] = i <= c ? x[i] : 0.0;
+  };
+  if (w0 < n) load(t);
+#pragma unroll 1
   for (int j = 0; j < k; ++j) {
-    double* wj = W + (int64_t)j * m;
+    if (t == j) {
+      double s = 0.0, x0 = 0.0, beta, tau, scal;
+#pragma unroll
+      for (int r = 0; r < MR; ++r) {
+        s += r > j ? x[r] * x[r] : 0.0;
+        x0 = r == j ? x[r] : x0;
+      }
+      reflector(x0, s, beta, tau, scal);
+      L.tau[j] = tau;
+#pragma unroll
+      for (int r = 0; r < MR; ++r) {
+        V[j][r] = r > j ? x[r] * scal : (r == j ? 1.0 : 0.0);
+        x[r] = r == j ? beta : x[r];
+      }
+    }
+    __syncthreads();
+    if (t > j && w0 < n) apply(j);
+  }
+  if (w0 < n) store_r(t);
+#pragma unroll 1
+  for (int c = t + NQ; c < n; c += NQ) {
+    load(c);
+#pragma unroll 1
+    for (int j = 0; j < k; ++j) apply(j);
+    store_r(c);
+  }
+  __syncthreads();   // src is read before q, which may be the same memory, is written
+  if (t < k) {
+#pragma unroll
+    for (int r = 0; r < MR; ++r) x[r] = r == t ? 1.0 : 0.0;
+#pragma unroll 1
+    for (int j = k - 1; j >= 0; --j) apply(j);
+#pragma unroll
+    for (int r = 0; r < MR; ++r)
+      if (r < m) q[J.q_trans ? (int64_t)t * m + r : (int64_t)r * k + t] = x[r];
+  }
+}
+
+// C[:, c0 .. c1) <- (I - V op(T) V^T) C over rows j0 .. m - 1 (C column-major,
+// leading dimension m; op(T) = T^T if trans); each wave takes 16 columns.
+__device__ __forceinline__ void qr_apply(double TNX_GLOBAL* C, int c0, int c1, int j0, int m, QrLds& L,
+                                         bool trans) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4, ldp = m + 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int ct = c0 + 16 * wave; ct < c1; ct += 16 * (NQ / 64)) {
+    const bool ok = ct + i < c1;
+    double TNX_GLOBAL* col = C + (int64_t)(ok ? ct + i : ct) * m;
+    tnx_d4 w1 = {0, 0, 0, 0}, w2 = {0, 0, 0, 0};
+    for (int r0 = j0; r0 < m; r0 += 8) {   // V^T C, lane group g: rows 2 g, 2 g + 1
+      const int r = r0 + 2 * g;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int rr = min(r + h, m - 1);
+        const double a = L.P[i * ldp + rr], b = col[rr];
+        const bool in = r + h < m;
+        w1 = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? a : 0.0, in && ok ? b : 0.0, w1, 0, 0, 0);
+      }
+    }
+    // w1's register s holds rows 4 s + g: the k of MFMA s as it is
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      w2 = __builtin_amdgcn_mfma_f64_16x16x4f64(trans ? L.T[4 * s + g][i] : L.T[i][4 * s + g], -w1[s],
+                                                w2, 0, 0, 0);
+    for (int r0 = j0; r0 < m; r0 += 16) {
+      tnx_d4 d;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) d[r] = col[min(r0 + g + 4 * r, m - 1)];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const double a = L.P[(4 * s + g) * ldp + min(r0 + i, m - 1)];
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a, w2[s], d, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (ok && r0 + g + 4 * r < m) col[r0 + g + 4 * r] = d[r];
+    }
+  }
+}
+
+// T of the block reflector H_0 ... H_15 = I - V T V^T from V (L.P) and tau
+// (columns past the block have V = 0 and tau = 0)
+__device__ __forceinline__ void qr_form_t(int j0, int jb, int m, QrLds& L) {
+  const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4, ldp = m + 1;
+  if (threadIdx.x < 64) {
+    tnx_d4 s4 = {0, 0, 0, 0};
+    for (int r0 = j0; r0 < m; r0 += 4) {
+      const double v = L.P[i * ldp + min(r0 + g, m - 1)];
+      const double x = r0 + g < m ? v : 0.0;
+      s4 = __builtin_amdgcn_mfma_f64_16x16x4f64(x, x, s4, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) L.S[g + 4 * r][i] = s4[r];
+    __builtin_amdgcn_wave_barrier();
+    // column c of T: T[a][c] = -tau_c sum_b T[a][b] S[b][c] (b < c); lane a
+    // holds row a in LDS (only it reads that row)
+    if (g == 0) {
+#pragma unroll 1
+      for (int c = 0; c < QS; ++c) {
+        const double tc = c < jb ? L.tau[j0 + c] : 0.0;
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int b = 0; b < QS; ++b) s[b & 3] += b < c ? L.T[i][b] * L.S[b][c] : 0.0;
+        L.T[i][c] = i == c ? tc : (i < c ? -tc * ((s[0] + s[1]) + (s[2] + s[3])) : 0.0);
+      }
+    }
+  }
+}
+
+// column-major m x n work matrix W (ld = m); Q scratch m x k after it.
+__device__ __forceinline__ void qr_blocked(const tnx_qr_job& J, QrLds& L) {
+  const int m = J.m, n = J.n, k = m < n ? m : n, t = threadIdx.x, ldp = m + 1;
+  const int lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  double TNX_GLOBAL* W = as_global<double>(J.work);
+  double TNX_GLOBAL* Q = W + (int64_t)m * n;
+  for (int j0 = 0; j0 < k; j0 += QS) {
+    const int jb = min(QS, k - j0), rows = m - j0;
+    for (int e = t; e < QS * rows; e += NQ) {
+      const int c = e / rows, r = j0 + e - c * rows;
+      L.P[c * ldp + r] = c < jb ? W[(int64_t)(j0 + c) * m + r] : 0.0;
+    }
+    __syncthreads();
+    // column jj: every wave forms the reflector from the unscaled column and
+    // applies it to one column right of it
+    for (int jj = 0; jj < jb; ++jj) {
+      const int j = j0 + jj, c = jj + 1 + wave;
+      const double* x = L.P + jj * ldp;
+      if (c < jb || wave == 0) {
+        double* y = L.P + (c < jb ? c : jj) * ldp;
+        double s = 0.0, d = 0.0;
+        for (int r = j + 1 + lane; r < m; r += 64) {
+          const double xr = x[r];
+          s += xr * xr;
+          d += xr * y[r];
+        }
+        s = tnx_wave_sum(s);
+        d = tnx_wave_sum(d);
+        double beta, tau, scal;
+        reflector(x[j], s, beta, tau, scal);
+        if (t == 0) {
+          L.beta[jj] = beta;
+          L.scal[jj] = scal;
+          L.tau[j] = tau;
+        }
+        if (c < jb && tau != 0.0) {
+          const double f = (y[j] + scal * d) * tau, fs = f * scal;
+          for (int r = j + 1 + lane; r < m; r += 64) y[r] -= fs * x[r];
+          if (lane == 0) y[j] -= f;
+        }
+      }
+      __syncthreads();
+    }
+    // R and V to W, V (unit lower trapezoidal) in P
+    for (int e = t; e < QS * rows; e += NQ) {
+      const int c = e / rows, r = j0 + e - c * rows;
+      if (c >= jb) continue;
+      double v = L.P[c * ldp + r];
+      if (r == j0 + c) {
+        W[(int64_t)(j0 + c) * m + r] = L.beta[c];
+        v = 1.0;
+      } else {
+        if (r > j0 + c) v *= L.scal[c];
+        W[(int64_t)(j0 + c) * m + r] = v;
+        if (r < j0 + c) v = 0.0;
+      }
+      L.P[c * ldp + r] = v;
+    }
+    __syncthreads();
+    qr_form_t(j0, jb, m, L);
+    __syncthreads();
+    qr_apply(W, j0 + jb, n, j0, m, L, true);
+    __syncthreads();
+  }
+  double TNX_GLOBAL* R = as_global<double>(J.r);
+  for (int64_t e = t; e < (int64_t)k * n; e += NQ) {
+    const int i = (int)(e / n), c = (int)(e - (int64_t)i * n);
+    R[e] = (i <= c) ? W[(int64_t)c * m + i] : 0.0;
+  }
+  // Q = H_0 ... H_{k-1} [I_k; 0], the blocks in reverse
+  for (int64_t e = t; e < (int64_t)m * k; e += NQ) {
+    const int c = (int)(e / m), r = (int)(e - (int64_t)c * m);
+    Q[e] = (r == c) ? 1.0 : 0.0;
+  }
+  for (int j0 = (k - 1) / QS * QS; j0 >= 0; j0 -= QS) {
+    const int jb = min(QS, k - j0), rows = m - j0;
+    for (int e = t; e < QS * rows; e += NQ) {
+      const int c = e / rows, r = j0 + e - c * rows;
+      L.P[c * ldp + r] = c >= jb || r < j0 + c ? 0.0 : r == j0 + c ? 1.0 : W[(int64_t)(j0 + c) * m + r];
+    }
+    __syncthreads();
+    qr_form_t(j0, jb, m, L);
+    __syncthreads();
+    qr_apply(Q, j0, k, j0, m, L, false);
+    __syncthreads();
+  }
+}
+
+// column by column: each reflector by one wave, its columns by all of them
+__device__ __forceinline__ void qr_columns(const tnx_qr_job& J, QrLds& L) {
+  const int m = J.m, n = J.n, k = m < n ? m : n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double TNX_GLOBAL* W = as_global<double>(J.work);
+  double TNX_GLOBAL* Q = W + (int64_t)m * n;
+  for (int j = 0; j < k; ++j) {
+    double TNX_GLOBAL* wj = W + (int64_t)j * m;
     if (wave == 0) {
       double s = 0.0;
       for (int r = j + 1 + lane; r < m; r += 64) s += wj[r] * wj[r];
       s = tnx_wave_sum(s);
-      const double x0 = wj[j];
       double beta, t, scal;
-      if (s == 0.0) {
-        beta = x0; t = 0.0; scal = 0.0;
-      } else {
-        double nrm = sqrt(x0 * x0 + s);
-        beta = x0 >= 0.0 ? -nrm : nrm;
-        t = (beta - x0) / beta;
-        scal = 1.0 / (x0 - beta);
-      }
+      reflector(wj[j], s, beta, t, scal);
       for (int r = j + 1 + lane; r < m; r += 64) wj[r] *= scal;
       if (lane == 0) {
         wj[j] = beta;
-        tau[j] = t;
+        L.tau[j] = t;
       }
     }
     __syncthreads();
-    const double tj = tau[j];
+    const double tj = L.tau[j];
     if (tj != 0.0) {
-      for (int c = j + 1 + wave; c < n; c += 4) {
-        double* wc = W + (int64_t)c * m;
+      for (int c = j + 1 + wave; c < n; c += NQ / 64) {
+        double TNX_GLOBAL* wc = W + (int64_t)c * m;
         double s = (lane == 0) ? wc[j] : 0.0;
         for (int r = j + 1 + lane; r < m; r += 64) s += wj[r] * wc[r];
         s = tnx_wave_sum(s) * tj;
@@ -72,25 +314,24 @@ __global__ __launch_bounds__(NT) void qr_kernel(const tnx_qr_job* __restrict__ j
     }
     __syncthreads();
   }
-
   // R (k x n, row-major): upper triangle of W
-  double* R = (double*)J.r;
-  for (int64_t e = threadIdx.x; e < (int64_t)k * n; e += NT) {
+  double TNX_GLOBAL* R = as_global<double>(J.r);
+  for (int64_t e = threadIdx.x; e < (int64_t)k * n; e += NQ) {
     int i = (int)(e / n), c = (int)(e - (int64_t)i * n);
     R[e] = (i <= c) ? W[(int64_t)c * m + i] : 0.0;
   }
   // Q = H_0 ... H_{k-1} [I_k; 0], column-major m x k, backward accumulation
-  for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NT) {
+  for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NQ) {
     int c = (int)(e / m), r = (int)(e - (int64_t)c * m);
     Q[e] = (r == c) ? 1.0 : 0.0;
   }
   __syncthreads();
   for (int j = k - 1; j >= 0; --j) {
-    const double tj = tau[j];
+    const double tj = L.tau[j];
     if (tj != 0.0) {
-      const double* v = W + (int64_t)j * m;  // v[j] = 1 implicit, v[r>j] stored
-      for (int c = j + wave; c < k; c += 4) {
-        double* qc = Q + (int64_t)c * m;
+      const double TNX_GLOBAL* v = W + (int64_t)j * m;  // v[j] = 1 implicit, v[r>j] stored
+      for (int c = j + wave; c < k; c += NQ / 64) {
+        double TNX_GLOBAL* qc = Q + (int64_t)c * m;
         double s = (lane == 0) ? qc[j] : 0.0;
         for (int r = j + 1 + lane; r < m; r += 64) s += v[r] * qc[r];
         s = tnx_wave_sum(s) * tj;
@@ -100,16 +341,41 @@ __global__ __launch_bounds__(NT) void qr_kernel(const tnx_qr_job* __restrict__ j
     }
     __syncthreads();
   }
-  double* q = (double*)J.q;
+}
+
+__global__ __launch_bounds__(NQ) void qr_kernel(const tnx_qr_job* __restrict__ jobs) {
+  extern __shared__ double lds[];
+  QrLds& L = *(QrLds*)lds;
+  const tnx_qr_job J = jobs[blockIdx.x];
+  const int m = J.m, n = J.n, k = m < n ? m : n;
+  if (k > KMAX || m <= 0 || n <= 0) return;  // rejected on the host
+  if (m <= QS) {
+    if (m <= 4) qr_small<4>(J, L);
+    else if (m <= 8) qr_small<8>(J, L);
+    else qr_small<QS>(J, L);
+    return;
+  }
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
+  double TNX_GLOBAL* W = as_global<double>(J.work);
+  const double TNX_GLOBAL* Q = W + (int64_t)m * n;
+  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
+    int r, c;
+    if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }   // src[c*ld+r] contiguous in r
+    else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }           // src[r*ld+c] contiguous in c
+    W[(int64_t)c * m + r] = src_at(src, J.ld, J.trans, r, c);
+  }
+  __syncthreads();
+  if (m <= QB_MAX && k >= QS) qr_blocked(J, L);
+  else qr_columns(J, L);
+  double TNX_GLOBAL* q = as_global<double>(J.q);
   if (J.q_trans) {
-    for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NT) q[e] = Q[e];
+    for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NQ) q[e] = Q[e];
   } else {
-    for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NT) {
+    for (int64_t e = threadIdx.x; e < (int64_t)m * k; e += NQ) {
       int r = (int)(e / k), c = (int)(e - (int64_t)r * k);
       q[e] = Q[(int64_t)c * m + r];
     }
   }
-  (void)bcast;
 }
 
 // One-sided Jacobi SVD; work: W (m x n col-major), V (n x n col-major).
@@ -120,7 +386,7 @@ __global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double* W = (double*)J.work;
   double* V = W + (int64_t)m * n;
-  const double* src = (const double*)J.src;
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
   __shared__ int rotated;
   __shared__ double sv[KMAX];
   __shared__ int order[KMAX];
@@ -551,7 +817,13 @@ extern "C" int tnx_qr_f64(const tnx_qr_job* jobs, int njob, tnx_stream_t stream)
     tnx_set_error("tnx_qr_f64: bad arguments");
     return TNX_EINVAL;
   }
-  hipLaunchKernelGGL(qr_kernel, dim3(njob), dim3(NT), 0, (hipStream_t)stream, jobs);
+  static bool attr_set = false;
+  if (!attr_set) {
+    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)sizeof(QrLds)));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(qr_kernel, dim3(njob), dim3(NQ), sizeof(QrLds), (hipStream_t)stream, jobs);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }

@@ -385,6 +385,41 @@ def test_svd_jacobi_f64(gpu, m, n, trans):
     assert np.allclose(U @ SVT, M, atol=1e-12 * np.abs(M).max())
 
 
+@pytest.mark.parametrize('m,n', [(1, 1), (1, 70), (4, 4), (5, 1500), (8, 3), (9, 16), (16, 16),
+                                 (16, 130), (17, 16), (17, 33), (33, 17), (48, 47), (300, 520),
+                                 (512, 40), (513, 20), (70, 15)])
+@pytest.mark.parametrize('trans', [0, 1])
+def test_qr_paths(gpu, m, n, trans):
+    """Every way through the QR (up to 16 rows; blocks of 16 columns up to
+    512 rows; column by column) at its edges, Q over its source, against
+    numpy's QR, whose reflectors have the same signs.  Householder QR: Q^T Q =
+    1 and Q R = M to a few unit roundoffs per reflector (1e-14 sqrt(m n))."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m * 31 + n)
+    k = min(m, n)
+    M = rng.randn(m, n)
+    buf = _dev(M.T.copy() if trans else M)      # holds M, then Q (k <= n)
+    r = torch.zeros(k * n, dtype=torch.float64, device='cuda')
+    work = torch.zeros(m * n + m * k, dtype=torch.float64, device='cuda')
+    job = np.array([(buf.data_ptr(), buf.data_ptr(), r.data_ptr(), work.data_ptr(), m, n,
+                     m if trans else n, trans, trans, 0)], dtype=L.QR_JOB)
+    (dj,) = _upload([job])
+    print('qr paths', m, n, trans, flush=True)
+    L.check(lib.tnx_qr_f64(_vp(dj.data_ptr()), 1, _stream()), 'qr')
+    torch.cuda.synchronize()
+    q = buf.reshape(-1)[:m * k].cpu().numpy()
+    Q = q.reshape(k, m).T if trans else q.reshape(m, k)
+    R = r.cpu().numpy().reshape(k, n)
+    tol = 1e-14 * np.sqrt(m * n)
+    assert np.abs(Q.T @ Q - np.eye(k)).max() < tol
+    assert np.abs(Q @ R - M).max() < tol * np.abs(M).max()
+    assert np.all(np.tril(R, -1) == 0.0)
+    ref = np.linalg.qr(M)[1]
+    assert np.all(np.sign(np.diag(R)) == np.sign(np.diag(ref)))
+
+
 def test_chol_inv_f64(gpu):
     """One launch over Gram matrices of every block shape (n = 1 .. 128,
     partial 16-blocks, leading dimension above n, one matrix with
