@@ -2,11 +2,12 @@
 // Cholesky factor of CholeskyQR3 and one-sided Jacobi (Hestenes) SVD
 // (entanglement spectrum moves).  One workgroup per matrix.
 #include "tnx_common.h"
+#include "jacobi_rot.h"
 
 namespace {
 
 constexpr int NT = 256;
-constexpr int NQ = 1024;    // lanes of the QR kernel
+constexpr int NQ = 1024;    // lanes of the QR and SVD kernels
 constexpr int KMAX = 4096;  // max columns of a gauge-move matrix
 
 __device__ __forceinline__ double src_at(const double TNX_GLOBAL* src, int ld, int trans, int r, int c) {
@@ -378,26 +379,45 @@ __global__ __launch_bounds__(NQ) void qr_kernel(const tnx_qr_job* __restrict__ j
   }
 }
 
-// One-sided Jacobi SVD; work: W (m x n col-major), V (n x n col-major).
-__global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__ jobs, int max_sweeps) {
-  const tnx_svd_job J = jobs[blockIdx.x];
-  const int m = J.m, n = J.n;
-  if (n > KMAX || m < n || n <= 0) return;  // rejected on the host
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  double* W = (double*)J.work;
-  double* V = W + (int64_t)m * n;
-  const double TNX_GLOBAL* src = as_global<const double>(J.src);
-  __shared__ int rotated;
-  __shared__ double sv[KMAX];
-  __shared__ int order[KMAX];
+// ------------------------------------------------ one-sided Jacobi SVD
+// W (m x n) and V (n x n), both column-major, in LDS when they fit
+// (SVD_LDS bytes: n = 80 for a square matrix) and in the job's work area
+// otherwise.  SVD_T = 16 lanes rotate a column pair, so the pairs of a round
+// run side by side up to n = 128; more lanes only repeat the scalar part of a
+// rotation, which is most of it (order 64: 64 lanes a pair 2.0 ms, 16 0.85).
+// Bound: a rotation's reductions and angle (latency).  ms (MI355X), four
+// wavefronts on columns in global memory -> this: order 16 0.32 -> 0.08, 32
+// 1.5 -> 0.24, 64 6.5 -> 0.85, with singular values over 20 decades 17.3 ->
+// 2.4, 128 (not in LDS) 37 -> 12.  Putting the larger column of a pair first,
+// as the block Jacobi does, costs sweeps here (1.2 ms at 64).
+constexpr size_t SVD_LDS = 100 * 1024;
+constexpr int SVD_T = 16;
 
-  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NT) {
+// sum over the 16 lanes of a row
+__device__ __forceinline__ double row_sum(double v) {
+  v = tnx_row_add<0x128>(v);
+  v = tnx_row_add<0x124>(v);
+  v = tnx_row_add<0x122>(v);
+  return tnx_row_add<0x121>(v);
+}
+
+template <typename PW>
+__device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, PW W, PW V, double* sv,
+                                         int* order, int& rotated) {
+  const int m = J.m, n = J.n;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int NW = NQ / 64;
+  const int l = lane & (SVD_T - 1);
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
+
+  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
     int r, c;
     if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }
     else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }
     W[(int64_t)c * m + r] = src_at(src, J.ld, J.trans, r, c);
   }
-  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NT) {
+  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NQ) {
     int c = (int)(e / n), r = (int)(e - (int64_t)c * n);
     V[e] = (r == c) ? 1.0 : 0.0;
   }
@@ -410,41 +430,41 @@ __global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__
     if (threadIdx.x == 0) rotated = 0;
     __syncthreads();
     for (int round = 0; round < np - 1; ++round) {
-      for (int p = wave; p < np / 2; p += 4) {
+      for (int p = threadIdx.x / SVD_T; p < np / 2; p += NQ / SVD_T) {
         // circle method: player np-1 fixed, others rotate
         int a = (p == 0) ? np - 1 : (round + p) % (np - 1);
         int b = (round + np - 1 - p) % (np - 1);
         if (p == 0) b = round % (np - 1);
         if (a >= n || b >= n || a == b) continue;
         if (a > b) { int t = a; a = b; b = t; }
-        double* wa = W + (int64_t)a * m;
-        double* wb = W + (int64_t)b * m;
+        const PW wa = W + (int64_t)a * m, wb = W + (int64_t)b * m;
         double al = 0.0, be = 0.0, ga = 0.0;
-        for (int r = lane; r < m; r += 64) {
+        for (int r = l; r < m; r += SVD_T) {
           const double x = wa[r], y = wb[r];
           al += x * x;
           be += y * y;
           ga += x * y;
         }
-        al = tnx_wave_sum(al);
-        be = tnx_wave_sum(be);
-        ga = tnx_wave_sum(ga);
-        if (ga != 0.0 && fabs(ga) > eps * sqrt(al * be)) {
-          if (lane == 0) rotated = 1;
-          const double zeta = (be - al) / (2.0 * ga);
-          const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-          const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
-          for (int r = lane; r < m; r += 64) {
-            const double x = wa[r], y = wb[r];
-            wa[r] = cs * x - sn * y;
-            wb[r] = sn * x + cs * y;
+        al = row_sum(al);
+        be = row_sum(be);
+        ga = row_sum(ga);
+        const double ab = al * be;
+        const bool rot = ga != 0.0 && fabs(ga) > eps * (ab > 0.0 ? ab * __builtin_amdgcn_rsq(ab) : 0.0);
+        const JacobiRot jr = jacobi_rot(al, be, ga, rot, false);
+        if (rot || jr.swap) {
+          if (l == 0 && rot) rotated = 1;
+          for (int r = l; r < m; r += SVD_T) {
+            double x = wa[r], y = wb[r];
+            jacobi_apply(jr, x, y);
+            wa[r] = x;
+            wb[r] = y;
           }
-          double* va = V + (int64_t)a * n;
-          double* vb = V + (int64_t)b * n;
-          for (int r = lane; r < n; r += 64) {
-            const double x = va[r], y = vb[r];
-            va[r] = cs * x - sn * y;
-            vb[r] = sn * x + cs * y;
+          const PW va = V + (int64_t)a * n, vb = V + (int64_t)b * n;
+          for (int r = l; r < n; r += SVD_T) {
+            double x = va[r], y = vb[r];
+            jacobi_apply(jr, x, y);
+            va[r] = x;
+            vb[r] = y;
           }
         }
       }
@@ -454,30 +474,30 @@ __global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__
     __syncthreads();
   }
   // singular values and descending order
-  for (int c = wave; c < n; c += 4) {
-    const double* wc = W + (int64_t)c * m;
+  for (int c = wave; c < n; c += NW) {
+    const PW wc = W + (int64_t)c * m;
     double s = 0.0;
     for (int r = lane; r < m; r += 64) s += wc[r] * wc[r];
     s = tnx_wave_sum(s);
     if (lane == 0) sv[c] = sqrt(s);
   }
   __syncthreads();
-  for (int c = threadIdx.x; c < n; c += NT) {
+  for (int c = threadIdx.x; c < n; c += NQ) {
     int rank = 0;
     const double x = sv[c];
     for (int o = 0; o < n; ++o) rank += (sv[o] > x) || (sv[o] == x && o < c);
     order[rank] = c;
   }
   __syncthreads();
-  double* s_out = (double*)J.s;
-  double* u = (double*)J.u;
-  double* svt = (double*)J.svt;
-  for (int i = threadIdx.x; i < n; i += NT) s_out[i] = sv[order[i]];
+  double TNX_GLOBAL* s_out = as_global<double>(J.s);
+  double TNX_GLOBAL* u = as_global<double>(J.u);
+  double TNX_GLOBAL* svt = as_global<double>(J.svt);
+  for (int i = threadIdx.x; i < n; i += NQ) s_out[i] = sv[order[i]];
   // U columns (normalised), sorted; zero columns are completed afterwards
-  for (int i = wave; i < n; i += 4) {
+  for (int i = wave; i < n; i += NW) {
     const int c = order[i];
     const double sc = sv[c] > 0.0 ? 1.0 / sv[c] : 0.0;
-    const double* wc = W + (int64_t)c * m;
+    const PW wc = W + (int64_t)c * m;
     for (int r = lane; r < m; r += 64) {
       const double v = wc[r] * sc;
       if (J.u_trans) u[(int64_t)i * m + r] = v;
@@ -485,7 +505,7 @@ __global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__
     }
   }
   // svt[i][col] = s_i * V[col][order i]
-  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NT) {
+  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NQ) {
     int i = (int)(e / n), col = (int)(e - (int64_t)i * n);
     const int c = order[i];
     svt[e] = sv[c] * V[(int64_t)c * n + col];
@@ -534,6 +554,23 @@ __global__ __launch_bounds__(NT) void svd_kernel(const tnx_svd_job* __restrict__
         }
       }
     }
+  }
+}
+
+__global__ __launch_bounds__(NQ) void svd_kernel(const tnx_svd_job* __restrict__ jobs, int max_sweeps) {
+  extern __shared__ double lds[];
+  __shared__ int rotated;
+  __shared__ double sv[KMAX];
+  __shared__ int order[KMAX];
+  const tnx_svd_job J = jobs[blockIdx.x];
+  const int m = J.m, n = J.n;
+  if (n > KMAX || m < n || n <= 0) return;  // rejected on the host
+  const int64_t wn = (int64_t)m * n;
+  if ((wn + (int64_t)n * n) * (int64_t)sizeof(double) <= (int64_t)SVD_LDS) {
+    svd_body<double*>(J, max_sweeps, lds, lds + wn, sv, order, rotated);
+  } else {
+    double TNX_GLOBAL* W = as_global<double>(J.work);
+    svd_body<double TNX_GLOBAL*>(J, max_sweeps, W, W + wn, sv, order, rotated);
   }
 }
 
@@ -835,7 +872,13 @@ extern "C" int tnx_svd_jacobi_f64(const tnx_svd_job* jobs, int njob, int max_swe
     tnx_set_error("tnx_svd_jacobi_f64: bad arguments");
     return TNX_EINVAL;
   }
-  hipLaunchKernelGGL(svd_kernel, dim3(njob), dim3(NT), 0, (hipStream_t)stream, jobs, max_sweeps);
+  static bool attr_set = false;
+  if (!attr_set) {
+    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)svd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)SVD_LDS));
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(svd_kernel, dim3(njob), dim3(NQ), SVD_LDS, (hipStream_t)stream, jobs, max_sweeps);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }

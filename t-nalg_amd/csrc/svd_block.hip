@@ -44,6 +44,7 @@
 // R may then be the work area itself (r == work, ld_r == n): forming B is a
 // copy onto itself.
 #include "tnx_common.h"
+#include "jacobi_rot.h"
 
 namespace {
 
@@ -107,39 +108,6 @@ __global__ __launch_bounds__(NT) void k_svdj_scale(const tnx_svdj_job* __restric
 
 __global__ void k_svdj_clear(int32_t* flag) {
   if (threadIdx.x == 0) *flag = 0;
-}
-
-// The rotation of the pair (x, y) with Gram entries a, c and g: x' = x - s (y +
-// tau x), y' = y + s (x - tau y), tau = s / (1 + cos); swap: the results
-// change places (x'' = y', y'' = -x'), so that the larger column comes first.
-// The tangent needs no more than the hardware's reciprocal and root (any
-// angle is a rotation; an approximate one leaves 1e-7 of g), the cosine and
-// tau are refined to working accuracy, so the transformation is orthogonal.
-struct Rot { double s, tau; bool rot, swap; };
-__device__ __forceinline__ Rot rot_of(double a, double c, double g, double eps2, double zero2) {
-  Rot r;
-  r.rot = g != 0.0 && a > zero2 && c > zero2 && g * g > eps2 * (a * c);
-  r.swap = c > a && a > zero2;   // never with a zero column (the padding of a panel among them)
-  const double h = c - a, g2 = r.rot ? 2.0 * g : 1.0;
-  const double w = fma(h, h, g2 * g2);
-  const double den = fabs(h) + w * __builtin_amdgcn_rsq(w);
-  const double t = (h >= 0.0 ? g2 : -g2) * __builtin_amdgcn_rcp(den);   // |t| <= 1
-  const double x = fma(t, t, 1.0);
-  double y = __builtin_amdgcn_rsq(x);              // cos = 1 / sqrt(1 + t^2)
-  const double e = fma(-x * y, y, 1.0);            // third order: e^3 of the root's 2^-20 or less
-  y = fma(y * e, fma(0.375, e, 0.5), y);
-  const double d = 1.0 + y;
-  double q = __builtin_amdgcn_rcp(d);
-  const double f = fma(-d, q, 1.0);
-  q = fma(q, fma(f, f, f), q);
-  r.s = r.rot ? y * t : 0.0;
-  r.tau = r.s * q;
-  return r;
-}
-__device__ __forceinline__ void rotate(const Rot& r, double& x, double& y) {
-  const double xn = fma(-r.s, fma(r.tau, x, y), x), yn = fma(r.s, fma(-r.tau, y, x), y);
-  x = r.swap ? yn : xn;
-  y = r.swap ? -xn : yn;
 }
 
 // Column c (0..31) of a panel: sub-blocks starting at columns ca and cb, cnt
@@ -311,15 +279,20 @@ __global__ __launch_bounds__(RT, 4) void k_svdj_round(const tnx_svdj_job* __rest
         const double (*G)[GLD] = L.m.G[cur];
         int up, vp, uq, vq;
         pair_of(PW, ir, qi, uq, vq);
-        const Rot rq = rot_of(G[uq][uq], G[vq][vq], G[uq][vq], eps2, zero2);
+        auto rotation = [&](int u, int v) {
+          const double a = G[u][u], c = G[v][v], gg = G[u][v];
+          const bool live = a > zero2 && c > zero2;   // no zero column (the padding among them)
+          return jacobi_rot(a, c, gg, live && gg * gg > eps2 * (a * c), live);
+        };
+        const JacobiRot rq = rotation(uq, vq);
         if (!q_half) {
           pair_of(PW, ir, pi, up, vp);
-          const Rot rp = rot_of(G[up][up], G[vp][vp], G[up][vp], eps2, zero2);
+          const JacobiRot rp = rotation(up, vp);
           double g11 = G[up][uq], g12 = G[up][vq], g21 = G[vp][uq], g22 = G[vp][vq];
-          rotate(rq, g11, g12);
-          rotate(rq, g21, g22);
-          rotate(rp, g11, g21);
-          rotate(rp, g12, g22);
+          jacobi_apply(rq, g11, g12);
+          jacobi_apply(rq, g21, g22);
+          jacobi_apply(rp, g11, g21);
+          jacobi_apply(rp, g12, g22);
           double (*H)[GLD] = L.m.G[cur ^ 1];
           H[up][uq] = g11;
           H[up][vq] = g12;
@@ -329,8 +302,8 @@ __global__ __launch_bounds__(RT, 4) void k_svdj_round(const tnx_svdj_job* __rest
           const double (*Q)[GLD] = L.m.Q[cur];
           double q11 = Q[2 * pi][uq], q12 = Q[2 * pi][vq];
           double q21 = Q[2 * pi + 1][uq], q22 = Q[2 * pi + 1][vq];
-          rotate(rq, q11, q12);
-          rotate(rq, q21, q22);
+          jacobi_apply(rq, q11, q12);
+          jacobi_apply(rq, q21, q22);
           double (*H)[GLD] = L.m.Q[cur ^ 1];
           H[2 * pi][uq] = q11;
           H[2 * pi][vq] = q12;

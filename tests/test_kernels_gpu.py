@@ -420,6 +420,37 @@ def test_qr_paths(gpu, m, n, trans):
     assert np.all(np.sign(np.diag(R)) == np.sign(np.diag(ref)))
 
 
+@pytest.mark.parametrize('m,n', [(1, 1), (3, 3), (17, 2), (31, 31), (64, 64), (80, 80), (81, 81),
+                                 (500, 21), (130, 129)])
+def test_svd_jacobi_in_and_out_of_lds(gpu, m, n):
+    """The single-workgroup Jacobi SVD below, at and above the order whose
+    columns fit in LDS, singular values over 12 decades in mixed columns: the
+    bounds of test_svd_jacobi_f64."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + 3 * n)
+    M = (rng.randn(m, n) * np.logspace(0, -12, n)) @ np.linalg.qr(rng.randn(n, n))[0]
+    src = _dev(M)
+    u = torch.zeros(m * n, dtype=torch.float64, device='cuda')
+    s = torch.zeros(n, dtype=torch.float64, device='cuda')
+    svt = torch.zeros(n * n, dtype=torch.float64, device='cuda')
+    work = torch.zeros(m * n + n * n, dtype=torch.float64, device='cuda')
+    job = np.array([(src.data_ptr(), u.data_ptr(), s.data_ptr(), svt.data_ptr(), work.data_ptr(),
+                     m, n, n, 0, 0, 0)], dtype=L.SVD_JOB)
+    (dj,) = _upload([job])
+    print('svd lds', m, n, flush=True)
+    L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), 1, 60, _stream()), 'svd')
+    torch.cuda.synchronize()
+    U, sv, SVT = (x.cpu().numpy() for x in (u, s, svt))
+    U, SVT = U.reshape(m, n), SVT.reshape(n, n)
+    ref = np.linalg.svd(M, compute_uv=False)
+    assert np.abs(sv - ref).max() < 1e-14 * ref[0] * max(1, n)
+    assert np.all(np.diff(sv) <= 0)
+    assert np.allclose(U.T @ U, np.eye(n), atol=1e-10)
+    assert np.allclose(U @ SVT, M, atol=1e-12 * np.abs(M).max())
+
+
 def test_chol_inv_f64(gpu):
     """One launch over Gram matrices of every block shape (n = 1 .. 128,
     partial 16-blocks, leading dimension above n, one matrix with
