@@ -395,10 +395,10 @@ constexpr int SVD_T = 16;
 
 // sum over the 16 lanes of a row
 __device__ __forceinline__ double row_sum(double v) {
-  v = tnx_row_add<0x128>(v);
-  v = tnx_row_add<0x124>(v);
-  v = tnx_row_add<0x122>(v);
-  return tnx_row_add<0x121>(v);
+  v += tnx_row_get<0x128>(v);
+  v += tnx_row_get<0x124>(v);
+  v += tnx_row_get<0x122>(v);
+  return v + tnx_row_get<0x121>(v);
 }
 
 template <typename PW>
@@ -837,12 +837,8 @@ extern "C" int tnx_chol_inv_f64(const tnx_chol_job* jobs, int njob, tnx_stream_t
     tnx_set_error("tnx_chol_inv_f64: bad arguments");
     return TNX_EINVAL;
   }
-  static bool attr_set = false;
-  if (!attr_set) {
-    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)chol_inv_kernel,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)CHOL_LDS));
-    attr_set = true;
-  }
+  static std::atomic<uint64_t> lds_set{0};
+  if (int rc = tnx_dynamic_lds((const void*)chol_inv_kernel, CHOL_LDS, lds_set)) return rc;
   hipLaunchKernelGGL(chol_inv_kernel, dim3(njob), dim3(NT), CHOL_LDS, (hipStream_t)stream, jobs);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
@@ -854,12 +850,8 @@ extern "C" int tnx_qr_f64(const tnx_qr_job* jobs, int njob, tnx_stream_t stream)
     tnx_set_error("tnx_qr_f64: bad arguments");
     return TNX_EINVAL;
   }
-  static bool attr_set = false;
-  if (!attr_set) {
-    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)qr_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)sizeof(QrLds)));
-    attr_set = true;
-  }
+  static std::atomic<uint64_t> lds_set{0};
+  if (int rc = tnx_dynamic_lds((const void*)qr_kernel, sizeof(QrLds), lds_set)) return rc;
   hipLaunchKernelGGL(qr_kernel, dim3(njob), dim3(NQ), sizeof(QrLds), (hipStream_t)stream, jobs);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
@@ -872,12 +864,8 @@ extern "C" int tnx_svd_jacobi_f64(const tnx_svd_job* jobs, int njob, int max_swe
     tnx_set_error("tnx_svd_jacobi_f64: bad arguments");
     return TNX_EINVAL;
   }
-  static bool attr_set = false;
-  if (!attr_set) {
-    TNX_CHECK_HIP(hipFuncSetAttribute((const void*)svd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)SVD_LDS));
-    attr_set = true;
-  }
+  static std::atomic<uint64_t> lds_set{0};
+  if (int rc = tnx_dynamic_lds((const void*)svd_kernel, SVD_LDS, lds_set)) return rc;
   hipLaunchKernelGGL(svd_kernel, dim3(njob), dim3(NQ), SVD_LDS, (hipStream_t)stream, jobs, max_sweeps);
   TNX_CHECK_LAUNCH();
   return TNX_OK;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdio.h>
+#include <atomic>
 #include <string>
 
 #include "../../include/tnalg_hip.h"
@@ -69,6 +70,18 @@ int tnx_gemm_grouped_ts(int mode, const tnx_gemm_problem* prob, int nprob,
     }                                                                            \
   } while (0)
 
+// Once per kernel and GPU: allow it `bytes` of dynamic LDS (a launch asks for
+// more than the default).  `done`: the kernel's bit set of GPUs, static.
+inline int tnx_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& done) {
+  int dev = 0;
+  TNX_CHECK_HIP(hipGetDevice(&dev));
+  const uint64_t bit = 1ull << (dev & 63);
+  if (done.load(std::memory_order_acquire) & bit) return TNX_OK;
+  TNX_CHECK_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  done.fetch_or(bit, std::memory_order_release);
+  return TNX_OK;
+}
+
 typedef double tnx_d4 __attribute__((ext_vector_type(4)));
 typedef float tnx_f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 tnx_bf8 __attribute__((ext_vector_type(8)));
@@ -105,17 +118,20 @@ __device__ __forceinline__ int tnx_xcd_remap(int bid, int nblocks) {
   return x * q + (x < r ? x : r) + i;
 }
 
-// One step of the butterfly below: v plus the value `DPP` (a row rotation of
-// the data-parallel primitives) brings from another lane of the 16-lane row.
-template <int DPP> __device__ __forceinline__ double tnx_row_add(double v) {
+// Lane exchanges of the butterflies below, all of them VALU operations
+// (through the LDS crossbar, __shfl_xor, each took about 120 cycles on the
+// path of every reduction).  tnx_row_get: the value that `DPP`, a rotation
+// within the 16-lane row, brings from another lane.
+template <int DPP> __device__ __forceinline__ double tnx_row_get(double v) {
   const long long x = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_mov_dpp((int)x, DPP, 0xf, 0xf, true);
   const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), DPP, 0xf, 0xf, true);
-  return v + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-// x[lane] + x[lane ^ 32] (HALF) or x[lane] + x[lane ^ 16], by the swap of the
-// odd rows of one register with the even rows of another.
-template <bool HALF> __device__ __forceinline__ double tnx_swap_add(double v) {
+// The values of lane and lane ^ 32 (HALF) or lane ^ 16, the one with the bit
+// clear in `p`, by the swap of the odd rows of one register with the even rows
+// of another.
+template <bool HALF> __device__ __forceinline__ void tnx_swap_get(double v, double& p, double& q) {
   const long long x = __double_as_longlong(v);
   const unsigned l = (unsigned)x, h = (unsigned)(x >> 32);
   typedef unsigned u2 __attribute__((ext_vector_type(2)));
@@ -127,21 +143,28 @@ template <bool HALF> __device__ __forceinline__ double tnx_swap_add(double v) {
     lo = __builtin_amdgcn_permlane16_swap(l, l, false, false);
     hi = __builtin_amdgcn_permlane16_swap(h, h, false, false);
   }
-  return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
-         __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+  p = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
+  q = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
 }
-// Sum over the wavefront, the same bits in every lane: the butterfly over lane
-// ^ 32, 16, 8, 4, 2, 1.  Within a 16-lane row a rotation by d = 8, 4, 2, 1
-// brings lane ^ d's value, as the values repeat with period 2 d by then.  All
-// steps are VALU operations: through the LDS crossbar (__shfl_xor) each of the
-// six took about 120 cycles on the path of every reduction.
+// Butterfly over lane ^ 32, 16, 8, 4, 2, 1, the same bits in every lane.  In a
+// 16-lane row a rotation by d = 8, 4, 2, 1 brings lane ^ d's value, as the
+// values repeat with period 2 d by then.
+template <typename F> __device__ __forceinline__ double tnx_wave_fold(double v, F f) {
+  double p, q;
+  tnx_swap_get<true>(v, p, q);
+  v = f(p, q);
+  tnx_swap_get<false>(v, p, q);
+  v = f(p, q);
+  v = f(v, tnx_row_get<0x128>(v));
+  v = f(v, tnx_row_get<0x124>(v));
+  v = f(v, tnx_row_get<0x122>(v));
+  return f(v, tnx_row_get<0x121>(v));
+}
 __device__ __forceinline__ double tnx_wave_sum(double v) {
-  v = tnx_swap_add<true>(v);
-  v = tnx_swap_add<false>(v);
-  v = tnx_row_add<0x128>(v);
-  v = tnx_row_add<0x124>(v);
-  v = tnx_row_add<0x122>(v);
-  return tnx_row_add<0x121>(v);
+  return tnx_wave_fold(v, [](double x, double y) { return x + y; });
+}
+__device__ __forceinline__ double tnx_wave_min(double v) {
+  return tnx_wave_fold(v, [](double x, double y) { return fmin(x, y); });
 }
 
 // Largest index i in [0, n) whose 32-bit field at byte offset `off` of the
