@@ -15,15 +15,13 @@
 // basis); the basis is stored in f64, or in f32 for a solve whose matvec
 // runs in f32 or bf16 (v_dtype: the basis passes then move half the bytes).
 // The matvec may run in f32 or bf16.
-// The (j+1)x(j+1) tridiagonal eigenproblem is solved on the device by 257-way
-// multisection of the Sturm count (one workgroup) followed by inverse
-// iteration with partial pivoting.
+// The (j+1)x(j+1) tridiagonal eigenproblem is solved on the device by one
+// wavefront: 65-way multisection, then a twisted factorisation.
 // A solve that has not converged after ncv steps is restarted implicitly
 // (Sorensen's implicitly restarted Lanczos with exact shifts, as ARPACK's
 // dsaupd does for eigsh): the ncv - k largest Ritz values are applied as
-// shifts of implicit QR steps on the tridiagonal matrix, which compresses the
-// factorisation to k = min(LZ_KEEP, ncv - 1) vectors spanning the k lowest
-// Ritz vectors; the next cycle continues the Lanczos recurrence from step k.
+// shifts to the tridiagonal matrix, which compresses the factorisation to
+// k = min(LZ_KEEP, ncv - 1) vectors spanning the k lowest Ritz vectors; the next cycle continues the Lanczos recurrence from step k.
 #include <mutex>
 
 #include "tnx_common.h"
@@ -194,112 +192,134 @@ __device__ __forceinline__ void reduce_partials(const double* part, int chunk_be
   }
 }
 
-// Number of eigenvalues of the symmetric tridiagonal (a, b) below x.
-__device__ inline int sturm_count(const double* a, const double* b, int k, double x) {
-  const double tiny = 1e-300;
-  int cnt = 0;
-  double q = a[0] - x;
-  if (q < 0) cnt++;
+// 1 / d to working accuracy (the hardware's approximation, third order)
+__device__ __forceinline__ double fast_rcp(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+__device__ __forceinline__ double fast_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Number of eigenvalues below x of the k x k symmetric tridiagonal with
+// diagonal a and squared couplings b2 (LDS), whose entries are of order one or
+// less: sign changes of the leading minors p_i = (a_i - x) p_{i-1} - b2_{i-1}
+// p_{i-2}, one dependent operation a row where the ratios of the minors
+// (Sturm's sequence) need a division.  A zero counts as a change; the pair is
+// scaled up when it gets small.
+__device__ __forceinline__ int count_below(const double* a, const double* b2, int k, double x) {
+  double p0 = 1.0, p1 = a[0] - x;
+  bool neg = p1 <= 0.0;
+  int cnt = neg;
+#pragma unroll 4
   for (int i = 1; i < k; ++i) {
-    if (fabs(q) < tiny) q = -tiny;
-    q = (a[i] - x) - b[i - 1] * b[i - 1] / q;
-    if (q < 0) cnt++;
+    const double p2 = fma(a[i] - x, p1, -b2[i - 1] * p0);
+    const bool change = neg ? p2 >= 0.0 : p2 <= 0.0;
+    cnt += change;
+    neg = neg != change;
+    const double sc = fmax(fabs(p1), fabs(p2)) < 1e-100 ? 1e100 : 1.0;
+    p0 = p1 * sc;
+    p1 = p2 * sc;
   }
   return cnt;
 }
 
-// Lowest eigenpair of the k x k tridiagonal (a, b), all NT lanes of the
-// block (a, b in LDS); thread 0 writes y[0..k) and *theta.  `work` is LDS
-// scratch of 5 * NCV_MAX doubles for the inverse iteration.  The bracket
-// shrinks 257-fold per round: lane t evaluates the Sturm count at the
-// (t + 1)-th of 256 interior points and the first point with a count >= 1
-// bounds the lowest eigenvalue.
-__device__ void tridiag_lowest(const double* a, const double* b, int k, double* y,
-                               double* theta, double* work) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Eigenpair idx (0: the lowest) of the k x k tridiagonal (a, b) in LDS, by one
+// wavefront (all 64 lanes): *theta and y[0..k) (LDS).  work: LDS scratch of
+// TRI_WORK doubles of the wavefront's own.
+// The bracket (the Gershgorin bounds; the smallest diagonal entry bounds the
+// lowest eigenvalue) shrinks 65-fold per round (64 interior points, one a
+// lane).  The vector is that of
+// the twisted factorisation: the pivots of T - theta from the top (D+) and
+// from the bottom (D-), two lanes side by side, meet at the row r of smallest
+// gamma_r = D+_r + D-_r - (a_r - theta), and z_r = 1 is continued by z_i = -b
+// z_{i+1} / D+_i above and -b z_{i-1} / D-_i below it: products of ratios,
+// accurate for the small components, the last of which is the residual
+// estimate.  A vanishing pivot is replaced by a tiny one (the next is then huge
+// and their ratios cancel).  The vector's sign is that of a positive component sum (as inverse iteration from a
+// constant vector gives).
+// Bound: the serial chains over k rows.  k_update_norm, most of which this is
+// (mean over k = 1..20, one solve, MI355X): 16.1 us with Sturm sequences by
+// division in 256 lanes and inverse iteration by one lane, 13.8 us so.
+constexpr int TRI_WORK = 4 * NCV_MAX;
+__device__ __forceinline__ void tridiag_pair(const double* a, const double* b, int k, int idx,
+                                             double* y, double* theta, double* work) {
+  const int lane = threadIdx.x & 63;
+  double* as = work;
+  double* b2 = work + NCV_MAX;
+  double* dp = work + 2 * NCV_MAX;   // D+, then D-
+  const bool in = lane < k;
+  const double al = in ? a[lane] : 0.0;
+  const double bl = lane + 1 < k ? b[lane] : 0.0;   // coupling of rows lane, lane + 1
+  const double bm = in && lane > 0 ? b[lane - 1] : 0.0;
+  const double inf = __builtin_huge_val();
+  double base = tnx_wave_min(in ? al - fabs(bl) - fabs(bm) : inf);
+  const double dmin = tnx_wave_min(in ? al : inf);
+  const double most = -tnx_wave_min(in ? -(al + fabs(bl) + fabs(bm)) : inf);
+  base -= 1e-12 * fmax(most - base, 1e-300);
+  // entries relative to `base`, over a power of two near the spectrum's width
+  const int ex = __builtin_amdgcn_frexp_exp(most - base);
+  if (in) {
+    as[lane] = __builtin_amdgcn_ldexp(al - base, -ex);
+    const double bs = __builtin_amdgcn_ldexp(bl, -ex);
+    b2[lane] = bs * bs;
+  }
+  __builtin_amdgcn_wave_barrier();
+  const double top = idx == 0 ? dmin : most;
+  double lo = 0.0, hi = __builtin_amdgcn_ldexp(top - base, -ex) * (1.0 + 1e-12);
+  const double stop = __builtin_amdgcn_ldexp(4.0 * 2.220446049250313e-16 * fmax(fabs(base), fabs(top)), -ex);
+  for (int round = 0; round < 16; ++round) {
+    const double w = (hi - lo) * (1.0 / 65.0);  // identical in every lane
+    if (65.0 * w <= stop + 1e-300) break;
+    const unsigned long long m = __ballot(count_below(as, b2, k, lo + w * (double)(lane + 1)) > idx);
+    const int f = m != 0ull ? __ffsll((long long)m) : 65;   // the first point above it (65: hi)
+    const double l0 = lo;
+    lo = l0 + w * (double)(f - 1);
+    if (f < 65) hi = l0 + w * (double)f;
+  }
+  const double th = 0.5 * (lo + hi);
   if (k == 1) {
-    if (threadIdx.x == 0) { y[0] = 1.0; *theta = a[0]; }
+    if (lane == 0) {
+      y[0] = 1.0;
+      *theta = a[0];
+    }
     return;
   }
-  __shared__ unsigned long long masks[NT / 64];
-  double lo = a[0], hi = a[0];
+  // pivots: even lanes from the top, odd lanes from the bottom
+  const bool up = lane & 1;
+  double* dw = dp + (up ? NCV_MAX : 0);
+  const double tiny = 1e-150;
+  double d = 1.0;
+#pragma unroll 4
   for (int i = 0; i < k; ++i) {
-    double r = (i > 0 ? fabs(b[i - 1]) : 0.0) + (i < k - 1 ? fabs(b[i]) : 0.0);
-    lo = fmin(lo, a[i] - r);
-    hi = fmax(hi, a[i] + r);
+    const int row = up ? k - 1 - i : i;
+    const double off = i == 0 ? 0.0 : b2[up ? row : row - 1];
+    d = (as[row] - th) - off * fast_rcp(d);
+    if (fabs(d) < tiny) d = tiny;
+    if (lane < 2) dw[row] = d;
   }
-  const double span = fmax(hi - lo, 1e-300);
-  lo -= 1e-12 * span;
-  hi += 1e-12 * span;
-  constexpr double NSUB = NT + 1;
-  for (int round = 0; round < 16; ++round) {
-    const double w = hi - lo;  // identical in every lane
-    if (w <= 4.0 * 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + 1e-300) break;
-    const double x = lo + w * (double)(threadIdx.x + 1) / NSUB;
-    const int cnt = sturm_count(a, b, k, x);
-    const unsigned long long m = __ballot(cnt >= 1);
-    if (lane == 0) masks[wave] = m;
-    __syncthreads();
-    int f = -1;
-    for (int q = 0; q < NT / 64; ++q)
-      if (masks[q] != 0ull) {
-        f = q * 64 + __ffsll((long long)masks[q]) - 1;
-        break;
-      }
-    __syncthreads();  // masks are rewritten next round
-    if (f < 0) {
-      lo = lo + w * (double)NT / NSUB;
-    } else {
-      const double xf = lo + w * (double)(f + 1) / NSUB;
-      const double xp = lo + w * (double)f / NSUB;
-      hi = xf;
-      lo = xp;
-    }
+  __builtin_amdgcn_wave_barrier();
+  const double gam = in ? fabs(dp[lane] + dp[NCV_MAX + lane] - (as[lane] - th)) : inf;
+  const double gmin = tnx_wave_min(gam);
+  const int r = __ffsll((long long)__ballot(gam == gmin)) - 1;
+  // ratio of z_lane to its neighbour on the side of r, then running products
+  double z = 1.0;
+  if (in && lane < r) z = -__builtin_amdgcn_ldexp(bl, -ex) * fast_rcp(dp[lane]);
+  else if (in && lane > r) z = -__builtin_amdgcn_ldexp(bm, -ex) * fast_rcp(dp[NCV_MAX + lane]);
+#pragma unroll
+  for (int o = 1; o < NCV_MAX; o <<= 1) {
+    const int from = lane < r ? lane + o : lane - o;
+    const double v = __shfl(z, from, 64);
+    if (lane < r ? from < r : from > r) z *= v;
   }
-  if (threadIdx.x != 0) return;
-  const double th = 0.5 * (lo + hi);
-  *theta = th;
-  // inverse iteration with partial pivoting on (T - th I)
-  double* z = work;
-  double* rhs = work + NCV_MAX;
-  double* u0 = work + 2 * NCV_MAX;
-  double* u1 = work + 3 * NCV_MAX;
-  double* u2 = work + 4 * NCV_MAX;
-  const double tiny = 2.220446049250313e-16 * span;
-  for (int i = 0; i < k; ++i) z[i] = 1.0 / sqrt((double)k);
-  for (int it = 0; it < 2; ++it) {
-    for (int i = 0; i < k; ++i) rhs[i] = z[i];
-    // current pivot-row candidate (cols i, i+1, i+2)
-    double p0 = a[0] - th, p1 = b[0], p2 = 0.0, pr = rhs[0];
-    for (int i = 0; i < k - 1; ++i) {
-      const double n0 = b[i], n1 = a[i + 1] - th, n2 = (i + 1 < k - 1) ? b[i + 1] : 0.0;
-      const double nr = rhs[i + 1];
-      if (fabs(p0) >= fabs(n0)) {
-        if (fabs(p0) < tiny) p0 = (p0 < 0 ? -tiny : tiny);
-        const double f = n0 / p0;
-        u0[i] = p0; u1[i] = p1; u2[i] = p2; rhs[i] = pr;
-        p0 = n1 - f * p1; p1 = n2 - f * p2; p2 = 0.0; pr = nr - f * pr;
-      } else {
-        const double f = p0 / n0;
-        u0[i] = n0; u1[i] = n1; u2[i] = n2; rhs[i] = nr;
-        const double q0 = p1 - f * n1, q1 = p2 - f * n2;
-        p0 = q0; p1 = q1; p2 = 0.0; pr = pr - f * nr;
-      }
-    }
-    if (fabs(p0) < tiny) p0 = (p0 < 0 ? -tiny : tiny);
-    u0[k - 1] = p0; u1[k - 1] = 0.0; u2[k - 1] = 0.0; rhs[k - 1] = pr;
-    for (int i = k - 1; i >= 0; --i) {
-      double s = rhs[i];
-      if (i + 1 < k) s -= u1[i] * z[i + 1];
-      if (i + 2 < k) s -= u2[i] * z[i + 2];
-      z[i] = s / u0[i];
-    }
-    double nrm = 0.0;
-    for (int i = 0; i < k; ++i) nrm += z[i] * z[i];
-    nrm = 1.0 / sqrt(nrm);
-    for (int i = 0; i < k; ++i) z[i] *= nrm;
-  }
-  for (int i = 0; i < k; ++i) y[i] = z[i];
+  z = in ? z : 0.0;
+  double f = fast_rsqrt(tnx_wave_sum(z * z));
+  if (tnx_wave_sum(z) < 0.0) f = -f;
+  if (in) y[lane] = z * f;
+  if (lane == 0) *theta = base + __builtin_amdgcn_ldexp(th, ex);
 }
 
 // dtype of a solve's x or w: the call's, or the solve's own field when the
@@ -587,7 +607,7 @@ __global__ __launch_bounds__(NT) void k_update_norm(const tnx_lanczos_solve* __r
   }
   LzState& st = L.st[s];
   __shared__ double a_s[NCV_MAX], b_s[NCV_MAX], y_s[NCV_MAX], th_s;
-  __shared__ double work[5 * NCV_MAX];
+  __shared__ double work[TRI_WORK];
   // alpha[0..j-1], beta[0..j-1] were written by earlier launches: every lane
   // loads its share (one round trip instead of a serial loop of j loads)
   for (int k = threadIdx.x; k < j; k += NT) {
@@ -604,7 +624,7 @@ __global__ __launch_bounds__(NT) void k_update_norm(const tnx_lanczos_solve* __r
     b_s[j] = beta_j;
   }
   __syncthreads();
-  tridiag_lowest(a_s, b_s, j + 1, y_s, &th_s, work);
+  if (threadIdx.x < 64) tridiag_pair(a_s, b_s, j + 1, 0, y_s, &th_s, work);
   __syncthreads();
   for (int k = threadIdx.x; k <= j; k += NT) st.y[k] = y_s[k];
   if (threadIdx.x == 0) {
@@ -629,42 +649,160 @@ __global__ __launch_bounds__(NT) void k_update_norm(const tnx_lanczos_solve* __r
   tnx_stamp_end(ts);
 }
 
-// Sturm count (eigenvalues below x) of the m x m tridiagonal held in
-// registers: a[i] diagonal, e[i] = b[i]^2 the squared coupling of i, i+1.
-__device__ __forceinline__ int sturm_count_reg(const double (&a)[NCV_MAX],
-                                               const double (&e)[NCV_MAX], int m, double x) {
-  const double tiny = 1e-300;
-  int cnt = 0;
-  double q = 1.0;
+// Implicit restart with the m - k largest Ritz values as shifts, from the k
+// lowest Ritz pairs (one wavefront; the pairs' vectors y[i][0..m) and values
+// th[i] in LDS).  What the shifted QR steps leave is determined by them: the
+// new basis spans V Y, its tridiagonal matrix has their values, and only its
+// last vector couples to V[m].  So in the coordinates of the Ritz vectors the
+// basis is the Lanczos basis of diag(th) built backwards: the last vector is
+// s / |s|, s_i = y_i[m-1], and a Lanczos recurrence from it gives the others
+// down to the first and the couplings (positive, as the QR steps leave them).
+// The one sign left is that of the first vector, prod (T - shift) e_1 in the
+// QR steps: (-1)^(m-k) along each Ritz vector, as the shifts lie above.
+// False, with nothing written, if two Ritz values are so close that their
+// vectors are not independent: those vectors are each accurate to rounding
+// over the gap only.
+// Writes the new alpha, beta[0..k-2], the coefficients C[0..m-1] and sigma,
+// the coupling of the new last vector to V[m].
+__device__ __forceinline__ bool restart_from_pairs(double (*y)[NCV_MAX], const double* th, int m,
+                                                   int k, double beta_m, LzState& st,
+                                                   double* sigma) {
+  const int lane = threadIdx.x & 63;
+  double v[LZ_KEEP];
 #pragma unroll
-  for (int i = 0; i < NCV_MAX; ++i) {
-    if (i < m) {
-      q = (i == 0) ? (a[0] - x) : (a[i] - x) - e[i - 1] / q;
-      if (q < 0) cnt++;
-      if (fabs(q) < tiny) q = -tiny;
+  for (int i = 0; i < LZ_KEEP; ++i) v[i] = i < k && lane < m ? y[i][lane] : 0.0;
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass)
+#pragma unroll
+    for (int i = 1; i < LZ_KEEP; ++i)
+      if (i < k) {
+#pragma unroll
+        for (int q = 0; q < i; ++q) v[i] -= tnx_wave_sum(v[q] * v[i]) * v[q];
+        const double nn = tnx_wave_sum(v[i] * v[i]);
+        if (!(nn > 1e-4)) return false;
+        v[i] *= fast_rsqrt(nn);
+      }
+  // From here every lane computes the same k x k numbers: z[c][i] is the
+  // component of new vector c along Ritz vector i.
+  double z[LZ_KEEP][LZ_KEEP], d[LZ_KEEP], s2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < LZ_KEEP; ++i) {
+    const double si = __shfl(v[i], m - 1, 64);
+    d[i] = i < k ? th[i] - th[0] : 0.0;
+    s2 += si * si;
+#pragma unroll
+    for (int c = 0; c < LZ_KEEP; ++c) z[c][i] = c == k - 1 ? si : 0.0;
+  }
+  const double spread = d[0] + fmax(fmax(d[1], d[2]), d[3]);
+  const double sn = sqrt(s2);
+  double al[LZ_KEEP], be[LZ_KEEP];
+#pragma unroll
+  for (int c = LZ_KEEP - 1; c >= 0; --c) {
+    if (c >= k) continue;
+    double w[LZ_KEEP], wn = 0.0;
+    if (c == k - 1) {
+#pragma unroll
+      for (int i = 0; i < LZ_KEEP; ++i) w[i] = sn > 0.0 ? z[c][i] : (i == 0 ? 1.0 : 0.0);
+      wn = sn > 0.0 ? s2 : 1.0;
+    } else {
+      // Theta z of the vector above, orthogonalised twice.  If nothing is left
+      // (an invariant subspace) any orthogonal vector will do: from the unit
+      // vector with the most room, and its coupling is zero to rounding.
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (u == 1 && wn > 1e-28 * spread * spread) continue;
+        int row = 0;
+        double room = 2.0;
+#pragma unroll
+        for (int i = 0; i < LZ_KEEP; ++i) {
+          double q = 0.0;
+#pragma unroll
+          for (int l = c + 1; l < LZ_KEEP; ++l) q += l < k ? z[l][i] * z[l][i] : 0.0;
+          if (i < k && q < room) {
+            room = q;
+            row = i;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < LZ_KEEP; ++i)
+          w[i] = u == 0 ? d[i] * z[c + 1 < LZ_KEEP ? c + 1 : c][i] : (i == row ? 1.0 : 0.0);
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass)
+#pragma unroll
+          for (int l = c + 1; l < LZ_KEEP; ++l)
+            if (l < k) {
+              double dot = 0.0;
+#pragma unroll
+              for (int i = 0; i < LZ_KEEP; ++i) dot += z[l][i] * w[i];
+#pragma unroll
+              for (int i = 0; i < LZ_KEEP; ++i) w[i] -= dot * z[l][i];
+            }
+        wn = 0.0;
+#pragma unroll
+        for (int i = 0; i < LZ_KEEP; ++i) wn += w[i] * w[i];
+        if (u == 0) be[c] = sqrt(wn);
+      }
+    }
+    const double f = 1.0 / sqrt(wn);
+    al[c] = 0.0;
+#pragma unroll
+    for (int i = 0; i < LZ_KEEP; ++i) {
+      z[c][i] = w[i] * f;
+      if (i < k) al[c] += th[i] * z[c][i] * z[c][i];
     }
   }
-  return cnt;
+  // the sign, from the largest component of the first vector
+  double big = 0.0, sg = 1.0;
+#pragma unroll
+  for (int i = 0; i < LZ_KEEP; ++i) {
+    const double y0 = __shfl(v[i], 0, 64);
+    if (i < k && fabs(z[0][i]) > big) {
+      big = fabs(z[0][i]);
+      sg = ((z[0][i] < 0.0) != (y0 < 0.0)) != (((m - k) & 1) != 0) ? -1.0 : 1.0;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < LZ_KEEP; ++c)
+    if (c < k) {
+      double q = 0.0;
+#pragma unroll
+      for (int i = 0; i < LZ_KEEP; ++i) q += v[i] * z[c][i];
+      if (lane < m) st.C[lane][c] = sg * q;
+      if (lane == 0) {
+        st.alpha[c] = al[c];
+        if (c + 1 < k) st.beta[c] = be[c];
+      }
+    }
+  if (lane < m) st.C[lane][k] = 0.0;
+  if (lane == 0) *sigma = beta_m * sg * sn;
+  return true;
 }
 
 // Implicit restart, solve part (one workgroup per solve, active solves
 // only), after a full cycle of m = ncv steps (V[m] is the normalised next
-// Lanczos vector, beta[m-1] its coefficient):
-//  1. the m - k largest Ritz values are the shifts: lane i bisects the
-//     Sturm count for eigenvalue k + i (a shift needs no more than ~1e-13
-//     relative accuracy: any shift gives a valid compressed factorisation,
-//     the exact ones remove the unwanted directions);
-//  2. lane 0 applies them as implicit QR steps to T = tridiag(alpha, beta)
-//     (a Givens bulge chase per shift, within the leading block when a
-//     subdiagonal entry has become negligible) and records the rotations;
-//  3. lane t < m accumulates row t of Q (the product of the rotations);
-//  4. the compressed factorisation: alpha[0..k), beta[0..k-1) from the
-//     rotated T, and the new residual direction
+// Lanczos vector, beta[m-1] its coefficient): the factorisation of length k
+// that implicit QR steps with the m - k largest Ritz values as shifts leave.
+//  1. wavefronts 0..k-1 find the k lowest Ritz pairs, and the new basis
+//     follows from them (restart_from_pairs);
+//  2. when Ritz values coincide to rounding, by the QR steps themselves:
+//     SH_LANES lanes search for eigenvalue k + i together, that many + 1
+//     parts a round (a shift needs no more than ~1e-13 relative accuracy: any
+//     shift gives a valid compressed factorisation); lane 0 applies the
+//     shifts to T = tridiag(alpha, beta) (a Givens bulge chase per shift,
+//     within the leading block when a subdiagonal entry has become
+//     negligible) in registers (statically indexed unrolled loops) and
+//     records the rotations; lane r (r < m) applies them to row r of the
+//     identity: the transformation Q;
+//  3. the new T (k x k) and the residual of the compressed factorisation
 //        r = bhat * V Q[:, k] + beta[m-1] Q[m-1, k-1] V[m],  beta[k-1] = |r|,
-//     give the coefficients C of the new basis rows 0..k (k_irl_apply).
-// The tridiagonal stays in registers (statically indexed unrolled loops) in
-// steps 1 and 2.  A residual that vanishes (an invariant subspace) ends the
-// solve as converged with its current Ritz pair.
+//     (bhat = 0 in case 1) give the coefficients C of the new basis rows
+//     0..k (k_irl_apply).
+// A residual that vanishes (an invariant subspace) ends the solve as
+// converged with its current Ritz pair.
+// Bound: latency, a few serial chains over m rows.  us for m = 20 (MI355X):
+// the QR steps with a library square root and one lane's bisection per shift
+// 164, with fast_rsqrt and SH_LANES lanes 103, from the Ritz pairs 20.5.
+constexpr int SH_LANES = 8;   // NT / NCV_MAX: every shift at once
 __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __restrict__ S,
                                                   int nsolve, void* state, int nchunks, int m,
                                                   int k) {
@@ -683,116 +821,140 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
     b_l[t] = st.beta[t];   // b[m-1]: coefficient of V[m]
   }
   __syncthreads();
-  const int np = m - k;
-  if (t < np) {
-    double a[NCV_MAX], e[NCV_MAX];
-    double lo = a_l[0], hi = a_l[0];
-#pragma unroll
-    for (int i = 0; i < NCV_MAX; ++i) {
-      a[i] = (i < m) ? a_l[i] : 0.0;
-      const double bi = (i < m - 1) ? b_l[i] : 0.0;
-      e[i] = bi * bi;
-      if (i < m) {
-        const double r = fabs(bi) + (i > 0 ? fabs(b_l[i - 1]) : 0.0);
-        lo = fmin(lo, a[i] - r);
-        hi = fmax(hi, a[i] + r);
-      }
-    }
-    const int idx = k + t;
-    for (int it = 0; it < 64; ++it) {
-      if (hi - lo <= 1e-13 * fmax(fabs(lo), fabs(hi)) + 1e-300) break;
-      const double mid = 0.5 * (lo + hi);
-      if (sturm_count_reg(a, e, m, mid) >= idx + 1) hi = mid;
-      else lo = mid;
-    }
-    sh[t] = 0.5 * (lo + hi);
+  __shared__ double yk[LZ_KEEP][NCV_MAX], thk[LZ_KEEP], tw[LZ_KEEP][TRI_WORK], sigma_s;
+  __shared__ int pairs_s;
+  static_assert(NT / 64 >= LZ_KEEP, "a wavefront per kept Ritz pair");
+  if (t / 64 < k) tridiag_pair(a_l, b_l, m, t / 64, yk[t / 64], &thk[t / 64], tw[t / 64]);
+  __syncthreads();
+  if (t < 64) {
+    const bool ok = restart_from_pairs(yk, thk, m, k, b_l[m - 1], st, &sigma_s);
+    if (t == 0) pairs_s = ok;
   }
   __syncthreads();
-  if (t == 0) {
-    double a[NCV_MAX], b[NCV_MAX];
-#pragma unroll
-    for (int i = 0; i < NCV_MAX; ++i) {
-      a[i] = (i < m) ? a_l[i] : 0.0;
-      b[i] = (i < m - 1) ? b_l[i] : 0.0;
-    }
-    for (int p = 0; p < np; ++p) {
-      int iend = m - 1;   // chase rows/cols 0..iend
-#pragma unroll
-      for (int u = NCV_MAX - 2; u >= 0; --u)
-        if (u < m - 1 && fabs(b[u]) <= 2.220446049250313e-16 * (fabs(a[u]) + fabs(a[u + 1])))
-          iend = u;   // the first negligible coupling from the top
-#pragma unroll
-      for (int u = 0; u < NCV_MAX - 1; ++u)
-        if (u == iend) b[u] = 0.0;
-      nrot[p] = iend;
-      double x = a[0] - sh[p], z = b[0], bulge = 0.0;
-#pragma unroll
-      for (int u = 0; u < NCV_MAX - 1; ++u) {
-        if (u < iend) {
-          // one reciprocal square root per rotation: the chase is a serial
-          // chain, and its entries are O(|T|), far from over- or underflow
-          double c = 1.0, sn = 0.0;
-          if (z != 0.0) {
-            const double ri = rsqrt(x * x + z * z);
-            c = x * ri;
-            sn = z * ri;
-          }
-          rc[p][u] = c;
-          rs[p][u] = sn;
-          if (u > 0) b[u - 1] = c * b[u - 1] + sn * bulge;
-          const double au = a[u], au1 = a[u + 1], bu = b[u];
-          a[u] = c * c * au + 2.0 * c * sn * bu + sn * sn * au1;
-          a[u + 1] = sn * sn * au - 2.0 * c * sn * bu + c * c * au1;
-          b[u] = c * sn * (au1 - au) + (c * c - sn * sn) * bu;
-          if (u + 1 < iend) {
-            bulge = sn * b[u + 1];
-            b[u + 1] = c * b[u + 1];
-            x = b[u];
-            z = bulge;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < LZ_KEEP; ++i) {
-      ak[i] = a[i];
-      bk[i] = b[i];
-    }
-  }
-  __syncthreads();
+  const bool pairs = pairs_s != 0;
   double q[NCV_MAX];   // row t of Q (static indices: kept in registers)
-#pragma unroll
-  for (int c = 0; c < NCV_MAX; ++c) q[c] = (c == t) ? 1.0 : 0.0;
-  if (t < m) {
-    for (int p = 0; p < np; ++p) {
-      const int n = nrot[p];
-#pragma unroll
-      for (int u = 0; u < NCV_MAX - 1; ++u) {
-        if (u < n) {
-          const double c = rc[p][u], sn = rs[p][u];
-          const double q0 = q[u], q1 = q[u + 1];
-          q[u] = c * q0 + sn * q1;
-          q[u + 1] = -sn * q0 + c * q1;
+  if (!pairs) {
+    const int np = m - k;
+    __shared__ double as_l[NCV_MAX], b2_l[NCV_MAX];
+    double lo = a_l[0], hi = a_l[0];
+    for (int i = 0; i < m; ++i) {
+      const double r = (i < m - 1 ? fabs(b_l[i]) : 0.0) + (i > 0 ? fabs(b_l[i - 1]) : 0.0);
+      lo = fmin(lo, a_l[i] - r);
+      hi = fmax(hi, a_l[i] + r);
+    }
+    // entries relative to the lower bound, over a power of two near the span
+    const int ex = __builtin_amdgcn_frexp_exp(fmax(hi - lo, 1e-300));
+    const double base = lo, amax = fmax(fabs(lo), fabs(hi));
+    if (t < m) {
+      as_l[t] = __builtin_amdgcn_ldexp(a_l[t] - base, -ex);
+      const double bs = t < m - 1 ? __builtin_amdgcn_ldexp(b_l[t], -ex) : 0.0;
+      b2_l[t] = bs * bs;
+    }
+    __syncthreads();
+    {
+      const int i = t / SH_LANES, l = t % SH_LANES, idx = k + i;
+      const double stop = __builtin_amdgcn_ldexp(1e-13 * amax, -ex) + 1e-300;
+      double x0 = 0.0, x1 = __builtin_amdgcn_ldexp(hi - base, -ex);
+      if (i < np) {
+        for (int it = 0; it < 20 && x1 - x0 > stop; ++it) {
+          const double w = (x1 - x0) * (1.0 / (SH_LANES + 1));
+          const bool above = count_below(as_l, b2_l, m, x0 + w * (double)(l + 1)) >= idx + 1;
+          // the group's lanes of the ballot: points from the first `above` on
+          const unsigned msk = (unsigned)(__ballot(above) >> ((t & 63) - l)) & ((1u << SH_LANES) - 1);
+          const int f = msk ? __ffs((int)msk) : SH_LANES + 1;
+          const double o = x0;
+          x0 = o + w * (double)(f - 1);
+          if (f <= SH_LANES) x1 = o + w * (double)f;
         }
+        if (l == 0) sh[i] = base + __builtin_amdgcn_ldexp(0.5 * (x0 + x1), ex);
       }
     }
-    if (t == m - 1) {
+    __syncthreads();
+    if (t == 0) {
+      double a[NCV_MAX], b[NCV_MAX];
 #pragma unroll
-      for (int c = 0; c < NCV_MAX; ++c)
-        if (c == k - 1) qmk = q[c];
+      for (int i = 0; i < NCV_MAX; ++i) {
+        a[i] = (i < m) ? a_l[i] : 0.0;
+        b[i] = (i < m - 1) ? b_l[i] : 0.0;
+      }
+      for (int p = 0; p < np; ++p) {
+        int iend = m - 1;   // chase rows/cols 0..iend
+#pragma unroll
+        for (int u = NCV_MAX - 2; u >= 0; --u)
+          if (u < m - 1 && fabs(b[u]) <= 2.220446049250313e-16 * (fabs(a[u]) + fabs(a[u + 1])))
+            iend = u;   // the first negligible coupling from the top
+#pragma unroll
+        for (int u = 0; u < NCV_MAX - 1; ++u)
+          if (u == iend) b[u] = 0.0;
+        nrot[p] = iend;
+        double x = a[0] - sh[p], z = b[0], bulge = 0.0;
+#pragma unroll
+        for (int u = 0; u < NCV_MAX - 1; ++u) {
+          if (u < iend) {
+            // one reciprocal square root per rotation: the chase is a serial
+            // chain, and its entries are O(|T|), far from over- or underflow
+            double c = 1.0, sn = 0.0;
+            if (z != 0.0) {
+              const double ri = fast_rsqrt(x * x + z * z);
+              c = x * ri;
+              sn = z * ri;
+            }
+            rc[p][u] = c;
+            rs[p][u] = sn;
+            if (u > 0) b[u - 1] = c * b[u - 1] + sn * bulge;
+            const double au = a[u], au1 = a[u + 1], bu = b[u];
+            a[u] = c * c * au + 2.0 * c * sn * bu + sn * sn * au1;
+            a[u + 1] = sn * sn * au - 2.0 * c * sn * bu + c * c * au1;
+            b[u] = c * sn * (au1 - au) + (c * c - sn * sn) * bu;
+            if (u + 1 < iend) {
+              bulge = sn * b[u + 1];
+              b[u + 1] = c * b[u + 1];
+              x = b[u];
+              z = bulge;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < LZ_KEEP; ++i) {
+        ak[i] = a[i];
+        bk[i] = b[i];
+      }
     }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NCV_MAX; ++c) q[c] = (c == t) ? 1.0 : 0.0;
+    if (t < m) {
+      for (int p = 0; p < np; ++p) {
+        const int n = nrot[p];
+#pragma unroll
+        for (int u = 0; u < NCV_MAX - 1; ++u) {
+          if (u < n) {
+            const double c = rc[p][u], sn = rs[p][u];
+            const double q0 = q[u], q1 = q[u + 1];
+            q[u] = c * q0 + sn * q1;
+            q[u + 1] = -sn * q0 + c * q1;
+          }
+        }
+      }
+      if (t == m - 1) {
+#pragma unroll
+        for (int c = 0; c < NCV_MAX; ++c)
+          if (c == k - 1) qmk = q[c];
+      }
+    }
+    __syncthreads();
   }
-  __syncthreads();
   if (t == 0) {
-    const double bhat = bk[k - 1];
-    const double sigma = st.beta[m - 1] * qmk;
+    const double bhat = pairs ? 0.0 : bk[k - 1];
+    const double sigma = pairs ? sigma_s : b_l[m - 1] * qmk;
     const double rho = hypot(bhat, sigma);
     bhat_s = bhat;
     rho_s = rho;
     double anorm = 0.0;
     for (int u = 0; u < m; ++u) anorm = fmax(anorm, fabs(a_l[u]) + fabs(b_l[u]));
-    for (int u = 0; u < k; ++u) st.alpha[u] = ak[u];
-    for (int u = 0; u + 1 < k; ++u) st.beta[u] = bk[u];
+    for (int u = 0; u < k && !pairs; ++u) st.alpha[u] = ak[u];
+    for (int u = 0; u + 1 < k && !pairs; ++u) st.beta[u] = bk[u];
     st.beta[k - 1] = rho;
     st.restarts += 1;
     for (int u = 0; u <= k; ++u) st.C[m][u] = 0.0;
@@ -805,7 +967,7 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
     }
   }
   __syncthreads();
-  if (t < m) {
+  if (t < m && !pairs) {
     const double f = rho_s > 0.0 ? bhat_s / rho_s : 0.0;
 #pragma unroll
     for (int c = 0; c < NCV_MAX; ++c) {

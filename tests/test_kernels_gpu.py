@@ -1100,3 +1100,64 @@ def test_fill_normal_stream(gpu):
     assert np.allclose(x[:256], ref, rtol=1e-14, atol=1e-14)
     ref = np.array([normal((1 << 40) + 99, far + g) for g in range(64)])
     assert np.allclose(d.cpu().numpy(), ref, rtol=1e-14, atol=1e-14)
+
+
+@pytest.mark.parametrize('ncv,low', [(2, -2.0), (3, -2.0), (5, -2.0), (20, -2.0), (32, -0.15),
+                                     (20, None)])
+def test_lanczos_restart_lengths(gpu, ncv, low):
+    """Implicit restarts at the shortest and longest cycles (1 to 4 kept
+    vectors), and (low None) of a chain whose leading 20 x 20 block has two of its
+    four lowest eigenvalues equal to rounding, in two wells, below a lowest
+    one that is not converged: those vectors are not independent, and the
+    restart after 20 steps falls back to the shifted QR steps.  Against
+    numpy.linalg.eigh: the residual test's 1e-10 / 1e-4 = 1e-6 (times 1 +
+    1e-4 |theta|) gives the Ritz value to 1e-6 ** 2 / gap (at least 0.1)."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    rng = np.random.RandomState(3)
+    pair = low is None
+    if pair:
+        n = 64
+        d = np.zeros(n)
+        d[[3, 10]] = -200.7
+        d[17:24] = -200.5
+        H = np.diag(d) + 0.3 * (np.eye(n, k=1) + np.eye(n, k=-1))
+        ev = np.linalg.eigvalsh(H[:20, :20])
+        assert ev[1] - ev[0] > 0.1 and ev[2] - ev[1] < 2e-13
+        v0 = np.eye(n)[0]
+    else:
+        n = 200
+        d = np.concatenate([[low], np.linspace(0.0, 10.0, n - 1)])
+        Q, _ = np.linalg.qr(rng.randn(n, n))
+        H = (Q * d) @ Q.T
+        H = (H + H.T) / 2
+        v0 = rng.randn(n)
+    e, U = np.linalg.eigh(H)
+    assert e[1] - e[0] > 0.1
+    Hd, init = _dev(H), _dev(v0)
+    V = torch.zeros((ncv + 1) * n, dtype=torch.float64, device='cuda')
+    w, x, out = (torch.zeros(n, dtype=torch.float64, device='cuda') for _ in range(3))
+    g2 = R.GemmList()
+    g2.add(w.data_ptr(), n, 1, 1, [(Hd.data_ptr(), n, 0, x.data_ptr(), 1, 0, n, 1.0)], active=0)
+    lz = L.lanczos_records([(V.data_ptr(), w.data_ptr(), x.data_ptr(), init.data_ptr(),
+                             out.data_ptr(), n, n, 0, 0, 1e-10 / 1e-4, 1e-4, 0.0, 0, 0)])
+    p, s = g2.arrays()
+    dp, ds, dlz = _upload([p, s, lz])
+    plan = L.MatvecPlan(0, 0, 0, 0, 0, 0, 0, 0, dp.data_ptr(), ds.data_ptr(), len(p),
+                        R.gemm_tiles(p), 0, 0, 0)
+    state = torch.zeros(int(lib.tnx_lanczos_state_bytes(1, 1, ncv)), dtype=torch.uint8,
+                        device='cuda')
+    res = np.zeros(1, dtype=L.LANCZOS_RESULT)
+    print('lanczos restart ncv', ncv, 'low', low, flush=True)
+    rc = lib.tnx_lanczos_run_ex(plan, _vp(dlz.data_ptr()), 1, 1, ncv, 400, ncv if pair else 1,
+                                0, 0, _vp(state.data_ptr()), _vp(res.ctypes.data), _stream())
+    assert rc == 0, (rc, lib.tnx_last_error(), res)
+    v = out.cpu().numpy()
+    assert res[0]['iters'] > ncv
+    assert abs(res[0]['theta'] - e[0]) < 1e-9 * abs(e[0]), (res, e[0])
+    assert abs(np.linalg.norm(v) - 1) < 1e-12
+    assert np.linalg.norm(H @ v - res[0]['theta'] * v) < 2e-6
+    # residual over the gap bounds the part outside the lowest eigenvector
+    assert abs(abs(v @ U[:, 0]) - 1) < (2e-6 / (e[1] - e[0])) ** 2
