@@ -29,8 +29,11 @@
 namespace {
 
 constexpr int NCV_MAX = 32;
-constexpr int CHUNK = 1024;  // 256 lanes x 4 elements
-constexpr int NT = 256;
+constexpr int CHUNK = 1024;
+constexpr int NP = 512;           // lanes of the kernels over a chunk
+constexpr int EPT = CHUNK / NP;   // elements of a lane
+constexpr int NW = NP / 64;
+constexpr int NT = 256;           // lanes of the restart's solve
 constexpr int LZ_KEEP = 4;   // vectors kept by an implicit restart (at most)
 constexpr double LZ_REORTH_SKIP = 1e-12;   // second projection left out below this (relative)
 constexpr double LZ_REORTH_SKIP_F32 = 1e-6;  // the same for an f32 basis (its rounding level)
@@ -50,9 +53,11 @@ struct LzState {
 // Vectors an implicit restart keeps for a call with ncv Krylov vectors.
 __host__ __device__ inline int lz_keep(int ncv) { return ncv - 1 < LZ_KEEP ? ncv - 1 : LZ_KEEP; }
 
-// partA / partB: per-chunk partial sums, [nchunks][NCV_MAX + 1].  Passes that
-// follow each other alternate between them (a kernel reads one while it
-// writes the other).
+// partA / partB: per-chunk partial sums, [NCV_MAX + 1][nchunks] (a solve's
+// partials of one sum are consecutive).  Passes that follow each other
+// alternate between them (a kernel reads one while it writes the other).
+// nact[0]: active solves; nact[1]: eigensolve blocks of the running
+// k_update_norm that are done.
 struct LzLayout {
   LzState* st;
   int32_t* act;
@@ -99,96 +104,147 @@ __device__ __forceinline__ ChunkInfo chunk_of(const tnx_lanczos_solve* solves, i
   return ci;
 }
 
-// Wavefront sum of s into red[wave][k] (a block sum is red[0..3][k] after a
-// barrier).
-__device__ __forceinline__ void wave_to_lds(double s, int k, double (*red)[NCV_MAX + 1]) {
-  s = tnx_wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = s;
+typedef double (*Red)[NCV_MAX + 1];   // wavefront sums, red[wave][k]
+
+// R = 4, 8 or 16 sums over the wavefront at once, of v[0..R), into
+// red[k0..k0 + R).  Each step of the butterfly halves the sums a lane carries
+// as well as the lanes that share one: the exchange moves one value of a pair
+// each way.  63 instructions for 16 sums, where 16 butterflies take 288.
+template <int R> __device__ __forceinline__ void wave_sums(const double* v, int k0, double* red) {
+  const int lane = threadIdx.x & 63;
+  double s[R / 2];
+#pragma unroll
+  for (int u = 0; u < R / 2; ++u) {
+    double p = v[u], q = v[u + R / 2];
+    tnx_swap<true>(p, q);
+    s[u] = p + q;
+  }
+#pragma unroll
+  for (int u = 0; u < R / 4; ++u) {
+    double p = s[u], q = s[u + R / 4];
+    tnx_swap<false>(p, q);
+    s[u] = p + q;
+  }
+  int k = (lane >> 5) * (R / 2) + ((lane >> 4) & 1) * (R / 4);
+  if constexpr (R >= 8) {
+    const bool up = lane & 8;
+#pragma unroll
+    for (int u = 0; u < R / 8; ++u) {
+      const double keep = up ? s[u + R / 8] : s[u], give = up ? s[u] : s[u + R / 8];
+      s[u] = keep + tnx_row_get<0x128>(give);
+    }
+    k += up ? R / 8 : 0;
+  } else {
+    s[0] += tnx_row_get<0x128>(s[0]);
+  }
+  if constexpr (R == 16) {   // 0x141: lane ^ 7, the other half of the 8 lanes
+    const bool up = lane & 4;
+    const double keep = up ? s[1] : s[0], give = up ? s[0] : s[1];
+    s[0] = keep + tnx_row_get<0x141>(give);
+    k += up ? 1 : 0;
+  } else {
+    s[0] += tnx_row_get<0x141>(s[0]);
+  }
+  s[0] += tnx_row_get<0x4e>(s[0]);   // lane ^ 2, then lane ^ 1
+  s[0] += tnx_row_get<0xb1>(s[0]);
+  if ((lane & (64 / R - 1)) == 0) red[k0 + k] = s[0];
+}
+// L sums (a multiple of 4, up to 32)
+template <int L> __device__ __forceinline__ void wave_sums_all(const double (&v)[L], double* red) {
+  constexpr int A = L & 16, B = L & 8;
+  if constexpr (L == 32) wave_sums<16>(v + 16, 16, red);
+  if constexpr (L >= 16) wave_sums<16>(v, 0, red);
+  if constexpr (L < 32 && B != 0) wave_sums<8>(v + A, A, red);
+  if constexpr ((L & 4) != 0) wave_sums<4>(v + A + B, A + B, red);
 }
 
-// Partial dots V[k] . x over this chunk for k = 0..j, wave sums into
-// red[wave][k].  Rows are taken four at a time so their loads are in flight
-// together (the loop is latency bound otherwise).
-template <typename VT>
-__device__ __forceinline__ void chunk_dots(const VT* __restrict__ V, int ldv, int j, int i0,
-                                           int i1, const double (&x)[CHUNK / NT],
-                                           double (*red)[NCV_MAX + 1]) {
-  for (int k0 = 0; k0 <= j; k0 += 4) {
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
+// sum of the NW wavefronts' entries k
+__device__ __forceinline__ double red_total(const double (*red)[NCV_MAX + 1], int k) {
+  return ((red[0][k] + red[1][k]) + (red[2][k] + red[3][k])) +
+         ((red[4][k] + red[5][k]) + (red[6][k] + red[7][k]));
+}
+
+// Elements of lane t of a chunk: i0 + t, i0 + t + NP.  elem: the element's
+// index, that of the chunk's last element past its end.
+__device__ __forceinline__ int elem(const ChunkInfo& ci, int q) {
+  return min(ci.i0 + q * NP + (int)threadIdx.x, ci.i1 - 1);
+}
+__device__ __forceinline__ bool inside(const ChunkInfo& ci, int q) {
+  return ci.i0 + q * NP + (int)threadIdx.x < ci.i1;
+}
+
+// This chunk's elements of L basis rows, row min(u, j) for u = 0..L - 1, all
+// loads in flight together.
+template <typename VT, int L>
+__device__ __forceinline__ void load_rows(const VT TNX_GLOBAL* V, int ldv, int j,
+                                          const ChunkInfo& ci, VT (&v)[L][EPT]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = k0 + u;
-      if (k <= j) {
-        const VT* row = V + (int64_t)k * ldv;
+  for (int u = 0; u < L; ++u) {
+    const VT TNX_GLOBAL* row = V + (int64_t)min(u, j) * ldv;
 #pragma unroll
-        for (int q = 0; q < CHUNK / NT; ++q) {
-          const int i = i0 + q * NT + threadIdx.x;
-          if (i < i1) s[u] += (double)row[i] * x[q];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (k0 + u <= j) wave_to_lds(s[u], k0 + u, red);
+    for (int q = 0; q < EPT; ++q) v[u][q] = row[elem(ci, q)];
   }
+}
+
+// Dots of the L rows with x (zero past the chunk's end), wavefront sums into
+// red[wave].
+template <typename VT, int L>
+__device__ __forceinline__ void rows_dots(const VT (&v)[L][EPT], const double (&x)[EPT], Red red) {
+  double s[L];
+#pragma unroll
+  for (int u = 0; u < L; ++u) {
+    s[u] = 0.0;
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) s[u] += (double)v[u][q] * x[q];
+  }
+  wave_sums_all(s, red[threadIdx.x >> 6]);
 }
 
 // x -= sum_{k<=j} h[k] V[k] over this chunk (rows four at a time).
 template <typename VT>
-__device__ __forceinline__ void chunk_axpy(const VT* __restrict__ V, int ldv, int j, int i0,
-                                           int i1, const double* h, double (&x)[CHUNK / NT]) {
+__device__ __forceinline__ void chunk_axpy(const VT TNX_GLOBAL* V, int ldv, int j,
+                                           const ChunkInfo& ci, const double* h,
+                                           double (&x)[EPT]) {
   for (int k0 = 0; k0 <= j; k0 += 4) {
-    double v[4][CHUNK / NT];
+    double v[4][EPT];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < EPT; ++q)
+        v[u][q] = (double)V[(int64_t)min(k0 + u, j) * ldv + elem(ci, q)];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int k = k0 + u;
-      const VT* row = V + (int64_t)(k <= j ? k : j) * ldv;
+      const double hk = k0 + u <= j ? h[min(k0 + u, j)] : 0.0;
 #pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) {
-        const int i = i0 + q * NT + threadIdx.x;
-        v[u][q] = (k <= j && i < i1) ? (double)row[i] : 0.0;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int kk = (k0 + u <= j) ? k0 + u : j;
-      const double hk = (k0 + u <= j) ? h[kk] : 0.0;
-#pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) x[q] -= hk * v[u][q];
+      for (int q = 0; q < EPT; ++q) x[q] -= hk * v[u][q];
     }
   }
 }
 
-// Block-wide sum of one value per thread into red[0..3][0].
-__device__ __forceinline__ void block_sums(const double* v, int nv, double (*red)[NCV_MAX + 1]) {
-  (void)nv;
-  wave_to_lds(v[0], 0, red);
-  __syncthreads();
-}
-
 // Sum the partials of one solve (chunks [chunk_begin, chunk_begin + nch))
-// for k in [0, nk) into dst[k] (all NT lanes; dst is read after a barrier).
-// The partials were written by the previous kernel on the stream.  Wave w
-// sums the entries k = w, w + 4, ...: its 64 lanes stride over the chunks
-// and four entries are read per pass, so the loads are in flight together.
-// The summation order depends only on nch, so every block of a solve gets
-// the same bits.
-__device__ __forceinline__ void reduce_partials(const double* part, int chunk_begin, int nch,
-                                                int nk, double* dst) {
+// for k in [0, nk) into dst[k], zeros for k in [nk, npad) (all NP lanes; dst
+// is read after a barrier).  The partials were written by the previous kernel
+// on the stream.  Wave w sums the entries k = w, w + NW, ...: its 64 lanes
+// stride over the chunks and four entries are read per pass, so the loads are
+// in flight together.  The summation order depends only on nch, so every
+// block of a solve gets the same bits.
+__device__ __forceinline__ void reduce_partials(const double* part, int nchunks, int chunk_begin,
+                                                int nch, int nk, int npad, double* dst) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int k0 = wave; k0 < nk; k0 += 16) {
+  __shared__ double out[NW][4];
+  const double TNX_GLOBAL* p = as_global<const double>((uint64_t)part) + chunk_begin;
+  for (int k0 = wave; k0 < npad; k0 += 4 * NW) {
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c = lane; c < nch; c += 64) {
-      const double* p = part + (int64_t)(chunk_begin + c) * (NCV_MAX + 1);
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (k0 + 4 * u < nk) s[u] += p[k0 + 4 * u];
+      for (int u = 0; u < 4; ++u) {
+        const int k = k0 + u * NW;
+        s[u] += k < nk ? p[(int64_t)min(k, nk - 1) * nchunks + c] : 0.0;
+      }
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const double v = tnx_wave_sum(s[u]);
-      if (lane == 0 && k0 + 4 * u < nk) dst[k0 + 4 * u] = v;
-    }
+    wave_sums<4>(s, 0, out[wave]);
+    __builtin_amdgcn_wave_barrier();
+    if (lane < 4 && k0 + lane * NW < npad) dst[k0 + lane * NW] = out[wave][lane];
   }
 }
 
@@ -330,12 +386,6 @@ __device__ __forceinline__ int dtype_of(int call_dtype, int32_t own) {
 
 // ---------------------------------------------------------------- kernels
 
-// Block sum of one value per thread (all NT lanes; result in every lane).
-__device__ __forceinline__ double block_total(double v, double (*red)[NCV_MAX + 1]) {
-  block_sums(&v, 1, red);
-  return (red[0][0] + red[1][0]) + (red[2][0] + red[3][0]);
-}
-
 // act[s], read once per block through LDS: block 0 of a solve may clear it
 // while the solve's other blocks run k_update_norm, and every lane of a block
 // must take the same early return.
@@ -346,65 +396,101 @@ __device__ __forceinline__ bool solve_active(const int32_t* act, int s) {
   return a != 0;
 }
 
-// chunk partial of ||init||^2 -> partA[block][0]
-__global__ __launch_bounds__(NT) void k_init_norm(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+// chunk partial of ||init||^2 -> partA[0][chunk]
+__global__ __launch_bounds__(NP) void k_init_norm(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                                   void* state, int nchunks) {
   LzLayout L = lz_layout(state, nsolve, nchunks);
   ChunkInfo ci = chunk_of(S, nsolve);
   const tnx_lanczos_solve D = S[ci.s];
-  const double* v = (const double*)D.init;
+  const double TNX_GLOBAL* v = as_global<const double>(D.init);
   double acc = 0.0;
-  for (int i = ci.i0 + threadIdx.x; i < ci.i1; i += NT) acc += v[i] * v[i];
-  __shared__ double red[4][NCV_MAX + 1];
-  const double tot = block_total(acc, red);
-  if (threadIdx.x == 0) L.partA[(int64_t)blockIdx.x * (NCV_MAX + 1)] = tot;
+  for (int q = 0; q < EPT; ++q)
+    if (inside(ci, q)) acc += v[elem(ci, q)] * v[elem(ci, q)];
+  __shared__ double red[NW][NCV_MAX + 1];
+  acc = tnx_wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][0] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) L.partA[blockIdx.x] = red_total(red, 0);
 }
 
 // scale = 1 / ||init|| (summed by every block); V[0] = init * scale (a flat
 // vector when init == 0); x = cast(V[0]).  Block 0 of the solve resets the
 // solve's state and marks it active.
-__global__ __launch_bounds__(NT) void k_init_scale(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+__global__ __launch_bounds__(NP) void k_init_scale(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                                    void* state, int nchunks, int x_dtype) {
   LzLayout L = lz_layout(state, nsolve, nchunks);
   ChunkInfo ci = chunk_of(S, nsolve);
   const tnx_lanczos_solve D = S[ci.s];
   __shared__ double tot;
-  reduce_partials(L.partA, D.chunk_begin, ci.nch, 1, &tot);
+  reduce_partials(L.partA, nchunks, D.chunk_begin, ci.nch, 1, 1, &tot);
   __syncthreads();
   const double sc = tot > 0.0 ? 1.0 / sqrt(tot) : -1.0;
-  if (ci.c == 0 && threadIdx.x == 0) {
+  if (ci.c == 0 && threadIdx.x < NCV_MAX) {
     LzState& st = L.st[ci.s];
-    st.scale = sc;
-    st.converged = 0;
-    st.iters = 0;
-    st.jlast = 0;
-    st.restarts = 0;
-    st.theta = 0.0;
-    st.resid = 0.0;
-    st.y[0] = 1.0;
-    for (int k = 1; k < NCV_MAX; ++k) st.y[k] = 0.0;
-    L.act[ci.s] = 1;
+    st.y[threadIdx.x] = threadIdx.x == 0 ? 1.0 : 0.0;
+    if (threadIdx.x == 0) {
+      st.scale = sc;
+      st.converged = 0;
+      st.iters = 0;
+      st.jlast = 0;
+      st.restarts = 0;
+      st.theta = 0.0;
+      st.resid = 0.0;
+      L.act[ci.s] = 1;
+    }
   }
-  const double* v = (const double*)D.init;
+  const double TNX_GLOBAL* v = as_global<const double>(D.init);
   const double flat = 1.0 / sqrt((double)D.n);
   const int xd = dtype_of(x_dtype, D.x_dtype);
   const bool vf = D.v_dtype == TNX_F32;
-  for (int i = ci.i0 + threadIdx.x; i < ci.i1; i += NT) {
+  for (int q = 0; q < EPT; ++q) {
+    if (!inside(ci, q)) continue;
+    const int i = elem(ci, q);
     double val = sc > 0.0 ? v[i] * sc : flat;
     if (vf) {
       // the basis row as stored: the start vector rounded to f32
       const float vv = (float)val;
-      ((float*)D.V)[i] = vv;
+      as_global<float>(D.V)[i] = vv;
       val = (double)vv;
     } else {
-      ((double*)D.V)[i] = val;
+      as_global<double>(D.V)[i] = val;
     }
     tnx_store((void*)D.x, xd, i, val);
   }
 }
 
-// pass 1: chunk partials of V[k] . w, k <= j -> partA
-__global__ __launch_bounds__(NT) void k_dots(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+// The two projections of a Krylov step (k_dots, k_update_dots) hold the
+// chunk's part of all basis rows in registers: LV >= j + 1 rows (a multiple
+// of 4, chosen by the host), so every load is issued before the first is
+// used, and the second projection reads nothing again.
+// Bound: latency at a few chunks, else the basis rows' bandwidth.
+// us a call, dots and update/dots, f64 basis, mean over the cycles of 20
+// (MI355X): one solve of 2 chunks 8.7 + 11.3 with 256 lanes, generic pointers,
+// rows four at a time and a butterfly per sum, now 3.5 + 4.7; 16 solves of 32
+// chunks 21 + 27, now 9 + 11.
+
+// chunk partials of V[k] . w, k <= j -> partA
+template <typename VT, int LV>
+__device__ __forceinline__ void dots_body(const tnx_lanczos_solve& D, const LzLayout& L,
+                                          const ChunkInfo& ci, int nchunks, int j, int wd) {
+  __shared__ double red[NW][NCV_MAX + 1];
+  VT v[LV][EPT];
+  load_rows(as_global<const VT>(D.V), D.ldv, j, ci, v);
+  double w[EPT];
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    w[q] = tnx_load((const void*)D.w, wd, elem(ci, q));
+    if (!inside(ci, q)) w[q] = 0.0;
+  }
+  rows_dots(v, w, red);
+  __syncthreads();
+  if ((int)threadIdx.x <= j)
+    L.partA[(int64_t)threadIdx.x * nchunks + blockIdx.x] = red_total(red, threadIdx.x);
+}
+
+// pass 1
+template <int LV>
+__global__ __launch_bounds__(NP) void k_dots(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                              void* state, int nchunks, int j, int w_dtype,
                                              unsigned long long* ts) {
   tnx_stamp_begin(ts);
@@ -413,24 +499,60 @@ __global__ __launch_bounds__(NT) void k_dots(const tnx_lanczos_solve* __restrict
   if (L.act[ci.s] == 0) return;
   const tnx_lanczos_solve D = S[ci.s];
   const int wd = dtype_of(w_dtype, D.w_dtype);
-  double w[CHUNK / NT];
-#pragma unroll
-  for (int q = 0; q < CHUNK / NT; ++q) {
-    int i = ci.i0 + q * NT + threadIdx.x;
-    w[q] = (i < ci.i1) ? tnx_load((const void*)D.w, wd, i) : 0.0;
-  }
-  __shared__ double red[4][NCV_MAX + 1];
-  if (D.v_dtype == TNX_F32) chunk_dots((const float*)D.V, D.ldv, j, ci.i0, ci.i1, w, red);
-  else chunk_dots((const double*)D.V, D.ldv, j, ci.i0, ci.i1, w, red);
-  __syncthreads();
-  for (int k = threadIdx.x; k <= j; k += NT)
-    L.partA[(int64_t)blockIdx.x * (NCV_MAX + 1) + k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  if (D.v_dtype == TNX_F32) dots_body<float, LV>(D, L, ci, nchunks, j, wd);
+  else dots_body<double, LV>(D, L, ci, nchunks, j, wd);
   tnx_stamp_end(ts);
 }
 
 // h1 = sum of the pass-1 partials; r = w - sum h1[k] V[k] -> V[j+1];
-// pass 2: chunk partials of V[k] . r (k <= j) and of ||r||^2 (slot j+1) -> partB
-__global__ __launch_bounds__(NT) void k_update_dots(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+// pass 2: chunk partials of V[k] . r (k <= j) and of ||r||^2 (slot j+1) -> partB.
+// With an f32 basis r (kept in f64 registers for its dots and norm) is parked
+// in row j+1 rounded to f32; the next pass normalises the parked row.
+template <typename VT, int LV>
+__device__ __forceinline__ void update_dots_body(const tnx_lanczos_solve& D, const LzLayout& L,
+                                                 const ChunkInfo& ci, int nchunks, int j, int wd) {
+  __shared__ double red[NW][NCV_MAX + 1];
+  __shared__ double h[NCV_MAX + 1];
+  VT v[LV][EPT];
+  load_rows(as_global<const VT>(D.V), D.ldv, j, ci, v);
+  double r[EPT];
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    r[q] = tnx_load((const void*)D.w, wd, elem(ci, q));
+    if (!inside(ci, q)) r[q] = 0.0;
+  }
+  reduce_partials(L.partA, nchunks, D.chunk_begin, ci.nch, j + 1, LV, h);
+  __syncthreads();
+  if (ci.c == 0 && (int)threadIdx.x <= j) L.st[ci.s].h1[threadIdx.x] = h[threadIdx.x];
+#pragma unroll
+  for (int u = 0; u < LV; ++u) {
+    const double hu = h[u];
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) r[q] -= hu * (double)v[u][q];
+  }
+  VT TNX_GLOBAL* Vn = as_global<VT>(D.V) + (int64_t)(j + 1) * D.ldv;
+  double nn = 0.0;  // ||r||^2
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    if (inside(ci, q)) Vn[elem(ci, q)] = (VT)r[q];
+    else r[q] = 0.0;
+    nn += r[q] * r[q];
+  }
+  rows_dots(v, r, red);
+  nn = tnx_wave_sum(nn);
+  __shared__ double rn[NW];
+  if ((threadIdx.x & 63) == 0) rn[threadIdx.x >> 6] = nn;
+  __syncthreads();
+  if ((int)threadIdx.x <= j) {
+    L.partB[(int64_t)threadIdx.x * nchunks + blockIdx.x] = red_total(red, threadIdx.x);
+  } else if ((int)threadIdx.x == j + 1) {
+    L.partB[(int64_t)threadIdx.x * nchunks + blockIdx.x] =
+        ((rn[0] + rn[1]) + (rn[2] + rn[3])) + ((rn[4] + rn[5]) + (rn[6] + rn[7]));
+  }
+}
+
+template <int LV>
+__global__ __launch_bounds__(NP) void k_update_dots(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                                     void* state, int nchunks, int j, int w_dtype,
                                                     unsigned long long* ts) {
   tnx_stamp_begin(ts);
@@ -438,50 +560,83 @@ __global__ __launch_bounds__(NT) void k_update_dots(const tnx_lanczos_solve* __r
   ChunkInfo ci = chunk_of(S, nsolve);
   if (L.act[ci.s] == 0) return;
   const tnx_lanczos_solve D = S[ci.s];
-  __shared__ double h[NCV_MAX + 1];
-  reduce_partials(L.partA, D.chunk_begin, ci.nch, j + 1, h);
-  __syncthreads();
-  if (ci.c == 0)
-    for (int k = threadIdx.x; k <= j; k += NT) L.st[ci.s].h1[k] = h[k];
   const int wd = dtype_of(w_dtype, D.w_dtype);
-  double r[CHUNK / NT];
-#pragma unroll
-  for (int q = 0; q < CHUNK / NT; ++q) {
-    int i = ci.i0 + q * NT + threadIdx.x;
-    r[q] = (i < ci.i1) ? tnx_load((const void*)D.w, wd, i) : 0.0;
-  }
-  __shared__ double red[4][NCV_MAX + 1];
-  if (D.v_dtype == TNX_F32) {
-    // r (kept in f64 registers for its dots and norm) is parked in row j+1
-    // rounded to f32; the next pass normalises the parked row
-    const float* V = (const float*)D.V;
-    chunk_axpy(V, D.ldv, j, ci.i0, ci.i1, h, r);
-    float* Vn = (float*)D.V + (int64_t)(j + 1) * D.ldv;
-#pragma unroll
-    for (int q = 0; q < CHUNK / NT; ++q) {
-      int i = ci.i0 + q * NT + threadIdx.x;
-      if (i < ci.i1) Vn[i] = (float)r[q];
-    }
-    chunk_dots(V, D.ldv, j, ci.i0, ci.i1, r, red);
-  } else {
-    const double* V = (const double*)D.V;
-    chunk_axpy(V, D.ldv, j, ci.i0, ci.i1, h, r);
-    double* Vn = (double*)D.V + (int64_t)(j + 1) * D.ldv;
-#pragma unroll
-    for (int q = 0; q < CHUNK / NT; ++q) {
-      int i = ci.i0 + q * NT + threadIdx.x;
-      if (i < ci.i1) Vn[i] = r[q];
-    }
-    chunk_dots(V, D.ldv, j, ci.i0, ci.i1, r, red);
-  }
-  double nn = 0.0;  // ||r||^2 (r is zero past the chunk end)
-#pragma unroll
-  for (int q = 0; q < CHUNK / NT; ++q) nn += r[q] * r[q];
-  wave_to_lds(nn, j + 1, red);
-  __syncthreads();
-  for (int k = threadIdx.x; k <= j + 1; k += NT)
-    L.partB[(int64_t)blockIdx.x * (NCV_MAX + 1) + k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  if (D.v_dtype == TNX_F32) update_dots_body<float, LV>(D, L, ci, nchunks, j, wd);
+  else update_dots_body<double, LV>(D, L, ci, nchunks, j, wd);
   tnx_stamp_end(ts);
+}
+
+// The active count after a step, written to the host by the last eigensolve
+// block of k_update_norm to finish (every block has made its convergence
+// decision by then): each block adds itself to the done count nact[1] and, if
+// its solve converged, takes it off the active count nact[0], in one 64-bit
+// atomic; the one that completes the count writes the active count to `host`
+// (pinned memory the host reads after the launch's event) and clears the done
+// count for the next launch.  No block waits for another.
+__device__ __forceinline__ void publish_nact(const LzLayout& L, int nsolve, bool converged,
+                                             int32_t* host) {
+  if (threadIdx.x != 0) return;
+  unsigned long long* both = (unsigned long long*)L.nact;
+  const unsigned long long add = (1ull << 32) - (converged ? 1 : 0);
+  const unsigned long long now =
+      __hip_atomic_fetch_add(both, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+  if ((now >> 32) == (unsigned long long)nsolve) {
+    if (host != nullptr) *(volatile int32_t*)host = (int32_t)(unsigned)now;
+    __hip_atomic_store(both, now & 0xffffffffull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// beta_j = sqrt(||r||^2 - ||h2||^2) from the sums h[0..j] = h2, h[j+1] =
+// ||r||^2 (LDS), the same bits in every wavefront; *skip: the second
+// projection is negligible.
+__device__ __forceinline__ double new_coupling(const double* h, int j, int v_dtype, bool* skip) {
+  const int lane = threadIdx.x & 63;
+  const double hl = lane <= j ? h[lane] : 0.0;
+  const double hh = tnx_wave_sum(hl * hl);
+  const double bb = fmax(h[j + 1] - hh, 0.0);
+  const double sk = v_dtype == TNX_F32 ? LZ_REORTH_SKIP_F32 : LZ_REORTH_SKIP;
+  *skip = hh <= sk * sk * bb;
+  return sqrt(bb);
+}
+
+// alpha_j and beta_j of a solve, the tridiagonal eigenproblem and the
+// convergence test, by one wavefront (LDS: a, b with entries 0..j-1 loaded,
+// y, work).  True if the solve converged (its active flag is cleared).
+__device__ __forceinline__ bool finish_step(const tnx_lanczos_solve& D, const LzLayout& L, int s,
+                                            int j, double alpha, double beta, int min_iters,
+                                            double* a, double* b, double* y, double* work) {
+  const int lane = threadIdx.x & 63;
+  LzState& st = L.st[s];
+  __shared__ double th_s;
+  if (lane == 0) {
+    a[j] = alpha;
+    b[j] = beta;
+  }
+  __builtin_amdgcn_wave_barrier();
+  tridiag_pair(a, b, j + 1, 0, y, &th_s, work);
+  __builtin_amdgcn_wave_barrier();
+  if (lane <= j) st.y[lane] = y[lane];
+  const double anorm = -tnx_wave_min(
+      lane <= j ? -(fabs(a[lane]) + (lane > 0 ? fabs(b[lane - 1]) : 0.0)) : 0.0);
+  const double th = th_s;
+  const double res = fabs(beta * y[j]);
+  const double thr = fmax(D.tol_scale * fabs(1.0 - D.tau * th), D.floor_rel * fabs(th));
+  const bool breakdown = beta <= 1e-14 * fmax(anorm, 1e-300);
+  const bool full = (j + 1 >= D.n);
+  const bool conv = full || breakdown || ((j + 1 >= min_iters) && res <= thr);
+  if (lane == 0) {
+    st.alpha[j] = alpha;
+    st.beta[j] = beta;
+    st.iters += 1;
+    st.theta = th;
+    st.resid = res;
+    st.jlast = j;
+    if (conv) {
+      st.converged = 1;
+      __hip_atomic_store(L.act + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  return conv;
 }
 
 // h2 = sum of the pass-2 partials (slots 0..j), ||r||^2 = slot j+1;
@@ -489,7 +644,7 @@ __global__ __launch_bounds__(NT) void k_update_dots(const tnx_lanczos_solve* __r
 // V is orthonormal; ||h2|| is at rounding level next to ||r|| except at a
 // Lanczos breakdown, which the test below catches).
 // Chunk blocks: V[j+1] = (r - V h2) / beta_j and x = cast(V[j+1]) over
-// their chunk, when another Krylov vector follows.  When the second
+// their chunk.  When the second
 // projection is below LZ_REORTH_SKIP relative to beta_j (the usual case:
 // r is already orthogonal to V to that level after the first pass), the
 // correction is left out and V is not read: V[j+1] = r / beta_j, whose
@@ -504,148 +659,71 @@ __global__ __launch_bounds__(NT) void k_update_dots(const tnx_lanczos_solve* __r
 // convergence).  They come first in the grid, so the serial eigensolve
 // starts with the chunks' pass (blocks [nsolve, nsolve + nchunks)) instead
 // of after it.
-// The active count after a step, written to the host by the last eigensolve
-// block of k_update_norm to finish (every block has made its convergence
-// decision by then): each block counts itself in nact[1] after a fence; the
-// one that completes the count reads nact, writes it to `host` (pinned
-// memory the host reads after the launch's event) and clears the count for
-// the next launch.  No block waits for another.
-__device__ __forceinline__ void publish_nact(const LzLayout& L, int nsolve, int32_t* host) {
-  if (threadIdx.x != 0) return;
-  __threadfence();
-  if (atomicAdd(L.nact + 1, 1) == nsolve - 1) {
-    __threadfence();
-    const int32_t v = __hip_atomic_load(L.nact, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (host != nullptr) {
-      *(volatile int32_t*)host = v;
-      __threadfence_system();
+template <typename VT>
+__device__ __forceinline__ void normalize_body(const tnx_lanczos_solve& D, const ChunkInfo& ci,
+                                               int j, int xd, const LzLayout& L, int nchunks) {
+  __shared__ double h[NCV_MAX + 1];
+  const VT TNX_GLOBAL* V = as_global<const VT>(D.V);
+  VT TNX_GLOBAL* Vn = as_global<VT>(D.V) + (int64_t)(j + 1) * D.ldv;
+  double r[EPT];
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) r[q] = (double)Vn[elem(ci, q)];
+  reduce_partials(L.partB, nchunks, D.chunk_begin, ci.nch, j + 2, j + 2, h);
+  __syncthreads();
+  bool skip;
+  const double beta = new_coupling(h, j, D.v_dtype, &skip);
+  const double inv = 1.0 / beta;
+  if (!skip) chunk_axpy(V, D.ldv, j, ci, h, r);
+#pragma unroll
+  for (int q = 0; q < EPT; ++q)
+    if (inside(ci, q)) {
+      // x is the basis row as stored, so the next matvec acts on it
+      const VT v = (VT)(r[q] * inv);
+      Vn[elem(ci, q)] = v;
+      tnx_store((void*)D.x, xd, elem(ci, q), (double)v);
     }
-    __hip_atomic_store(L.nact + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
 }
 
-__global__ __launch_bounds__(NT) void k_update_norm(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+__global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                                     void* state, int nchunks, int j, int x_dtype,
-                                                    int normalize, int min_iters,
-                                                    int32_t* nact_host, unsigned long long* ts) {
+                                                    int min_iters, int32_t* nact_host,
+                                                    unsigned long long* ts) {
   tnx_stamp_begin(ts);
   LzLayout L = lz_layout(state, nsolve, nchunks);
-  const bool solver = (int)blockIdx.x < nsolve;
-  ChunkInfo ci;
-  int s;
-  if (solver) {
-    s = (int)blockIdx.x;
-  } else {
-    if (!normalize) return;
-    ci = chunk_of(S, nsolve, (int)blockIdx.x - nsolve);
-    s = ci.s;
-  }
-  if (!solve_active(L.act, s)) {
-    if (solver) publish_nact(L, nsolve, nact_host);
-    return;
-  }
-  const tnx_lanczos_solve D = S[s];
-  __shared__ double h[NCV_MAX + 1];
-  __shared__ double beta_s;
-  __shared__ int skip_s;
-  reduce_partials(L.partB, D.chunk_begin, (D.n + CHUNK - 1) / CHUNK, j + 2, h);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double hh = 0.0;
-    for (int k = 0; k <= j; ++k) hh += h[k] * h[k];
-    const double bb = fmax(h[j + 1] - hh, 0.0);
-    beta_s = sqrt(bb);
-    const double sk = D.v_dtype == TNX_F32 ? LZ_REORTH_SKIP_F32 : LZ_REORTH_SKIP;
-    skip_s = hh <= sk * sk * bb;
-  }
-  __syncthreads();
-  const double beta_j = beta_s;
-  if (!solver) {
-    const double inv = 1.0 / beta_j;
+  if ((int)blockIdx.x >= nsolve) {
+    const ChunkInfo ci = chunk_of(S, nsolve, (int)blockIdx.x - nsolve);
+    if (!solve_active(L.act, ci.s)) return;
+    const tnx_lanczos_solve D = S[ci.s];
     const int xd = dtype_of(x_dtype, D.x_dtype);
-    double r[CHUNK / NT];
-    if (D.v_dtype == TNX_F32) {
-      const float* V = (const float*)D.V;
-      float* Vn = (float*)D.V + (int64_t)(j + 1) * D.ldv;
-#pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) {
-        int i = ci.i0 + q * NT + threadIdx.x;
-        r[q] = (i < ci.i1) ? (double)Vn[i] : 0.0;
-      }
-      if (!skip_s) chunk_axpy(V, D.ldv, j, ci.i0, ci.i1, h, r);
-#pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) {
-        int i = ci.i0 + q * NT + threadIdx.x;
-        if (i < ci.i1) {
-          // x is the basis row as stored, so the next matvec acts on it
-          const float v = (float)(r[q] * inv);
-          Vn[i] = v;
-          tnx_store((void*)D.x, xd, i, (double)v);
-        }
-      }
-    } else {
-      const double* V = (const double*)D.V;
-      double* Vn = (double*)D.V + (int64_t)(j + 1) * D.ldv;
-#pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) {
-        int i = ci.i0 + q * NT + threadIdx.x;
-        r[q] = (i < ci.i1) ? Vn[i] : 0.0;
-      }
-      if (!skip_s) chunk_axpy(V, D.ldv, j, ci.i0, ci.i1, h, r);
-#pragma unroll
-      for (int q = 0; q < CHUNK / NT; ++q) {
-        int i = ci.i0 + q * NT + threadIdx.x;
-        if (i < ci.i1) {
-          const double v = r[q] * inv;
-          Vn[i] = v;
-          tnx_store((void*)D.x, xd, i, v);
-        }
-      }
-    }
+    if (D.v_dtype == TNX_F32) normalize_body<float>(D, ci, j, xd, L, nchunks);
+    else normalize_body<double>(D, ci, j, xd, L, nchunks);
     tnx_stamp_end(ts);
     return;
   }
+  const int s = (int)blockIdx.x;
+  if (!solve_active(L.act, s)) {
+    publish_nact(L, nsolve, false, nact_host);
+    return;
+  }
+  const tnx_lanczos_solve D = S[s];
   LzState& st = L.st[s];
-  __shared__ double a_s[NCV_MAX], b_s[NCV_MAX], y_s[NCV_MAX], th_s;
-  __shared__ double work[TRI_WORK];
+  __shared__ double h[NCV_MAX + 1];
+  __shared__ double a_s[NCV_MAX], b_s[NCV_MAX], y_s[NCV_MAX], work[TRI_WORK];
   // alpha[0..j-1], beta[0..j-1] were written by earlier launches: every lane
   // loads its share (one round trip instead of a serial loop of j loads)
-  for (int k = threadIdx.x; k < j; k += NT) {
-    a_s[k] = st.alpha[k];
-    b_s[k] = st.beta[k];
+  if ((int)threadIdx.x < j) {
+    a_s[threadIdx.x] = st.alpha[threadIdx.x];
+    b_s[threadIdx.x] = st.beta[threadIdx.x];
   }
-  for (int k = threadIdx.x; k <= j; k += NT) st.h2[k] = h[k];
-  if (threadIdx.x == 0) {
-    const double alpha = st.h1[j] + h[j];
-    st.alpha[j] = alpha;
-    st.beta[j] = beta_j;
-    st.iters += 1;
-    a_s[j] = alpha;
-    b_s[j] = beta_j;
-  }
+  const double h1j = st.h1[j];
+  reduce_partials(L.partB, nchunks, D.chunk_begin, (D.n + CHUNK - 1) / CHUNK, j + 2, j + 2, h);
   __syncthreads();
-  if (threadIdx.x < 64) tridiag_pair(a_s, b_s, j + 1, 0, y_s, &th_s, work);
-  __syncthreads();
-  for (int k = threadIdx.x; k <= j; k += NT) st.y[k] = y_s[k];
-  if (threadIdx.x == 0) {
-    const double beta = b_s[j];
-    const double th = th_s;
-    const double res = fabs(beta * y_s[j]);
-    st.theta = th;
-    st.resid = res;
-    st.jlast = j;
-    const double thr = fmax(D.tol_scale * fabs(1.0 - D.tau * th), D.floor_rel * fabs(th));
-    double anorm = 0.0;
-    for (int k = 0; k <= j; ++k) anorm = fmax(anorm, fabs(a_s[k]) + (k > 0 ? fabs(b_s[k - 1]) : 0.0));
-    const bool breakdown = beta <= 1e-14 * fmax(anorm, 1e-300);
-    const bool full = (j + 1 >= D.n);
-    if (full || breakdown || ((j + 1 >= min_iters) && res <= thr)) {
-      st.converged = 1;
-      __hip_atomic_store(L.act + s, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      atomicSub(L.nact, 1);
-    }
-  }
-  publish_nact(L, nsolve, nact_host);
+  if (threadIdx.x >= 64) return;
+  if ((int)threadIdx.x <= j) st.h2[threadIdx.x] = h[threadIdx.x];
+  bool skip;
+  const double beta = new_coupling(h, j, D.v_dtype, &skip);
+  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, min_iters, a_s, b_s, y_s, work);
+  publish_nact(L, nsolve, conv, nact_host);
   tnx_stamp_end(ts);
 }
 
@@ -978,37 +1056,55 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
 }
 
 // Rows V'[u] = sum_t C[t][u] V[t] (u <= k, t <= m) of this chunk in place,
-// x = cast(V'[k]) as stored.
+// x = cast(V'[k]) as stored.  Rows are read eight at a time, so their loads
+// are in flight together.
 template <typename VT>
-__device__ __forceinline__ void irl_apply_rows(VT* V, const tnx_lanczos_solve& D,
+__device__ __forceinline__ void irl_apply_rows(const tnx_lanczos_solve& D,
                                                const double (*C)[LZ_KEEP + 1],
                                                const ChunkInfo& ci, int m, int k, int xd) {
-  for (int i = ci.i0 + threadIdx.x; i < ci.i1; i += NT) {
-    double acc[LZ_KEEP + 1];
+  VT TNX_GLOBAL* V = as_global<VT>(D.V);
+  double acc[EPT][LZ_KEEP + 1];
 #pragma unroll
-    for (int u = 0; u <= LZ_KEEP; ++u) acc[u] = 0.0;
-    for (int t = 0; t <= m; ++t) {
-      const double v = (double)V[(int64_t)t * D.ldv + i];
+  for (int q = 0; q < EPT; ++q)
 #pragma unroll
-      for (int u = 0; u <= LZ_KEEP; ++u)
-        if (u <= k) acc[u] += C[t][u] * v;
-    }
+    for (int u = 0; u <= LZ_KEEP; ++u) acc[q][u] = 0.0;
+  for (int t0 = 0; t0 <= m; t0 += 8) {
+    VT v[8][EPT];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int q = 0; q < EPT; ++q) v[r][q] = V[(int64_t)min(t0 + r, m) * D.ldv + elem(ci, q)];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (t0 + r <= m) {
+#pragma unroll
+        for (int u = 0; u <= LZ_KEEP; ++u)
+          if (u <= k) {
+            const double c = C[t0 + r][u];
+#pragma unroll
+            for (int q = 0; q < EPT; ++q) acc[q][u] += c * (double)v[r][q];
+          }
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    if (!inside(ci, q)) continue;
     double xk = 0.0;
 #pragma unroll
     for (int u = 0; u <= LZ_KEEP; ++u)
       if (u <= k) {
-        const VT st = (VT)acc[u];
-        V[(int64_t)u * D.ldv + i] = st;
+        const VT st = (VT)acc[q][u];
+        V[(int64_t)u * D.ldv + elem(ci, q)] = st;
         if (u == k) xk = (double)st;
       }
-    tnx_store((void*)D.x, xd, i, xk);
+    tnx_store((void*)D.x, xd, elem(ci, q), xk);
   }
 }
 
 // Implicit restart, basis part (chunk workgroups of the active solves): the
 // new rows V'[u] = sum_t C[t][u] V[t] (u <= k, t <= m) in place (every
 // element is read in full before it is written), x = cast(V'[k]).
-__global__ __launch_bounds__(NT) void k_irl_apply(const tnx_lanczos_solve* __restrict__ S,
+__global__ __launch_bounds__(NP) void k_irl_apply(const tnx_lanczos_solve* __restrict__ S,
                                                   int nsolve, void* state, int nchunks, int m,
                                                   int k, int x_dtype) {
   LzLayout L = lz_layout(state, nsolve, nchunks);
@@ -1017,17 +1113,44 @@ __global__ __launch_bounds__(NT) void k_irl_apply(const tnx_lanczos_solve* __res
   const tnx_lanczos_solve D = S[ci.s];
   const LzState& st = L.st[ci.s];
   __shared__ double C[NCV_MAX + 1][LZ_KEEP + 1];
-  for (int e = threadIdx.x; e < (m + 1) * (LZ_KEEP + 1); e += NT)
+  for (int e = threadIdx.x; e < (m + 1) * (LZ_KEEP + 1); e += NP)
     C[e / (LZ_KEEP + 1)][e % (LZ_KEEP + 1)] = st.C[e / (LZ_KEEP + 1)][e % (LZ_KEEP + 1)];
   __syncthreads();
   const int xd = dtype_of(x_dtype, D.x_dtype);
-  if (D.v_dtype == TNX_F32) irl_apply_rows((float*)D.V, D, C, ci, m, k, xd);
-  else irl_apply_rows((double*)D.V, D, C, ci, m, k, xd);
+  if (D.v_dtype == TNX_F32) irl_apply_rows<float>(D, C, ci, m, k, xd);
+  else irl_apply_rows<double>(D, C, ci, m, k, xd);
+}
+
+// out = sum_k y[k] V[k] of a chunk, eight rows' loads in flight at a time
+template <typename VT>
+__device__ __forceinline__ void final_rows(const tnx_lanczos_solve& D, const ChunkInfo& ci,
+                                           const double* y, int kk) {
+  const VT TNX_GLOBAL* V = as_global<const VT>(D.V);
+  double acc[EPT];
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) acc[q] = 0.0;
+  for (int t0 = 0; t0 < kk; t0 += 8) {
+    VT v[8][EPT];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int q = 0; q < EPT; ++q)
+        v[r][q] = V[(int64_t)min(t0 + r, kk - 1) * D.ldv + elem(ci, q)];
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (t0 + r < kk) {
+#pragma unroll
+        for (int q = 0; q < EPT; ++q) acc[q] += y[t0 + r] * (double)v[r][q];
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < EPT; ++q)
+    if (inside(ci, q)) as_global<double>(D.out)[elem(ci, q)] = acc[q];
 }
 
 // out = sum_k y[k] V[k] for every solve; the first chunk's block of each
 // solve also writes its result record to `res`
-__global__ __launch_bounds__(NT) void k_final(const tnx_lanczos_solve* __restrict__ S, int nsolve,
+__global__ __launch_bounds__(NP) void k_final(const tnx_lanczos_solve* __restrict__ S, int nsolve,
                                               void* state, int nchunks,
                                               tnx_lanczos_result* res) {
   LzLayout L = lz_layout(state, nsolve, nchunks);
@@ -1040,25 +1163,12 @@ __global__ __launch_bounds__(NT) void k_final(const tnx_lanczos_solve* __restric
     res[ci.s].iters = st.iters;
     res[ci.s].converged = st.converged;
   }
-  const int kk = st.jlast + 1;
-  double* out = (double*)D.out;
-  if (D.v_dtype == TNX_F32) {
-    const float* V = (const float*)D.V;
-    for (int i = ci.i0 + threadIdx.x; i < ci.i1; i += NT) {
-      double s = 0.0;
-      for (int k = 0; k < kk; ++k) s += st.y[k] * (double)V[(int64_t)k * D.ldv + i];
-      out[i] = s;
-    }
-  } else {
-    const double* V = (const double*)D.V;
-    for (int i = ci.i0 + threadIdx.x; i < ci.i1; i += NT) {
-      double s = 0.0;
-      for (int k = 0; k < kk; ++k) s += st.y[k] * V[(int64_t)k * D.ldv + i];
-      out[i] = s;
-    }
-  }
+  __shared__ double y[NCV_MAX];
+  if (threadIdx.x < NCV_MAX) y[threadIdx.x] = st.y[threadIdx.x];
+  __syncthreads();
+  if (D.v_dtype == TNX_F32) final_rows<float>(D, ci, y, st.jlast + 1);
+  else final_rows<double>(D, ci, y, st.jlast + 1);
 }
-
 
 // pinned staging for the polled active count and the results
 struct Pinned {
@@ -1128,11 +1238,27 @@ int issue_start(const tnx_lanczos_solve* solves, int nsolve, void* state, int nc
   static_assert(sizeof(LzState) % sizeof(uint64_t) == 0, "LzState is whole words");
   hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((words + 255) / 256 < 1024 ? (words + 255) / 256 : 1024)),
                      dim3(256), 0, s, (uint64_t*)L.st, words, L.nact, nsolve);
-  hipLaunchKernelGGL(k_init_norm, dim3(nchunks), dim3(NT), 0, s, solves, nsolve, state, nchunks);
-  hipLaunchKernelGGL(k_init_scale, dim3(nchunks), dim3(NT), 0, s, solves, nsolve, state, nchunks,
+  hipLaunchKernelGGL(k_init_norm, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks);
+  hipLaunchKernelGGL(k_init_scale, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks,
                      x_dtype);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
+}
+
+// The projections' instances for Krylov index j: the next multiple of 4 above
+// j rows in registers.
+typedef void (*BasisKernel)(const tnx_lanczos_solve*, int, void*, int, int, int,
+                            unsigned long long*);
+struct BasisPass {
+  BasisKernel dots, update_dots;
+};
+BasisPass basis_pass(int j) {
+  static const BasisPass table[NCV_MAX / 4] = {
+      {k_dots<4>, k_update_dots<4>},   {k_dots<8>, k_update_dots<8>},
+      {k_dots<12>, k_update_dots<12>}, {k_dots<16>, k_update_dots<16>},
+      {k_dots<20>, k_update_dots<20>}, {k_dots<24>, k_update_dots<24>},
+      {k_dots<28>, k_update_dots<28>}, {k_dots<32>, k_update_dots<32>}};
+  return table[j / 4];
 }
 
 // Krylov step j of every active solve: each plan's matvec, then the dots,
@@ -1145,7 +1271,7 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   LzLayout L = lz_layout(state, nsolve, nchunks);
   for (int p = 0; p < nplan; ++p)
     if (int rc = tnx_heff_matvec(plans + p, L.act, stream)) return rc;
-  const dim3 grid(nchunks), block(NT);
+  const dim3 grid(nchunks), block(NP);
   // sampled timing (one plan: its modes give the x and w element sizes, and
   // the basis element size under the policy that a low-precision matvec
   // has an f32 basis); algorithmic bytes over the nchunks * CHUNK
@@ -1161,19 +1287,20 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   tnx_prof_count(TNX_PC_UPDATE_DOTS, E * (vrows + ws + vs));
   tnx_prof_count(TNX_PC_UPDATE_NORM, E * (2.0 * vs + xs));
   int mk = prof ? tnx_prof_mark(TNX_PC_DOTS, s) : -1;
-  hipLaunchKernelGGL(k_dots, grid, block, 0, s, solves, nsolve, state, nchunks, j, w_dtype,
+  const BasisPass pass = basis_pass(j);
+  hipLaunchKernelGGL(pass.dots, grid, block, 0, s, solves, nsolve, state, nchunks, j, w_dtype,
                      tnx_prof_ts(mk));
   tnx_prof_done(mk, s, E * (vrows + ws));
   mk = prof ? tnx_prof_mark(TNX_PC_UPDATE_DOTS, s) : -1;
-  hipLaunchKernelGGL(k_update_dots, grid, block, 0, s, solves, nsolve, state, nchunks, j, w_dtype,
-                     tnx_prof_ts(mk));
+  hipLaunchKernelGGL(pass.update_dots, grid, block, 0, s, solves, nsolve, state, nchunks, j,
+                     w_dtype, tnx_prof_ts(mk));
   tnx_prof_done(mk, s, E * (vrows + ws + vs));
   // the chunk blocks normalise V[j+1] at every step, the last of a cycle
   // included (an implicit restart combines V[ncv] into the new basis)
   (void)ncv;
   mk = prof ? tnx_prof_mark(TNX_PC_UPDATE_NORM, s) : -1;
   hipLaunchKernelGGL(k_update_norm, dim3(nchunks + nsolve), block, 0, s, solves, nsolve, state,
-                     nchunks, j, x_dtype, 1, min_iters, nact_host, tnx_prof_ts(mk));
+                     nchunks, j, x_dtype, min_iters, nact_host, tnx_prof_ts(mk));
   // (r read, V[j+1] and x written; the basis rows of the second correction,
   // read only when it is not negligible, are not counted)
   tnx_prof_done(mk, s, E * (2.0 * vs + xs));
@@ -1188,7 +1315,7 @@ int issue_restart(const tnx_lanczos_solve* solves, int nsolve, void* state, int 
   const int k = lz_keep(ncv);
   hipLaunchKernelGGL(k_irl_solve, dim3(nsolve), dim3(NT), 0, s, solves, nsolve, state, nchunks,
                      ncv, k);
-  hipLaunchKernelGGL(k_irl_apply, dim3(nchunks), dim3(NT), 0, s, solves, nsolve, state, nchunks,
+  hipLaunchKernelGGL(k_irl_apply, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks,
                      ncv, k, x_dtype);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
@@ -1197,7 +1324,7 @@ int issue_restart(const tnx_lanczos_solve* solves, int nsolve, void* state, int 
 // Eigenvectors into every solve's `out`, results into `res` (device-visible).
 int issue_finish(const tnx_lanczos_solve* solves, int nsolve, void* state, int nchunks,
                  tnx_lanczos_result* res, hipStream_t s) {
-  hipLaunchKernelGGL(k_final, dim3(nchunks), dim3(NT), 0, s, solves, nsolve, state, nchunks, res);
+  hipLaunchKernelGGL(k_final, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks, res);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }

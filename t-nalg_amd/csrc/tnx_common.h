@@ -94,17 +94,19 @@ template <typename T> __device__ __forceinline__ T TNX_GLOBAL* as_global(uint64_
   return (T TNX_GLOBAL*)p;
 }
 
-// Load element idx of a buffer of runtime dtype as double.
+// Load element idx of a buffer (global memory) of runtime dtype as double.
 __device__ __forceinline__ double tnx_load(const void* p, int dtype, int64_t idx) {
-  if (dtype == TNX_F64) return ((const double*)p)[idx];
-  if (dtype == TNX_F32) return (double)((const float*)p)[idx];
-  return (double)(float)((const __bf16*)p)[idx];
+  const uint64_t a = (uint64_t)p;
+  if (dtype == TNX_F64) return as_global<const double>(a)[idx];
+  if (dtype == TNX_F32) return (double)as_global<const float>(a)[idx];
+  return (double)(float)as_global<const __bf16>(a)[idx];
 }
 
 __device__ __forceinline__ void tnx_store(void* p, int dtype, int64_t idx, double v) {
-  if (dtype == TNX_F64) ((double*)p)[idx] = v;
-  else if (dtype == TNX_F32) ((float*)p)[idx] = (float)v;
-  else ((__bf16*)p)[idx] = (__bf16)(float)v;
+  const uint64_t a = (uint64_t)p;
+  if (dtype == TNX_F64) as_global<double>(a)[idx] = v;
+  else if (dtype == TNX_F32) as_global<float>(a)[idx] = (float)v;
+  else as_global<__bf16>(a)[idx] = (__bf16)(float)v;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs of MI355X, each with
@@ -128,20 +130,18 @@ template <int DPP> __device__ __forceinline__ double tnx_row_get(double v) {
   const int hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), DPP, 0xf, 0xf, true);
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-// The values of lane and lane ^ 32 (HALF) or lane ^ 16, the one with the bit
-// clear in `p`, by the swap of the odd rows of one register with the even rows
-// of another.
-template <bool HALF> __device__ __forceinline__ void tnx_swap_get(double v, double& p, double& q) {
-  const long long x = __double_as_longlong(v);
-  const unsigned l = (unsigned)x, h = (unsigned)(x >> 32);
+// Exchange of the odd halves (HALF: lanes 32-63; else the odd 16-lane rows) of
+// p with the even ones of q.
+template <bool HALF> __device__ __forceinline__ void tnx_swap(double& p, double& q) {
+  const long long x = __double_as_longlong(p), y = __double_as_longlong(q);
   typedef unsigned u2 __attribute__((ext_vector_type(2)));
   u2 lo, hi;
   if constexpr (HALF) {
-    lo = __builtin_amdgcn_permlane32_swap(l, l, false, false);
-    hi = __builtin_amdgcn_permlane32_swap(h, h, false, false);
+    lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
   } else {
-    lo = __builtin_amdgcn_permlane16_swap(l, l, false, false);
-    hi = __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
   }
   p = __longlong_as_double(((long long)hi[0] << 32) | lo[0]);
   q = __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
@@ -150,10 +150,10 @@ template <bool HALF> __device__ __forceinline__ void tnx_swap_get(double v, doub
 // 16-lane row a rotation by d = 8, 4, 2, 1 brings lane ^ d's value, as the
 // values repeat with period 2 d by then.
 template <typename F> __device__ __forceinline__ double tnx_wave_fold(double v, F f) {
-  double p, q;
-  tnx_swap_get<true>(v, p, q);
-  v = f(p, q);
-  tnx_swap_get<false>(v, p, q);
+  double p = v, q = v;   // after a swap: the value of the lane with the bit clear, set
+  tnx_swap<true>(p, q);
+  p = q = f(p, q);
+  tnx_swap<false>(p, q);
   v = f(p, q);
   v = f(v, tnx_row_get<0x128>(v));
   v = f(v, tnx_row_get<0x124>(v));

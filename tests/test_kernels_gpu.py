@@ -1161,3 +1161,70 @@ def test_lanczos_restart_lengths(gpu, ncv, low):
     assert np.linalg.norm(H @ v - res[0]['theta'] * v) < 2e-6
     # residual over the gap bounds the part outside the lowest eigenvector
     assert abs(abs(v @ U[:, 0]) - 1) < (2e-6 / (e[1] - e[0])) ** 2
+
+
+@pytest.mark.parametrize('v32', [False, True])
+@pytest.mark.parametrize('alone', [False, True])
+def test_lanczos_chunk_edges(gpu, v32, alone):
+    """A full cycle of 32 steps at sizes around the 512-lane and 1024-element
+    chunk edges, rows at an odd stride, all solves in one call or each alone:
+    the basis stays orthonormal (1e-10 in f64; 32 rows rounded to f32, 2e-6),
+    the Ritz value is that of the operator projected on the basis, the padding
+    between rows is untouched, and both ways of calling give the same bits."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    ncv, pad, sizes = 32, 3, [40, 511, 512, 513, 1023, 1024, 1025, 2049]
+    np_t, tol = (np.float32, 2e-6) if v32 else (np.float64, 1e-10)
+
+    def run(idx):
+        keep, solves = [], []
+        g2 = R.GemmList()
+        for q, k in enumerate(idx):
+            n = sizes[k]
+            rng = np.random.RandomState(100 + k)
+            A = rng.randn(n, n)
+            H = 0.01 * (A + A.T) / 2 + np.diag(np.linspace(0.0, 10.0, n))
+            Hd, init = _dev(H), _dev(rng.randn(n))
+            V = _dev(np.full((ncv + 1, n + pad), 7.0, dtype=np_t))
+            w, x, out = (torch.zeros(n, dtype=torch.float64, device='cuda') for _ in range(3))
+            keep.append((Hd, init, V, w, x, out, H))
+            g2.add(w.data_ptr(), n, 1, 1, [(Hd.data_ptr(), n, 0, x.data_ptr(), 1, 0, n, 1.0)],
+                   active=q)
+            solves.append((V.data_ptr(), w.data_ptr(), x.data_ptr(), init.data_ptr(),
+                           out.data_ptr(), n, n + pad, 0, 0, 1e-30, 1e-4, 0.0, 0, 0,
+                           L.F32 if v32 else L.F64, 0))
+        lz = L.lanczos_records(solves)
+        ch = (lz['n'] + L.LZ_CHUNK - 1) // L.LZ_CHUNK
+        lz['chunk_begin'] = np.concatenate([[0], np.cumsum(ch)[:-1]])
+        p, s = g2.arrays()
+        dp, ds, dlz = _upload([p, s, lz])
+        plan = L.MatvecPlan(0, 0, 0, 0, 0, 0, 0, 0, dp.data_ptr(), ds.data_ptr(), len(p),
+                            R.gemm_tiles(p), 0, 0, 0)
+        state = torch.zeros(int(lib.tnx_lanczos_state_bytes(len(idx), int(ch.sum()), ncv)),
+                            dtype=torch.uint8, device='cuda')
+        res = np.zeros(len(idx), dtype=L.LANCZOS_RESULT)
+        rc = lib.tnx_lanczos_run_ex(plan, _vp(dlz.data_ptr()), len(idx), int(ch.sum()), ncv, 0,
+                                    ncv, 0, 0, _vp(state.data_ptr()), _vp(res.ctypes.data),
+                                    _stream())
+        assert rc == L.ENOCONV, (rc, lib.tnx_last_error())
+        return [(res[q], t[2].cpu().numpy(), t[5].cpu().numpy(), t[6])
+                for q, t in enumerate(keep)]
+
+    print('lanczos chunk edges', sizes, 'f32 basis', v32, 'alone', alone, flush=True)
+    got = run(list(range(len(sizes))))
+    if alone:
+        for k, (r, V, out, _) in enumerate(got):
+            (r1, V1, out1, _), = run([k])
+            assert r1['theta'] == r['theta'] and r1['resid'] == r['resid'], sizes[k]
+            assert np.array_equal(V1, V) and np.array_equal(out1, out), sizes[k]
+        return
+    for n, (r, V, out, H) in zip(sizes, got):
+        assert r['iters'] == ncv
+        assert np.all(V[:, n:] == 7.0), n
+        B = V[:, :n].astype(np.float64)
+        assert np.abs(B @ B.T - np.eye(ncv + 1)).max() < tol, n
+        th = np.linalg.eigvalsh(B[:ncv] @ H @ B[:ncv].T)[0]
+        assert abs(r['theta'] - th) < 10 * tol, (n, r, th)
+        assert abs(np.linalg.norm(out) - 1) < 10 * tol, n
