@@ -16,7 +16,7 @@
 // runs in f32 or bf16 (v_dtype: the basis passes then move half the bytes).
 // The matvec may run in f32 or bf16.
 // The (j+1)x(j+1) tridiagonal eigenproblem is solved on the device by one
-// wavefront: 65-way multisection, then a twisted factorisation.
+// wavefront: multisection with secant steps, then a twisted factorisation.
 // A solve that has not converged after ncv steps is restarted implicitly
 // (Sorensen's implicitly restarted Lanczos with exact shifts, as ARPACK's
 // dsaupd does for eigsh): the ncv - k largest Ritz values are applied as
@@ -260,83 +260,123 @@ __device__ __forceinline__ double fast_rsqrt(double x) {
   return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// Number of eigenvalues below x of the k x k symmetric tridiagonal with
-// diagonal a and squared couplings b2 (LDS), whose entries are of order one or
-// less: sign changes of the leading minors p_i = (a_i - x) p_{i-1} - b2_{i-1}
-// p_{i-2}, one dependent operation a row where the ratios of the minors
-// (Sturm's sequence) need a division.  A zero counts as a change; the pair is
-// scaled up when it gets small.
-__device__ __forceinline__ int count_below(const double* a, const double* b2, int k, double x) {
-  double p0 = 1.0, p1 = a[0] - x;
-  bool neg = p1 <= 0.0;
-  int cnt = neg;
-#pragma unroll 4
-  for (int i = 1; i < k; ++i) {
-    const double p2 = fma(a[i] - x, p1, -b2[i - 1] * p0);
-    const bool change = neg ? p2 >= 0.0 : p2 <= 0.0;
-    cnt += change;
-    neg = neg != change;
-    const double sc = fmax(fabs(p1), fabs(p2)) < 1e-100 ? 1e100 : 1.0;
-    p0 = p1 * sc;
-    p1 = p2 * sc;
+// A symmetric tridiagonal problem in LDS, scaled: rows 0..pad_rows(k) - 1 with
+// diagonal a[i] and squared couplings c2[i] of rows i - 1 and i (c2[0] = 0),
+// entries of order one or less; rows from k on are decoupled, above the
+// spectrum.
+constexpr int MINOR_ROWS = 8;   // rows whose LDS reads are issued together
+__device__ __forceinline__ int pad_rows(int k) { return (k + MINOR_ROWS - 1) & -MINOR_ROWS; }
+constexpr double PAD_DIAG = 4.0;
+
+// MINOR_ROWS more leading minors p_i = (a_i - x) p_{i-1} - c2_i p_{i-2} from
+// row i0: one dependent operation a row, where the ratios of the minors
+// (Sturm's sequence) need a division.  The pair is then scaled up if both
+// have got small: MINOR_ROWS rows cannot take them from there to underflow,
+// short of an x within rounding of an eigenvalue, where any count will do.
+// CHANGES: *acc += the sign changes (a zero takes either sign); else the sign
+// bit of *acc is set once a minor is negative.
+template <bool CHANGES>
+__device__ __forceinline__ void minors(const double* a, const double* c2, int i0, double x,
+                                       double& p0, double& p1, int& acc, int& scaled) {
+  double ar[MINOR_ROWS], cr[MINOR_ROWS];
+#pragma unroll
+  for (int u = 0; u < MINOR_ROWS; ++u) {
+    ar[u] = a[i0 + u] - x;
+    cr[u] = c2[i0 + u];
   }
+#pragma unroll
+  for (int u = 0; u < MINOR_ROWS; ++u) {
+    const double p2 = fma(ar[u], p1, -cr[u] * p0);
+    if constexpr (CHANGES) acc += (unsigned)(__double2hiint(p1) ^ __double2hiint(p2)) >> 31;
+    else acc |= __double2hiint(p2);
+    p0 = p1;
+    p1 = p2;
+  }
+  const bool small = fmax(fabs(p0), fabs(p1)) < 1e-100;
+  const double sc = small ? 1e100 : 1.0;
+  scaled += small;
+  p0 *= sc;
+  p1 *= sc;
+}
+
+// Number of eigenvalues below x of the problem's k rows.
+__device__ __forceinline__ int count_below(const double* a, const double* c2, int k, double x) {
+  double p0 = 0.0, p1 = 1.0;
+  int cnt = 0, scaled = 0;
+  for (int i0 = 0; i0 < pad_rows(k); i0 += MINOR_ROWS)
+    minors<true>(a, c2, i0, x, p0, p1, cnt, scaled);
   return cnt;
+}
+
+// Eigenvalue idx of the problem's k rows in [lo, hi], to `stop`, by one
+// wavefront: each round 64 points, one a lane, the bracket being the
+// neighbouring points around the eigenvalue.  The points are evenly spaced
+// (65-fold per round), or, once the determinant has opposite signs at the
+// ends of the bracket, at distances halving towards the secant's zero from
+// both ends: its error is of second order in the bracket, so four or five
+// rounds take the place of nine.  A secant round that gains less than an even
+// one is followed by an even one.  LOWEST: idx = 0.
+template <bool LOWEST>
+__device__ __forceinline__ double multisect(const double* a, const double* c2, int k, int idx,
+                                            double lo, double hi, double stop) {
+  const int lane = threadIdx.x & 63;
+  bool secant = false;
+  double g = 0.0;
+  for (int round = 0; round < 24; ++round) {
+    const double w = hi - lo;  // all of these identical in every lane
+    if (w <= stop) break;
+    const double even = lo + w * (1.0 / 65.0) * (double)(lane + 1);
+    const double near = lane < 32 ? g - __builtin_amdgcn_ldexp(g - lo, -(lane + 1))
+                                  : g + __builtin_amdgcn_ldexp(hi - g, lane - 64);
+    const double x = secant ? near : even;
+    double p0 = 0.0, p1 = 1.0;
+    int acc = 0, scaled = 0;
+    for (int i0 = 0; i0 < pad_rows(k); i0 += MINOR_ROWS)
+      minors<!LOWEST>(a, c2, i0, x, p0, p1, acc, scaled);
+    const unsigned long long m = __ballot(LOWEST ? acc < 0 : acc > idx);
+    const int f = m != 0ull ? __builtin_ctzll(m) : 64;   // first lane above it
+    const int lu = min(f, 63), ll = max(f, 1) - 1;
+    auto from = [](double v, int l) {
+      const long long b = __double_as_longlong(v);
+      const int lo32 = __builtin_amdgcn_readlane((int)b, l);
+      const int hi32 = __builtin_amdgcn_readlane((int)(b >> 32), l);
+      return __longlong_as_double(((long long)hi32 << 32) | (unsigned)lo32);
+    };
+    const double xu = from(x, lu), xl = from(x, ll), vu = from(p1, lu), vl = from(p1, ll);
+    const bool both = f > 0 && f < 64 && __builtin_amdgcn_readlane(scaled, lu) ==
+                                             __builtin_amdgcn_readlane(scaled, ll);
+    if (f < 64) hi = xu;
+    if (f > 0) lo = xl;
+    const bool gained = 65.0 * (hi - lo) <= w;
+    g = lo + (hi - lo) * vl * fast_rcp(vl - vu);
+    secant = both && (gained || !secant) && g > lo && g < hi && ((vl < 0.0) != (vu < 0.0));
+  }
+  return 0.5 * (lo + hi);
 }
 
 // Eigenpair idx (0: the lowest) of the k x k tridiagonal (a, b) in LDS, by one
 // wavefront (all 64 lanes): *theta and y[0..k) (LDS).  work: LDS scratch of
 // TRI_WORK doubles of the wavefront's own.
-// The bracket (the Gershgorin bounds; the smallest diagonal entry bounds the
-// lowest eigenvalue) shrinks 65-fold per round (64 interior points, one a
-// lane).  The vector is that of
-// the twisted factorisation: the pivots of T - theta from the top (D+) and
-// from the bottom (D-), two lanes side by side, meet at the row r of smallest
+// The eigenvalue is searched between the Gershgorin bounds (the smallest
+// diagonal entry bounds the lowest).  The vector is that of the twisted
+// factorisation: the pivots of T - theta from the top (D+) and from the bottom
+// (D-), each the ratio of neighbouring minors, meet at the row r of smallest
 // gamma_r = D+_r + D-_r - (a_r - theta), and z_r = 1 is continued by z_i = -b
 // z_{i+1} / D+_i above and -b z_{i-1} / D-_i below it: products of ratios,
 // accurate for the small components, the last of which is the residual
-// estimate.  A vanishing pivot is replaced by a tiny one (the next is then huge
-// and their ratios cancel).  The vector's sign is that of a positive component sum (as inverse iteration from a
-// constant vector gives).
+// estimate.  A vanishing pivot is replaced by a tiny one and one over a
+// vanishing minor by a huge one (their ratios cancel).  The vector's sign is
+// that of a positive component sum (as inverse iteration from a constant
+// vector gives).
 // Bound: the serial chains over k rows.  k_update_norm, most of which this is
 // (mean over k = 1..20, one solve, MI355X): 16.1 us with Sturm sequences by
-// division in 256 lanes and inverse iteration by one lane, 13.8 us so.
-constexpr int TRI_WORK = 4 * NCV_MAX;
+// division in 256 lanes and inverse iteration by one lane, 12.2 with minors and
+// even rounds only, 8.3 so.
+constexpr int TRI_WORK = 6 * NCV_MAX + 2;
+template <bool LOWEST>
 __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, int k, int idx,
                                              double* y, double* theta, double* work) {
   const int lane = threadIdx.x & 63;
-  double* as = work;
-  double* b2 = work + NCV_MAX;
-  double* dp = work + 2 * NCV_MAX;   // D+, then D-
-  const bool in = lane < k;
-  const double al = in ? a[lane] : 0.0;
-  const double bl = lane + 1 < k ? b[lane] : 0.0;   // coupling of rows lane, lane + 1
-  const double bm = in && lane > 0 ? b[lane - 1] : 0.0;
-  const double inf = __builtin_huge_val();
-  double base = tnx_wave_min(in ? al - fabs(bl) - fabs(bm) : inf);
-  const double dmin = tnx_wave_min(in ? al : inf);
-  const double most = -tnx_wave_min(in ? -(al + fabs(bl) + fabs(bm)) : inf);
-  base -= 1e-12 * fmax(most - base, 1e-300);
-  // entries relative to `base`, over a power of two near the spectrum's width
-  const int ex = __builtin_amdgcn_frexp_exp(most - base);
-  if (in) {
-    as[lane] = __builtin_amdgcn_ldexp(al - base, -ex);
-    const double bs = __builtin_amdgcn_ldexp(bl, -ex);
-    b2[lane] = bs * bs;
-  }
-  __builtin_amdgcn_wave_barrier();
-  const double top = idx == 0 ? dmin : most;
-  double lo = 0.0, hi = __builtin_amdgcn_ldexp(top - base, -ex) * (1.0 + 1e-12);
-  const double stop = __builtin_amdgcn_ldexp(4.0 * 2.220446049250313e-16 * fmax(fabs(base), fabs(top)), -ex);
-  for (int round = 0; round < 16; ++round) {
-    const double w = (hi - lo) * (1.0 / 65.0);  // identical in every lane
-    if (65.0 * w <= stop + 1e-300) break;
-    const unsigned long long m = __ballot(count_below(as, b2, k, lo + w * (double)(lane + 1)) > idx);
-    const int f = m != 0ull ? __ffsll((long long)m) : 65;   // the first point above it (65: hi)
-    const double l0 = lo;
-    lo = l0 + w * (double)(f - 1);
-    if (f < 65) hi = l0 + w * (double)f;
-  }
-  const double th = 0.5 * (lo + hi);
   if (k == 1) {
     if (lane == 0) {
       y[0] = 1.0;
@@ -344,27 +384,80 @@ __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, i
     }
     return;
   }
-  // pivots: even lanes from the top, odd lanes from the bottom
-  const bool up = lane & 1;
-  double* dw = dp + (up ? NCV_MAX : 0);
-  const double tiny = 1e-150;
-  double d = 1.0;
-#pragma unroll 4
-  for (int i = 0; i < k; ++i) {
-    const int row = up ? k - 1 - i : i;
-    const double off = i == 0 ? 0.0 : b2[up ? row : row - 1];
-    d = (as[row] - th) - off * fast_rcp(d);
-    if (fabs(d) < tiny) d = tiny;
-    if (lane < 2) dw[row] = d;
+  double* as = work;
+  double* c2 = work + NCV_MAX;             // NCV_MAX + 1 entries
+  double* mn = work + 2 * NCV_MAX + 2;     // minors: top, top before, bottom, bottom before
+  const bool in = lane < k;
+  const double al = in ? a[lane] : 0.0;
+  const double bl = lane + 1 < k ? b[lane] : 0.0;   // coupling of rows lane, lane + 1
+  const double bm = in && lane > 0 ? b[lane - 1] : 0.0;
+  const double inf = __builtin_huge_val();
+  double base = tnx_wave_min(in ? al - fabs(bl) - fabs(bm) : inf);
+  const double most = -tnx_wave_min(in ? -(al + fabs(bl) + fabs(bm)) : inf);
+  const double top = LOWEST ? tnx_wave_min(in ? al : inf) : most;
+  base -= 1e-12 * fmax(most - base, 1e-300);
+  // entries relative to `base`, over a power of two near the spectrum's width
+  const int ex = __builtin_amdgcn_frexp_exp(most - base);
+  if (lane <= NCV_MAX) {
+    const double bs = __builtin_amdgcn_ldexp(bm, -ex);
+    if (lane < NCV_MAX) as[lane] = in ? __builtin_amdgcn_ldexp(al - base, -ex) : PAD_DIAG;
+    c2[lane] = bs * bs;
   }
   __builtin_amdgcn_wave_barrier();
-  const double gam = in ? fabs(dp[lane] + dp[NCV_MAX + lane] - (as[lane] - th)) : inf;
+  const double stop = __builtin_amdgcn_ldexp(
+      4.0 * 2.220446049250313e-16 * fmax(fabs(base), fabs(top)), -ex) + 1e-300;
+  const double th = multisect<LOWEST>(
+      as, c2, k, idx, 0.0, __builtin_amdgcn_ldexp(top - base, -ex) * (1.0 + 1e-12), stop);
+  // minors: lane 0 from the top, lane 1 from the bottom, with the one before
+  // each at the same scale
+  const bool up = lane & 1;
+  const int kk = pad_rows(k);
+  double* mw = mn + (up ? 2 * NCV_MAX : 0);
+  double p0 = 0.0, p1 = 1.0;
+  for (int i0 = 0; i0 < kk; i0 += MINOR_ROWS) {
+    double ar[MINOR_ROWS], cr[MINOR_ROWS], p[MINOR_ROWS + 1];
+#pragma unroll
+    for (int u = 0; u < MINOR_ROWS; ++u) {
+      ar[u] = as[up ? kk - 1 - (i0 + u) : i0 + u] - th;
+      cr[u] = c2[up ? kk - (i0 + u) : i0 + u];
+    }
+    p[0] = p1;
+#pragma unroll
+    for (int u = 0; u < MINOR_ROWS; ++u) {
+      const double p2 = fma(ar[u], p1, -cr[u] * p0);
+      p0 = p1;
+      p[u + 1] = p1 = p2;
+    }
+    if (lane < 2) {
+#pragma unroll
+      for (int u = 0; u < MINOR_ROWS; ++u) {
+        const int row = up ? kk - 1 - (i0 + u) : i0 + u;
+        mw[row] = p[u + 1];
+        mw[NCV_MAX + row] = p[u];
+      }
+    }
+    const double sc = fmax(fabs(p0), fabs(p1)) < 1e-100 ? 1e100 : 1.0;
+    p0 *= sc;
+    p1 *= sc;
+  }
+  __builtin_amdgcn_wave_barrier();
+  const double tiny = 1e-150;
+  double dt = 1.0, db = 1.0;   // pivots of row `lane`
+  if (in) {
+    const double t1 = mn[lane], t0 = mn[NCV_MAX + lane];
+    const double u1 = mn[2 * NCV_MAX + lane], u0 = mn[3 * NCV_MAX + lane];
+    dt = fabs(t0) < 1e-290 ? 1e150 : t1 * fast_rcp(t0);
+    db = fabs(u0) < 1e-290 ? 1e150 : u1 * fast_rcp(u0);
+    if (fabs(dt) < tiny) dt = tiny;
+    if (fabs(db) < tiny) db = tiny;
+  }
+  const double gam = in ? fabs(dt + db - (as[lane] - th)) : inf;
   const double gmin = tnx_wave_min(gam);
   const int r = __ffsll((long long)__ballot(gam == gmin)) - 1;
   // ratio of z_lane to its neighbour on the side of r, then running products
   double z = 1.0;
-  if (in && lane < r) z = -__builtin_amdgcn_ldexp(bl, -ex) * fast_rcp(dp[lane]);
-  else if (in && lane > r) z = -__builtin_amdgcn_ldexp(bm, -ex) * fast_rcp(dp[NCV_MAX + lane]);
+  if (in && lane < r) z = -__builtin_amdgcn_ldexp(bl, -ex) * fast_rcp(dt);
+  else if (in && lane > r) z = -__builtin_amdgcn_ldexp(bm, -ex) * fast_rcp(db);
 #pragma unroll
   for (int o = 1; o < NCV_MAX; o <<= 1) {
     const int from = lane < r ? lane + o : lane - o;
@@ -386,9 +479,8 @@ __device__ __forceinline__ int dtype_of(int call_dtype, int32_t own) {
 
 // ---------------------------------------------------------------- kernels
 
-// act[s], read once per block through LDS: block 0 of a solve may clear it
-// while the solve's other blocks run k_update_norm, and every lane of a block
-// must take the same early return.
+// act[s], read once per block through LDS, so that every lane of a block
+// takes the same early return whenever another block clears it.
 __device__ __forceinline__ bool solve_active(const int32_t* act, int s) {
   __shared__ int a;
   if (threadIdx.x == 0) a = __hip_atomic_load(act + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -613,7 +705,7 @@ __device__ __forceinline__ bool finish_step(const tnx_lanczos_solve& D, const Lz
     b[j] = beta;
   }
   __builtin_amdgcn_wave_barrier();
-  tridiag_pair(a, b, j + 1, 0, y, &th_s, work);
+  tridiag_pair<true>(a, b, j + 1, 0, y, &th_s, work);
   __builtin_amdgcn_wave_barrier();
   if (lane <= j) st.y[lane] = y[lane];
   const double anorm = -tnx_wave_min(
@@ -663,6 +755,9 @@ template <typename VT>
 __device__ __forceinline__ void normalize_body(const tnx_lanczos_solve& D, const ChunkInfo& ci,
                                                int j, int xd, const LzLayout& L, int nchunks) {
   __shared__ double h[NCV_MAX + 1];
+  __shared__ int active;
+  if (threadIdx.x == 0)
+    active = __hip_atomic_load(L.act + ci.s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const VT TNX_GLOBAL* V = as_global<const VT>(D.V);
   VT TNX_GLOBAL* Vn = as_global<VT>(D.V) + (int64_t)(j + 1) * D.ldv;
   double r[EPT];
@@ -670,6 +765,7 @@ __device__ __forceinline__ void normalize_body(const tnx_lanczos_solve& D, const
   for (int q = 0; q < EPT; ++q) r[q] = (double)Vn[elem(ci, q)];
   reduce_partials(L.partB, nchunks, D.chunk_begin, ci.nch, j + 2, j + 2, h);
   __syncthreads();
+  if (active == 0) return;
   bool skip;
   const double beta = new_coupling(h, j, D.v_dtype, &skip);
   const double inv = 1.0 / beta;
@@ -692,7 +788,6 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
   LzLayout L = lz_layout(state, nsolve, nchunks);
   if ((int)blockIdx.x >= nsolve) {
     const ChunkInfo ci = chunk_of(S, nsolve, (int)blockIdx.x - nsolve);
-    if (!solve_active(L.act, ci.s)) return;
     const tnx_lanczos_solve D = S[ci.s];
     const int xd = dtype_of(x_dtype, D.x_dtype);
     if (D.v_dtype == TNX_F32) normalize_body<float>(D, ci, j, xd, L, nchunks);
@@ -701,10 +796,10 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
     return;
   }
   const int s = (int)blockIdx.x;
-  if (!solve_active(L.act, s)) {
-    publish_nact(L, nsolve, false, nact_host);
-    return;
-  }
+  // (only this block clears the flag in this launch; all loads are issued
+  // before it is looked at)
+  const int active =
+      __hip_atomic_load(L.act + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const tnx_lanczos_solve D = S[s];
   LzState& st = L.st[s];
   __shared__ double h[NCV_MAX + 1];
@@ -719,6 +814,10 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
   reduce_partials(L.partB, nchunks, D.chunk_begin, (D.n + CHUNK - 1) / CHUNK, j + 2, j + 2, h);
   __syncthreads();
   if (threadIdx.x >= 64) return;
+  if (active == 0) {
+    publish_nact(L, nsolve, false, nact_host);
+    return;
+  }
   if ((int)threadIdx.x <= j) st.h2[threadIdx.x] = h[threadIdx.x];
   bool skip;
   const double beta = new_coupling(h, j, D.v_dtype, &skip);
@@ -879,7 +978,7 @@ __device__ __forceinline__ bool restart_from_pairs(double (*y)[NCV_MAX], const d
 // converged with its current Ritz pair.
 // Bound: latency, a few serial chains over m rows.  us for m = 20 (MI355X):
 // the QR steps with a library square root and one lane's bisection per shift
-// 164, with fast_rsqrt and SH_LANES lanes 103, from the Ritz pairs 20.5.
+// 164, with fast_rsqrt and SH_LANES lanes 103, from the Ritz pairs 14.4.
 constexpr int SH_LANES = 8;   // NT / NCV_MAX: every shift at once
 __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __restrict__ S,
                                                   int nsolve, void* state, int nchunks, int m,
@@ -902,7 +1001,7 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
   __shared__ double yk[LZ_KEEP][NCV_MAX], thk[LZ_KEEP], tw[LZ_KEEP][TRI_WORK], sigma_s;
   __shared__ int pairs_s;
   static_assert(NT / 64 >= LZ_KEEP, "a wavefront per kept Ritz pair");
-  if (t / 64 < k) tridiag_pair(a_l, b_l, m, t / 64, yk[t / 64], &thk[t / 64], tw[t / 64]);
+  if (t / 64 < k) tridiag_pair<false>(a_l, b_l, m, t / 64, yk[t / 64], &thk[t / 64], tw[t / 64]);
   __syncthreads();
   if (t < 64) {
     const bool ok = restart_from_pairs(yk, thk, m, k, b_l[m - 1], st, &sigma_s);
@@ -913,7 +1012,7 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
   double q[NCV_MAX];   // row t of Q (static indices: kept in registers)
   if (!pairs) {
     const int np = m - k;
-    __shared__ double as_l[NCV_MAX], b2_l[NCV_MAX];
+    __shared__ double as_l[NCV_MAX], c2_l[NCV_MAX];
     double lo = a_l[0], hi = a_l[0];
     for (int i = 0; i < m; ++i) {
       const double r = (i < m - 1 ? fabs(b_l[i]) : 0.0) + (i > 0 ? fabs(b_l[i - 1]) : 0.0);
@@ -923,10 +1022,10 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
     // entries relative to the lower bound, over a power of two near the span
     const int ex = __builtin_amdgcn_frexp_exp(fmax(hi - lo, 1e-300));
     const double base = lo, amax = fmax(fabs(lo), fabs(hi));
-    if (t < m) {
-      as_l[t] = __builtin_amdgcn_ldexp(a_l[t] - base, -ex);
-      const double bs = t < m - 1 ? __builtin_amdgcn_ldexp(b_l[t], -ex) : 0.0;
-      b2_l[t] = bs * bs;
+    if (t < NCV_MAX) {
+      as_l[t] = t < m ? __builtin_amdgcn_ldexp(a_l[t] - base, -ex) : PAD_DIAG;
+      const double bs = t > 0 && t < m ? __builtin_amdgcn_ldexp(b_l[t - 1], -ex) : 0.0;
+      c2_l[t] = bs * bs;
     }
     __syncthreads();
     {
@@ -936,7 +1035,7 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
       if (i < np) {
         for (int it = 0; it < 20 && x1 - x0 > stop; ++it) {
           const double w = (x1 - x0) * (1.0 / (SH_LANES + 1));
-          const bool above = count_below(as_l, b2_l, m, x0 + w * (double)(l + 1)) >= idx + 1;
+          const bool above = count_below(as_l, c2_l, m, x0 + w * (double)(l + 1)) >= idx + 1;
           // the group's lanes of the ballot: points from the first `above` on
           const unsigned msk = (unsigned)(__ballot(above) >> ((t & 63) - l)) & ((1u << SH_LANES) - 1);
           const int f = msk ? __ffs((int)msk) : SH_LANES + 1;
