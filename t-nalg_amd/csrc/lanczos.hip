@@ -826,6 +826,127 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
   tnx_stamp_end(ts);
 }
 
+// k_dots, k_update_dots and k_update_norm of one Krylov step in one launch, for
+// solves of at most NG chunks: a workgroup per solve, NP lanes per chunk, the
+// basis rows and r in registers throughout and the sums through LDS.  The
+// sums are those of the three passes in the same order (a solve's result does
+// not depend on what it shares a call with).
+// Bound: latency, mostly the eigensolve's, and one CU's loads of the basis rows.
+// us a step, mean over the cycles of 20 (MI355X), and two launches fewer: one
+// chunk 8.3, two 13.3, the three passes 17.  More chunks in a workgroup would
+// read their rows (650 KB for four) at one CU's rate.
+template <typename VT, int LV, int NG>
+__device__ __forceinline__ void step_small_body(const tnx_lanczos_solve& D, const LzLayout& L,
+                                                int s, int nsolve, int j, int wd, int xd,
+                                                int min_iters, int32_t* nact_host) {
+  __shared__ double red[NG * NW][NCV_MAX + 1], rn[NG * NW];
+  __shared__ double h[NCV_MAX + 1];
+  __shared__ double a_s[NCV_MAX], b_s[NCV_MAX], y_s[NCV_MAX], work[TRI_WORK];
+  const int t = threadIdx.x, g = t / NP;
+  // lanes g NP .. g NP + NP - 1 have chunk g (elem, inside add the lane)
+  ChunkInfo ci;
+  ci.i0 = g * (CHUNK - NP);
+  ci.i1 = min(D.n, (g + 1) * CHUNK);
+  LzState& st = L.st[s];
+  VT v[LV][EPT];
+  load_rows(as_global<const VT>(D.V), D.ldv, j, ci, v);
+  double r[EPT];
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    r[q] = tnx_load((const void*)D.w, wd, elem(ci, q));
+    if (!inside(ci, q)) r[q] = 0.0;
+  }
+  if (t < j) {
+    a_s[t] = st.alpha[t];
+    b_s[t] = st.beta[t];
+  }
+  rows_dots(v, r, red);
+  __syncthreads();
+  auto total = [&](int k) {
+    double x = red_total(red, k);
+    if constexpr (NG == 2) x += red_total(red + NW, k);
+    return x;
+  };
+  if (t < LV) {
+    const double x = t <= j ? total(t) : 0.0;
+    h[t] = x;
+    if (t <= j) st.h1[t] = x;
+  }
+  __syncthreads();
+  const double h1j = h[j];
+#pragma unroll
+  for (int u = 0; u < LV; ++u) {
+    const double hu = h[u];
+#pragma unroll
+    for (int q = 0; q < EPT; ++q) r[q] -= hu * (double)v[u][q];
+  }
+  double nn = 0.0;
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) {
+    if (!inside(ci, q)) r[q] = 0.0;
+    nn += r[q] * r[q];
+  }
+  rows_dots(v, r, red);
+  nn = tnx_wave_sum(nn);
+  if ((t & 63) == 0) rn[t >> 6] = nn;
+  __syncthreads();
+  if (t <= j) {
+    h[t] = total(t);
+  } else if (t == j + 1) {
+    double x = ((rn[0] + rn[1]) + (rn[2] + rn[3])) + ((rn[4] + rn[5]) + (rn[6] + rn[7]));
+    if constexpr (NG == 2)
+      x += ((rn[8] + rn[9]) + (rn[10] + rn[11])) + ((rn[12] + rn[13]) + (rn[14] + rn[15]));
+    h[t] = x;
+  }
+  __syncthreads();
+  bool skip;
+  const double beta = new_coupling(h, j, D.v_dtype, &skip);
+  const double inv = 1.0 / beta;
+#pragma unroll
+  for (int q = 0; q < EPT; ++q) r[q] = (double)(VT)r[q];   // as the three passes park it
+  if (!skip) {
+#pragma unroll
+    for (int u = 0; u < LV; ++u) {
+      const double hu = u <= j ? h[u] : 0.0;
+#pragma unroll
+      for (int q = 0; q < EPT; ++q) r[q] -= hu * (double)v[u][q];
+    }
+  }
+  VT TNX_GLOBAL* Vn = as_global<VT>(D.V) + (int64_t)(j + 1) * D.ldv;
+#pragma unroll
+  for (int q = 0; q < EPT; ++q)
+    if (inside(ci, q)) {
+      const VT x = (VT)(r[q] * inv);
+      Vn[elem(ci, q)] = x;
+      tnx_store((void*)D.x, xd, elem(ci, q), (double)x);
+    }
+  if (t >= 64) return;
+  if (t <= j) st.h2[t] = h[t];
+  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, min_iters, a_s, b_s, y_s, work);
+  publish_nact(L, nsolve, conv, nact_host);
+}
+
+template <int LV, int NG>
+__global__ __launch_bounds__(NG * NP) void k_step_small(const tnx_lanczos_solve* __restrict__ S,
+                                                        int nsolve, void* state, int nchunks,
+                                                        int j, int w_dtype, int x_dtype,
+                                                        int min_iters, int32_t* nact_host) {
+  const LzLayout L = lz_layout(state, nsolve, nchunks);
+  const int s = (int)blockIdx.x;
+  // (only this block clears the flag in this launch, and not before the first
+  // barrier, which every lane passes after it has read the flag)
+  if (__hip_atomic_load(L.act + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+    publish_nact(L, nsolve, false, nact_host);
+    return;
+  }
+  const tnx_lanczos_solve D = S[s];
+  const int wd = dtype_of(w_dtype, D.w_dtype), xd = dtype_of(x_dtype, D.x_dtype);
+  if (D.v_dtype == TNX_F32)
+    step_small_body<float, LV, NG>(D, L, s, nsolve, j, wd, xd, min_iters, nact_host);
+  else
+    step_small_body<double, LV, NG>(D, L, s, nsolve, j, wd, xd, min_iters, nact_host);
+}
+
 // Implicit restart with the m - k largest Ritz values as shifts, from the k
 // lowest Ritz pairs (one wavefront; the pairs' vectors y[i][0..m) and values
 // th[i] in LDS).  What the shifted QR steps leave is determined by them: the
@@ -1351,6 +1472,20 @@ typedef void (*BasisKernel)(const tnx_lanczos_solve*, int, void*, int, int, int,
 struct BasisPass {
   BasisKernel dots, update_dots;
 };
+typedef void (*SmallKernel)(const tnx_lanczos_solve*, int, void*, int, int, int, int, int,
+                            int32_t*);
+// The one-launch step for solves of at most `chunks` chunks, or null: two
+// chunks are 1024 lanes, whose registers hold 20 basis rows.
+SmallKernel small_pass(int j, int chunks) {
+  static const SmallKernel one[NCV_MAX / 4] = {
+      k_step_small<4, 1>,  k_step_small<8, 1>,  k_step_small<12, 1>, k_step_small<16, 1>,
+      k_step_small<20, 1>, k_step_small<24, 1>, k_step_small<28, 1>, k_step_small<32, 1>};
+  static const SmallKernel two[5] = {k_step_small<4, 2>, k_step_small<8, 2>, k_step_small<12, 2>,
+                                     k_step_small<16, 2>, k_step_small<20, 2>};
+  if (chunks == 1) return one[j / 4];
+  return chunks == 2 && j < 20 ? two[j / 4] : nullptr;
+}
+
 BasisPass basis_pass(int j) {
   static const BasisPass table[NCV_MAX / 4] = {
       {k_dots<4>, k_update_dots<4>},   {k_dots<8>, k_update_dots<8>},
@@ -1385,6 +1520,15 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   tnx_prof_count(TNX_PC_DOTS, E * (vrows + ws));
   tnx_prof_count(TNX_PC_UPDATE_DOTS, E * (vrows + ws + vs));
   tnx_prof_count(TNX_PC_UPDATE_NORM, E * (2.0 * vs + xs));
+  // Every solve has a chunk at least, so none has more than this.  (Sampled
+  // timing keeps the three passes, which it reports one by one.)
+  const int most = nchunks - nsolve + 1;
+  if (const SmallKernel small = prof ? nullptr : small_pass(j, most)) {
+    hipLaunchKernelGGL(small, dim3(nsolve), dim3(most * NP), 0, s, solves, nsolve, state, nchunks,
+                       j, w_dtype, x_dtype, min_iters, nact_host);
+    TNX_CHECK_LAUNCH();
+    return TNX_OK;
+  }
   int mk = prof ? tnx_prof_mark(TNX_PC_DOTS, s) : -1;
   const BasisPass pass = basis_pass(j);
   hipLaunchKernelGGL(pass.dots, grid, block, 0, s, solves, nsolve, state, nchunks, j, w_dtype,
