@@ -335,15 +335,17 @@ class InfiniteRun:
                     kj.append((_vp(a.Rb, nn * N), n, d, chi,
                                [(_vp(a.Tmn, (nn * Dm + k) * d * d), d,
                                  _vp(envR, k * chi), Dm * chi, 1.0) for k in range(Dm)]))
-                segs = []
+                segs, segs_t = [], []
                 for nn in range(Dm):
                     Lp, Rp = _vp(a.Lb, nn * N), _vp(a.Rb, nn * N)
                     t0, t1 = _vp(a.T1, nn * N), _vp(a.T1, (Dm + nn) * N)
                     g1.add(t0, n, n, n, [(Lp, n, 0, x, n, 0, n, 1.0)], active=q)
                     g1.add(t1, n, n, n, [(Lp, n, 1, x, n, 0, n, 1.0)], active=q)
                     segs.append((t0, n, 0, Rp, n, 1, n, -0.5))
-                    segs.append((t1, n, 0, Rp, n, 0, n, -0.5))
-                g2.add(w, n, n, n, segs, active=q)
+                    segs_t.append((t1, n, 0, Rp, n, 0, n, -0.5))
+                # segments of one layout follow each other: the kernel streams
+                # them without a pause, and starts over at a change
+                g2.add(w, n, n, n, segs + segs_t, active=q)
                 lz.append((_vp(a.V), w, x, _vp(a.init), _vp(a.psi), N, N, min(NCV, N), 0,
                            0.0, 0.0, MPO_FLOOR, L.F64, L.F64))
                 # environment updates: Y_k = L_k A, Z_n = R_n B^T; env = A^T Y, B Z
