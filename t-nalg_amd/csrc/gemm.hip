@@ -225,12 +225,14 @@ __device__ __forceinline__ void mma_chunk(typename Tr<MODE>::V4 (&acc)[MB][MB], 
 
 // The problem that owns 64x64 tile `bid`: problems of a launch are mostly of
 // one size, so the record at its share of the range is tried first (one
-// round of loads), then the search.
+// round of loads, scalar ones, as the whole record is then mostly in the
+// cache), then the search.
 __device__ __forceinline__ int find_problem(const tnx_gemm_problem* __restrict__ probs, int nprob,
                                             int bid, int ntiles) {
-  const int guess = (int)((int64_t)bid * nprob / ntiles);
-  const int lo = probs[guess].tile_begin;
-  const int hi = guess + 1 < nprob ? probs[guess + 1].tile_begin : ntiles;
+  const tnx_gemm_problem TNX_CONST* P = (const tnx_gemm_problem TNX_CONST*)(uint64_t)probs;
+  const int guess = __builtin_amdgcn_readfirstlane((int)((int64_t)bid * nprob / ntiles));
+  const int lo = P[guess].tile_begin;
+  const int hi = guess + 1 < nprob ? P[min(guess + 1, nprob - 1)].tile_begin : ntiles;
   if (bid >= lo && bid < hi) return guess;
   return tnx_find_owner(probs, sizeof(tnx_gemm_problem), offsetof(tnx_gemm_problem, tile_begin),
                         nprob, bid);
@@ -243,10 +245,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
-
-// Descriptor records are read through the scalar cache: they do not change
-// during the launch, and the vector counter then counts operand loads only.
-#define TNX_CONST __attribute__((address_space(4)))
 
 // whether a segment's operands can be fetched by 16-byte pieces
 template <typename O, bool KA, bool KBc>
@@ -381,7 +379,11 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
   const tnx_gemm_problem TNX_CONST* cp = (const tnx_gemm_problem TNX_CONST*)(uint64_t)probs + pi;
   const tnx_gemm_seg TNX_CONST* cs = (const tnx_gemm_seg TNX_CONST*)(uint64_t)segs;
   const tnx_gemm_problem TNX_CONST& P = *cp;
-  if (P.active >= 0 && active != nullptr && active[P.active] == 0) return;
+  // (flags change between launches only: a scalar load, waited for with the
+  // records)
+  const int on = P.active >= 0 && active != nullptr
+                     ? ((const int32_t TNX_CONST*)(uint64_t)active)[P.active] : 1;
+  if (on == 0) return;
   const int tiles_n = (P.N + 63) / 64;
   const int t_local = bid - P.tile_begin;
   const int tr = t_local / tiles_n, tc = t_local - tr * tiles_n;

@@ -5,6 +5,8 @@
 // and the library's error/version entry points.
 #include <stdarg.h>
 
+#include <type_traits>
+
 #include "tnx_common.h"
 
 static thread_local std::string g_last_error;
@@ -27,238 +29,275 @@ constexpr int MIX_DMAX = 4;   // largest physical dimension (the operator table 
 // registers of a lane hold PPT x d sources and PPT x d sums either way).
 __host__ __device__ constexpr int mix_ppt(int d) { return d <= 2 ? 4 : 2; }
 
-// One lane per (a, b) pair, PPT pairs per lane: the d source values
-// src[a, :, b] of a term are loaded once and mixed by the d x d operator in
-// registers, so each output element costs one load per term.  Terms are the
-// outer loop: a term's record and operator are read once per lane, and the
-// loads of the lane's pairs are issued together.
-template <int DM>
-__device__ __forceinline__ void mix_body(const tnx_mix_job& J, int blk,
-                                         const tnx_mix_term* __restrict__ terms,
-                                         const double* __restrict__ ops) {
-  constexpr int PPT = mix_ppt(DM);
-  const int d = J.d, Dr = J.Dr;
+template <int DT> struct Elem { typedef double T; };
+template <> struct Elem<TNX_F32> { typedef float T; };
+template <> struct Elem<TNX_BF16> { typedef __bf16 T; };
+template <typename TI> __device__ __forceinline__ double widen(TI v) { return (double)v; }
+template <> __device__ __forceinline__ double widen<__bf16>(__bf16 v) { return (double)(float)v; }
+
+// a buffer whose groups of 4 elements are one piece
+__device__ __forceinline__ bool aligned4(uint64_t p, int dtype) {
+  const int isz = dtype == TNX_F64 ? 8 : dtype == TNX_F32 ? 4 : 2;
+  return (p & (uint64_t)(4 * isz - 1)) == 0;
+}
+
+// Four consecutive elements at e (a multiple of 4) of an aligned4 buffer.
+template <int DT>
+__device__ __forceinline__ void store4(uint64_t p, int64_t e, const double (&v)[4], bool add) {
+  typedef typename Elem<DT>::T TI;
+  typedef TI V4 __attribute__((ext_vector_type(4)));
+  V4 TNX_GLOBAL* d = as_global<V4>(p) + e / 4;
+  V4 o;
+  if (add) o = *d;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const double x = add ? v[q] + widen<TI>(o[q]) : v[q];
+    if constexpr (DT == TNX_BF16) o[q] = (TI)(float)x;
+    else o[q] = (TI)x;
+  }
+  *d = o;
+}
+
+// Element e of a destination of dtype DT (+)= v.
+template <int DT>
+__device__ __forceinline__ void store1(uint64_t p, int64_t e, double v, bool add) {
+  typedef typename Elem<DT>::T TI;
+  TI TNX_GLOBAL* d = as_global<TI>(p) + e;
+  if (add) v += widen<TI>(*d);
+  if constexpr (DT == TNX_BF16) *d = (TI)(float)v;
+  else *d = (TI)v;
+}
+
+// One workgroup of a job whose sources all have dtype DT: 256 lanes, PPT
+// (a, b) pairs each; the D source values of a term and pair are mixed by the
+// D x D operator in registers, so each output element costs one load per term.
+// TB terms at a time: their records, then their operators (scalar loads) and
+// every source element, before the first is used.  An element gets its terms in order, whichever instance runs
+// it (the same bits).
+// VEC (d <= 2, Dr % 4 == 0, everything aligned4): the lane's 4 pairs are
+// consecutive, in one row, and a row is one load or store; otherwise the pairs
+// are 256 apart.
+// Bound: latency for a few blocks (owner, job, terms and sources follow each
+// other), else memory.  us a matvec's launch (MI355X), by terms one at a time,
+// a record and an operator waited for in each, and now: a 30 x 27 problem 6.3
+// and 4.9; 64 of 128 x 128 in bf16 (41 MB) 20.1 and 16.4, in f64 (147 MB) 25.9
+// and 24.2.
+template <int D, bool VEC, int DT, int TB>
+__device__ __forceinline__ void mix_body(const tnx_mix_job TNX_CONST& J, int blk,
+                                         const tnx_mix_term TNX_CONST* T,
+                                         const double TNX_CONST* ops) {
+  constexpr int PPT = mix_ppt(D);
+  static_assert(!VEC || PPT == 4, "a row's piece is 4 elements");
+  typedef typename Elem<DT>::T TI;
+  typedef TI V4 __attribute__((ext_vector_type(4)));
+  const int Dr = J.Dr, count = J.term_count;
   const int npairs = J.Dl * Dr;
-  const int base = blk * 256 * PPT;
-  int64_t e0[PPT];  // element (a, 0, b) of each pair
+  int64_t e0[PPT];  // element (a, 0, b) of each pair (past the end: of the last one)
   bool ok[PPT];
 #pragma unroll
   for (int q = 0; q < PPT; ++q) {
-    const int p = base + q * 256 + threadIdx.x;
+    const int p = blk * 256 * PPT + (VEC ? 4 * (int)threadIdx.x + q : q * 256 + (int)threadIdx.x);
     ok[q] = p < npairs;
-    const int a = ok[q] ? p / Dr : 0;
-    e0[q] = ok[q] ? (int64_t)a * d * Dr + (p - a * Dr) : 0;
-  }
-  double acc[PPT][DM];
-#pragma unroll
-  for (int q = 0; q < PPT; ++q)
-#pragma unroll
-    for (int s = 0; s < DM; ++s) acc[q][s] = 0.0;
-  for (int ti = J.term_begin; ti < J.term_begin + J.term_count; ++ti) {
-    const tnx_mix_term T = terms[ti];
-    double x[PPT][DM];
-#pragma unroll
-    for (int q = 0; q < PPT; ++q)
-#pragma unroll
-      for (int t = 0; t < DM; ++t)
-        x[q][t] = (ok[q] && t < d) ? tnx_load((const void*)T.src, T.src_dtype,
-                                              e0[q] + (int64_t)t * Dr) : 0.0;
-    if (T.op < 0) {
-#pragma unroll
-      for (int q = 0; q < PPT; ++q)
-#pragma unroll
-        for (int s = 0; s < DM; ++s) acc[q][s] += T.coef * x[q][s];
+    if (VEC && q > 0) {
+      e0[q] = e0[0] + q;
     } else {
-      double O[DM * DM];
-      const double* Op = ops + (int64_t)T.op * d * d;
-#pragma unroll
-      for (int s = 0; s < DM; ++s)
-#pragma unroll
-        for (int t = 0; t < DM; ++t)
-          O[s * DM + t] = (s < d && t < d) ? Op[s * d + t] : 0.0;
-#pragma unroll
-      for (int q = 0; q < PPT; ++q)
-#pragma unroll
-        for (int s = 0; s < DM; ++s) {
-          if (s < d) {
-            double v = 0.0;
-#pragma unroll
-            for (int t = 0; t < DM; ++t)
-              if (t < d) v += O[s * DM + t] * x[q][t];
-            acc[q][s] += T.coef * v;
-          }
-        }
+      const int pc = min(p, npairs - (VEC ? 4 : 1));
+      const int a = pc / Dr;
+      e0[q] = (int64_t)a * D * Dr + (pc - a * Dr);
     }
   }
+  double acc[D][PPT];
 #pragma unroll
-  for (int q = 0; q < PPT; ++q) {
-    if (!ok[q]) continue;
+  for (int s = 0; s < D; ++s)
 #pragma unroll
-    for (int s = 0; s < DM; ++s) {
-      if (s < d) {
-        const int64_t e = e0[q] + (int64_t)s * Dr;
-        double v = acc[q][s];
-        if (J.accumulate) v += tnx_load((const void*)J.dst, J.dst_dtype, e);
-        tnx_store((void*)J.dst, J.dst_dtype, e, v);
+    for (int q = 0; q < PPT; ++q) acc[s][q] = 0.0;
+  for (int t0 = 0; t0 < count; t0 += TB) {
+    const int n = count - t0;
+    uint64_t src[TB];
+    double coef[TB], O[TB][D * D];
+    int op[TB];
+    TI x[TB][D][PPT];
+#pragma unroll
+    for (int u = 0; u < TB; ++u) {
+      const tnx_mix_term TNX_CONST& t = T[min(t0 + u, count - 1)];
+      src[u] = t.src;
+      coef[u] = t.coef;
+      op[u] = t.op;
+    }
+#pragma unroll
+    for (int u = 0; u < TB; ++u) {
+      const double TNX_CONST* Op = ops + (int64_t)max(op[u], 0) * (D * D);
+      if (op[u] >= 0) {
+#pragma unroll
+        for (int k = 0; k < D * D; ++k) O[u][k] = Op[k];
       }
     }
-  }
-}
-
-// Four consecutive elements [e, e + 4) of a buffer of runtime dtype, as
-// double; the caller guarantees that e is a multiple of 4 and the buffer
-// 4-element aligned, so the load is one 8-, 16- or two 16-byte accesses.
-// The conversions are tnx_load's.
-__device__ __forceinline__ void tnx_load4(const void* p, int dtype, int64_t e, double (&v)[4]) {
-  if (dtype == TNX_F64) {
-    const double2 a = *(const double2*)((const double*)p + e);
-    const double2 b = *(const double2*)((const double*)p + e + 2);
-    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-  } else if (dtype == TNX_F32) {
-    const float4 a = *(const float4*)((const float*)p + e);
-    v[0] = (double)a.x; v[1] = (double)a.y; v[2] = (double)a.z; v[3] = (double)a.w;
-  } else {
-    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-    const bf4 a = *(const bf4*)((const __bf16*)p + e);
-    v[0] = (double)(float)a[0]; v[1] = (double)(float)a[1];
-    v[2] = (double)(float)a[2]; v[3] = (double)(float)a[3];
-  }
-}
-
-__device__ __forceinline__ void tnx_store4(void* p, int dtype, int64_t e, const double (&v)[4]) {
-  if (dtype == TNX_F64) {
-    *(double2*)((double*)p + e) = make_double2(v[0], v[1]);
-    *(double2*)((double*)p + e + 2) = make_double2(v[2], v[3]);
-  } else if (dtype == TNX_F32) {
-    *(float4*)((float*)p + e) = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
-  } else {
-    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-    bf4 a;
-    a[0] = (__bf16)(float)v[0]; a[1] = (__bf16)(float)v[1];
-    a[2] = (__bf16)(float)v[2]; a[3] = (__bf16)(float)v[3];
-    *(bf4*)((__bf16*)p + e) = a;
-  }
-}
-
-__device__ __forceinline__ bool aligned4(const void* p, int dtype) {
-  const int isz = dtype == TNX_F64 ? 8 : dtype == TNX_F32 ? 4 : 2;
-  return ((uintptr_t)p & (uintptr_t)(4 * isz - 1)) == 0;
-}
-
-// d <= 2 jobs whose rows hold a multiple of 4 pairs (Dr % 4 == 0): lane t
-// takes the 4 consecutive pairs [base + 4t, base + 4t + 4), all in one row,
-// so each source row of a term is one vector load per lane and a wave reads
-// 256 consecutive elements.  Same arithmetic per element as mix_body (terms
-// in order, the operator applied to the d sources of the pair), so the same
-// bits.  A term or destination that is not 4-element aligned takes scalar
-// accesses.
-__device__ __forceinline__ void mix_body_vec2(const tnx_mix_job& J, int blk,
-                                              const tnx_mix_term* __restrict__ terms,
-                                              const double* __restrict__ ops) {
-  const int d = J.d, Dr = J.Dr;
-  const int npairs = J.Dl * Dr;
-  const int p0 = blk * 256 * 4 + 4 * threadIdx.x;
-  if (p0 >= npairs) return;
-  const int a = p0 / Dr;
-  const int64_t e0 = (int64_t)a * d * Dr + (p0 - a * Dr);
-  double acc[2][4];
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
+    for (int u = 0; u < TB; ++u)
+      if (u < n) {
+        const TI TNX_GLOBAL* sp = as_global<const TI>(src[u]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[s][q] = 0.0;
-  for (int ti = J.term_begin; ti < J.term_begin + J.term_count; ++ti) {
-    const tnx_mix_term T = terms[ti];
-    double x[2][4];
-    const bool vec = aligned4((const void*)T.src, T.src_dtype);
+        for (int t = 0; t < D; ++t) {
+          const int64_t row = (int64_t)t * Dr;
+          if constexpr (VEC) {
+            const V4 v = *(const V4 TNX_GLOBAL*)(sp + e0[0] + row);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if (t < d) {
-        if (vec) {
-          tnx_load4((const void*)T.src, T.src_dtype, e0 + (int64_t)t * Dr, x[t]);
+            for (int q = 0; q < 4; ++q) x[u][t][q] = v[q];
+          } else {
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) x[u][t][q] = sp[e0[q] + row];
+          }
+        }
+      }
+#pragma unroll
+    for (int u = 0; u < TB; ++u)
+      if (u < n) {
+        double w[D][PPT];
+#pragma unroll
+        for (int t = 0; t < D; ++t)
+#pragma unroll
+          for (int q = 0; q < PPT; ++q) w[t][q] = widen<TI>(x[u][t][q]);
+        if (op[u] < 0) {
+#pragma unroll
+          for (int s = 0; s < D; ++s)
+#pragma unroll
+            for (int q = 0; q < PPT; ++q) acc[s][q] += coef[u] * w[s][q];
         } else {
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            x[t][q] = tnx_load((const void*)T.src, T.src_dtype, e0 + (int64_t)t * Dr + q);
-        }
-      } else {
+          for (int s = 0; s < D; ++s)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[t][q] = 0.0;
+            for (int q = 0; q < PPT; ++q) {
+              double m = 0.0;
+#pragma unroll
+              for (int t = 0; t < D; ++t) m += O[u][s * D + t] * w[t][q];
+              acc[s][q] += coef[u] * m;
+            }
+        }
       }
-    }
-    if (T.op < 0) {
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc[s][q] += T.coef * x[s][q];
-    } else {
-      double O[4];
-      const double* Op = ops + (int64_t)T.op * d * d;
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) O[s * 2 + t] = (s < d && t < d) ? Op[s * d + t] : 0.0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          if (s < d) {
-            double v = 0.0;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-              if (t < d) v += O[s * 2 + t] * x[t][q];
-            acc[s][q] += T.coef * v;
-          }
-        }
-    }
   }
-  const bool vec = aligned4((const void*)J.dst, J.dst_dtype);
+  const bool add = J.accumulate != 0;
+  auto store = [&](auto tag) {
+    constexpr int DD = decltype(tag)::value;
 #pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    if (s < d) {
-      const int64_t e = e0 + (int64_t)s * Dr;
-      double v[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = acc[s][q];
-      if (vec) {
-        if (J.accumulate) {
-          double o[4];
-          tnx_load4((const void*)J.dst, J.dst_dtype, e, o);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) v[q] += o[q];
-        }
-        tnx_store4((void*)J.dst, J.dst_dtype, e, v);
+    for (int s = 0; s < D; ++s) {
+      const int64_t row = (int64_t)s * Dr;
+      if constexpr (VEC) {
+        if (ok[0]) store4<DD>(J.dst, e0[0] + row, acc[s], add);
       } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          double w = v[q];
-          if (J.accumulate) w += tnx_load((const void*)J.dst, J.dst_dtype, e + q);
-          tnx_store((void*)J.dst, J.dst_dtype, e + q, w);
-        }
+        for (int q = 0; q < PPT; ++q)
+          if (ok[q]) store1<DD>(J.dst, e0[q] + row, acc[s][q], add);
       }
     }
+  };
+  if (J.dst_dtype == TNX_F64) store(std::integral_constant<int, TNX_F64>());
+  else if (J.dst_dtype == TNX_F32) store(std::integral_constant<int, TNX_F32>());
+  else store(std::integral_constant<int, TNX_BF16>());
+}
+
+// The same for a job whose sources differ in dtype: element by element.
+__device__ __forceinline__ void mix_mixed(const tnx_mix_job TNX_CONST& J, int blk,
+                                          const tnx_mix_term TNX_CONST* T,
+                                          const double TNX_CONST* ops) {
+  const int d = J.d, Dr = J.Dr, per = 256 * mix_ppt(d);
+  const int end = min(J.Dl * Dr, (blk + 1) * per);
+  for (int p = blk * per + (int)threadIdx.x; p < end; p += 256) {
+    const int a = p / Dr;
+    const int64_t e0 = (int64_t)a * d * Dr + (p - a * Dr);
+    double acc[MIX_DMAX] = {0.0, 0.0, 0.0, 0.0};
+    for (int u = 0; u < J.term_count; ++u) {
+      const double coef = T[u].coef;
+      double x[MIX_DMAX];
+#pragma unroll
+      for (int t = 0; t < MIX_DMAX; ++t)
+        x[t] = tnx_load((const void*)T[u].src, T[u].src_dtype, e0 + (int64_t)min(t, d - 1) * Dr);
+      const double TNX_CONST* O = ops + (int64_t)max(T[u].op, 0) * d * d;
+#pragma unroll
+      for (int s = 0; s < MIX_DMAX; ++s) {
+        double m = x[s];
+        if (T[u].op >= 0) {
+          m = 0.0;
+#pragma unroll
+          for (int t = 0; t < MIX_DMAX; ++t)
+            if (s < d && t < d) m += O[s * d + t] * x[t];
+        }
+        acc[s] += coef * m;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < MIX_DMAX; ++s)
+      if (s < d) {
+        const int64_t e = e0 + (int64_t)s * Dr;
+        if (J.accumulate) acc[s] += tnx_load((const void*)J.dst, J.dst_dtype, e);
+        tnx_store((void*)J.dst, J.dst_dtype, e, acc[s]);
+      }
   }
 }
 
-// TAG only names the instance: 1 for the matvec's mixer (so profiles can tell
-// its launches from the environment, cast and copy mixes), 0 otherwise.
-template <int TAG>
+// The job that owns block `bid`: jobs of a launch are mostly of one size, so
+// the record at its share of the range is tried first, then the search.
+__device__ __forceinline__ int find_job(const tnx_mix_job* jobs, int njob, int bid, int nblocks) {
+  const tnx_mix_job TNX_CONST* J = (const tnx_mix_job TNX_CONST*)(uint64_t)jobs;
+  const int guess = __builtin_amdgcn_readfirstlane((int)((int64_t)bid * njob / nblocks));
+  const int lo = J[guess].block_begin;
+  const int hi = guess + 1 < njob ? J[min(guess + 1, njob - 1)].block_begin : nblocks;
+  if (bid >= lo && bid < hi) return guess;
+  return tnx_find_owner(jobs, sizeof(tnx_mix_job), offsetof(tnx_mix_job, block_begin), njob, bid);
+}
+
+// DT: the matvec's mixer, whose sources have the dtype of its first GEMM's
+// operands (a job with others goes element by element); -1: any mix.  With
+// one dtype's bodies the bf16 instance needs 77 registers instead of 99, and
+// more workgroups are in flight.
+template <int DT>
 __global__ __launch_bounds__(256) void mix_kernel(const tnx_mix_job* __restrict__ jobs, int njob,
                                                   const tnx_mix_term* __restrict__ terms,
                                                   const double* __restrict__ ops,
                                                   const int32_t* __restrict__ active,
                                                   unsigned long long* ts) {
   tnx_stamp_begin(ts);
-  const int bid = blockIdx.x;
-  const int ji = tnx_find_owner(jobs, sizeof(tnx_mix_job), offsetof(tnx_mix_job, block_begin),
-                                njob, bid);
-  const tnx_mix_job J = jobs[ji];
-  if (J.active >= 0 && active != nullptr && active[J.active] == 0) return;
-  if (J.d <= 2 && J.Dr % 4 == 0)
-    mix_body_vec2(J, bid - J.block_begin, terms, ops);
-  else if (J.d <= 2)
-    mix_body<2>(J, bid - J.block_begin, terms, ops);
-  else
-    mix_body<MIX_DMAX>(J, bid - J.block_begin, terms, ops);
+  const int bid = tnx_xcd_remap(blockIdx.x, gridDim.x);
+  const int ji = __builtin_amdgcn_readfirstlane(find_job(jobs, njob, bid, gridDim.x));
+  const tnx_mix_job TNX_CONST& J = ((const tnx_mix_job TNX_CONST*)(uint64_t)jobs)[ji];
+  const int on = J.active >= 0 && active != nullptr
+                     ? ((const int32_t TNX_CONST*)(uint64_t)active)[J.active] : 1;
+  if (on == 0) return;
+  const double TNX_CONST* O = (const double TNX_CONST*)(uint64_t)ops;
+  const int blk = bid - J.block_begin;
+  // the sources' dtype and alignments
+  const tnx_mix_term TNX_CONST* T = (const tnx_mix_term TNX_CONST*)(uint64_t)terms + J.term_begin;
+  const int count = J.term_count, dt = count > 0 ? T[0].src_dtype : TNX_F64;
+  bool same = true, vec = J.d <= 2 && J.Dr % 4 == 0 && aligned4(J.dst, J.dst_dtype);
+  for (int u0 = 0; u0 < count; u0 += 4)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const tnx_mix_term TNX_CONST& t = T[min(u0 + u, count - 1)];
+      same = same && t.src_dtype == dt;
+      vec = vec && aligned4(t.src, t.src_dtype);
+    }
+#define TNX_MIX(DT)                                                  \
+  if (vec && J.d == 2) mix_body<2, true, DT, 4>(J, blk, T, O);       \
+  else if (vec) mix_body<1, true, DT, 4>(J, blk, T, O);              \
+  else if (J.d == 1) mix_body<1, false, DT, 4>(J, blk, T, O);        \
+  else if (J.d == 2) mix_body<2, false, DT, 2>(J, blk, T, O);        \
+  else if (J.d == 3) mix_body<3, false, DT, 1>(J, blk, T, O);        \
+  else mix_body<4, false, DT, 1>(J, blk, T, O)
+  if constexpr (DT >= 0) {
+    if (same && dt == DT) {
+      TNX_MIX(DT);
+    } else {
+      mix_mixed(J, blk, T, O);
+    }
+  } else if (!same) {
+    mix_mixed(J, blk, T, O);
+  } else if (dt == TNX_F64) {
+    TNX_MIX(TNX_F64);
+  } else if (dt == TNX_F32) {
+    TNX_MIX(TNX_F32);
+  } else {
+    TNX_MIX(TNX_BF16);
+  }
+#undef TNX_MIX
   tnx_stamp_end(ts);
 }
 
@@ -395,26 +434,26 @@ extern "C" int tnx_abi_sizes(int32_t* sizes, int n) {
 }
 
 static int launch_mix(const tnx_mix_job* job, int njob, const tnx_mix_term* term, int nblocks,
-                      const double* ops, const int32_t* active, tnx_stream_t stream, bool matvec,
+                      const double* ops, const int32_t* active, tnx_stream_t stream, int dt,
                       unsigned long long* ts = nullptr) {
   if (nblocks == 0 || njob == 0) return TNX_OK;
   if (job == nullptr || term == nullptr || nblocks < 0 || njob < 0) {
     tnx_set_error("tnx_mix: bad arguments (njob=%d nblocks=%d)", njob, nblocks);
     return TNX_EINVAL;
   }
-  if (matvec)
-    hipLaunchKernelGGL(mix_kernel<1>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, job, njob,
-                       term, ops, active, ts);
-  else
-    hipLaunchKernelGGL(mix_kernel<0>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, job, njob,
-                       term, ops, active, ts);
+  auto kernel = dt == TNX_F64    ? mix_kernel<TNX_F64>
+                : dt == TNX_F32  ? mix_kernel<TNX_F32>
+                : dt == TNX_BF16 ? mix_kernel<TNX_BF16>
+                                 : mix_kernel<-1>;
+  hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, job, njob, term, ops,
+                     active, ts);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }
 
 extern "C" int tnx_mix(const tnx_mix_job* job, int njob, const tnx_mix_term* term, int nblocks,
                        const double* ops, const int32_t* active, tnx_stream_t stream) {
-  return launch_mix(job, njob, term, nblocks, ops, active, stream, false);
+  return launch_mix(job, njob, term, nblocks, ops, active, stream, -1);
 }
 
 extern "C" int tnx_trace_dot(const tnx_dot_job* jobs, int njob, double* out, tnx_stream_t stream) {
@@ -454,8 +493,10 @@ extern "C" int tnx_heff_matvec(const tnx_matvec_plan* plan, const int32_t* activ
   if (rc) return rc;
   tnx_prof_done(mk, s, plan->work[0]);
   mk = (prof && plan->mix_nblocks > 0) ? tnx_prof_mark(TNX_PC_MIX, s) : -1;
+  const int m1 = plan->mode & 0xff;
   rc = launch_mix(plan->mix_job, plan->mix_njob, plan->mix_term, plan->mix_nblocks, plan->ops, active,
-                  stream, true, tnx_prof_ts(mk));
+                  stream, m1 == TNX_GEMM_F64 ? TNX_F64 : m1 == TNX_GEMM_F32 ? TNX_F32 : TNX_BF16,
+                  tnx_prof_ts(mk));
   if (rc) return rc;
   tnx_prof_done(mk, s, plan->work[1]);
   mk = prof ? tnx_prof_mark(gemm_class(plan->mode2, 1), s) : -1;

@@ -94,6 +94,10 @@ template <typename T> __device__ __forceinline__ T TNX_GLOBAL* as_global(uint64_
   return (T TNX_GLOBAL*)p;
 }
 
+// Descriptor records are read through the scalar cache: nothing changes them
+// during a launch, and the vector counter then counts operand loads only.
+#define TNX_CONST __attribute__((address_space(4)))
+
 // Load element idx of a buffer (global memory) of runtime dtype as double.
 __device__ __forceinline__ double tnx_load(const void* p, int dtype, int64_t idx) {
   const uint64_t a = (uint64_t)p;

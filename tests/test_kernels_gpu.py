@@ -1228,3 +1228,51 @@ def test_lanczos_chunk_edges(gpu, v32, alone):
         th = np.linalg.eigvalsh(B[:ncv] @ H @ B[:ncv].T)[0]
         assert abs(r['theta'] - th) < 10 * tol, (n, r, th)
         assert abs(np.linalg.norm(out) - 1) < 10 * tol, n
+
+
+@pytest.mark.parametrize('d', [1, 2, 3, 4])
+@pytest.mark.parametrize('nterm', [1, 2, 4, 5, 9])
+def test_mix_term_batches(gpu, d, nterm):
+    """Numbers of terms around the batch of 4, every physical dimension, rows
+    with and without a multiple of 4 pairs, a job over several workgroups, and
+    sources of one or of mixed dtypes: numpy on the rounded inputs to 1e-13 of
+    the largest entry, and the same bits from a destination that is not
+    4-element aligned."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    rng = np.random.RandomState(10 * d + nterm)
+    ops = rng.randn(5, d, d)
+    opsd = _dev(ops.reshape(-1))
+    kinds = [(torch.float64, L.F64), (torch.float32, L.F32), (torch.bfloat16, L.BF16)]
+    mx = R.MixList()
+    keep, expect, outs = [], [], []
+    for (Dl, Dr) in [(7, 8), (5, 3), (70, 36), (41, 33)]:
+        for mixed in (0, 1):
+            terms, ref = [], np.zeros((Dl, d, Dr))
+            for k in range(nterm):
+                tt, code = kinds[k % 3 if mixed else (Dl + Dr) % 3]
+                x = torch.from_numpy(rng.randn(Dl, d, Dr)).to(tt).cuda()
+                keep.append(x)
+                xr = x.to(torch.float64).cpu().numpy()
+                op = (k % 6) - 1
+                c = rng.randn()
+                terms.append((x.data_ptr(), code, c, op))
+                ref = ref + c * (xr if op < 0 else np.einsum('st,atb->asb', ops[op], xr))
+            for shift in (0, 1):
+                dst = torch.zeros(Dl * d * Dr + 1, dtype=torch.float64, device='cuda')
+                outs.append(dst[shift:shift + Dl * d * Dr])
+                expect.append(ref)
+                mx.add(outs[-1].data_ptr(), L.F64, Dl, d, Dr, terms)
+    j, t = mx.arrays()
+    dj, dt = _upload([j, t])
+    print('mix batches d', d, 'terms', nterm, flush=True)
+    L.check(lib.tnx_mix(_vp(dj.data_ptr()), len(j), _vp(dt.data_ptr()), R.mix_blocks(j),
+                        _vp(opsd.data_ptr()), None, _stream()), 'mix')
+    torch.cuda.synchronize()
+    got = [o.cpu().numpy() for o in outs]
+    for k, (g, r) in enumerate(zip(got, expect)):
+        assert np.abs(g - r.reshape(-1)).max() <= 1e-13 * max(np.abs(r).max(), 1.0), (k, r.shape)
+    for k in range(0, len(got), 2):
+        assert np.array_equal(got[k], got[k + 1]), k
