@@ -248,18 +248,6 @@ __device__ __forceinline__ void reduce_partials(const double* part, int nchunks,
   }
 }
 
-// 1 / d to working accuracy (the hardware's approximation, third order)
-__device__ __forceinline__ double fast_rcp(double d) {
-  const double r = __builtin_amdgcn_rcp(d);
-  const double e = fma(-d, r, 1.0);
-  return fma(r, fma(e, e, e), r);
-}
-__device__ __forceinline__ double fast_rsqrt(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(0.375, e, 0.5), y);
-}
-
 // A symmetric tridiagonal problem in LDS, scaled: rows 0..pad_rows(k) - 1 with
 // diagonal a[i] and squared couplings c2[i] of rows i - 1 and i (c2[0] = 0),
 // entries of order one or less; rows from k on are decoupled, above the
@@ -348,7 +336,7 @@ __device__ __forceinline__ double multisect(const double* a, const double* c2, i
     if (f < 64) hi = xu;
     if (f > 0) lo = xl;
     const bool gained = 65.0 * (hi - lo) <= w;
-    g = lo + (hi - lo) * vl * fast_rcp(vl - vu);
+    g = lo + (hi - lo) * vl * tnx_rcp(vl - vu);
     secant = both && (gained || !secant) && g > lo && g < hi && ((vl < 0.0) != (vu < 0.0));
   }
   return 0.5 * (lo + hi);
@@ -446,8 +434,8 @@ __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, i
   if (in) {
     const double t1 = mn[lane], t0 = mn[NCV_MAX + lane];
     const double u1 = mn[2 * NCV_MAX + lane], u0 = mn[3 * NCV_MAX + lane];
-    dt = fabs(t0) < 1e-290 ? 1e150 : t1 * fast_rcp(t0);
-    db = fabs(u0) < 1e-290 ? 1e150 : u1 * fast_rcp(u0);
+    dt = fabs(t0) < 1e-290 ? 1e150 : t1 * tnx_rcp(t0);
+    db = fabs(u0) < 1e-290 ? 1e150 : u1 * tnx_rcp(u0);
     if (fabs(dt) < tiny) dt = tiny;
     if (fabs(db) < tiny) db = tiny;
   }
@@ -456,8 +444,8 @@ __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, i
   const int r = __ffsll((long long)__ballot(gam == gmin)) - 1;
   // ratio of z_lane to its neighbour on the side of r, then running products
   double z = 1.0;
-  if (in && lane < r) z = -__builtin_amdgcn_ldexp(bl, -ex) * fast_rcp(dt);
-  else if (in && lane > r) z = -__builtin_amdgcn_ldexp(bm, -ex) * fast_rcp(db);
+  if (in && lane < r) z = -__builtin_amdgcn_ldexp(bl, -ex) * tnx_rcp(dt);
+  else if (in && lane > r) z = -__builtin_amdgcn_ldexp(bm, -ex) * tnx_rcp(db);
 #pragma unroll
   for (int o = 1; o < NCV_MAX; o <<= 1) {
     const int from = lane < r ? lane + o : lane - o;
@@ -465,7 +453,7 @@ __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, i
     if (lane < r ? from < r : from > r) z *= v;
   }
   z = in ? z : 0.0;
-  double f = fast_rsqrt(tnx_wave_sum(z * z));
+  double f = tnx_rsqrt(tnx_wave_sum(z * z));
   if (tnx_wave_sum(z) < 0.0) f = -f;
   if (in) y[lane] = z * f;
   if (lane == 0) *theta = base + __builtin_amdgcn_ldexp(th, ex);
@@ -978,7 +966,7 @@ __device__ __forceinline__ bool restart_from_pairs(double (*y)[NCV_MAX], const d
         for (int q = 0; q < i; ++q) v[i] -= tnx_wave_sum(v[q] * v[i]) * v[q];
         const double nn = tnx_wave_sum(v[i] * v[i]);
         if (!(nn > 1e-4)) return false;
-        v[i] *= fast_rsqrt(nn);
+        v[i] *= tnx_rsqrt(nn);
       }
   // From here every lane computes the same k x k numbers: z[c][i] is the
   // component of new vector c along Ritz vector i.
@@ -1099,7 +1087,7 @@ __device__ __forceinline__ bool restart_from_pairs(double (*y)[NCV_MAX], const d
 // converged with its current Ritz pair.
 // Bound: latency, a few serial chains over m rows.  us for m = 20 (MI355X):
 // the QR steps with a library square root and one lane's bisection per shift
-// 164, with fast_rsqrt and SH_LANES lanes 103, from the Ritz pairs 14.4.
+// 164, with tnx_rsqrt and SH_LANES lanes 103, from the Ritz pairs 14.4.
 constexpr int SH_LANES = 8;   // NT / NCV_MAX: every shift at once
 __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __restrict__ S,
                                                   int nsolve, void* state, int nchunks, int m,
@@ -1193,7 +1181,7 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
             // chain, and its entries are O(|T|), far from over- or underflow
             double c = 1.0, sn = 0.0;
             if (z != 0.0) {
-              const double ri = fast_rsqrt(x * x + z * z);
+              const double ri = tnx_rsqrt(x * x + z * z);
               c = x * ri;
               sn = z * ri;
             }

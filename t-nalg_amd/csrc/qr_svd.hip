@@ -6,7 +6,6 @@
 
 namespace {
 
-constexpr int NT = 256;
 constexpr int NQ = 1024;    // lanes of the QR and SVD kernels
 constexpr int KMAX = 4096;  // max columns of a gauge-move matrix
 
@@ -574,49 +573,34 @@ __global__ __launch_bounds__(NQ) void svd_kernel(const tnx_svd_job* __restrict__
   }
 }
 
-// Cholesky factor + inverse of one n x n SPD matrix (n <= 128), 256 lanes,
+// Cholesky factor + inverse of one n x n SPD matrix (n <= 128), 1024 lanes,
 // in 16 x 16 blocks (nb = ceil(n / 16) block rows; the padding is the
 // identity).  Right-looking, with the inverse carried along: eliminating
 // [S | I] = R^T [R | F] gives R and F = R^{-T}, so R^{-1} = F^T comes out of
 // the same steps.  Per panel p:
 //   1. the owner wave of the diagonal block factors S_pp = R_pp^T R_pp in
-//      registers (the block in the v_mfma_f64_16x16x4_f64 output layout,
-//      row k read by lane shuffles, one reciprocal square root per step),
-//      F_pp = R_pp^{-T} from the same steps;
+//      registers, a column a lane, F_pp = R_pp^{-T} from the same steps;
 //   2. row panel p on MFMA: R_pb = F_pp S_pb (b > p), F_pe = F_pp E_pe (e < p);
 //   3. trailing update on MFMA: S_ab -= R_pa^T R_pb (p < a <= b) and
 //      E_ae -= R_pa^T F_pe (a > p, e <= p).
-// Wave w owns block columns w and 7 - w of the upper part (S -> R) and of
-// the strictly lower part (E -> F): 16 blocks of 4 accumulator registers per
-// lane, about the same work per wave in every phase.  The owner of the next
-// diagonal block updates it first and factors it while the other waves
-// finish the trailing update; two barriers per panel.  LDS holds the row
-// panels as they are formed (R above the diagonal, F below it, F_pp in its
-// own buffer), which are the MFMA operands of the later phases and the
-// output at the end.
+// The 8 x 8 blocks (the upper part S -> R, the strictly lower one E -> F) are
+// dealt to the 4 x 4 waves cyclically, four accumulator blocks a wave.  The
+// owner of the next diagonal block updates it first and factors it while the
+// other waves finish the trailing update; two barriers per panel.  An
+// accumulator block is in the layout of the MFMA's B operand, so the row panel
+// is formed in its owners' registers.  LDS holds the row panels as they are
+// formed (R above the diagonal, F below it, F_pp in its own buffer), which are
+// the operands of the later phases and the output at the end.
+// Bound: the serial chain of the diagonal blocks, 16 pivots each.  us (MI355X),
+// with 256 lanes and the diagonal block in the MFMA layout, its rows moved by
+// lane shuffles, and now: n = 128 57 and 30, the chains of a run at chi 64
+// (n <= 128) 18.9 and 12.7, at chi 16 (n <= 32) 6.3 and 4.8.
+constexpr int NC = 1024;
 constexpr int CHOL_NMAX = 128;
 constexpr double CHOL_NEAR_ID = 1e-10;  // largest |S - I| entry of the first-order path
 constexpr int CB_LD = CHOL_NMAX + 1;    // LDS row stride: row and column reads hit distinct banks
 constexpr int CB_XLD = 17;              // row stride of the F_pp blocks
 constexpr size_t CHOL_LDS = sizeof(double) * (CHOL_NMAX * CB_LD + 8 * 16 * CB_XLD);
-
-// block (a, b) of accumulator slot s of wave w: slots 0, 1 the diagonal
-// blocks (w, w), (7-w, 7-w); 2..8 the blocks above them in those columns;
-// 9..15 the blocks below them (the F part)
-__device__ __forceinline__ void chol_slot(int w, int s, int& a, int& b) {
-  const int c0 = w, c1 = 7 - w;
-  if (s == 0) {
-    a = c0; b = c0;
-  } else if (s == 1) {
-    a = c1; b = c1;
-  } else if (s <= 8) {
-    const int t = s - 2;
-    if (t < w) { a = t; b = c0; } else { a = t - w; b = c1; }
-  } else {
-    const int t = s - 9;
-    if (t < 7 - w) { a = c0 + 1 + t; b = c0; } else { a = 8 - w + (t - (7 - w)); b = c1; }
-  }
-}
 
 // 16 x 16 block in the MFMA output layout: row (lane / 16) + 4 r, column lane % 16
 __device__ __forceinline__ tnx_d4 chol_ld(const double* p, int ld, int lane) {
@@ -650,93 +634,115 @@ __device__ __forceinline__ double chol_readlane(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// d (the diagonal block, output layout) -> R_pp with zeros below the
-// diagonal; f -> F_pp = R_pp^{-T}.  Step k: R[k][j] = D[k][j] / sqrt(D[k][k])
-// (j > k), F[k][j] = E[k][j] / sqrt(D[k][k]); rows i > k lose R[k][i] times
-// row k of R and of F.  Row k sits in lanes 16 (k % 4) .. +15, register k / 4.
-__device__ __forceinline__ void chol_diag(tnx_d4& d, tnx_d4& f, int lane, int& bad) {
-  const int j = lane & 15, g = lane >> 4;
+// The diagonal block D (LDS, 16 rows of CB_LD) -> R_pp with zeros below the
+// diagonal; F (16 rows of CB_XLD) = R_pp^{-T}.  One wave: lane j < 16 holds
+// column j of D, lane 16 + j that of E (the identity at first).  Step k: row k
+// of both times 1 / sqrt(D[k][k]); rows i > k lose R[k][i], a lane's value read
+// into a scalar, times row k.  Row k + 1 goes first, so that the root of its
+// pivot is under way while the others are updated.
+__device__ __forceinline__ void chol_diag(double* D, double* F, int lane, int& bad) {
+  const int j = lane & 15;
+  const bool inv = lane & 16;
+  double d[16];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) f[r] = (g + 4 * r == j) ? 1.0 : 0.0;
+  for (int i = 0; i < 16; ++i) d[i] = inv ? (i == j ? 1.0 : 0.0) : D[i * CB_LD + j];
+  double piv = chol_readlane(d[0], 0);
+  double x = fmax(piv, 1e-300), y = __builtin_amdgcn_rsq(x);   // (not positive, NaN: 1e-300)
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    const int kr = k >> 2, src = 16 * (k & 3);
-    double piv = chol_readlane(d[kr], src + k);
-    const double dkj = __shfl(d[kr], src + j, 64);
-    const double ekj = __shfl(f[kr], src + j, 64);
-    double dki[4];
+    bad |= !(piv > 0.0);
+    // sqrt(piv) = piv / sqrt(piv): one root on the serial chain
+    d[k] = (lane == k ? x : d[k]) * tnx_rsqrt_step(x, y);
+    if (k == 15) break;
+    d[k + 1] = fma(-chol_readlane(d[k], k + 1), d[k], d[k + 1]);
+    piv = chol_readlane(d[k + 1], k + 1);
+    x = fmax(piv, 1e-300);
+    y = __builtin_amdgcn_rsq(x);
+    __builtin_amdgcn_sched_barrier(0);
+    double r[16];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) dki[r] = __shfl(d[kr], src + g + 4 * r, 64);
-    if (!(piv > 0.0)) {
-      piv = 1e-300;
-      bad = 1;
-    }
-    // one reciprocal square root on the serial chain instead of sqrt + divide
-    const double rk = rsqrt(piv), sq = piv * rk;
-    const double rkj = (j > k) ? dkj * rk : (j == k ? sq : 0.0);
-    const double fkj = ekj * rk;
+    for (int i = k + 2; i < 16; ++i) r[i] = chol_readlane(d[k], i);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (g + 4 * r > k) {
-        const double rki = dki[r] * rk;
-        d[r] = fma(-rki, rkj, d[r]);
-        f[r] = fma(-rki, fkj, f[r]);
-      }
-    }
-    if (g == (k & 3)) {
-      d[kr] = rkj;
-      f[kr] = fkj;
+    for (int i = k + 2; i < 16; ++i) d[i] = fma(-r[i], d[k], d[i]);
+  }
+  if (lane < 32) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (inv) F[i * CB_XLD + j] = d[i];
+      else D[i * CB_LD + j] = i <= j ? d[i] : 0.0;
     }
   }
 }
 
-__global__ __launch_bounds__(NT) void chol_inv_kernel(const tnx_chol_job* __restrict__ jobs) {
+__global__ __launch_bounds__(NC) void chol_inv_kernel(const tnx_chol_job* __restrict__ jobs) {
   extern __shared__ double lds[];
   double* Sl = lds;                          // CHOL_NMAX rows of CB_LD
   double* Xd = lds + CHOL_NMAX * CB_LD;      // F_pp, 16 rows of CB_XLD per panel
   const tnx_chol_job J = jobs[blockIdx.x];
   const int n = J.n;
   if (n <= 0 || n > CHOL_NMAX) return;  // rejected on the host
-  const double* G = (const double*)J.g;
   const int ld = J.ld > 0 ? J.ld : n;
   const int nb = (n + 15) >> 4, np = 16 * nb;
-  __shared__ double red[8];
+  __shared__ double red[2][NC / 64];
   __shared__ int bad_s;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // G padded with the identity; trace (shift) and largest |G - I| entry
+  constexpr int NR = CHOL_NMAX / (NC / 64);   // rows of a wave
   double trace = 0.0, emax = 0.0;
-  for (int i = wave; i < np; i += 4)
-    for (int j = lane; j < np; j += 64) {
-      double v = (i == j) ? 1.0 : 0.0;
-      if (i < n && j < n) {
-        const double gv = G[(int64_t)i * ld + j];
-        if (i == j) trace += gv;
-        emax = fmax(emax, fabs(gv - v));
-        v = gv;
-      }
-      Sl[i * CB_LD + j] = v;
+  {
+    const double TNX_GLOBAL* G = as_global<const double>(J.g);
+    double v[NR][2];
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+      if (NC / 64 * t >= np) break;
+      const double TNX_GLOBAL* row = G + (int64_t)min(wave + NC / 64 * t, n - 1) * ld;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) v[t][c] = row[(unsigned)min(lane + 64 * c, n - 1)];
     }
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+      if (NC / 64 * t >= np) break;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int i = wave + NC / 64 * t, j = lane + 64 * c;
+        const double id = i == j ? 1.0 : 0.0;
+        if (i < n && j < n) {
+          if (i == j) trace += v[t][c];
+          emax = fmax(emax, fabs(v[t][c] - id));
+        } else {
+          v[t][c] = id;
+        }
+        if (i < np && j < np) Sl[i * CB_LD + j] = v[t][c];
+      }
+    }
+  }
   trace = tnx_wave_sum(trace);
-  for (int o = 32; o > 0; o >>= 1) emax = fmax(emax, __shfl_xor(emax, o, 64));
+  emax = tnx_wave_fold(emax, [](double x, double y) { return fmax(x, y); });
   if (lane == 0) {
-    red[wave] = trace;
-    red[4 + wave] = emax;
+    red[0][wave] = trace;
+    red[1][wave] = emax;
   }
   if (threadIdx.x == 0) bad_s = 0;
   __syncthreads();
-  const double shift = J.shift_scale * (J.shift_ref ? *(const double*)J.shift_ref
-                                                    : ((red[0] + red[1]) + (red[2] + red[3])));
-  const double em = fmax(fmax(red[4], red[5]), fmax(red[6], red[7]));
-  double* R = (double*)J.r;
-  double* Ri = (double*)J.rinv;
+  double tsum = 0.0, em = 0.0;
+#pragma unroll
+  for (int w = 0; w < NC / 64; ++w) {
+    tsum += red[0][w];
+    em = fmax(em, red[1][w]);
+  }
+  const double shift =
+      J.shift_scale * (J.shift_ref ? *as_global<const double>(J.shift_ref) : tsum);
+  double TNX_GLOBAL* R = as_global<double>(J.r);
+  double TNX_GLOBAL* Ri = as_global<double>(J.rinv);
   // Near-identity Gram matrix (the last pass of CholeskyQR3, whose panel is
   // already orthonormal to working accuracy): with S = I + E, ||E||_max <=
   // CHOL_NEAR_ID and no shift, R = I + U (U = strict upper part of E plus
   // half its diagonal) and R^{-1} = I - U hold up to O(E^2) <= 1e-20, below
   // the rounding of the factorisation, and need no sequential steps.
   if (shift == 0.0 && em <= CHOL_NEAR_ID) {
-    for (int i = wave; i < n; i += 4)
+    for (int i = wave; i < n; i += NC / 64)
       for (int j = lane; j < n; j += 64) {
         const double sv = Sl[i * CB_LD + j];
         const double u = j > i ? sv : (j == i ? 0.5 * (sv - 1.0) : 0.0);
@@ -747,75 +753,75 @@ __global__ __launch_bounds__(NT) void chol_inv_kernel(const tnx_chol_job* __rest
     if (threadIdx.x == 0 && J.status != 0) *(int32_t*)J.status = 0;
     return;
   }
-  int sa[16], sb[16];
-  tnx_d4 acc[16];
+  // block (sa, sb) of slot s: slot 0 or 3 is a diagonal block of waves 0, 5, 10, 15
+  const int wa = wave >> 2, wb = wave & 3;
+  tnx_d4 acc[4];
 #pragma unroll
-  for (int s = 0; s < 16; ++s) {
-    chol_slot(wave, s, sa[s], sb[s]);
+  for (int s = 0; s < 4; ++s) {
+    const int sa = wa + 4 * (s >> 1), sb = wb + 4 * (s & 1);
     acc[s] = tnx_d4{0.0, 0.0, 0.0, 0.0};
-    if (s <= 8 && sb[s] < nb) {
-      acc[s] = chol_ld(Sl + 16 * sa[s] * CB_LD + 16 * sb[s], CB_LD, lane);
-      if (sa[s] == sb[s]) {   // the shift on the diagonal (not on the padding)
+    if (sa <= sb && sb < nb) {
+      acc[s] = chol_ld(Sl + 16 * sa * CB_LD + 16 * sb, CB_LD, lane);
+      if (sa == sb) {   // the shift on the diagonal (not on the padding)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int i = 16 * sa[s] + (lane >> 4) + 4 * r;
+          const int i = 16 * sa + (lane >> 4) + 4 * r;
           if ((lane >> 4) + 4 * r == (lane & 15) && i < n) acc[s][r] += shift;
         }
       }
     }
   }
   int bad = 0;
+#pragma unroll 1
   for (int p = 0; p < nb; ++p) {
-    const double* Pp = Sl + 16 * p * CB_LD;       // row panel p
-    if (p > 0) {   // trailing update of panel p-1, diagonal blocks first
-      const double* Pq = Pp - 16 * CB_LD;
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-        if (sa[s] > p - 1 && sa[s] < nb)
-          acc[s] = chol_mma(acc[s], Pq + 16 * sa[s], 1, CB_LD, Pq + 16 * sb[s], CB_LD, lane, -1.0);
+    int ln = lane;   // opaque: what follows from the lane is formed anew, not
+    asm volatile("" : "+v"(ln));   // kept in registers (and spilled) across panels
+    double* Pp = Sl + 16 * p * CB_LD;             // row panel p
+    double* Fp = Xd + 16 * p * CB_XLD;
+    const double* Pq = Pp - 16 * CB_LD;           // and p - 1 (p > 0)
+    const double* Fq = Fp - 16 * CB_XLD;
+    if (wave == 5 * (p & 3)) {   // the diagonal block: trailing update, then its factor
+      __builtin_amdgcn_s_setprio(3);
+      tnx_d4 dd = p < 4 ? acc[0] : acc[3];
+      if (p > 0) dd = chol_mma(dd, Pq + 16 * p, 1, CB_LD, Pq + 16 * p, CB_LD, ln, -1.0);
+      chol_st(Pp + 16 * p, CB_LD, ln, dd);
+      __builtin_amdgcn_wave_barrier();
+      chol_diag(Pp + 16 * p, Fp, ln, bad);
+      __builtin_amdgcn_s_setprio(0);
     }
-    if (min(p, 7 - p) == wave) {   // factor the diagonal block of panel p
-      tnx_d4 dd = (p == wave) ? acc[0] : acc[1], ff;
-      chol_diag(dd, ff, lane, bad);
-      chol_st(Sl + 16 * p * CB_LD + 16 * p, CB_LD, lane, dd);
-      chol_st(Xd + 16 * p * CB_XLD, CB_XLD, lane, ff);
+    if (p > 0) {   // trailing update of panel p - 1
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int sa = wa + 4 * (s >> 1), sb = wb + 4 * (s & 1);
+        if (sa < p || sa >= nb || sb >= nb || (sa == p && sb == p)) continue;
+        if (sb < sa && sb >= p) continue;   // E_ab starts with panel b
+        const bool diag = sb == p - 1;
+        acc[s] = chol_mma(acc[s], Pq + 16 * sa, 1, CB_LD, diag ? Fq : Pq + 16 * sb,
+                          diag ? CB_XLD : CB_LD, ln, -1.0);
+      }
     }
-    if (p > 0) {
-      const double* Pq = Pp - 16 * CB_LD;
-      const double* Fq = Xd + 16 * (p - 1) * CB_XLD;
-#pragma unroll
-      for (int s = 2; s < 9; ++s)
-        if (sa[s] > p - 1 && sb[s] < nb)
-          acc[s] = chol_mma(acc[s], Pq + 16 * sa[s], 1, CB_LD, Pq + 16 * sb[s], CB_LD, lane, -1.0);
-#pragma unroll
-      for (int s = 9; s < 16; ++s)
-        if (sa[s] > p - 1 && sa[s] < nb && sb[s] <= p - 1) {
-          const bool diag = sb[s] == p - 1;
-          acc[s] = chol_mma(acc[s], Pq + 16 * sa[s], 1, CB_LD, diag ? Fq : Pq + 16 * sb[s],
-                            diag ? CB_XLD : CB_LD, lane, -1.0);
-        }
-    }
-    // row panel p of S (above the diagonal) and E (below it) as updated
-#pragma unroll
-    for (int s = 2; s < 16; ++s)
-      if (sa[s] == p && sb[s] < nb) chol_st(Sl + 16 * p * CB_LD + 16 * sb[s], CB_LD, lane, acc[s]);
     __syncthreads();
     // R_pb = F_pp S_pb, F_pe = F_pp E_pe
-    const double* Fp = Xd + 16 * p * CB_XLD;
+    if (wa == (p & 3)) {
 #pragma unroll
-    for (int s = 2; s < 16; ++s)
-      if (sa[s] == p && sb[s] < nb) {
-        const tnx_d4 c = chol_mma(tnx_d4{0.0, 0.0, 0.0, 0.0}, Fp, CB_XLD, 1, Pp + 16 * sb[s], CB_LD,
-                                  lane, 1.0);
-        chol_st(Sl + 16 * p * CB_LD + 16 * sb[s], CB_LD, lane, c);
+      for (int s = 0; s < 4; ++s) {
+        const int sa = wa + 4 * (s >> 1), sb = wb + 4 * (s & 1);
+        if (sa != p || sb == p || sb >= nb) continue;
+        tnx_d4 c = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          c = __builtin_amdgcn_mfma_f64_16x16x4f64(Fp[(ln & 15) * CB_XLD + 4 * r + (ln >> 4)],
+                                                   acc[s][r], c, 0, 0, 0);
+        chol_st(Pp + 16 * sb, CB_LD, ln, c);
       }
+    }
     __syncthreads();
   }
   if (bad && lane == 0) bad_s = 1;
   __syncthreads();
   // R (upper) and R^{-1} = F^T: F_pp from its buffer, the blocks below the
   // diagonal of F from the lower part of Sl
-  for (int i = wave; i < n; i += 4)
+  for (int i = wave; i < n; i += NC / 64)
     for (int j = lane; j < n; j += 64) {
       double rv = 0.0, xv = 0.0;
       if (j >= i) {
@@ -839,7 +845,7 @@ extern "C" int tnx_chol_inv_f64(const tnx_chol_job* jobs, int njob, tnx_stream_t
   }
   static std::atomic<uint64_t> lds_set{0};
   if (int rc = tnx_dynamic_lds((const void*)chol_inv_kernel, CHOL_LDS, lds_set)) return rc;
-  hipLaunchKernelGGL(chol_inv_kernel, dim3(njob), dim3(NT), CHOL_LDS, (hipStream_t)stream, jobs);
+  hipLaunchKernelGGL(chol_inv_kernel, dim3(njob), dim3(NC), CHOL_LDS, (hipStream_t)stream, jobs);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }

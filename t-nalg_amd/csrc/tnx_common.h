@@ -171,6 +171,22 @@ __device__ __forceinline__ double tnx_wave_min(double v) {
   return tnx_wave_fold(v, [](double x, double y) { return fmin(x, y); });
 }
 
+// 1 / d and 1 / sqrt(x) to working accuracy, normal arguments: the hardware's
+// approximation and a third-order step, a fraction of a division's or library
+// root's chain.
+__device__ __forceinline__ double tnx_rcp(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = fma(-d, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+__device__ __forceinline__ double tnx_rsqrt_step(double x, double y) {   // y ~ 1 / sqrt(x)
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ double tnx_rsqrt(double x) {
+  return tnx_rsqrt_step(x, __builtin_amdgcn_rsq(x));
+}
+
 // Largest index i in [0, n) whose 32-bit field at byte offset `off` of the
 // i-th record (records of `rec` bytes) is <= key.  The fields are prefix
 // sums (non-decreasing, first one 0, key >= 0), so i is the record owning
