@@ -429,44 +429,59 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
   const TC TNX_GLOBAL* C0 = as_global<const TC>(P.c0);
   const int gj = col0 + wc + NB * (lane & 15);
   const bool wide = gj + NB <= P.N;
+  typedef TC VC __attribute__((ext_vector_type(NB), aligned(sizeof(TC))));
+  auto row_of = [&](int i, int r) {
+    const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
+    return row0 + wr + MB * rr + i;
+  };
+  // C0 first, all of it (elements past the edges: of the last row or column):
+  // no load can pass a store it might alias
+  TC c0[MB][4][NB];
+  if (C0 != nullptr) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const TC TNX_GLOBAL* row = C0 + (int64_t)min(row_of(i, r), P.M - 1) * P.ldc0;
+        if (wide) {
+          if constexpr (NB == 1) c0[i][r][0] = row[gj];
+          else {
+            const VC c = *(const VC TNX_GLOBAL*)(row + gj);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) c0[i][r][j] = c[j];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) c0[i][r][j] = row[min(gj + j, P.N - 1)];
+        }
+      }
+  }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
-      const int gi = row0 + wr + MB * rr + i;
+      const int gi = row_of(i, r);
       if (gi >= P.M) continue;
-      typedef TC VC __attribute__((ext_vector_type(NB), aligned(sizeof(TC))));
+      TC v[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        double x = (double)acc[i][j][r];
+        if (C0 != nullptr) x += P.beta * to_d(c0[i][r][j]);
+        v[j] = from_d<TC>(x);
+      }
+      TC TNX_GLOBAL* row = Cp + (int64_t)gi * P.ldc;
       if (wide) {
-        double v[NB];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) v[j] = (double)acc[i][j][r];
-        if (C0 != nullptr) {
-          TC c0[NB];
-          if constexpr (NB == 1) c0[0] = C0[(int64_t)gi * P.ldc0 + gj];
-          else {
-            const VC c = *(const VC TNX_GLOBAL*)(C0 + (int64_t)gi * P.ldc0 + gj);
-#pragma unroll
-            for (int j = 0; j < NB; ++j) c0[j] = c[j];
-          }
-#pragma unroll
-          for (int j = 0; j < NB; ++j) v[j] += P.beta * to_d(c0[j]);
-        }
-        if constexpr (NB == 1) Cp[(int64_t)gi * P.ldc + gj] = from_d<TC>(v[0]);
+        if constexpr (NB == 1) row[gj] = v[0];
         else {
           VC c;
 #pragma unroll
-          for (int j = 0; j < NB; ++j) c[j] = from_d<TC>(v[j]);
-          *(VC TNX_GLOBAL*)(Cp + (int64_t)gi * P.ldc + gj) = c;
+          for (int j = 0; j < NB; ++j) c[j] = v[j];
+          *(VC TNX_GLOBAL*)(row + gj) = c;
         }
       } else {
 #pragma unroll
         for (int j = 0; j < NB; ++j)
-          if (gj + j < P.N) {
-            double v = (double)acc[i][j][r];
-            if (C0 != nullptr) v += P.beta * to_d(C0[(int64_t)gi * P.ldc0 + gj + j]);
-            Cp[(int64_t)gi * P.ldc + gj + j] = from_d<TC>(v);
-          }
+          if (gj + j < P.N) row[gj + j] = v[j];
       }
     }
   if (ts != nullptr) {
