@@ -400,31 +400,12 @@ __device__ __forceinline__ double row_sum(double v) {
   return v + tnx_row_get<0x121>(v);
 }
 
+// Rotates the columns of W (m x n) until they are orthogonal, V (n x n) along.
 template <typename PW>
-__device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, PW W, PW V, double* sv,
-                                         int* order, int& rotated) {
-  const int m = J.m, n = J.n;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  constexpr int NW = NQ / 64;
-  const int l = lane & (SVD_T - 1);
-  const double TNX_GLOBAL* src = as_global<const double>(J.src);
-
-  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
-    int r, c;
-    if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }
-    else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }
-    W[(int64_t)c * m + r] = src_at(src, J.ld, J.trans, r, c);
-  }
-  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NQ) {
-    int c = (int)(e / n), r = (int)(e - (int64_t)c * n);
-    V[e] = (r == c) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-
+__device__ __forceinline__ void jacobi_sweeps(PW W, int m, PW V, int n, double eps, int max_sweeps,
+                                              int& rotated) {
+  const int l = threadIdx.x & (SVD_T - 1);
   const int np = (n + 1) & ~1;  // players in the round-robin tournament
-  // rotate while |a.b| > m*eps*|a||b| (columns orthogonal to working accuracy)
-  const double eps = 2.220446049250313e-16 * (double)(m > 8 ? m : 8);
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     if (threadIdx.x == 0) rotated = 0;
     __syncthreads();
@@ -472,13 +453,21 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
     if (rotated == 0) break;
     __syncthreads();
   }
-  // singular values and descending order
-  for (int c = wave; c < n; c += NW) {
+}
+
+// Singular values sv (LDS) = column norms of W, order = their descending order.
+template <typename PW>
+__device__ __forceinline__ void sort_columns(PW W, int m, int n, double* sv, int* order) {
+  const int lane = threadIdx.x & 63;
+  for (int c = threadIdx.x >> 6; c < n; c += NQ / 64) {
     const PW wc = W + (int64_t)c * m;
     double s = 0.0;
     for (int r = lane; r < m; r += 64) s += wc[r] * wc[r];
     s = tnx_wave_sum(s);
-    if (lane == 0) sv[c] = sqrt(s);
+    if (lane == 0) {
+      sv[c] = sqrt(s);
+      order[c] = c;   // (values that do not compare leave entries unset below)
+    }
   }
   __syncthreads();
   for (int c = threadIdx.x; c < n; c += NQ) {
@@ -488,6 +477,32 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
     order[rank] = c;
   }
   __syncthreads();
+}
+
+template <typename PW>
+__device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, PW W, PW V, double* sv,
+                                         int* order, int& rotated) {
+  const int m = J.m, n = J.n;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int NW = NQ / 64;
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
+
+  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
+    int r, c;
+    if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }
+    else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }
+    W[(int64_t)c * m + r] = src_at(src, J.ld, J.trans, r, c);
+  }
+  for (int64_t e = threadIdx.x; e < (int64_t)n * n; e += NQ) {
+    int c = (int)(e / n), r = (int)(e - (int64_t)c * n);
+    V[e] = (r == c) ? 1.0 : 0.0;
+  }
+  __syncthreads();
+
+  // rotate while |a.b| > m*eps*|a||b| (columns orthogonal to working accuracy)
+  jacobi_sweeps(W, m, V, n, 2.220446049250313e-16 * (double)(m > 8 ? m : 8), max_sweeps, rotated);
+  sort_columns(W, m, n, sv, order);
   double TNX_GLOBAL* s_out = as_global<double>(J.s);
   double TNX_GLOBAL* u = as_global<double>(J.u);
   double TNX_GLOBAL* svt = as_global<double>(J.svt);
@@ -556,6 +571,163 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
   }
 }
 
+// The same by way of M P = Q R (Householder, the largest remaining column
+// first): the columns of X = R^T are rotated, X W = B, so that M = Q W B^T P^T,
+// u = Q W, diag(s) vt = B^T P^T.  With singular values that decay the columns of
+// X start nearly sorted and nearly orthogonal, those of M do not: 24 sweeps
+// become 7 (order 64, values over 10 or 16 decades), 10 of a random matrix 9,
+// and a tall M is rotated as an n x n matrix.  u comes out orthonormal whatever
+// the rank.  A (m x n), X and V (n x n) in LDS, m <= 64 ROWS.  M is scaled by a
+// power of two, so that squares of its entries stay in range.
+// us (MI355X), columns of M -> this: order 64 with values over 10 decades 2030 ->
+// 785, over 20 2430 -> 775, random 840 -> 930; 128 x 40 over 10 decades 1150 ->
+// 394, random 550 -> 456; order 16 132 -> 84, random 84 -> 91.
+constexpr int SVD_QR_M = 256;
+constexpr int SVD_QR_N = 72;   // columns at most (SVD_LDS holds m n + 2 n^2 doubles)
+template <int ROWS>
+__device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps, double* A, double* X,
+                                            double* V, double* sv, int* order, int& rotated) {
+  const int m = J.m, n = J.n;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int NW = NQ / 64;
+  __shared__ double nrm[SVD_QR_N], v0s[SVD_QR_N], fs[SVD_QR_N], beta[SVD_QR_N];
+  const double TNX_GLOBAL* src = as_global<const double>(J.src);
+  double big = 0.0;
+  for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
+    int r, c;
+    if (J.trans) { c = (int)(e / m); r = (int)(e - (int64_t)c * m); }
+    else { r = (int)(e / n); c = (int)(e - (int64_t)r * n); }
+    const double x = src_at(src, J.ld, J.trans, r, c);
+    A[(int64_t)c * m + r] = x;
+    big = fmax(big, fabs(x));
+  }
+  big = tnx_wave_fold(big, [](double x, double y) { return fmax(x, y); });
+  if (lane == 0) sv[wave] = big;
+  __syncthreads();
+  big = sv[lane & (NW - 1)];
+  big = tnx_wave_fold(big, [](double x, double y) { return fmax(x, y); });
+  const int ex = __builtin_amdgcn_frexp_exp(big);
+  for (int e = threadIdx.x; e < m * n; e += NQ) A[e] = __builtin_amdgcn_ldexp(A[e], -ex);
+  for (int e = threadIdx.x; e < n * n; e += NQ) {
+    const int c = e / n;
+    V[e] = (e - c * n == c) ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  for (int c = wave; c < n; c += NW) {
+    double t = 0.0;
+    for (int r = lane; r < m; r += 64) t += A[c * m + r] * A[c * m + r];
+    t = tnx_wave_sum(t);
+    if (lane == 0) nrm[c] = t;
+  }
+  __syncthreads();
+  // pivoted order, a copy per wave: lane j has the column at position j, and
+  // that at 64 + j
+  int p0 = lane, p1 = 64 + lane;
+  auto at = [&](int j) {
+    return j < 64 ? __builtin_amdgcn_readlane(p0, j) : __builtin_amdgcn_readlane(p1, j - 64);
+  };
+  for (int k = 0; k < n; ++k) {
+    // position of the largest remaining column (the first of equal ones)
+    const double n0 = lane >= k && lane < n ? nrm[p0] : -1.0;
+    const double n1 = 64 + lane >= k && 64 + lane < n ? nrm[p1] : -1.0;
+    const double top = tnx_wave_fold(fmax(n0, n1), [](double x, double y) { return fmax(x, y); });
+    const unsigned long long m0 = __ballot(n0 == top), m1 = __ballot(n1 == top);
+    const int best = m0 ? __builtin_ctzll(m0) : m1 ? 64 + __builtin_ctzll(m1) : k;   // (NaN: k)
+    const int ck = at(k), cb = at(best);
+    if (lane == (k & 63)) (k < 64 ? p0 : p1) = cb;
+    if (lane == (best & 63)) (best < 64 ? p0 : p1) = ck;
+    // reflector I - f v v^T, v = (x_k - beta, x_{k+1}, ...)
+    const double* x = A + cb * m;
+    double v[ROWS], ss = 0.0;
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) {
+      const int r = lane + 64 * t;
+      v[t] = r >= k && r < m ? x[r] : 0.0;
+      ss += v[t] * v[t];
+    }
+    ss = tnx_wave_sum(ss);
+    const double xk = x[k], nx = sqrt(ss);
+    const double b = xk > 0.0 ? -nx : nx, v0 = xk - b;
+    const double f = nx > 0.0 ? 1.0 / (nx * (nx + fabs(xk))) : 0.0;
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t)
+      if (lane + 64 * t == k) v[t] = v0;
+    if (threadIdx.x == 0) {
+      v0s[k] = v0;
+      fs[k] = f;
+      beta[k] = b;
+    }
+    for (int j = k + 1 + wave; j < n; j += NW) {
+      double* a = A + at(j) * m;
+      double y[ROWS], d = 0.0, t2 = 0.0;
+#pragma unroll
+      for (int t = 0; t < ROWS; ++t) {
+        const int r = lane + 64 * t;
+        y[t] = r < m ? a[r] : 0.0;
+        d += v[t] * y[t];
+      }
+      d = f * tnx_wave_sum(d);
+#pragma unroll
+      for (int t = 0; t < ROWS; ++t) {
+        const int r = lane + 64 * t;
+        y[t] -= d * v[t];
+        if (r >= k && r < m) a[r] = y[t];
+        if (r > k) t2 += y[t] * y[t];
+      }
+      t2 = tnx_wave_sum(t2);
+      if (lane == 0) nrm[at(j)] = t2;
+    }
+    __syncthreads();
+  }
+  // X: column i is row i of R
+  for (int i = wave; i < n; i += NW)
+    for (int c = lane; c < n; c += 64) {
+      const int pc = c < 64 ? p0 : p1;   // (c = lane or 64 + lane)
+      X[i * n + c] = c > i ? A[pc * m + i] : c == i ? beta[i] : 0.0;
+    }
+  __syncthreads();
+  jacobi_sweeps(X, n, V, n, 2.220446049250313e-16 * (double)(m > 8 ? m : 8), max_sweeps, rotated);
+  sort_columns(X, n, n, sv, order);
+  double TNX_GLOBAL* s_out = as_global<double>(J.s);
+  double TNX_GLOBAL* u = as_global<double>(J.u);
+  double TNX_GLOBAL* svt = as_global<double>(J.svt);
+  for (int i = threadIdx.x; i < n; i += NQ) s_out[i] = __builtin_amdgcn_ldexp(sv[order[i]], ex);
+  for (int i = wave; i < n; i += NW) {
+    const int c = order[i];
+    for (int q = lane; q < n; q += 64) 
+      svt[(int64_t)i * n + (q < 64 ? p0 : p1)] = __builtin_amdgcn_ldexp(X[c * n + q], ex);
+    double z[ROWS];
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) {
+      const int r = lane + 64 * t;
+      z[t] = r < n ? V[c * n + r] : 0.0;
+    }
+    for (int k = n - 1; k >= 0; --k) {
+      const double* x = A + at(k) * m;
+      const double v0 = v0s[k];
+      double v[ROWS], d = 0.0;
+#pragma unroll
+      for (int t = 0; t < ROWS; ++t) {
+        const int r = lane + 64 * t;
+        v[t] = r > k && r < m ? x[r] : r == k ? v0 : 0.0;
+        d += v[t] * z[t];
+      }
+      d = fs[k] * tnx_wave_sum(d);
+#pragma unroll
+      for (int t = 0; t < ROWS; ++t) z[t] -= d * v[t];
+    }
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) {
+      const int r = lane + 64 * t;
+      if (r < m) {
+        if (J.u_trans) u[(int64_t)i * m + r] = z[t];
+        else u[(int64_t)r * n + i] = z[t];
+      }
+    }
+  }
+}
+
 __global__ __launch_bounds__(NQ) void svd_kernel(const tnx_svd_job* __restrict__ jobs, int max_sweeps) {
   extern __shared__ double lds[];
   __shared__ int rotated;
@@ -565,7 +737,13 @@ __global__ __launch_bounds__(NQ) void svd_kernel(const tnx_svd_job* __restrict__
   const int m = J.m, n = J.n;
   if (n > KMAX || m < n || n <= 0) return;  // rejected on the host
   const int64_t wn = (int64_t)m * n;
-  if ((wn + (int64_t)n * n) * (int64_t)sizeof(double) <= (int64_t)SVD_LDS) {
+  if (m <= SVD_QR_M && n <= SVD_QR_N &&
+      (wn + 2 * (int64_t)n * n) * (int64_t)sizeof(double) <= (int64_t)SVD_LDS) {
+    double *X = lds + wn, *V = X + n * n;
+    if (m <= 64) svd_body_qr<1>(J, max_sweeps, lds, X, V, sv, order, rotated);
+    else if (m <= 128) svd_body_qr<2>(J, max_sweeps, lds, X, V, sv, order, rotated);
+    else svd_body_qr<4>(J, max_sweeps, lds, X, V, sv, order, rotated);
+  } else if ((wn + (int64_t)n * n) * (int64_t)sizeof(double) <= (int64_t)SVD_LDS) {
     svd_body<double*>(J, max_sweeps, lds, lds + wn, sv, order, rotated);
   } else {
     double TNX_GLOBAL* W = as_global<double>(J.work);

@@ -1276,3 +1276,55 @@ def test_mix_term_batches(gpu, d, nterm):
         assert np.abs(g - r.reshape(-1)).max() <= 1e-13 * max(np.abs(r).max(), 1.0), (k, r.shape)
     for k in range(0, len(got), 2):
         assert np.array_equal(got[k], got[k + 1]), k
+
+
+@pytest.mark.parametrize('m,n', [(1, 1), (7, 7), (64, 64), (65, 65), (66, 66), (256, 16), (257, 16),
+                                 (90, 33)])
+@pytest.mark.parametrize('kind', ['decay', 'rank', 'zero', 'small'])
+def test_svd_jacobi_by_qr(gpu, m, n, kind):
+    """Sizes at the edges of the SVD that starts with a pivoted QR (m <= 256, m n
+    + 2 n^2 doubles in LDS) and the one on the columns: values over 16 decades,
+    the zero matrix and (by QR) rank deficiency with zero columns and entries of
+    1e-170, both layouts.  M = U diag(s) V^T to 1e-14 max(m, 8) ||M||, U
+    orthonormal to 1e-14 max(m, 8) (the rotations stop at m eps), s as numpy's
+    to 1e-14 n s_0."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    by_qr = m <= 256 and n <= 65
+    if kind in ('small', 'rank') and not by_qr:
+        pytest.skip('the rotations on the columns square the entries, and their completion of many '
+                    'exact null columns can run out of unit vectors')
+    rng = np.random.RandomState(m + n)
+    M = rng.randn(m, n)
+    if kind == 'decay':
+        Q, R = np.linalg.qr(M)
+        M = (Q * 10.0 ** (-16 * np.arange(n) / n)) @ np.linalg.qr(rng.randn(n, n))[0]
+    elif kind == 'rank':
+        M = M[:, :(n + 1) // 2] @ rng.randn((n + 1) // 2, n)
+        M[:, ::5] = 0.0
+    elif kind == 'zero':
+        M = np.zeros((m, n))
+    elif kind == 'small':
+        M = M * 1e-170
+    ref = np.linalg.svd(M, compute_uv=False)
+    nM = max(np.linalg.norm(M / (ref[0] or 1.0)), 1e-300)
+    tol = 1e-14 * max(m, 8)
+    for trans in (0, 1):
+        src = _dev(M.T if trans else M)
+        u, s, vt, w = (torch.zeros(k, dtype=torch.float64, device='cuda')
+                       for k in (m * n, n, n * n, m * n + n * n))
+        job = np.array([(src.data_ptr(), u.data_ptr(), s.data_ptr(), vt.data_ptr(), w.data_ptr(),
+                         m, n, m if trans else n, trans, trans, 0)], dtype=L.SVD_JOB)
+        (dj,) = _upload([job])
+        print('svd by qr', m, n, kind, 'trans', trans, flush=True)
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), 1, 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        U = u.cpu().numpy()
+        U = U.reshape(n, m).T if trans else U.reshape(m, n)
+        S, V = s.cpu().numpy(), vt.cpu().numpy().reshape(n, n)
+        sc = ref[0] or 1.0
+        assert np.all(np.diff(S) <= 0)
+        assert np.abs(S - ref).max() <= 1e-14 * n * sc
+        assert np.abs(U.T @ U - np.eye(n)).max() <= tol
+        assert np.linalg.norm(U @ (V / sc) - M / sc) <= tol * nM
