@@ -9,19 +9,23 @@
 // swapped.  The tangent needs no more than the hardware's reciprocal and root
 // (any angle is a rotation; an approximate one leaves 1e-7 of g); it is formed
 // from the entries over a power of two near the larger one, so nothing over-
-// or underflows.  The cosine and tau are refined to working accuracy (third
+// or underflows (without SCALE the caller keeps their squares in range).  The cosine and tau are refined to working accuracy (third
 // order: the cube of the approximation's 2^-20 or less), so the transformation
 // is orthogonal; in this form its rounding errors are those of the small
 // numbers s and tau, not of cos.
 struct JacobiRot { double s, tau; bool swap; };
 
+template <bool SCALE = true>
 __device__ __forceinline__ JacobiRot jacobi_rot(double a, double c, double g, bool rot, bool order) {
   JacobiRot r;
   r.swap = order && c > a;
-  double h = c - a;
-  const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(h), fabs(g)));
-  h = __builtin_amdgcn_ldexp(h, ex);
-  const double g2 = rot ? 2.0 * __builtin_amdgcn_ldexp(g, ex) : 1.0;
+  double h = rot ? c - a : 0.0;
+  if constexpr (SCALE) {
+    const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(h), fabs(g)));
+    h = __builtin_amdgcn_ldexp(h, ex);
+    g = __builtin_amdgcn_ldexp(g, ex);
+  }
+  const double g2 = rot ? 2.0 * g : 1.0;
   const double w = fma(h, h, g2 * g2);
   const double den = fabs(h) + w * __builtin_amdgcn_rsq(w);
   const double t = (h >= 0.0 ? g2 : -g2) * __builtin_amdgcn_rcp(den);   // |t| <= 1

@@ -24,11 +24,13 @@
 // those of the small numbers s and t: relative error of the singular values
 // 1.5e-15 (n = 128, 200) where c x - s y on the columns had 1.5e-14 to 4e-14.
 // ms (MI355X), rotations of columns in LDS -> this: one matrix of order 64 1.8
-// -> 0.8, 128 6.5 -> 1.8, 256 21.8 -> 5.6, 1024 195 -> 61; 16 of order 256
-// 23.1 -> 6.5, with singular values over 10 decades in rows of any size 75.6
-// -> 17.0; values only, 500 of order 128 15.8 -> 10.2.
-// Bound: latency.  A round (n = 128 about 25 us) is 31 steps of one barrier,
-// each a chain of some 40 dependent f64 operations for the angles; Gram matrix
+// -> 0.8, 128 6.6 -> 1.6, 256 21.9 -> 5.0, 1024 195 -> 58; 16 of order 256
+// 23.1 -> 5.9, with singular values over 10 decades in rows of any size 75.9
+// -> 15.5; values only, 500 of order 128 16.0 -> 8.7.
+// Bound: latency.  A round (n = 128 about 21 us; 25 with the rows' angles
+// formed anew instead of taken from the lane that has them, and the reads of a
+// step behind its angle) is 31 steps of one barrier, each a chain of some 30
+// dependent f64 operations for the angle; Gram matrix
 // and products are the rest.  Tried and not kept: two sweeps over a Gram
 // matrix (fewer rounds, more steps: 128 2.7 ms), two for panels whose column
 // norms differ by 1e4 (10 decades 5.4 -> 8.9 ms), angles in f32 (no gain), 256
@@ -186,7 +188,7 @@ __global__ __launch_bounds__(RT, 4) void k_svdj_round(const tnx_svdj_job* __rest
   // Gram entries are scaled by a power of two near 1 / ||R||_F^2, so that
   // products of them neither over- nor underflow
   const double fro2 = norms_of(J)[n];
-  const double scale = (fro2 > 1e-300 && fro2 < 1e300) ? ldexp(1.0, -ilogb(fro2)) : 1.0;
+  const double scale = (fro2 > 1e-300 && fro2 < 1.7e308) ? ldexp(1.0, -ilogb(fro2)) : 1.0;
   const double eps = 2.220446049250313e-16 * (double)(n > 8 ? n : 8), eps2 = eps * eps;
   const double zero2 = eps2 * fro2 * scale;  // column norm^2 of numerical zero
   const int cnt = bw < SB ? bw : SB, nsub = bw < SB ? 1 : bw / SB;
@@ -273,43 +275,45 @@ __global__ __launch_bounds__(RT, 4) void k_svdj_round(const tnx_svdj_job* __rest
       __syncthreads();
       if (turned == 0) continue;
       any = 1;
+      // A lane holds elements (r1, r2) x (uq, vq): of G, rows and columns of two
+      // rotations, or of Q, rows 2 pi and 2 pi + 1.  The indices of the next
+      // step are formed ahead of the barrier, all LDS reads ahead of the angle.
+      static_assert(offsetof(decltype(L.m), Q) == sizeof(L.m.G), "Q follows G");
+      double* const M = &L.m.G[0][0][0];
+      constexpr int COPY = PW * GLD;          // elements of one copy of G or Q
+      const int half = q_half ? 2 * COPY : 0;
+      int uq, vq, r1 = 2 * pi, r2 = 2 * pi + 1;
+      pair_of(PW, 0, qi, uq, vq);
+      if (!q_half) pair_of(PW, 0, pi, r1, r2);
 #pragma unroll 1
       for (int ir = 0; ir < PW - 1; ++ir) {
-        const int cur = ir & 1;
-        const double (*G)[GLD] = L.m.G[cur];
-        int up, vp, uq, vq;
-        pair_of(PW, ir, qi, uq, vq);
-        auto rotation = [&](int u, int v) {
-          const double a = G[u][u], c = G[v][v], gg = G[u][v];
-          const bool live = a > zero2 && c > zero2;   // no zero column (the padding among them)
-          return jacobi_rot(a, c, gg, live && gg * gg > eps2 * (a * c), live);
-        };
-        const JacobiRot rq = rotation(uq, vq);
+        const double* G = M + (ir & 1) * COPY;
+        const double* S = G + half;
+        double* D = M + ((ir & 1) ^ 1) * COPY + half;
+        const int ru = (int)__umul24(uq, GLD), rv = (int)__umul24(vq, GLD);
+        const int o1 = (int)__umul24(r1, GLD), o2 = (int)__umul24(r2, GLD);
+        const double a = G[ru + uq], c = G[rv + vq], gg = G[ru + vq];
+        double x11 = S[o1 + uq], x12 = S[o1 + vq], x21 = S[o2 + uq], x22 = S[o2 + vq];
+        const bool live = a > zero2 && c > zero2;   // no zero column (the padding among them)
+        // (entries of a live pair are above 1e-45: the squares stay in range)
+        const JacobiRot rq = jacobi_rot<false>(a, c, gg, live && gg * gg > eps2 * (a * c), live);
+        jacobi_apply(rq, x11, x12);
+        jacobi_apply(rq, x21, x22);
         if (!q_half) {
-          pair_of(PW, ir, pi, up, vp);
-          const JacobiRot rp = rotation(up, vp);
-          double g11 = G[up][uq], g12 = G[up][vq], g21 = G[vp][uq], g22 = G[vp][vq];
-          jacobi_apply(rq, g11, g12);
-          jacobi_apply(rq, g21, g22);
-          jacobi_apply(rp, g11, g21);
-          jacobi_apply(rp, g12, g22);
-          double (*H)[GLD] = L.m.G[cur ^ 1];
-          H[up][uq] = g11;
-          H[up][vq] = g12;
-          H[vp][uq] = g21;
-          H[vp][vq] = g22;
-        } else {
-          const double (*Q)[GLD] = L.m.Q[cur];
-          double q11 = Q[2 * pi][uq], q12 = Q[2 * pi][vq];
-          double q21 = Q[2 * pi + 1][uq], q22 = Q[2 * pi + 1][vq];
-          jacobi_apply(rq, q11, q12);
-          jacobi_apply(rq, q21, q22);
-          double (*H)[GLD] = L.m.Q[cur ^ 1];
-          H[2 * pi][uq] = q11;
-          H[2 * pi][vq] = q12;
-          H[2 * pi + 1][uq] = q21;
-          H[2 * pi + 1][vq] = q22;
+          // the rows' rotation: the one lane pi has for its column
+          JacobiRot rp;
+          rp.s = __shfl(rq.s, pi, 64);
+          rp.tau = __shfl(rq.tau, pi, 64);
+          rp.swap = (__ballot(rq.swap) >> pi) & 1;
+          jacobi_apply(rp, x11, x21);
+          jacobi_apply(rp, x12, x22);
         }
+        D[o1 + uq] = x11;
+        D[o1 + vq] = x12;
+        D[o2 + uq] = x21;
+        D[o2 + vq] = x22;
+        pair_of(PW, ir + 1, qi, uq, vq);
+        if (!q_half) pair_of(PW, ir + 1, pi, r1, r2);
         __syncthreads();
       }
       const double (*Q)[GLD] = L.m.Q[(PW - 1) & 1];
