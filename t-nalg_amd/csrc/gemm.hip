@@ -393,6 +393,43 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = (wave >> 1) * 16 * MB, wc = (wave & 1) * 16 * NB;
+  // C: lane % 16 is the column index of a block; the row index of
+  // accumulator element r is 4 (lane / 16) + r for the f32-output MFMAs
+  // and lane / 16 + 4 r for v_mfma_f64_16x16x4_f64 (measured on gfx950)
+  TC TNX_GLOBAL* Cp = as_global<TC>(P.c);
+  const TC TNX_GLOBAL* C0 = as_global<const TC>(P.c0);
+  const int gj = col0 + wc + NB * (lane & 15);
+  const bool full = gj + NB <= P.N;   // the lane's columns all exist
+  typedef TC VC __attribute__((ext_vector_type(NB), aligned(sizeof(TC))));
+  auto row_of = [&](int i, int r) {
+    const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
+    return row0 + wr + MB * rr + i;
+  };
+  // All of C0 before the first store (no load can pass a store it might
+  // alias; elements past the edges: of the last row or column), and before the
+  // products where the registers allow it.
+  TC c0[MB][4][NB];
+  auto load_c0 = [&]() {
+    if (C0 == nullptr) return;
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const TC TNX_GLOBAL* row = C0 + (int64_t)min(row_of(i, r), P.M - 1) * P.ldc0;
+        if (full) {
+          if constexpr (NB == 1) c0[i][r][0] = row[gj];
+          else {
+            const VC c = *(const VC TNX_GLOBAL*)(row + gj);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) c0[i][r][j] = c[j];
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) c0[i][r][j] = row[min(gj + j, P.N - 1)];
+        }
+      }
+  };
+  if constexpr (MB == 1) load_c0();
   V4 acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
@@ -422,40 +459,7 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
 #undef TNX_STREAM
   }
 
-  // C: lane % 16 is the column index of a block; the row index of
-  // accumulator element r is 4 (lane / 16) + r for the f32-output MFMAs
-  // and lane / 16 + 4 r for v_mfma_f64_16x16x4_f64 (measured on gfx950)
-  TC TNX_GLOBAL* Cp = as_global<TC>(P.c);
-  const TC TNX_GLOBAL* C0 = as_global<const TC>(P.c0);
-  const int gj = col0 + wc + NB * (lane & 15);
-  const bool wide = gj + NB <= P.N;
-  typedef TC VC __attribute__((ext_vector_type(NB), aligned(sizeof(TC))));
-  auto row_of = [&](int i, int r) {
-    const int rr = (MODE == TNX_GEMM_F64) ? ((lane >> 4) + 4 * r) : ((lane >> 4) * 4 + r);
-    return row0 + wr + MB * rr + i;
-  };
-  // C0 first, all of it (elements past the edges: of the last row or column):
-  // no load can pass a store it might alias
-  TC c0[MB][4][NB];
-  if (C0 != nullptr) {
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const TC TNX_GLOBAL* row = C0 + (int64_t)min(row_of(i, r), P.M - 1) * P.ldc0;
-        if (wide) {
-          if constexpr (NB == 1) c0[i][r][0] = row[gj];
-          else {
-            const VC c = *(const VC TNX_GLOBAL*)(row + gj);
-#pragma unroll
-            for (int j = 0; j < NB; ++j) c0[i][r][j] = c[j];
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < NB; ++j) c0[i][r][j] = row[min(gj + j, P.N - 1)];
-        }
-      }
-  }
+  if constexpr (MB > 1) load_c0();
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -470,7 +474,7 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
         v[j] = from_d<TC>(x);
       }
       TC TNX_GLOBAL* row = Cp + (int64_t)gi * P.ldc;
-      if (wide) {
+      if (full) {
         if constexpr (NB == 1) row[gj] = v[0];
         else {
           VC c;
