@@ -91,25 +91,39 @@ __global__ __launch_bounds__(NT) void k_svdj_init(const tnx_svdj_job* __restrict
 }
 
 // ||R||_F^2 of each job into work[2 n^2 + n] (one workgroup per job, a fixed
-// summation order, so the zero test below does not depend on the batch).
-__global__ __launch_bounds__(NT) void k_svdj_scale(const tnx_svdj_job* __restrict__ jobs) {
+// summation order, so the zero test below does not depend on the batch); the
+// sweeps' flag cleared.
+constexpr int NS = 1024;
+__global__ __launch_bounds__(NS) void k_svdj_scale(const tnx_svdj_job* __restrict__ jobs,
+                                                   int32_t* flag) {
   const tnx_svdj_job J = jobs[blockIdx.x];
   const int64_t nn = (int64_t)J.n * J.n;
-  double* B = (double*)J.work;
+  const double TNX_GLOBAL* B = as_global<const double>(J.work);
   double s = 0.0;
-  for (int64_t i = threadIdx.x; i < nn; i += NT) {
+#pragma unroll 4
+  for (int64_t i = threadIdx.x; i < nn; i += NS) {
     const double b = B[i];
     s += b * b;
   }
   s = tnx_wave_sum(s);
-  __shared__ double red[NT / 64];
+  __shared__ double red[NS / 64];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) norms_of(J)[J.n] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < NS / 64; ++w) t += red[w];
+    norms_of(J)[J.n] = t;
+    if (blockIdx.x == 0) *flag = 0;
+  }
 }
 
-__global__ void k_svdj_clear(int32_t* flag) {
-  if (threadIdx.x == 0) *flag = 0;
+// The flag of a sweep to the host (pinned memory, read after an event), cleared
+// for the next one.  (A copy and a clear were two launches of 3.7 us.)
+__global__ void k_svdj_publish(int32_t* flag, volatile int32_t* host) {
+  if (threadIdx.x == 0) {
+    *host = *flag;
+    *flag = 0;
+  }
 }
 
 // Column c (0..31) of a panel: sub-blocks starting at columns ca and cb, cnt
@@ -390,7 +404,7 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
   if (g_flag_pin == nullptr)
     TNX_CHECK_HIP(hipHostMalloc((void**)&g_flag_pin, 64, hipHostMallocDefault));
   hipLaunchKernelGGL(k_svdj_init, dim3(max_n < 1024 ? max_n : 1024, njob), dim3(NT), 0, s, jobs);
-  hipLaunchKernelGGL(k_svdj_scale, dim3(njob), dim3(NT), 0, s, jobs);
+  hipLaunchKernelGGL(k_svdj_scale, dim3(njob), dim3(NS), 0, s, jobs, flag);
   TNX_CHECK_LAUNCH();
   // The flag of a sweep is read while the next one runs: a sweep after the
   // last is a Gram matrix per panel and nothing else (n = 128: 30 us for one
@@ -405,12 +419,11 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
   bool converged = false;
   hipError_t err = hipSuccess;
   for (int sweep = 0; sweep < max_sweeps && !converged && err == hipSuccess; ++sweep) {
-    hipLaunchKernelGGL(k_svdj_clear, dim3(1), dim3(64), 0, s, flag);
     for (int r = 0; r < max_nblk - 1; ++r)
       hipLaunchKernelGGL(k_svdj_round, dim3(npairs), dim3(RT), 0, s, jobs, njob, r, flag);
+    hipLaunchKernelGGL(k_svdj_publish, dim3(1), dim3(64), 0, s, flag,
+                       (volatile int32_t*)g_flag_pin + (sweep & 1));
     err = hipGetLastError();
-    if (err == hipSuccess)
-      err = hipMemcpyAsync(g_flag_pin + (sweep & 1), flag, sizeof(int32_t), hipMemcpyDeviceToHost, s);
     if (err == hipSuccess) err = hipEventRecord(ev[sweep & 1], s);
     // the previous sweep's flag, or after the last allowed sweep its own too
     for (int k = sweep > 0 ? sweep - 1 : 0; err == hipSuccess && !converged && k <= sweep; ++k) {
