@@ -354,7 +354,7 @@ MATVEC_PMC_TRAFFIC = {
 MATVEC_PMC_FLOPS = 2.15e9   # flops of each GEMM launch of those counter runs
 
 
-KERNEL_OF_CLASS = {'gemm f64': 'gemm_grouped_kernel<0>/<4>', 'gemm f32': 'gemm_grouped_kernel<1>',
+KERNEL_OF_CLASS = {'gemm f64': 'gemm_grouped_kernel<0>', 'gemm f32': 'gemm_grouped_kernel<1>',
                    'gemm bf16 matvec T': 'gemm_grouped_kernel<3>',
                    'gemm bf16 matvec w': 'gemm_grouped_kernel<2>', 'mixer': 'mix_kernel',
                    'k_dots': 'k_dots', 'k_update_dots': 'k_update_dots',

@@ -164,9 +164,9 @@ int tnx_abi_sizes(int32_t* sizes, int n);
  * / right2left) as used by MPSClass.py:837-858 and MPSClass.py:555-611.
  * ntiles = total 64x64 tiles; active = device int flags or NULL.
  * mode = tnx_gemm_mode | (variant << 8): a mode may have several kernel
- * variants (LDS staging depth and occupancy), all giving the same bits;
- * variant 0 is the default.  The matvec plan's mode / mode2 fields take the
- * same encoding.                                                           */
+ * variants (workgroup shapes), all giving the same bits; variant 0 is the
+ * default, chosen by the number of tiles.  The matvec plan's mode / mode2
+ * fields take the same encoding.                                           */
 int tnx_gemm_grouped(int mode, const tnx_gemm_problem* prob, int nprob,
                      const tnx_gemm_seg* seg, int ntiles, const int32_t* active,
                      tnx_stream_t stream);
