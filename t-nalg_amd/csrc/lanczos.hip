@@ -303,13 +303,13 @@ __device__ __forceinline__ int count_below(const double* a, const double* c2, in
 // ends of the bracket, at distances halving towards the secant's zero from
 // both ends: its error is of second order in the bracket, so four or five
 // rounds take the place of nine.  A secant round that gains less than an even
-// one is followed by an even one.  LOWEST: idx = 0.
+// one is followed by an even one.  g: a first guess in the place of the
+// secant's zero, if it lies inside the bracket.  LOWEST: idx = 0.
 template <bool LOWEST>
 __device__ __forceinline__ double multisect(const double* a, const double* c2, int k, int idx,
-                                            double lo, double hi, double stop) {
+                                            double lo, double hi, double stop, double g) {
   const int lane = threadIdx.x & 63;
-  bool secant = false;
-  double g = 0.0;
+  bool secant = g > lo && g < hi;
   for (int round = 0; round < 24; ++round) {
     const double w = hi - lo;  // all of these identical in every lane
     if (w <= stop) break;
@@ -344,7 +344,7 @@ __device__ __forceinline__ double multisect(const double* a, const double* c2, i
 
 // Eigenpair idx (0: the lowest) of the k x k tridiagonal (a, b) in LDS, by one
 // wavefront (all 64 lanes): *theta and y[0..k) (LDS).  work: LDS scratch of
-// TRI_WORK doubles of the wavefront's own.
+// TRI_WORK doubles of the wavefront's own; guess: of the eigenvalue, or NaN.
 // The eigenvalue is searched between the Gershgorin bounds (the smallest
 // diagonal entry bounds the lowest).  The vector is that of the twisted
 // factorisation: the pivots of T - theta from the top (D+) and from the bottom
@@ -359,11 +359,12 @@ __device__ __forceinline__ double multisect(const double* a, const double* c2, i
 // Bound: the serial chains over k rows.  k_update_norm, most of which this is
 // (mean over k = 1..20, one solve, MI355X): 16.1 us with Sturm sequences by
 // division in 256 lanes and inverse iteration by one lane, 12.2 with minors and
-// even rounds only, 8.3 so.
+// even rounds only, 8.3 with secant points, 7.9 from the last eigenvalue on.
 constexpr int TRI_WORK = 6 * NCV_MAX + 2;
 template <bool LOWEST>
 __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, int k, int idx,
-                                             double* y, double* theta, double* work) {
+                                             double* y, double* theta, double* work,
+                                             double guess) {
   const int lane = threadIdx.x & 63;
   if (k == 1) {
     if (lane == 0) {
@@ -395,7 +396,8 @@ __device__ __forceinline__ void tridiag_pair(const double* a, const double* b, i
   const double stop = __builtin_amdgcn_ldexp(
       4.0 * 2.220446049250313e-16 * fmax(fabs(base), fabs(top)), -ex) + 1e-300;
   const double th = multisect<LOWEST>(
-      as, c2, k, idx, 0.0, __builtin_amdgcn_ldexp(top - base, -ex) * (1.0 + 1e-12), stop);
+      as, c2, k, idx, 0.0, __builtin_amdgcn_ldexp(top - base, -ex) * (1.0 + 1e-12), stop,
+      __builtin_amdgcn_ldexp(guess - base, -ex));
   // minors: lane 0 from the top, lane 1 from the bottom, with the one before
   // each at the same scale
   const bool up = lane & 1;
@@ -683,8 +685,9 @@ __device__ __forceinline__ double new_coupling(const double* h, int j, int v_dty
 // convergence test, by one wavefront (LDS: a, b with entries 0..j-1 loaded,
 // y, work).  True if the solve converged (its active flag is cleared).
 __device__ __forceinline__ bool finish_step(const tnx_lanczos_solve& D, const LzLayout& L, int s,
-                                            int j, double alpha, double beta, int min_iters,
-                                            double* a, double* b, double* y, double* work) {
+                                            int j, double alpha, double beta, double last_theta,
+                                            int min_iters, double* a, double* b, double* y,
+                                            double* work) {
   const int lane = threadIdx.x & 63;
   LzState& st = L.st[s];
   __shared__ double th_s;
@@ -693,7 +696,9 @@ __device__ __forceinline__ bool finish_step(const tnx_lanczos_solve& D, const Lz
     b[j] = beta;
   }
   __builtin_amdgcn_wave_barrier();
-  tridiag_pair<true>(a, b, j + 1, 0, y, &th_s, work);
+  // the lowest eigenvalue only falls as the matrix grows: the last one is a
+  // close guess
+  tridiag_pair<true>(a, b, j + 1, 0, y, &th_s, work, last_theta);
   __builtin_amdgcn_wave_barrier();
   if (lane <= j) st.y[lane] = y[lane];
   const double anorm = -tnx_wave_min(
@@ -798,7 +803,7 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
     a_s[threadIdx.x] = st.alpha[threadIdx.x];
     b_s[threadIdx.x] = st.beta[threadIdx.x];
   }
-  const double h1j = st.h1[j];
+  const double h1j = st.h1[j], last = st.theta;
   reduce_partials(L.partB, nchunks, D.chunk_begin, (D.n + CHUNK - 1) / CHUNK, j + 2, j + 2, h);
   __syncthreads();
   if (threadIdx.x >= 64) return;
@@ -809,7 +814,7 @@ __global__ __launch_bounds__(NP) void k_update_norm(const tnx_lanczos_solve* __r
   if ((int)threadIdx.x <= j) st.h2[threadIdx.x] = h[threadIdx.x];
   bool skip;
   const double beta = new_coupling(h, j, D.v_dtype, &skip);
-  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, min_iters, a_s, b_s, y_s, work);
+  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, last, min_iters, a_s, b_s, y_s, work);
   publish_nact(L, nsolve, conv, nact_host);
   tnx_stamp_end(ts);
 }
@@ -844,6 +849,7 @@ __device__ __forceinline__ void step_small_body(const tnx_lanczos_solve& D, cons
     r[q] = tnx_load((const void*)D.w, wd, elem(ci, q));
     if (!inside(ci, q)) r[q] = 0.0;
   }
+  const double last = st.theta;
   if (t < j) {
     a_s[t] = st.alpha[t];
     b_s[t] = st.beta[t];
@@ -910,7 +916,7 @@ __device__ __forceinline__ void step_small_body(const tnx_lanczos_solve& D, cons
     }
   if (t >= 64) return;
   if (t <= j) st.h2[t] = h[t];
-  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, min_iters, a_s, b_s, y_s, work);
+  const bool conv = finish_step(D, L, s, j, h1j + h[j], beta, last, min_iters, a_s, b_s, y_s, work);
   publish_nact(L, nsolve, conv, nact_host);
 }
 
@@ -1110,7 +1116,9 @@ __global__ __launch_bounds__(NT) void k_irl_solve(const tnx_lanczos_solve* __res
   __shared__ double yk[LZ_KEEP][NCV_MAX], thk[LZ_KEEP], tw[LZ_KEEP][TRI_WORK], sigma_s;
   __shared__ int pairs_s;
   static_assert(NT / 64 >= LZ_KEEP, "a wavefront per kept Ritz pair");
-  if (t / 64 < k) tridiag_pair<false>(a_l, b_l, m, t / 64, yk[t / 64], &thk[t / 64], tw[t / 64]);
+  if (t / 64 < k) 
+    tridiag_pair<false>(a_l, b_l, m, t / 64, yk[t / 64], &thk[t / 64], tw[t / 64],
+                        __builtin_nan(""));
   __syncthreads();
   if (t < 64) {
     const bool ok = restart_from_pairs(yk, thk, m, k, b_l[m - 1], st, &sigma_s);
