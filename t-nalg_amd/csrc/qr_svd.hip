@@ -391,6 +391,10 @@ __global__ __launch_bounds__(NQ) void qr_kernel(const tnx_qr_job* __restrict__ j
 // as the block Jacobi does, costs sweeps here (1.2 ms at 64).
 constexpr size_t SVD_LDS = 100 * 1024;
 constexpr int SVD_T = 16;
+// the SVD by way of a QR: rows, and columns, at most (SVD_LDS holds m n + 2 n^2
+// doubles)
+constexpr int SVD_QR_M = 256;
+constexpr int SVD_QR_N = 72;
 
 // sum over the 16 lanes of a row
 __device__ __forceinline__ double row_sum(double v) {
@@ -445,6 +449,77 @@ __device__ __forceinline__ void jacobi_sweeps(PW W, int m, PW V, int n, double e
             jacobi_apply(jr, x, y);
             va[r] = x;
             vb[r] = y;
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (rotated == 0) break;
+    __syncthreads();
+  }
+}
+
+// The same for two n x n matrices in LDS, n <= 16 NE: a lane's NE elements of the
+// pair's columns of W and V stay in registers from the dot products to the
+// store, all reads ahead of the angle.  Bound: latency, one such chain a round
+// (order 64 over 10 decades 609 us in all, 785 with the elements read again for
+// each use and the pair found by remainders; 8 or 32 lanes a pair 980 and 890).
+template <int NE>
+__device__ __forceinline__ void jacobi_sweeps_lds(double* W, double* V, int n, double eps,
+                                                  int max_sweeps, int& rotated) {
+  const int l = threadIdx.x & (SVD_T - 1), p = threadIdx.x / SVD_T;
+  const int np = (n + 1) & ~1;   // players in the round-robin tournament
+  static_assert(NQ / SVD_T >= SVD_QR_N / 2, "every pair of a round at once");
+  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    if (threadIdx.x == 0) rotated = 0;
+    __syncthreads();
+    for (int round = 0; round < np - 1; ++round) {
+      // circle method: player np-1 fixed, others rotate
+      int a = round + p, b = round + np - 1 - p;
+      a = p == 0 ? np - 1 : a >= np - 1 ? a - (np - 1) : a;
+      b = p == 0 ? round : b >= np - 1 ? b - (np - 1) : b;
+      if (p < np / 2 && max(a, b) < n) {
+        const int u = min(a, b), v = max(a, b);
+        double* wa = W + u * n;
+        double* wb = W + v * n;
+        double* va = V + u * n;
+        double* vb = V + v * n;
+        double x[NE], y[NE], xv[NE], yv[NE];
+#pragma unroll
+        for (int e = 0; e < NE; ++e) {
+          const int r = min(l + SVD_T * e, n - 1);
+          x[e] = wa[r];
+          y[e] = wb[r];
+          xv[e] = va[r];
+          yv[e] = vb[r];
+        }
+        double al = 0.0, be = 0.0, ga = 0.0;
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+          if (l + SVD_T * e < n) {
+            al += x[e] * x[e];
+            be += y[e] * y[e];
+            ga += x[e] * y[e];
+          }
+        al = row_sum(al);
+        be = row_sum(be);
+        ga = row_sum(ga);
+        const double ab = al * be;
+        const bool rot = ga != 0.0 && fabs(ga) > eps * (ab > 0.0 ? ab * __builtin_amdgcn_rsq(ab) : 0.0);
+        if (rot) {
+          const JacobiRot jr = jacobi_rot(al, be, ga, rot, false);
+          if (l == 0) rotated = 1;
+#pragma unroll
+          for (int e = 0; e < NE; ++e) {
+            jacobi_apply(jr, x[e], y[e]);
+            jacobi_apply(jr, xv[e], yv[e]);
+            if (l + SVD_T * e < n) {
+              const int r = l + SVD_T * e;
+              wa[r] = x[e];
+              wb[r] = y[e];
+              va[r] = xv[e];
+              vb[r] = yv[e];
+            }
           }
         }
       }
@@ -580,10 +655,8 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
 // the rank.  A (m x n), X and V (n x n) in LDS, m <= 64 ROWS.  M is scaled by a
 // power of two, so that squares of its entries stay in range.
 // us (MI355X), columns of M -> this: order 64 with values over 10 decades 2030 ->
-// 785, over 20 2430 -> 775, random 840 -> 930; 128 x 40 over 10 decades 1150 ->
-// 394, random 550 -> 456; order 16 132 -> 84, random 84 -> 91.
-constexpr int SVD_QR_M = 256;
-constexpr int SVD_QR_N = 72;   // columns at most (SVD_LDS holds m n + 2 n^2 doubles)
+// 609, random 840 -> 717; 128 x 40 over 10 decades 1150 -> 302, random 550 ->
+// 343; order 16 132 -> 67, random 84 -> 71; order 8 41 -> 29.
 template <int ROWS>
 __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps, double* A, double* X,
                                             double* V, double* sv, int* order, int& rotated) {
@@ -687,7 +760,12 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
       X[i * n + c] = c > i ? A[pc * m + i] : c == i ? beta[i] : 0.0;
     }
   __syncthreads();
-  jacobi_sweeps(X, n, V, n, 2.220446049250313e-16 * (double)(m > 8 ? m : 8), max_sweeps, rotated);
+  const double eps = 2.220446049250313e-16 * (double)(m > 8 ? m : 8);
+  if (n <= 16) jacobi_sweeps_lds<1>(X, V, n, eps, max_sweeps, rotated);
+  else if (n <= 32) jacobi_sweeps_lds<2>(X, V, n, eps, max_sweeps, rotated);
+  else if (n <= 48) jacobi_sweeps_lds<3>(X, V, n, eps, max_sweeps, rotated);
+  else if (n <= 64) jacobi_sweeps_lds<4>(X, V, n, eps, max_sweeps, rotated);
+  else jacobi_sweeps_lds<5>(X, V, n, eps, max_sweeps, rotated);
   sort_columns(X, n, n, sv, order);
   double TNX_GLOBAL* s_out = as_global<double>(J.s);
   double TNX_GLOBAL* u = as_global<double>(J.u);
