@@ -664,7 +664,10 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int NW = NQ / 64;
-  __shared__ double nrm[SVD_QR_N], v0s[SVD_QR_N], fs[SVD_QR_N], beta[SVD_QR_N];
+  // nrm: norms^2 of the remaining columns, two copies.  Step k reads one and
+  // writes the other, so that a wave which comes to its choice late chooses
+  // from the same norms as the rest (the waves' orders must not differ).
+  __shared__ double nrm[2][SVD_QR_N], v0s[SVD_QR_N], fs[SVD_QR_N], beta[SVD_QR_N];
   const double TNX_GLOBAL* src = as_global<const double>(J.src);
   double big = 0.0;
   for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
@@ -691,7 +694,7 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
     double t = 0.0;
     for (int r = lane; r < m; r += 64) t += A[c * m + r] * A[c * m + r];
     t = tnx_wave_sum(t);
-    if (lane == 0) nrm[c] = t;
+    if (lane == 0) nrm[0][c] = t;
   }
   __syncthreads();
   // pivoted order, a copy per wave: lane j has the column at position j, and
@@ -702,8 +705,9 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   };
   for (int k = 0; k < n; ++k) {
     // position of the largest remaining column (the first of equal ones)
-    const double n0 = lane >= k && lane < n ? nrm[p0] : -1.0;
-    const double n1 = 64 + lane >= k && 64 + lane < n ? nrm[p1] : -1.0;
+    const double* now = nrm[k & 1];
+    const double n0 = lane >= k && lane < n ? now[p0] : -1.0;
+    const double n1 = 64 + lane >= k && 64 + lane < n ? now[p1] : -1.0;
     const double top = tnx_wave_fold(fmax(n0, n1), [](double x, double y) { return fmax(x, y); });
     const unsigned long long m0 = __ballot(n0 == top), m1 = __ballot(n1 == top);
     const int best = m0 ? __builtin_ctzll(m0) : m1 ? 64 + __builtin_ctzll(m1) : k;   // (NaN: k)
@@ -749,7 +753,7 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
         if (r > k) t2 += y[t] * y[t];
       }
       t2 = tnx_wave_sum(t2);
-      if (lane == 0) nrm[at(j)] = t2;
+      if (lane == 0) nrm[(k & 1) ^ 1][at(j)] = t2;
     }
     __syncthreads();
   }

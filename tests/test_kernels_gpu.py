@@ -1327,3 +1327,50 @@ def test_svd_jacobi_by_qr(gpu, m, n, kind):
         assert np.abs(S - ref).max() <= 1e-14 * n * sc
         assert np.abs(U.T @ U - np.eye(n)).max() <= tol
         assert np.linalg.norm(U @ (V / sc) - M / sc) <= tol * nM
+
+
+@pytest.mark.parametrize('m,n', [(8, 8), (32, 32), (65, 65), (150, 30)])
+@pytest.mark.parametrize('kind', ['isometry', 'multiple', 'hadamard', 'pairs'])
+def test_svd_columns_of_equal_norm(gpu, m, n, kind):
+    """The SVD by way of a pivoted QR where the choice of the pivot hangs on the
+    last bit: an isometry, a multiple of one, columns of +-1 (equal norms that
+    the downdates keep nearly equal) and every column twice.  The waves choose
+    for themselves, and their orders must not differ.  Bounds of
+    test_svd_jacobi_by_qr, several launches of 64 jobs."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + n)
+    njob = 64
+    tol = 1e-14 * max(m, 8)
+    mats = []
+    for _ in range(njob):
+        M = np.linalg.qr(rng.randn(m, n))[0]
+        if kind == 'multiple':
+            M = M * 3.7e5
+        elif kind == 'hadamard':
+            M = np.where(rng.randn(m, n) < 0, -1.0, 1.0)
+        elif kind == 'pairs':
+            M[:, 1::2] = M[:, 0:2 * (n // 2):2]
+        mats.append(M)
+    src = _dev(np.stack(mats))
+    u, s, vt, w = (torch.zeros(njob, k, dtype=torch.float64, device='cuda')
+                   for k in (m * n, n, n * n, m * n + n * n))
+    jobs = np.array([(src[k].data_ptr(), u[k].data_ptr(), s[k].data_ptr(), vt[k].data_ptr(),
+                      w[k].data_ptr(), m, n, n, 0, 0, 0) for k in range(njob)], dtype=L.SVD_JOB)
+    (dj,) = _upload([jobs])
+    first = None
+    for rep in range(3):
+        print('svd equal norms', m, n, kind, 'rep', rep, flush=True)
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), njob, 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        got = [x.cpu().numpy() for x in (u, s, vt)]
+        if first is None:
+            first = got
+        assert all(np.array_equal(a, b) for a, b in zip(got, first))
+    for k, M in enumerate(mats):
+        U, S, V = first[0][k].reshape(m, n), first[1][k], first[2][k].reshape(n, n)
+        ref = np.linalg.svd(M, compute_uv=False)
+        assert np.abs(S - ref).max() <= 1e-14 * n * ref[0]
+        assert np.abs(U.T @ U - np.eye(n)).max() <= tol
+        assert np.linalg.norm(U @ V - M) <= tol * np.linalg.norm(M)
