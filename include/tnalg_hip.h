@@ -51,6 +51,14 @@ enum tnx_gemm_mode {
   TNX_GEMM_BF16_BF16 = 3, /* bf16 x bf16 -> MFMA bf16 (f32 acc) -> bf16     */
 };
 
+/* Flag of a GEMM mode, TNX_GEMM_F64 only: an element's products are summed in
+ * the order of k, segment after segment.  A matvec plan with the flag in its
+ * `mode` has the Lanczos calls keep to a fixed order of every sum too, and a
+ * tnx_svd_job asks for the same by `in_order`.  For callers whose results hang
+ * on the last bit (a truncation between equal Schmidt values): with the flag
+ * they do not change when the other kernels are regrouped for speed.        */
+#define TNX_GEMM_IN_ORDER 0x10000
+
 /* One K-segment of a grouped GEMM problem: C += alpha * op(A) * op(B).
  * op(A) is M x K: A[i*lda+k] (transA=0) or A[k*lda+i] (transA=1).
  * op(B) is K x N: B[k*ldb+j] (transB=0) or B[j*ldb+k] (transB=1).           */
@@ -165,8 +173,8 @@ int tnx_abi_sizes(int32_t* sizes, int n);
  * ntiles = total 64x64 tiles; active = device int flags or NULL.
  * mode = tnx_gemm_mode | (variant << 8): a mode may have several kernel
  * variants (workgroup shapes), all giving the same bits; variant 0 is the
- * default, chosen by the number of tiles.  The matvec plan's mode / mode2
- * fields take the same encoding.                                           */
+ * default, chosen by the number of tiles.  TNX_GEMM_IN_ORDER may be added to
+ * TNX_GEMM_F64.  The matvec plan's mode / mode2 fields take the same encoding. */
 int tnx_gemm_grouped(int mode, const tnx_gemm_problem* prob, int nprob,
                      const tnx_gemm_seg* seg, int ntiles, const int32_t* active,
                      tnx_stream_t stream);
@@ -284,7 +292,7 @@ int tnx_chol_inv_f64(const tnx_chol_job* jobs, int njob, tnx_stream_t stream);
 typedef struct tnx_svd_job {
   uint64_t src, u, s, svt, work;
   int32_t m, n, ld, trans;
-  int32_t u_trans, reserved;
+  int32_t u_trans, in_order; /* in_order != 0: see TNX_GEMM_IN_ORDER           */
 } tnx_svd_job; /* 64 bytes */
 int tnx_svd_jacobi_f64(const tnx_svd_job* jobs, int njob, int max_sweeps, tnx_stream_t stream);
 

@@ -130,8 +130,12 @@ template <typename TI, int TT, int MB> struct Operand {
     }
   }
 
-  // Half chunk h of the wave's rows from `row` (within the tile)
-  template <bool KC> struct Raw {
+  // Half chunk h of the wave's rows from `row` (within the tile).  SEQ (f64):
+  // MFMA t takes k = 4 t + g of the half chunk from lane group g, so that the
+  // sum over k runs in the order of the index (8-byte instead of 16-byte LDS
+  // reads: GEMM 2 of an order-64 problem and its like 10.1 instead of 9.5 us).
+  template <bool KC, bool SEQ> struct Raw {
+    static_assert(!SEQ || sizeof(TI) == 8, "in-order sums are f64");
     // [k][row]: KL loads of MB elements (16-bit ones as whole words)
     static constexpr int W = KC ? 4 : (MB * (int)sizeof(TI) + 3) / 4;
     uint32_t w[KC ? MB : KL][W];
@@ -142,15 +146,25 @@ template <typename TI, int TT, int MB> struct Operand {
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
           const int rr = row + MB * m + i;
-          const u4 v = lds[rr * 8 + ((4 * h + g) ^ swz(rr))];
+          if constexpr (SEQ) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x) w[i][x] = v[x];
+            for (int t = 0; t < KL; ++t) {
+              const u4* p = lds + rr * 8 + ((4 * h + 2 * t + (g >> 1)) ^ swz(rr));
+              const double v = ((const double*)p)[g & 1];
+              __builtin_memcpy(&w[i][2 * t], &v, 8);
+            }
+          } else {
+            const u4 v = lds[rr * 8 + ((4 * h + g) ^ swz(rr))];
+#pragma unroll
+            for (int x = 0; x < 4; ++x) w[i][x] = v[x];
+          }
         }
       } else {
-        const char* p = (const char*)lds + ((h * (KB / 2) + KL * g) * TT + row + MB * m) * (int)sizeof(TI);
+        const char* p = (const char*)lds +
+                        ((h * (KB / 2) + (SEQ ? 1 : KL) * g) * TT + row + MB * m) * (int)sizeof(TI);
 #pragma unroll
         for (int s = 0; s < KL; ++s) {
-          const char* q = p + s * TT * (int)sizeof(TI);
+          const char* q = p + s * (SEQ ? 4 : 1) * TT * (int)sizeof(TI);
           if constexpr (MB * sizeof(TI) == 2) w[s][0] = *(const uint16_t*)q;
           else {
             typedef uint32_t V __attribute__((ext_vector_type(W)));
@@ -185,15 +199,15 @@ template <typename TI, int TT, int MB> struct Operand {
 };
 
 // acc += the staged chunk's A B, the wave's rows from wr and columns from wc
-template <int MODE, int TT, int MB, bool KA, bool KBc>
+template <int MODE, bool SEQ, int TT, int MB, bool KA, bool KBc>
 __device__ __forceinline__ void mma_chunk(typename Tr<MODE>::V4 (&acc)[MB][MB], const u4* As,
                                           const u4* Bs, int wr, int wc) {
   typedef typename Tr<MODE>::TI TI;
   typedef Operand<TI, TT, MB> O;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    typename O::template Raw<KA> a;
-    typename O::template Raw<KBc> b;
+    typename O::template Raw<KA, SEQ> a;
+    typename O::template Raw<KBc, SEQ> b;
     a.read(As, wr, h);
     b.read(Bs, wc, h);
     if constexpr (O::HALF) {
@@ -258,7 +272,7 @@ __device__ __forceinline__ bool wide(int M, int N, int K) {
 // ahead of the staged one, across the segments; past the last chunk it is
 // fetched again, unused (no branch around the loads, so that the waits count
 // them and never drain them).
-template <int MODE, int TT, int PD, bool KA, bool KBc, bool WIDE>
+template <int MODE, bool SEQ, int TT, int PD, bool KA, bool KBc, bool WIDE>
 __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][TT / 32],
                                           const tnx_gemm_seg TNX_CONST* segs, int s, int s_end,
                                           int M, int N, int row0, int col0, int wr, int wc,
@@ -326,7 +340,7 @@ __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][
   // refilled
   auto step = [&](int u) {
     const int d = (u + 1) % PD, stage = u & 1;
-    mma_chunk<MODE, TT, MB, KA, KBc>(acc, As[stage], Bs[stage], wr, wc);
+    mma_chunk<MODE, SEQ, TT, MB, KA, KBc>(acc, As[stage], Bs[stage], wr, wc);
     commit(d, stage ^ 1);
     fetch(d);
     lds_barrier();
@@ -357,7 +371,7 @@ __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][
 // Tried and not kept: operands straight from global memory to the MFMA
 // registers (an operand contiguous in k then touches 16 lines per load: f64
 // 58 of 73 and 42 where both are), 128 x 128 workgroups (f64 32, f32 63).
-template <int MODE, int TT, int PD, int W>
+template <int MODE, bool SEQ, int TT, int PD, int W>
 __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_problem* __restrict__ probs,
                                                            int nprob,
                                                            const tnx_gemm_seg* __restrict__ segs,
@@ -448,9 +462,9 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
     typedef Operand<typename T::TI, TT, MB> O;
 #define TNX_STREAM(KA, KBc)                                                                 \
   s = wide<O, KA, KBc>(P.M, P.N, K)                                                         \
-          ? run_stream<MODE, TT, PD, KA, KBc, true>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
+          ? run_stream<MODE, SEQ, TT, PD, KA, KBc, true>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
                                                     wc, As, Bs)                             \
-          : run_stream<MODE, TT, PD, KA, KBc, false>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
+          : run_stream<MODE, SEQ, TT, PD, KA, KBc, false>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
                                                      wc, As, Bs)
     if (!ta && tb) TNX_STREAM(true, true);
     else if (!ta) TNX_STREAM(true, false);
@@ -507,10 +521,10 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
 // 256 tiles 12.5 / 8.3).
 static int gemm_small_tiles(int mode) { return mode <= TNX_GEMM_F32 ? 256 : 128; }
 
-template <int MODE, int TT, int PD, int W>
+template <int MODE, bool SEQ, int TT, int PD, int W>
 static void launch_gemm(const tnx_gemm_problem* prob, int nprob, const tnx_gemm_seg* seg, int ntiles,
                         const int32_t* active, hipStream_t s, unsigned long long* ts) {
-  hipLaunchKernelGGL((gemm_grouped_kernel<MODE, TT, PD, W>), dim3(TT == 32 ? 4 * ntiles : ntiles),
+  hipLaunchKernelGGL((gemm_grouped_kernel<MODE, SEQ, TT, PD, W>), dim3(TT == 32 ? 4 * ntiles : ntiles),
                      dim3(256), 0, s, prob, nprob, seg, ntiles, active, ts);
 }
 
@@ -542,7 +556,9 @@ int tnx_gemm_grouped_ts(int mode, const tnx_gemm_problem* prob, int nprob,
   }
   const int base = mode & 0xFF, var = (mode >> 8) & 0xFF;
   const int nvar = tnx_gemm_variants(base);
-  if (nvar < 0 || (mode >> 16) != 0 || var >= nvar) {
+  const bool in_order = (mode & TNX_GEMM_IN_ORDER) != 0;
+  if (nvar < 0 || (mode & ~(TNX_GEMM_IN_ORDER | 0xFFFF)) != 0 || var >= nvar ||
+      (in_order && base != TNX_GEMM_F64)) {
     tnx_set_error("tnx_gemm_grouped: unknown mode %d (variant %d)", base, var);
     return TNX_EINVAL;
   }
@@ -551,14 +567,20 @@ int tnx_gemm_grouped_ts(int mode, const tnx_gemm_problem* prob, int nprob,
   // variant 0 takes the shape of the rule, variant 1 the other one; the 32x32
   // grid has four workgroups a tile, which a launch's x extent must hold
   const bool small = ((ntiles <= gemm_small_tiles(base)) != (var == 1)) && ntiles < (1 << 29);
-#define TNX_GEMM_LAUNCH(MODE, PDS, WS, PDL, WL)                                           \
-  if (small) launch_gemm<MODE, 32, PDS, WS>(prob, nprob, seg, ntiles, active, s, ts);     \
-  else launch_gemm<MODE, 64, PDL, WL>(prob, nprob, seg, ntiles, active, s, ts)
+#define TNX_GEMM_LAUNCH(MODE, SEQ, PDS, WS, PDL, WL)                                          \
+  if (small) launch_gemm<MODE, SEQ, 32, PDS, WS>(prob, nprob, seg, ntiles, active, s, ts);     \
+  else launch_gemm<MODE, SEQ, 64, PDL, WL>(prob, nprob, seg, ntiles, active, s, ts)
   switch (base) {
-    case TNX_GEMM_F64: TNX_GEMM_LAUNCH(TNX_GEMM_F64, 3, 4, 1, 3); break;
-    case TNX_GEMM_F32: TNX_GEMM_LAUNCH(TNX_GEMM_F32, 3, 4, 1, 3); break;
-    case TNX_GEMM_BF16_F32: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_F32, 4, 3, 1, 2); break;
-    default: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_BF16, 4, 3, 1, 2); break;
+    case TNX_GEMM_F64:
+      if (in_order) {
+        TNX_GEMM_LAUNCH(TNX_GEMM_F64, true, 3, 4, 1, 3);
+      } else {
+        TNX_GEMM_LAUNCH(TNX_GEMM_F64, false, 3, 4, 1, 3);
+      }
+      break;
+    case TNX_GEMM_F32: TNX_GEMM_LAUNCH(TNX_GEMM_F32, false, 3, 4, 1, 3); break;
+    case TNX_GEMM_BF16_F32: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_F32, false, 4, 3, 1, 2); break;
+    default: TNX_GEMM_LAUNCH(TNX_GEMM_BF16_BF16, false, 4, 3, 1, 2); break;
   }
 #undef TNX_GEMM_LAUNCH
   TNX_CHECK_LAUNCH();

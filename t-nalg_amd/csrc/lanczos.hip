@@ -17,6 +17,8 @@
 // The matvec may run in f32 or bf16.
 // The (j+1)x(j+1) tridiagonal eigenproblem is solved on the device by one
 // wavefront: multisection with secant steps, then a twisted factorisation.
+// (A call whose plan asks for sums in a fixed order takes the passes of
+// lanczos_in_order.h.)
 // A solve that has not converged after ncv steps is restarted implicitly
 // (Sorensen's implicitly restarted Lanczos with exact shifts, as ARPACK's
 // dsaupd does for eigsh): the ncv - k largest Ritz values are applied as
@@ -1386,6 +1388,8 @@ __global__ __launch_bounds__(NP) void k_final(const tnx_lanczos_solve* __restric
   else final_rows<double>(D, ci, y, st.jlast + 1);
 }
 
+#include "lanczos_in_order.h"
+
 // pinned staging for the polled active count and the results
 struct Pinned {
   int32_t* nact = nullptr;
@@ -1448,15 +1452,17 @@ int check_args(const char* who, const tnx_matvec_plan* plans, int nplan,
 // The launches of a call before its first Krylov step: state zeroed, every
 // solve active, start vectors normalised into V[0] and x.
 int issue_start(const tnx_lanczos_solve* solves, int nsolve, void* state, int nchunks,
-                int x_dtype, hipStream_t s) {
+                int x_dtype, bool in_order, hipStream_t s) {
   LzLayout L = lz_layout(state, nsolve, nchunks);
   const size_t words = sizeof(LzState) * (size_t)nsolve / sizeof(uint64_t);
   static_assert(sizeof(LzState) % sizeof(uint64_t) == 0, "LzState is whole words");
   hipLaunchKernelGGL(k_zero_words, dim3((unsigned)((words + 255) / 256 < 1024 ? (words + 255) / 256 : 1024)),
                      dim3(256), 0, s, (uint64_t*)L.st, words, L.nact, nsolve);
-  hipLaunchKernelGGL(k_init_norm, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks);
-  hipLaunchKernelGGL(k_init_scale, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks,
-                     x_dtype);
+  const dim3 grid(nchunks), block(in_order ? IT : NP);
+  hipLaunchKernelGGL(in_order ? io_init_norm : k_init_norm, grid, block, 0, s, solves, nsolve, state,
+                     nchunks);
+  hipLaunchKernelGGL(in_order ? io_init_scale : k_init_scale, grid, block, 0, s, solves, nsolve,
+                     state, nchunks, x_dtype);
   TNX_CHECK_LAUNCH();
   return TNX_OK;
 }
@@ -1482,7 +1488,17 @@ SmallKernel small_pass(int j, int chunks) {
   return chunks == 2 && j < 20 ? two[j / 4] : nullptr;
 }
 
-BasisPass basis_pass(int j) {
+// whether a call's passes keep to the fixed order of sums
+bool call_in_order(const tnx_matvec_plan* plans) {
+  return (plans[0].mode & TNX_GEMM_IN_ORDER) != 0;
+}
+
+BasisPass basis_pass(int j, bool in_order) {
+  static const BasisPass fixed[NCV_MAX / 4] = {
+      {io_pass1<4>, io_pass2<4>},   {io_pass1<8>, io_pass2<8>},   {io_pass1<12>, io_pass2<12>},
+      {io_pass1<16>, io_pass2<16>}, {io_pass1<20>, io_pass2<20>}, {io_pass1<24>, io_pass2<24>},
+      {io_pass1<28>, io_pass2<28>}, {io_pass1<32>, io_pass2<32>}};
+  if (in_order) return fixed[j / 4];
   static const BasisPass table[NCV_MAX / 4] = {
       {k_dots<4>, k_update_dots<4>},   {k_dots<8>, k_update_dots<8>},
       {k_dots<12>, k_update_dots<12>}, {k_dots<16>, k_update_dots<16>},
@@ -1501,7 +1517,8 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   LzLayout L = lz_layout(state, nsolve, nchunks);
   for (int p = 0; p < nplan; ++p)
     if (int rc = tnx_heff_matvec(plans + p, L.act, stream)) return rc;
-  const dim3 grid(nchunks), block(NP);
+  const bool in_order = call_in_order(plans);
+  const dim3 grid(nchunks), block(in_order ? IT : NP);
   // sampled timing (one plan: its modes give the x and w element sizes, and
   // the basis element size under the policy that a low-precision matvec
   // has an f32 basis); algorithmic bytes over the nchunks * CHUNK
@@ -1519,14 +1536,14 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   // Every solve has a chunk at least, so none has more than this.  (Sampled
   // timing keeps the three passes, which it reports one by one.)
   const int most = nchunks - nsolve + 1;
-  if (const SmallKernel small = prof ? nullptr : small_pass(j, most)) {
+  if (const SmallKernel small = prof || in_order ? nullptr : small_pass(j, most)) {
     hipLaunchKernelGGL(small, dim3(nsolve), dim3(most * NP), 0, s, solves, nsolve, state, nchunks,
                        j, w_dtype, x_dtype, min_iters, nact_host);
     TNX_CHECK_LAUNCH();
     return TNX_OK;
   }
   int mk = prof ? tnx_prof_mark(TNX_PC_DOTS, s) : -1;
-  const BasisPass pass = basis_pass(j);
+  const BasisPass pass = basis_pass(j, in_order);
   hipLaunchKernelGGL(pass.dots, grid, block, 0, s, solves, nsolve, state, nchunks, j, w_dtype,
                      tnx_prof_ts(mk));
   tnx_prof_done(mk, s, E * (vrows + ws));
@@ -1538,8 +1555,8 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
   // included (an implicit restart combines V[ncv] into the new basis)
   (void)ncv;
   mk = prof ? tnx_prof_mark(TNX_PC_UPDATE_NORM, s) : -1;
-  hipLaunchKernelGGL(k_update_norm, dim3(nchunks + nsolve), block, 0, s, solves, nsolve, state,
-                     nchunks, j, x_dtype, min_iters, nact_host, tnx_prof_ts(mk));
+  hipLaunchKernelGGL(in_order ? io_pass3 : k_update_norm, dim3(nchunks + nsolve), block, 0, s,
+                     solves, nsolve, state, nchunks, j, x_dtype, min_iters, nact_host, tnx_prof_ts(mk));
   // (r read, V[j+1] and x written; the basis rows of the second correction,
   // read only when it is not negligible, are not counted)
   tnx_prof_done(mk, s, E * (2.0 * vs + xs));
@@ -1550,10 +1567,11 @@ int issue_step(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve*
 // Implicit restart of the still-active solves after a full cycle: the next
 // cycle continues from Krylov step lz_keep(ncv).
 int issue_restart(const tnx_lanczos_solve* solves, int nsolve, void* state, int nchunks, int ncv,
-                  int x_dtype, hipStream_t s) {
+                  int x_dtype, bool in_order, hipStream_t s) {
   const int k = lz_keep(ncv);
-  hipLaunchKernelGGL(k_irl_solve, dim3(nsolve), dim3(NT), 0, s, solves, nsolve, state, nchunks,
-                     ncv, k);
+  static_assert(IT == NT, "one block size for both");
+  hipLaunchKernelGGL(in_order ? io_irl_solve : k_irl_solve, dim3(nsolve), dim3(NT), 0, s, solves,
+                     nsolve, state, nchunks, ncv, k);
   hipLaunchKernelGGL(k_irl_apply, dim3(nchunks), dim3(NP), 0, s, solves, nsolve, state, nchunks,
                      ncv, k, x_dtype);
   TNX_CHECK_LAUNCH();
@@ -1590,7 +1608,7 @@ int lanczos_run(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve
   if (int rc = ensure_pinned(nsolve)) return rc;
   hipStream_t s = (hipStream_t)stream;
   LzLayout L = lz_layout(state, nsolve, nchunks);
-  if (int rc = issue_start(solves, nsolve, state, nchunks, x_dtype, s)) return rc;
+  if (int rc = issue_start(solves, nsolve, state, nchunks, x_dtype, call_in_order(plans), s)) return rc;
 
   hipEvent_t ev[2];
   TNX_CHECK_HIP(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
@@ -1603,7 +1621,8 @@ int lanczos_run(const tnx_matvec_plan* plans, int nplan, const tnx_lanczos_solve
   int issued = 0;  // events recorded so far
   const bool sampled = tnx_prof_call_begin();
   for (int r = 0; r <= max_restarts && !done && !rc; ++r) {
-    if (r > 0 && (rc = issue_restart(solves, nsolve, state, nchunks, ncv, x_dtype, s))) break;
+    if (r > 0 && (rc = issue_restart(solves, nsolve, state, nchunks, ncv, x_dtype,
+                                     call_in_order(plans), s))) break;
     for (int j = (r > 0 ? lz_keep(ncv) : 0); j < ncv && !done; ++j) {
       tnx_prof_set(sampled && r == 0 && j == 0);
       // lagged poll: the step writes its active count to pin[slot], then
@@ -1760,7 +1779,9 @@ extern "C" int tnx_lanczos_run_multi_static(const tnx_matvec_plan* plans, int np
   tnx_lanczos_result* dres = (tnx_lanczos_result*)((char*)base + state_bytes);
   hipStream_t s = (hipStream_t)stream;
   LzLayout L = lz_layout(state, nsolve, nchunks);
-  if (int rc = issue_start(solves, nsolve, state, nchunks, TNX_DTYPE_PER_SOLVE, s)) return rc;
+  const bool in_order = call_in_order(plans);
+  if (int rc = issue_start(solves, nsolve, state, nchunks, TNX_DTYPE_PER_SOLVE, in_order, s))
+    return rc;
   // Every Krylov step of a cycle is queued without polling: a solve that has
   // converged is masked on the device, so its arithmetic, and the result,
   // are those of tnx_lanczos_run_multi.  The active count is read at the end
@@ -1769,7 +1790,8 @@ extern "C" int tnx_lanczos_run_multi_static(const tnx_matvec_plan* plans, int np
   const bool sampled = tnx_prof_call_begin();
   for (int r = 0; r <= max_restarts && !done; ++r) {
     if (r > 0)
-      if (int rc = issue_restart(solves, nsolve, state, nchunks, ncv, TNX_DTYPE_PER_SOLVE, s))
+      if (int rc = issue_restart(solves, nsolve, state, nchunks, ncv, TNX_DTYPE_PER_SOLVE,
+                                 in_order, s))
         return rc;
     for (int j = (r > 0 ? lz_keep(ncv) : 0); j < ncv; ++j) {
       tnx_prof_set(sampled && r == 0 && j == 0);

@@ -14,6 +14,7 @@ from .build import LIB_PATH
 
 F64, F32, BF16 = 0, 1, 2
 GEMM_F64, GEMM_F32, GEMM_BF16_F32, GEMM_BF16_BF16 = 0, 1, 2, 3
+GEMM_IN_ORDER = 0x10000   # flag of GEMM_F64: every sum of the call in a fixed order
 
 GEMM_SEG = np.dtype([('a', '<u8'), ('b', '<u8'), ('lda', '<i4'), ('ldb', '<i4'),
                      ('transA', '<i4'), ('transB', '<i4'), ('K', '<i4'), ('reserved', '<i4'),
@@ -46,7 +47,7 @@ QR_JOB = np.dtype([('src', '<u8'), ('q', '<u8'), ('r', '<u8'), ('work', '<u8'),
                    ('q_trans', '<i4'), ('reserved', '<i4')])
 SVD_JOB = np.dtype([('src', '<u8'), ('u', '<u8'), ('s', '<u8'), ('svt', '<u8'), ('work', '<u8'),
                     ('m', '<i4'), ('n', '<i4'), ('ld', '<i4'), ('trans', '<i4'),
-                    ('u_trans', '<i4'), ('reserved', '<i4')])
+                    ('u_trans', '<i4'), ('in_order', '<i4')])
 NORM_JOB = np.dtype([('x', '<u8'), ('n', '<i8')])
 FILL_JOB = np.dtype([('dst', '<u8'), ('n', '<i8'), ('seed', '<u8'), ('offset', '<i8')])
 KRON_TERM = np.dtype([('a', '<u8'), ('b', '<u8'), ('lda', '<i4'), ('ldb', '<i4'),

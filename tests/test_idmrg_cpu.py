@@ -142,3 +142,39 @@ def test_unsupported_configurations_raise():
         MpsInfinite('translation_invariant', 2, 4, 4, n_site=2, dmrg_type='white', device='cpu')
     with pytest.raises(ValueError):
         MpsInfinite('center_ort', 4, 4, 2, n_site=2, dmrg_type='mpo', device='cpu')
+
+
+@pytest.mark.parametrize('dtype', ['mpo', 'white'])
+def test_every_call_asks_for_sums_in_order(dtype):
+    """What a run returns can hang on the last bits (a degenerate pair of
+    Schmidt values at the cut), so its products, eigensolves and splits ask the
+    library for a fixed order of every sum."""
+    from idmrg_emul import EmulatedLib, _addr, _records
+    from tnalg_amd import _lib as L
+    from tnalg_amd.idmrg import InfiniteRun, MpsInfinite
+    seen = []
+
+    class Lib(EmulatedLib):
+        def tnx_gemm_grouped(self, mode, *a):
+            seen.append(('gemm', mode))
+            return super().tnx_gemm_grouped(mode, *a)
+
+        def tnx_svd_jacobi_f64(self, jobs, njob, *a):
+            seen.extend(('svd', int(j['in_order'])) for j in _records(_addr(jobs), L.SVD_JOB, njob))
+            return super().tnx_svd_jacobi_f64(jobs, njob, *a)
+
+        def tnx_lanczos_run_ex(self, plan, *a):
+            seen.append(('lanczos', plan.mode))
+            seen.append(('lanczos', plan.mode2))
+            return super().tnx_lanczos_run_ex(plan, *a)
+
+    para = _para(dtype, 3, True, sweeps=2, jxy=0.4, hx=0.2, hz=0.3)
+    h = P.hamiltonian_heisenberg('half', para['jxy'], para['jxy'], para['jz'], para['hx'] / 2,
+                                 para['hz'] / 2)
+    A = MpsInfinite('center_ort', 4 if dtype == 'mpo' else 2, 3, 4, n_site=2, is_symme_env=True,
+                    dmrg_type=dtype, hamilt_index=para['hamilt_index'],
+                    rng=np.random.RandomState(3), device='cpu')
+    InfiniteRun([A], [para], [h], lib=Lib(), stream=lambda: None).run()
+    want = {'gemm': L.GEMM_F64 | L.GEMM_IN_ORDER, 'lanczos': L.GEMM_F64 | L.GEMM_IN_ORDER, 'svd': 1}
+    assert {k for k, _ in seen} == set(want)
+    assert all(v == want[k] for k, v in seen)

@@ -1374,3 +1374,139 @@ def test_svd_columns_of_equal_norm(gpu, m, n, kind):
         assert np.abs(S - ref).max() <= 1e-14 * n * ref[0]
         assert np.abs(U.T @ U - np.eye(n)).max() <= tol
         assert np.linalg.norm(U @ V - M) <= tol * np.linalg.norm(M)
+
+
+@pytest.mark.parametrize('n', [1, 3, 14, 32, 33, 64, 65, 130])
+def test_gemm_in_order(gpu, n):
+    """TNX_GEMM_IN_ORDER at the edges of its tiles (n x n outputs of K = n and
+    2 n + 1), every combination of layouts, both workgroup shapes: numpy to
+    1e-12 as the f64 mode, the same bits from both shapes, and refused for the
+    other precisions and for other bits of the mode."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    rng = np.random.RandomState(n)
+    g, keep, outs, refs = R.GemmList(), [], [], []
+    for ta in (0, 1):
+        for tb in (0, 1):
+            segs, ref = [], 0.0
+            for K, alpha in ((n, 1.0), (2 * n + 1, -0.37)):
+                A, B = rng.randn(n, K), rng.randn(K, n)
+                Ad, Bd = _dev(A.T if ta else A), _dev(B.T if tb else B)
+                keep += [Ad, Bd]
+                segs.append((Ad.data_ptr(), Ad.shape[1], ta, Bd.data_ptr(), Bd.shape[1], tb, K, alpha))
+                ref = ref + alpha * (A @ B)
+            C0 = rng.randn(n, n)
+            C0d, C = _dev(C0), torch.zeros(n, n, dtype=torch.float64, device='cuda')
+            keep.append(C0d)
+            outs.append(C)
+            refs.append(ref + 0.3 * C0)
+            g.add(C.data_ptr(), n, n, n, segs, c0=C0d.data_ptr(), ldc0=n, beta=0.3)
+    p, s = g.arrays()
+    dp, ds = _upload([p, s])
+    nt = R.gemm_tiles(p)
+    got = []
+    for var in (0, 1):
+        print('gemm in order', n, 'variant', var, flush=True)
+        L.check(lib.tnx_gemm_grouped(L.GEMM_F64 | L.GEMM_IN_ORDER | (var << 8), _vp(dp.data_ptr()), len(p),
+                                     _vp(ds.data_ptr()), nt, None, _stream()), 'gemm')
+        torch.cuda.synchronize()
+        got.append([C.cpu().numpy().copy() for C in outs])
+    for a, b, ref in zip(got[0], got[1], refs):
+        assert np.abs(a - ref).max() <= 1e-12 * max(np.abs(ref).max(), 1.0)
+        assert np.array_equal(a, b)
+    for mode in (L.GEMM_F32 | L.GEMM_IN_ORDER, L.GEMM_BF16_F32 | L.GEMM_IN_ORDER, L.GEMM_F64 | 0x20000):
+        assert lib.tnx_gemm_grouped(mode, _vp(dp.data_ptr()), len(p), _vp(ds.data_ptr()), nt, None,
+                                    _stream()) == L.EINVAL
+
+
+@pytest.mark.parametrize('m,n', [(1, 1), (7, 7), (33, 32), (80, 80), (81, 81), (200, 9)])
+def test_svd_jacobi_in_order(gpu, m, n):
+    """A job with in_order in and out of LDS (order 80), singular values over 12
+    decades, both layouts: bounds of test_svd_jacobi_in_and_out_of_lds."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + 5 * n)
+    M = (rng.randn(m, n) * np.logspace(0, -12, n)) @ np.linalg.qr(rng.randn(n, n))[0]
+    ref = np.linalg.svd(M, compute_uv=False)
+    for trans in (0, 1):
+        src = _dev(M.T if trans else M)
+        u, s, vt, w = (torch.zeros(k, dtype=torch.float64, device='cuda')
+                       for k in (m * n, n, n * n, m * n + n * n))
+        job = np.array([(src.data_ptr(), u.data_ptr(), s.data_ptr(), vt.data_ptr(), w.data_ptr(),
+                         m, n, m if trans else n, trans, trans, 1)], dtype=L.SVD_JOB)
+        (dj,) = _upload([job])
+        print('svd in order', m, n, 'trans', trans, flush=True)
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), 1, 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        U = u.cpu().numpy()
+        U = U.reshape(n, m).T if trans else U.reshape(m, n)
+        S, V = s.cpu().numpy(), vt.cpu().numpy().reshape(n, n)
+        assert np.abs(S - ref).max() < 1e-14 * ref[0] * max(1, n)
+        assert np.all(np.diff(S) <= 0)
+        assert np.allclose(U.T @ U, np.eye(n), atol=1e-10)
+        assert np.allclose(U @ V, M, atol=1e-12 * np.abs(M).max())
+
+
+@pytest.mark.parametrize('ncv,v_dtype', [(2, 0), (7, 0), (20, 0), (32, 0), (20, 1)])
+def test_lanczos_in_order(gpu, ncv, v_dtype):
+    """A call whose plan asks for sums in a fixed order: one chunk, ends of chunks
+    and several chunks, alone and together, f64 and f32 basis.  Eigenvalue to
+    1e-9 and vector to 1e-8 of numpy's (f32 basis: 1e-5 and 1e-4) as
+    test_lanczos_batched, and the same bits alone as together."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    sizes = [3, 64, 1024, 1025, 3000]
+    rng = np.random.RandomState(ncv)
+    mats, inits = [], []
+    for n in sizes:
+        A = rng.randn(n, n)
+        diag = np.linspace(0.0, 10.0, n)
+        diag[0] = -2.0
+        mats.append(0.002 * (A + A.T) / 2 + np.diag(diag))
+        inits.append(rng.randn(n))
+    tol = 1e-8 if v_dtype == 0 else 1e-4   # residual: eigenvalue off by its square over the gap of 2
+
+    def run(idx):
+        keep, solves, outs = [], [], []
+        g2 = R.GemmList()
+        for k, i in enumerate(idx):
+            n = sizes[i]
+            Hd, init = _dev(mats[i]), _dev(inits[i])
+            V = torch.zeros((ncv + 1) * n, dtype=torch.float32 if v_dtype else torch.float64, device='cuda')
+            w, x, out = (torch.zeros(n, dtype=torch.float64, device='cuda') for _ in range(3))
+            keep += [Hd, init, V, w, x]
+            outs.append(out)
+            g2.add(w.data_ptr(), n, 1, 1, [(Hd.data_ptr(), n, 0, x.data_ptr(), 1, 0, n, 1.0)], active=k)
+            solves.append((V.data_ptr(), w.data_ptr(), x.data_ptr(), init.data_ptr(), out.data_ptr(), n,
+                           n, min(ncv, n), 0, tol, 1e-4, 0.0, 0, 0, v_dtype))
+        lz = L.lanczos_records(solves)
+        ch = (lz['n'] + L.LZ_CHUNK - 1) // L.LZ_CHUNK
+        lz['chunk_begin'] = np.concatenate([[0], np.cumsum(ch)[:-1]])
+        nch = int(ch.sum())
+        p, s = g2.arrays()
+        dp, ds, dlz = _upload([p, s, lz])
+        mode = L.GEMM_F64 | L.GEMM_IN_ORDER
+        plan = L.MatvecPlan(0, 0, 0, 0, 0, 0, 0, 0, dp.data_ptr(), ds.data_ptr(), len(p),
+                            R.gemm_tiles(p), 0, mode, mode)
+        state = torch.zeros(int(lib.tnx_lanczos_state_bytes(len(idx), nch, ncv)), dtype=torch.uint8,
+                            device='cuda')
+        res = np.zeros(len(idx), dtype=L.LANCZOS_RESULT)
+        print('lanczos in order ncv', ncv, 'basis', v_dtype, 'solves', [sizes[i] for i in idx], flush=True)
+        rc = lib.tnx_lanczos_run_ex(plan, _vp(dlz.data_ptr()), len(idx), nch, ncv, 400, 1, 0, 0,
+                                    _vp(state.data_ptr()), _vp(res.ctypes.data), _stream())
+        torch.cuda.synchronize()
+        assert rc == 0, (rc, lib.tnx_last_error())
+        return [(float(res[k]['theta']), outs[k].cpu().numpy()) for k in range(len(idx))]
+
+    together = run(range(len(sizes)))
+    for i in range(len(sizes)):
+        (th, out), = run([i])
+        assert th == together[i][0] and np.array_equal(out, together[i][1])
+        e, v = np.linalg.eigh(mats[i])
+        assert abs(th - e[0]) <= (1e-5 if v_dtype else 1e-9) * abs(e[0])
+        assert abs(abs(out @ v[:, 0]) / np.linalg.norm(out) - 1) <= (1e-4 if v_dtype else 1e-8)
