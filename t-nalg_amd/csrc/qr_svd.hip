@@ -763,10 +763,13 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   for (int k = 0; k < n; ++k) {
     // position of the largest remaining column (the first of equal ones)
     const double* now = nrm[k & 1];
-    const double n0 = lane >= k && lane < n ? now[p0] : -1.0;
-    const double n1 = 64 + lane >= k && 64 + lane < n ? now[p1] : -1.0;
+    const bool in0 = lane >= k && lane < n, in1 = 64 + lane >= k && 64 + lane < n;
+    const double n0 = in0 ? now[p0] : -1.0;
+    const double n1 = in1 ? now[p1] : -1.0;
     const double top = tnx_wave_fold(fmax(n0, n1), [](double x, double y) { return fmax(x, y); });
-    const unsigned long long m0 = __ballot(n0 == top), m1 = __ballot(n1 == top);
+    // (only positions that remain: where all of their norms are NaN, top is the
+    // -1 of the others)
+    const unsigned long long m0 = __ballot(in0 && n0 == top), m1 = __ballot(in1 && n1 == top);
     const int best = m0 ? __builtin_ctzll(m0) : m1 ? 64 + __builtin_ctzll(m1) : k;   // (NaN: k)
     const int ck = at(k), cb = at(best);
     if (lane == (k & 63)) (k < 64 ? p0 : p1) = cb;

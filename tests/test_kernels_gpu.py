@@ -1510,3 +1510,46 @@ def test_lanczos_in_order(gpu, ncv, v_dtype):
         e, v = np.linalg.eigh(mats[i])
         assert abs(th - e[0]) <= (1e-5 if v_dtype else 1e-9) * abs(e[0])
         assert abs(abs(out @ v[:, 0]) / np.linalg.norm(out) - 1) <= (1e-4 if v_dtype else 1e-8)
+
+
+@pytest.mark.parametrize('m,n', [(1, 1), (5, 4), (64, 64), (65, 65), (200, 20), (66, 66)])
+@pytest.mark.parametrize('kind', ['all', 'column', 'entry', 'inf'])
+def test_svd_of_nan_stays_in_its_own_buffers(gpu, m, n, kind):
+    """A job whose matrix holds NaN (all of it, a column, one entry) or an infinity
+    next to a finite one: it ends, writes nothing outside its own u, s and vt
+    (guard values on both sides of each) and the finite job's result is that of a
+    call of its own, bit for bit."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m * n)
+    good = rng.randn(m, n)
+    bad = rng.randn(m, n)
+    if kind == 'all':
+        bad[:] = np.nan
+    elif kind == 'column':
+        bad[:, n // 2] = np.nan
+    else:
+        bad[m // 2, n // 2] = np.nan if kind == 'entry' else np.inf
+    G = 128
+    sizes = (m * n, n, n * n, m * n + n * n)
+
+    def run(mats):
+        bufs = [[torch.full((k + 2 * G,), 7.25, dtype=torch.float64, device='cuda') for k in sizes]
+                for _ in mats]
+        srcs = [_dev(M) for M in mats]
+        jobs = np.array([(x.data_ptr(),) + tuple(b.data_ptr() + 8 * G for b in bs) + (m, n, n, 0, 0, 0)
+                         for x, bs in zip(srcs, bufs)], dtype=L.SVD_JOB)
+        (dj,) = _upload([jobs])
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), len(mats), 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        return [[b.cpu().numpy() for b in bs] for bs in bufs]
+
+    print('svd of nan', m, n, kind, flush=True)
+    both = run([bad, good])
+    (alone,) = run([good])
+    for bs in both:
+        for b in bs:
+            assert np.all(b[:G] == 7.25) and np.all(b[-G:] == 7.25)
+    for a, b in zip(both[1][:3], alone[:3]):
+        assert np.array_equal(a, b)
