@@ -395,6 +395,7 @@ constexpr int SVD_T = 16;
 // doubles)
 constexpr int SVD_QR_M = 256;
 constexpr int SVD_QR_N = 72;
+constexpr int SVD_TOP = 240;
 
 // sum over the 16 lanes of a row
 __device__ __forceinline__ double row_sum(double v) {
@@ -517,7 +518,7 @@ __device__ __forceinline__ void jacobi_sweeps_in_order(PW W, int m, PW V, int n,
 // The same for two n x n matrices in LDS, n <= 16 NE: a lane's NE elements of the
 // pair's columns of W and V stay in registers from the dot products to the
 // store, all reads ahead of the angle.  Bound: latency, one such chain a round
-// (order 64 over 10 decades 609 us in all, 785 with the elements read again for
+// (order 64 over 10 decades 659 us in all, some 180 more with the elements read again for
 // each use and the pair found by remainders; 8 or 32 lanes a pair 980 and 890).
 template <int NE>
 __device__ __forceinline__ void jacobi_sweeps_lds(double* W, double* V, int n, double eps,
@@ -585,8 +586,38 @@ __device__ __forceinline__ void jacobi_sweeps_lds(double* W, double* V, int n, d
   }
 }
 
+// Squares of entries below a norm^2 of SQ_SMALL lose bits to underflow: such a
+// norm is formed from the entries over a power of two near the largest.
+constexpr double SQ_SMALL = 1e-280;
+
+// Exponent of the largest entry of a wavefront's vector, ROWS a lane.
+template <int ROWS> __device__ __forceinline__ int column_exp(const double (&v)[ROWS]) {
+  double big = 0.0;
+#pragma unroll
+  for (int t = 0; t < ROWS; ++t) big = fmax(big, fabs(v[t]));
+  return __builtin_amdgcn_frexp_exp(
+      tnx_wave_fold(big, [](double x, double y) { return fmax(x, y); }));
+}
+
+// What stands for the norm^2 of such a vector: below SQ_SMALL, above zero if any
+// entry is, rising with the norm (its logarithm, linear between powers of two).
+template <int ROWS> __device__ __forceinline__ double small_key(const double (&v)[ROWS]) {
+  const int e = column_exp(v);
+  double s = 0.0;
+#pragma unroll
+  for (int t = 0; t < ROWS; ++t) {
+    const double x = __builtin_amdgcn_ldexp(v[t], -e);
+    s += x * x;
+  }
+  s = sqrt(tnx_wave_sum(s));
+  if (s == 0.0) return 0.0;
+  const int e2 = __builtin_amdgcn_frexp_exp(s);
+  const double f = (double)(e + e2) + 2.0 * __builtin_amdgcn_ldexp(s, -e2);
+  return SQ_SMALL * (0.5 + f * (1.0 / 4096.0));
+}
+
 // Singular values sv (LDS) = column norms of W, order = their descending order.
-template <typename PW>
+template <bool SCALE, typename PW>
 __device__ __forceinline__ void sort_columns(PW W, int m, int n, double* sv, int* order) {
   const int lane = threadIdx.x & 63;
   for (int c = threadIdx.x >> 6; c < n; c += NQ / 64) {
@@ -594,8 +625,23 @@ __device__ __forceinline__ void sort_columns(PW W, int m, int n, double* sv, int
     double s = 0.0;
     for (int r = lane; r < m; r += 64) s += wc[r] * wc[r];
     s = tnx_wave_sum(s);
+    int ex = 0;
+    if constexpr (SCALE) {
+      if (s < SQ_SMALL) {
+        double big = 0.0;
+        for (int r = lane; r < m; r += 64) big = fmax(big, fabs(wc[r]));
+        ex = __builtin_amdgcn_frexp_exp(
+            tnx_wave_fold(big, [](double x, double y) { return fmax(x, y); }));
+        s = 0.0;
+        for (int r = lane; r < m; r += 64) {
+          const double x = __builtin_amdgcn_ldexp(wc[r], -ex);
+          s += x * x;
+        }
+        s = tnx_wave_sum(s);
+      }
+    }
     if (lane == 0) {
-      sv[c] = sqrt(s);
+      sv[c] = SCALE ? __builtin_amdgcn_ldexp(sqrt(s), ex) : sqrt(s);
       order[c] = c;   // (values that do not compare leave entries unset below)
     }
   }
@@ -634,7 +680,7 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
   const double eps = 2.220446049250313e-16 * (double)(m > 8 ? m : 8);
   if constexpr (IN_ORDER) jacobi_sweeps_in_order(W, m, V, n, eps, max_sweeps, rotated);
   else jacobi_sweeps(W, m, V, n, eps, max_sweeps, rotated);
-  sort_columns(W, m, n, sv, order);
+  sort_columns<false>(W, m, n, sv, order);
   double TNX_GLOBAL* s_out = as_global<double>(J.s);
   double TNX_GLOBAL* u = as_global<double>(J.u);
   double TNX_GLOBAL* svt = as_global<double>(J.svt);
@@ -710,10 +756,13 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
 // become 7 (order 64, values over 10 or 16 decades), 10 of a random matrix 9,
 // and a tall M is rotated as an n x n matrix.  u comes out orthonormal whatever
 // the rank.  A (m x n), X and V (n x n) in LDS, m <= 64 ROWS.  M is scaled by a
-// power of two, so that squares of its entries stay in range.
+// power of two, its largest entry to 2^SVD_TOP: products of two columns' norms^2
+// (n <= 72, m <= 256) stay below 2^1024, and squares keep their bits down to
+// columns 1e-210 of the largest.  A reflector is formed from its column over a
+// power of two of its own, so that its products with any other column stay in range.
 // us (MI355X), columns of M -> this: order 64 with values over 10 decades 2030 ->
-// 609, random 840 -> 717; 128 x 40 over 10 decades 1150 -> 302, random 550 ->
-// 343; order 16 132 -> 67, random 84 -> 71; order 8 41 -> 29.
+// 659, random 840 -> 699; 128 x 40 over 10 decades 1150 -> 312, random 550 ->
+// 351; order 16 132 -> 68, random 84 -> 73; order 8 41 -> 31.
 template <int ROWS>
 __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps, double* A, double* X,
                                             double* V, double* sv, int* order, int& rotated) {
@@ -725,6 +774,7 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   // writes the other, so that a wave which comes to its choice late chooses
   // from the same norms as the rest (the waves' orders must not differ).
   __shared__ double nrm[2][SVD_QR_N], v0s[SVD_QR_N], fs[SVD_QR_N], beta[SVD_QR_N];
+  __shared__ int vex[SVD_QR_N];   // power of two of reflector k
   const double TNX_GLOBAL* src = as_global<const double>(J.src);
   double big = 0.0;
   for (int64_t e = threadIdx.x; e < (int64_t)m * n; e += NQ) {
@@ -740,7 +790,7 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   __syncthreads();
   big = sv[lane & (NW - 1)];
   big = tnx_wave_fold(big, [](double x, double y) { return fmax(x, y); });
-  const int ex = __builtin_amdgcn_frexp_exp(big);
+  const int ex = __builtin_amdgcn_frexp_exp(big) - SVD_TOP;
   for (int e = threadIdx.x; e < m * n; e += NQ) A[e] = __builtin_amdgcn_ldexp(A[e], -ex);
   for (int e = threadIdx.x; e < n * n; e += NQ) {
     const int c = e / n;
@@ -748,9 +798,14 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   }
   __syncthreads();
   for (int c = wave; c < n; c += NW) {
-    double t = 0.0;
-    for (int r = lane; r < m; r += 64) t += A[c * m + r] * A[c * m + r];
+    double y[ROWS], t = 0.0;
+#pragma unroll
+    for (int q = 0; q < ROWS; ++q) {
+      y[q] = lane + 64 * q < m ? A[c * m + lane + 64 * q] : 0.0;
+      t += y[q] * y[q];
+    }
     t = tnx_wave_sum(t);
+    if (t < SQ_SMALL) t = small_key<ROWS>(y);
     if (lane == 0) nrm[0][c] = t;
   }
   __syncthreads();
@@ -784,7 +839,19 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
       ss += v[t] * v[t];
     }
     ss = tnx_wave_sum(ss);
-    const double xk = x[k], nx = sqrt(ss);
+    int e = __builtin_amdgcn_frexp_exp(ss) >> 1;
+    const bool small = ss < SQ_SMALL;   // (the same in every lane)
+    if (small) e = column_exp(v);
+    ss = __builtin_amdgcn_ldexp(ss, -2 * e);
+#pragma unroll
+    for (int t = 0; t < ROWS; ++t) v[t] = __builtin_amdgcn_ldexp(v[t], -e);
+    if (small) {
+      ss = 0.0;
+#pragma unroll
+      for (int t = 0; t < ROWS; ++t) ss += v[t] * v[t];
+      ss = tnx_wave_sum(ss);
+    }
+    const double xk = __builtin_amdgcn_ldexp(x[k], -e), nx = sqrt(ss);
     const double b = xk > 0.0 ? -nx : nx, v0 = xk - b;
     const double f = nx > 0.0 ? 1.0 / (nx * (nx + fabs(xk))) : 0.0;
 #pragma unroll
@@ -793,7 +860,8 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
     if (threadIdx.x == 0) {
       v0s[k] = v0;
       fs[k] = f;
-      beta[k] = b;
+      beta[k] = __builtin_amdgcn_ldexp(b, e);
+      vex[k] = e;
     }
     for (int j = k + 1 + wave; j < n; j += NW) {
       double* a = A + at(j) * m;
@@ -813,16 +881,25 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
         if (r > k) t2 += y[t] * y[t];
       }
       t2 = tnx_wave_sum(t2);
+      if (t2 < SQ_SMALL) {
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t)
+          if (lane + 64 * t <= k || lane + 64 * t >= m) y[t] = 0.0;
+        t2 = small_key<ROWS>(y);
+      }
       if (lane == 0) nrm[(k & 1) ^ 1][at(j)] = t2;
     }
     __syncthreads();
   }
-  // X: column i is row i of R
-  for (int i = wave; i < n; i += NW)
+  // X: column i is row i of R; the reflectors (rows below) over their powers
+  for (int i = wave; i < n; i += NW) {
     for (int c = lane; c < n; c += 64) {
       const int pc = c < 64 ? p0 : p1;   // (c = lane or 64 + lane)
       X[i * n + c] = c > i ? A[pc * m + i] : c == i ? beta[i] : 0.0;
     }
+    double* x = A + at(i) * m;
+    for (int r = i + 1 + lane; r < m; r += 64) x[r] = __builtin_amdgcn_ldexp(x[r], -vex[i]);
+  }
   __syncthreads();
   const double eps = 2.220446049250313e-16 * (double)(m > 8 ? m : 8);
   if (n <= 16) jacobi_sweeps_lds<1>(X, V, n, eps, max_sweeps, rotated);
@@ -830,7 +907,7 @@ __device__ __forceinline__ void svd_body_qr(const tnx_svd_job& J, int max_sweeps
   else if (n <= 48) jacobi_sweeps_lds<3>(X, V, n, eps, max_sweeps, rotated);
   else if (n <= 64) jacobi_sweeps_lds<4>(X, V, n, eps, max_sweeps, rotated);
   else jacobi_sweeps_lds<5>(X, V, n, eps, max_sweeps, rotated);
-  sort_columns(X, n, n, sv, order);
+  sort_columns<true>(X, n, n, sv, order);
   double TNX_GLOBAL* s_out = as_global<double>(J.s);
   double TNX_GLOBAL* u = as_global<double>(J.u);
   double TNX_GLOBAL* svt = as_global<double>(J.svt);

@@ -1553,3 +1553,55 @@ def test_svd_of_nan_stays_in_its_own_buffers(gpu, m, n, kind):
             assert np.all(b[:G] == 7.25) and np.all(b[-G:] == 7.25)
     for a, b in zip(both[1][:3], alone[:3]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize('m,n', [(2, 2), (3, 3), (8, 8), (33, 33), (65, 65), (150, 30)])
+@pytest.mark.parametrize('kind,decades', [('diag', 157), ('diag', 225), ('diag', 290), ('columns', 150),
+                                          ('columns', 225), ('columns', 290), ('rows', 200), ('block', 170)])
+def test_svd_graded_over_hundreds_of_decades(gpu, m, n, kind, decades):
+    """The SVD by way of a pivoted QR on finite matrices whose columns (or rows, or
+    diagonal entries) fall over hundreds of decades, so that squares of what
+    remains underflow: a diagonal one gives its entries (to rounding) as singular
+    values; u is orthonormal to 1e-14 max(m, 8) whatever is left of a column; every
+    column of U vt is that of M to 1e-14 max(m, 8) of its own norm (of ||M|| for
+    graded rows)."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + n + decades)
+    fall = 10.0 ** (-decades * np.arange(n) / max(n - 1, 1))
+    if kind == 'diag':
+        M = np.zeros((m, n))
+        M[np.arange(n), rng.permutation(n)] = fall * np.where(rng.randn(n) < 0, -1.0, 1.0)
+    elif kind == 'columns':
+        M = rng.randn(m, n) * fall[rng.permutation(n)]
+    elif kind == 'rows':
+        M = rng.randn(m, n) * np.resize(fall, m)[:, None]
+    else:
+        M = np.zeros((m, n))
+        h = (n + 1) // 2
+        M[:h, :h] = np.linalg.qr(rng.randn(h, h))[0] * 1e70
+        M[h:, h:] = rng.randn(m - h, n - h) * 10.0 ** (70 - decades)
+    tol = 1e-14 * max(m, 8)
+    for trans in (0, 1):
+        src = _dev(M.T if trans else M)
+        u, s, vt, w = (torch.zeros(k, dtype=torch.float64, device='cuda')
+                       for k in (m * n, n, n * n, m * n + n * n))
+        job = np.array([(src.data_ptr(), u.data_ptr(), s.data_ptr(), vt.data_ptr(), w.data_ptr(),
+                         m, n, m if trans else n, trans, trans, 0)], dtype=L.SVD_JOB)
+        (dj,) = _upload([job])
+        print('svd graded', m, n, kind, decades, 'trans', trans, flush=True)
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), 1, 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        U = u.cpu().numpy()
+        U = U.reshape(n, m).T if trans else U.reshape(m, n)
+        S, V = s.cpu().numpy(), vt.cpu().numpy().reshape(n, n)
+        assert np.all(np.isfinite(U)) and np.all(np.isfinite(V)) and np.all(np.isfinite(S))
+        assert np.all(np.diff(S) <= 0)
+        assert np.abs(U.T @ U - np.eye(n)).max() <= tol
+        if kind == 'diag':
+            assert np.all(np.abs(S - fall) <= 1e-14 * n * fall)
+        sc = np.abs(M).max(axis=0) if kind != 'rows' else np.full(n, np.abs(M).max())
+        sc = np.where(sc > 0, sc, 1.0)
+        off = np.linalg.norm(U @ (V / sc) - M / sc, axis=0)
+        assert np.all(off <= tol * np.linalg.norm(M / sc, axis=0).clip(1.0)), off.max()
