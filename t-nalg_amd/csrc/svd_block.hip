@@ -417,6 +417,7 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
     return TNX_EHIP;
   }
   bool converged = false;
+  int recorded = 0;   // sweeps with a recorded event
   hipError_t err = hipSuccess;
   for (int sweep = 0; sweep < max_sweeps && !converged && err == hipSuccess; ++sweep) {
     for (int r = 0; r < max_nblk - 1; ++r)
@@ -425,6 +426,7 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
                        (volatile int32_t*)g_flag_pin + (sweep & 1));
     err = hipGetLastError();
     if (err == hipSuccess) err = hipEventRecord(ev[sweep & 1], s);
+    if (err == hipSuccess) ++recorded;
     // the previous sweep's flag, or after the last allowed sweep its own too
     for (int k = sweep > 0 ? sweep - 1 : 0; err == hipSuccess && !converged && k <= sweep; ++k) {
       if (k == sweep && sweep + 1 < max_sweeps) break;
@@ -432,14 +434,22 @@ extern "C" int tnx_svd_block_jacobi(const tnx_svdj_job* jobs, int njob, int npai
       converged = err == hipSuccess && ((volatile int32_t*)g_flag_pin)[k & 1] == 0;
     }
   }
+  if (err == hipSuccess) {
+    hipLaunchKernelGGL(k_svdj_norms, dim3((max_n + 3) / 4, njob), dim3(NT), 0, s, jobs);
+    hipLaunchKernelGGL(k_svdj_sort, dim3(max_n, njob), dim3(NT), 0, s, jobs);
+    err = hipGetLastError();
+  }
+  // The sweep queued past the last one publishes too: its write must be over
+  // before this thread's next call, which may be on another stream, reads the
+  // slots (the wait is for that sweep; norms and order run meanwhile).
+  const hipError_t last =
+      err == hipSuccess ? hipEventSynchronize(ev[(recorded - 1) & 1]) : hipStreamSynchronize(s);
+  if (err == hipSuccess) err = last;
   (void)hipEventDestroy(ev[0]);
   (void)hipEventDestroy(ev[1]);
   if (err != hipSuccess) {
     tnx_set_error("tnx_svd_block_jacobi: %s", hipGetErrorString(err));
     return TNX_EHIP;
   }
-  hipLaunchKernelGGL(k_svdj_norms, dim3((max_n + 3) / 4, njob), dim3(NT), 0, s, jobs);
-  hipLaunchKernelGGL(k_svdj_sort, dim3(max_n, njob), dim3(NT), 0, s, jobs);
-  TNX_CHECK_LAUNCH();
   return converged ? TNX_OK : TNX_ENOCONV;
 }

@@ -1605,3 +1605,43 @@ def test_svd_graded_over_hundreds_of_decades(gpu, m, n, kind, decades):
         sc = np.where(sc > 0, sc, 1.0)
         off = np.linalg.norm(U @ (V / sc) - M / sc, axis=0)
         assert np.all(off <= tol * np.linalg.norm(M / sc, axis=0).clip(1.0)), off.max()
+
+
+def test_svd_block_jacobi_calls_on_two_streams(gpu):
+    """One thread, a call of order 1024 on one stream and at once calls of order
+    16 on another, several times: nothing that the first still has queued when it
+    returns (the sweep past its last one) may reach the flag slots the others
+    read.  Values to 1e-13 n of numpy's."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(31)
+
+    def job(n):
+        R = np.triu(rng.randn(n, n))
+        r, work, s = _dev(R), torch.zeros(2 * n * n + n + 1, dtype=torch.float64, device='cuda'), \
+            torch.zeros(n, dtype=torch.float64, device='cuda')
+        u, v = (torch.zeros(n * n, dtype=torch.float64, device='cuda') for _ in range(2))
+        bw, nblk = L.svdj_blocking(n)
+        rec = np.array([(r.data_ptr(), work.data_ptr(), u.data_ptr(), v.data_ptr(), s.data_ptr(),
+                         n, n, bw, nblk, 0, 0)], dtype=L.SVDJ_JOB)
+        (dj,) = _upload([rec])
+        return R, s, (r, work, u, v, dj), nblk, torch.zeros(4, dtype=torch.int32, device='cuda')
+
+    def call(j, stream):
+        R, s, keep, nblk, flag = j
+        L.check(lib.tnx_svd_block_jacobi(_vp(keep[-1].data_ptr()), 1, nblk // 2, nblk, R.shape[0],
+                                         _vp(flag.data_ptr()), 60, _vp(stream.cuda_stream)), 'svd')
+
+    big, small = [job(1024) for _ in range(2)], [[job(16) for _ in range(24)] for _ in range(2)]
+    torch.cuda.synchronize()
+    sa, sb = torch.cuda.Stream(), torch.cuda.Stream()
+    for k in range(2):
+        print('svd_block_jacobi two streams', k, flush=True)
+        call(big[k], sa)
+        for j in small[k]:
+            call(j, sb)
+    torch.cuda.synchronize()
+    for R, s, _, _, _ in big + small[0] + small[1]:
+        ref = np.linalg.svd(R, compute_uv=False)
+        assert np.abs(s.cpu().numpy() - ref).max() < 1e-13 * ref[0] * R.shape[0]
