@@ -71,10 +71,10 @@ SVDJ_NMAX = 1024
 OK, EINVAL, ENOCONV = 0, -1, -3   # tnx_status values
 
 
-def svdj_blocking(n):
+def svdj_blocking(n, values_only=False):
     """(bw, nblk) of tnx_svd_block_jacobi for order n: blocks of the 16
     columns a panel's Gram matrix takes from each side, nblk = ceil(n / 16)
-    rounded up to even."""
+    rounded up to even; the same for values-only jobs."""
     bw = 16
     nblk = -(-n // bw)
     return bw, nblk + (nblk % 2)

@@ -378,3 +378,12 @@ def test_gemm_kmax_and_tuner_encoding():
     assert t.mode_for(L.GEMM_F64, 512, 512) == L.GEMM_F64
     t.tune(L.GEMM_F32, 512, 512, None)      # a mode with one variant is not timed
     assert t.shape_class(L.GEMM_F32, 512, 512) not in t.table
+
+
+@pytest.mark.parametrize('n', [8, 16, 17, 128, 1000])
+def test_svdj_blocking_takes_values_only(n):
+    """Every argument that callers of the blocking pass: an even number of blocks
+    that covers the order, the same for values-only jobs."""
+    bw, nblk = L.svdj_blocking(n)
+    assert nblk % 2 == 0 and bw * nblk >= n and bw * (nblk - 2) < n
+    assert L.svdj_blocking(n, values_only=True) == L.svdj_blocking(n, False) == (bw, nblk)
