@@ -1035,6 +1035,11 @@ __device__ __forceinline__ double chol_readlane(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// What a pivot that is not positive (or NaN) is replaced by: the smallest normal
+// number, so that fmax leaves every other pivot as it is (a compare and selects
+// instead of it take 4% of the kernel).
+constexpr double CHOL_TINY = 2.2250738585072014e-308;
+
 // The diagonal block D (LDS, 16 rows of CB_LD) -> R_pp with zeros below the
 // diagonal; F (16 rows of CB_XLD) = R_pp^{-T}.  One wave: lane j < 16 holds
 // column j of D, lane 16 + j that of E (the identity at first).  Step k: row k
@@ -1048,7 +1053,7 @@ __device__ __forceinline__ void chol_diag(double* D, double* F, int lane, int& b
 #pragma unroll
   for (int i = 0; i < 16; ++i) d[i] = inv ? (i == j ? 1.0 : 0.0) : D[i * CB_LD + j];
   double piv = chol_readlane(d[0], 0);
-  double x = fmax(piv, 1e-300), y = __builtin_amdgcn_rsq(x);   // (not positive, NaN: 1e-300)
+  double x = fmax(piv, CHOL_TINY), y = __builtin_amdgcn_rsq(x);
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
     bad |= !(piv > 0.0);
@@ -1057,7 +1062,7 @@ __device__ __forceinline__ void chol_diag(double* D, double* F, int lane, int& b
     if (k == 15) break;
     d[k + 1] = fma(-chol_readlane(d[k], k + 1), d[k], d[k + 1]);
     piv = chol_readlane(d[k + 1], k + 1);
-    x = fmax(piv, 1e-300);
+    x = fmax(piv, CHOL_TINY);
     y = __builtin_amdgcn_rsq(x);
     __builtin_amdgcn_sched_barrier(0);
     double r[16];

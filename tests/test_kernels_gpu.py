@@ -1645,3 +1645,37 @@ def test_svd_block_jacobi_calls_on_two_streams(gpu):
     for R, s, _, _, _ in big + small[0] + small[1]:
         ref = np.linalg.svd(R, compute_uv=False)
         assert np.abs(s.cpu().numpy() - ref).max() < 1e-13 * ref[0] * R.shape[0]
+
+
+@pytest.mark.parametrize('n', [1, 16, 17, 128])
+def test_chol_inv_of_tiny_matrices(gpu, n):
+    """Entries of 1e-303, where a positive pivot is below the value that stands for
+    one that is not: R and its inverse are those of the matrix over 2^-1000,
+    scaled (to 1e-12 of the largest entry, condition below 10), status 0; a zero
+    pivot still gives status 1."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(n)
+    A = rng.randn(4 * n + 8, n)
+    S = A.T @ A / (4 * n + 8)
+    Z = S.copy()
+    Z[n // 2, :] = Z[:, n // 2] = 0.0
+    for M, bad in ((np.ldexp(S, -1006), 0), (Z, 1)):
+        g = _dev(M)
+        r, ri = (torch.zeros(n * n, dtype=torch.float64, device='cuda') for _ in range(2))
+        st = torch.full((1,), 7, dtype=torch.int32, device='cuda')
+        job = np.array([(g.data_ptr(), r.data_ptr(), ri.data_ptr(), st.data_ptr(), 0, n, n, 0.0)],
+                       dtype=L.CHOL_JOB)
+        (dj,) = _upload([job])
+        print('chol tiny', n, bad, flush=True)
+        L.check(lib.tnx_chol_inv_f64(_vp(dj.data_ptr()), 1, _stream()), 'chol')
+        torch.cuda.synchronize()
+        assert int(st.item()) == bad
+        if bad == 0:
+            ref = np.linalg.cholesky(S).T
+            inv = np.linalg.inv(ref)
+            got = np.ldexp(r.cpu().numpy().reshape(n, n), 503)
+            gi = np.ldexp(ri.cpu().numpy().reshape(n, n), -503)
+            assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+            assert np.abs(gi - inv).max() <= 1e-12 * np.abs(inv).max()
