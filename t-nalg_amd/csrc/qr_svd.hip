@@ -59,13 +59,28 @@ __device__ __forceinline__ void qr_small(const tnx_qr_job& J, QrLds& L) {
   const int m = J.m, n = J.n, k = m < n ? m : n, t = threadIdx.x;
   const int w0 = t & ~63;   // first column of the wave: waves without columns only keep the barriers
   const double TNX_GLOBAL* src = as_global<const double>(J.src);
+  int ld = J.ld, trans = J.trans;
+  // More columns than lanes: R is written before the last ones are read, so src
+  // is copied first if R may lie in it.
+  const uint64_t len = 8 * (trans ? (uint64_t)(n - 1) * ld + m : (uint64_t)(m - 1) * ld + n);
+  if (n > NQ && J.r < J.src + len && J.src < J.r + 8 * (uint64_t)k * n) {
+    double TNX_GLOBAL* W = as_global<double>(J.work);
+    for (int e = t; e < m * n; e += NQ) {
+      const int c = e / m;
+      W[e] = src_at(src, ld, trans, e - c * m, c);
+    }
+    __syncthreads();
+    src = W;
+    ld = m;
+    trans = 1;
+  }
   double TNX_GLOBAL* R = as_global<double>(J.r);
   double TNX_GLOBAL* q = as_global<double>(J.q);
   double (*V)[QS + 1] = L.S;   // V[j]: zeros, V[j][j] = 1, the reflector, zeros past m
   double x[MR];
   auto load = [&](int c) {
 #pragma unroll
-    for (int r = 0; r < MR; ++r) x[r] = (r < m && c < n) ? src_at(src, J.ld, J.trans, r, c) : 0.0;
+    for (int r = 0; r < MR; ++r) x[r] = (r < m && c < n) ? src_at(src, ld, trans, r, c) : 0.0;
   };
   auto apply = [&](int j) {   // (I - tau v v^T) x
     double s[2] = {0.0, 0.0};

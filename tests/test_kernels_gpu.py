@@ -1679,3 +1679,34 @@ def test_chol_inv_of_tiny_matrices(gpu, n):
             gi = np.ldexp(ri.cpu().numpy().reshape(n, n), -503)
             assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
             assert np.abs(gi - inv).max() <= 1e-12 * np.abs(inv).max()
+
+
+@pytest.mark.parametrize('m,n', [(4, 40), (16, 1024), (3, 1025), (16, 2500), (17, 600)])
+@pytest.mark.parametrize('where', ['r', 'q', 'apart'])
+def test_qr_outputs_in_the_source(gpu, m, n, where):
+    """R or Q written over the matrix itself, both layouts, up to and beyond the
+    1024 columns a workgroup holds: the bits of a call with buffers of their own."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + n)
+    M = rng.randn(m, n)
+    k = min(m, n)
+    for trans in (0, 1):
+        got = []
+        for alias in (None, where):
+            src = _dev(M.T if trans else M).reshape(-1)
+            q, r, w = (torch.zeros(c, dtype=torch.float64, device='cuda')
+                       for c in (m * k, k * n, m * n + m * k))
+            qp = src if alias == 'q' else q
+            rp = src if alias == 'r' else r
+            job = np.array([(src.data_ptr(), qp.data_ptr(), rp.data_ptr(), w.data_ptr(), m, n,
+                             m if trans else n, trans, 0, 0)], dtype=L.QR_JOB)
+            (dj,) = _upload([job])
+            print('qr in the source', m, n, where, 'trans', trans, flush=True)
+            L.check(lib.tnx_qr_f64(_vp(dj.data_ptr()), 1, _stream()), 'qr')
+            torch.cuda.synchronize()
+            got.append((qp[:m * k].cpu().numpy().copy(), rp[:k * n].cpu().numpy().copy()))
+        assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+        Q, R = got[0][0].reshape(m, k), got[0][1].reshape(k, n)
+        assert np.abs(Q @ R - M).max() <= 1e-14 * np.sqrt(m * n) * np.abs(M).max()
