@@ -407,9 +407,11 @@ __global__ __launch_bounds__(NQ) void qr_kernel(const tnx_qr_job* __restrict__ j
 constexpr size_t SVD_LDS = 100 * 1024;
 constexpr int SVD_T = 16;
 // the SVD by way of a QR: rows, and columns, at most (SVD_LDS holds m n + 2 n^2
-// doubles)
+// doubles, m >= n)
 constexpr int SVD_QR_M = 256;
-constexpr int SVD_QR_N = 72;
+constexpr int SVD_QR_N = 65;
+static_assert(3 * 8 * SVD_QR_N * SVD_QR_N <= (int)SVD_LDS &&
+                  3 * 8 * (SVD_QR_N + 1) * (SVD_QR_N + 1) > (int)SVD_LDS, "the largest square");
 constexpr int SVD_TOP = 240;
 
 // sum over the 16 lanes of a row
@@ -450,9 +452,9 @@ __device__ __forceinline__ void jacobi_sweeps(PW W, int m, PW V, int n, double e
         ga = row_sum(ga);
         const double ab = al * be;
         const bool rot = ga != 0.0 && fabs(ga) > eps * (ab > 0.0 ? ab * __builtin_amdgcn_rsq(ab) : 0.0);
-        const JacobiRot jr = jacobi_rot(al, be, ga, rot, false);
-        if (rot || jr.swap) {
-          if (l == 0 && rot) rotated = 1;
+        if (rot) {
+          const JacobiRot jr = jacobi_rot(al, be, ga, rot, false);
+          if (l == 0) rotated = 1;
           for (int r = l; r < m; r += SVD_T) {
             double x = wa[r], y = wb[r];
             jacobi_apply(jr, x, y);
@@ -772,7 +774,7 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
 // and a tall M is rotated as an n x n matrix.  u comes out orthonormal whatever
 // the rank.  A (m x n), X and V (n x n) in LDS, m <= 64 ROWS.  M is scaled by a
 // power of two, its largest entry to 2^SVD_TOP: products of two columns' norms^2
-// (n <= 72, m <= 256) stay below 2^1024, and squares keep their bits down to
+// (n <= 65, m <= 256) stay below 2^1024, and squares keep their bits down to
 // columns 1e-210 of the largest.  A reflector is formed from its column over a
 // power of two of its own, so that its products with any other column stay in range.
 // us (MI355X), columns of M -> this: order 64 with values over 10 decades 2030 ->
