@@ -337,26 +337,26 @@ def live_kernels(stats):
 # (--pmc FETCH_SIZE, then --pmc WRITE_SIZE; KiB per dispatch averaged over
 # the 23 launches after each loop marker, --pmc-summary), scaled by what the
 # counters read for the calibration copy of 256 MiB (FETCH_SIZE x 2.00,
-# WRITE_SIZE x 1.00).  The GEMMs are priced in flops (2.15e9 per launch at
+# WRITE_SIZE x 1.00), kernels of commit e9e96f8.  The GEMMs are priced in flops (2.15e9 per launch at
 # that step), so only the mixer has an algorithmic byte count; a GEMM
 # class's traffic in the bench line is its live average launch's flops
 # times the measured bytes per flop.
 MATVEC_PMC_TRAFFIC = {
-    'mixer matvec': {'bf16': (42.5e6, 50.3e6), 'fp32': (76.1e6, 92.3e6),
-                     'fp64': (152.1e6, 184.5e6)},
+    'mixer matvec': {'bf16': (42.2e6, 50.3e6), 'fp32': (75.7e6, 92.3e6),
+                     'fp64': (151.2e6, 184.5e6)},
     'gemm f64 matvec T = F x': {'fp64': (117.7e6, None)},
     'gemm f64 matvec w = U R^T': {'fp64': (134.4e6, None)},
-    'gemm f32 matvec T = F x': {'fp32': (63.5e6, None)},
-    'gemm f32 matvec w = U R^T': {'fp32': (63.5e6, None)},
+    'gemm f32 matvec T = F x': {'fp32': (59.0e6, None)},
+    'gemm f32 matvec w = U R^T': {'fp32': (67.4e6, None)},
     'gemm bf16 matvec T = F x': {'bf16': (29.7e6, None)},
-    'gemm bf16 matvec w = U R^T': {'bf16': (42.7e6, None)},
+    'gemm bf16 matvec w = U R^T': {'bf16': (42.2e6, None)},
 }
 MATVEC_PMC_FLOPS = 2.15e9   # flops of each GEMM launch of those counter runs
 
 
-KERNEL_OF_CLASS = {'gemm f64': 'gemm_grouped_kernel<0>', 'gemm f32': 'gemm_grouped_kernel<1>',
-                   'gemm bf16 matvec T': 'gemm_grouped_kernel<3>',
-                   'gemm bf16 matvec w': 'gemm_grouped_kernel<2>', 'mixer': 'mix_kernel',
+KERNEL_OF_CLASS = {'gemm f64': 'gemm_grouped_kernel<0, ..>', 'gemm f32': 'gemm_grouped_kernel<1, ..>',
+                   'gemm bf16 matvec T': 'gemm_grouped_kernel<3, ..>',
+                   'gemm bf16 matvec w': 'gemm_grouped_kernel<2, ..>', 'mixer': 'mix_kernel',
                    'k_dots': 'k_dots', 'k_update_dots': 'k_update_dots',
                    'k_update_norm': 'k_update_norm'}
 
