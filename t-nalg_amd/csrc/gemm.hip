@@ -60,9 +60,34 @@ template <typename TI, int TT, int MB> struct Operand {
   // count loads and leave the later ones in flight).  Rows past `lim` repeat
   // earlier ones (their products are not stored) and k past K earlier k,
   // which clear() zeroes when the chunk is staged.  WIDE: one 16-byte load a
-  // piece, for sizes that pieces divide (wide_ok); otherwise by elements.
+  // piece, for sizes that pieces divide, and of 16-bit elements for all of a piece
+  // at least (wide_ok): the piece that such a size ends in is loaded up to that
+  // end, and clear() or align() moves its elements to their places.  Otherwise by
+  // elements.  (Eight loads a piece are too many: 64 products of 100 x 200 x 400 in
+  // bf16 30 us by elements, 12 so.  Two or four are not: 8-byte elements lose up to
+  // 10% of a small launch to the moves.)
   template <bool KC> static __device__ __forceinline__ bool wide_ok(int lim, int K) {
-    return ((KC ? K : lim) % E) == 0;
+    const int n = KC ? K : lim;
+    return HALF ? n >= E : n % E == 0;
+  }
+  // the elements of r from the `sh`-th on, zeros behind them (sh >= E: zeros)
+  static __device__ __forceinline__ u4 from_element(u4 r, int sh) {
+    unsigned __int128 v = __builtin_bit_cast(unsigned __int128, r);
+    v = sh < E ? v >> (8 * (int)sizeof(TI) * sh) : (unsigned __int128)0;
+    return __builtin_bit_cast(u4, v);
+  }
+  // [k][row], WIDE: whether the rows of the tile end within a piece, and its place
+  static __device__ __forceinline__ bool ragged(int row0, int lim) {
+    return HALF && row0 + TT > lim && lim % E != 0;
+  }
+  static __device__ __forceinline__ void align(u4 (&r)[NP], int row0, int lim) {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));   // formed in the branch, not ahead of the stream
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+      const int sh = row0 + ((t + 256 * q) % PR) * E + E - lim;
+      if (sh > 0) r[q] = from_element(r[q], sh);
+    }
   }
   template <bool KC, bool WIDE>
   static __device__ __forceinline__ void fetch(u4 (&r)[NP], uint64_t b, int64_t ld, int row0,
@@ -103,10 +128,17 @@ template <typename TI, int TT, int MB> struct Operand {
   }
 
   // zero the pieces' elements from k index `valid` of the chunk on
-  template <bool KC> static __device__ __forceinline__ void clear(u4 (&r)[NP], int valid) {
+  template <bool KC, bool WIDE> static __device__ __forceinline__ void clear(u4 (&r)[NP], int valid) {
+    int t = threadIdx.x;
+    if constexpr (HALF) asm volatile("" : "+v"(t));
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
-      const int c = threadIdx.x + 256 * q;
+      const int c = t + 256 * q;
+      if constexpr (KC && WIDE && HALF) {
+        const int sh = (c & 7) * E + E - valid;
+        if (sh > 0) r[q] = from_element(r[q], sh);
+        continue;
+      }
       TI e[E];
       __builtin_memcpy(e, &r[q], 16);
 #pragma unroll
@@ -281,7 +313,11 @@ __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][
   typedef Operand<typename Tr<MODE>::TI, TT, MB> O;
   u4 ra[PD][O::NP], rb[PD][O::NP];
   double al[PD];
-  int kv[PD];           // k of the chunk that exist
+  // k of the chunk that exist; where the tile ends within a piece, so much less
+  // that every chunk of it takes the branch of the ends below
+  int kv[PD];
+  const bool edge_a = WIDE && !KA && O::ragged(row0, M), edge_b = WIDE && !KBc && O::ragged(col0, N);
+  const int less = edge_a || edge_b ? 1 << 30 : 0;
   // the stream's extent: its segments and chunks
   int chunks = 0, end = s;
   for (; end < s_end; ++end) {
@@ -299,7 +335,7 @@ __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][
     O::template fetch<KA, WIDE>(ra[d], A, lda, row0, M, k0, K);
     O::template fetch<KBc, WIDE>(rb[d], B, ldb, col0, N, k0, K);
     al[d] = alpha;
-    kv[d] = K - k0;
+    kv[d] = K - k0 - less;
     if (k0 + O::KB < K) {
       k0 += O::KB;
     } else {
@@ -320,8 +356,11 @@ __device__ __forceinline__ int run_stream(typename Tr<MODE>::V4 (&acc)[TT / 32][
   auto commit = [&](int d, int stage) {
     if (kv[d] < O::KB) {
       asm volatile("");   // a branch, not selects on every chunk
-      O::template clear<KA>(ra[d], kv[d]);
-      O::template clear<KBc>(rb[d], kv[d]);
+      const int valid = kv[d] + less;
+      if (edge_a) O::align(ra[d], row0, M);
+      if (edge_b) O::align(rb[d], col0, N);
+      O::template clear<KA, WIDE>(ra[d], valid);
+      O::template clear<KBc, WIDE>(rb[d], valid);
     }
     if (__double_as_longlong(al[d]) != 0x3FF0000000000000ll) {
       asm volatile("");

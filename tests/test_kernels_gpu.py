@@ -1710,3 +1710,56 @@ def test_qr_outputs_in_the_source(gpu, m, n, where):
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
         Q, R = got[0][0].reshape(m, k), got[0][1].reshape(k, n)
         assert np.abs(Q @ R - M).max() <= 1e-14 * np.sqrt(m * n) * np.abs(M).max()
+
+
+@pytest.mark.parametrize('mode', ['f64', 'f32', 'bf16_f32', 'bf16_bf16', 'in order'])
+@pytest.mark.parametrize('ta,tb', [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_gemm_ragged_sizes_are_exact(gpu, mode, ta, tb):
+    """Every remainder of a 16-byte piece in M, N and K, below and above a piece, a
+    chunk and a tile, tight and odd leading dimensions, buffers that start one
+    element past a 16-byte line: products of -1, 0 and 1, whose sums (below 256) every precision
+    holds exactly, must be numpy's to the last bit, whatever lies between the rows
+    (NaN), in both workgroup shapes."""
+    import torch
+    from tnalg_amd import _lib as L
+    from tnalg_amd import records as R
+    lib = L.load()
+    code, tin, tout, _ = MODES['f64' if mode == 'in order' else mode]
+    if mode == 'in order':
+        code |= L.GEMM_IN_ORDER
+    ti, to = getattr(torch, tin), getattr(torch, tout)
+    rng = np.random.RandomState(9)
+    g, keep, outs = R.GemmList(), [], []
+    dims = list(range(1, 19)) + [31, 32, 33, 39, 61, 63, 64, 65, 66, 71, 90, 101, 127]
+
+    def operand(rows, cols, pad):
+        buf = torch.full((1 + rows * (cols + pad),), float('nan'), dtype=torch.float64)
+        a = rng.randint(-1, 2, (rows, cols)).astype(float)
+        buf[1:].reshape(rows, cols + pad)[:, :cols] = torch.from_numpy(a)
+        d = buf.to(ti).cuda()
+        keep.append(d)
+        return a, d.data_ptr() + d.element_size(), cols + pad
+
+    for i in range(400):
+        M, N, K, K2 = (int(dims[rng.randint(len(dims))]) for _ in range(4))
+        segs, ref = [], 0.0
+        for k, alpha in ((K, 1.0), (min(K2, 100), -1.0)):
+            A, ap, lda = operand(*((k, M) if ta else (M, k)), (0, 3)[i & 1])
+            B, bp, ldb = operand(*((N, k) if tb else (k, N)), (0, 5)[(i >> 1) & 1])
+            segs.append((ap, lda, ta, bp, ldb, tb, k, alpha))
+            ref = ref + alpha * ((A.T if ta else A) @ (B.T if tb else B))
+        C = torch.full((M, N + 2), 9.0, dtype=to, device='cuda')
+        outs.append((C, ref, (M, N, K, K2)))
+        g.add(C.data_ptr(), M, N, N + 2, segs)
+    p, s = g.arrays()
+    dp, ds = _upload([p, s])
+    for var in (0, 1):
+        print('gemm ragged', mode, ta, tb, 'variant', var, flush=True)
+        L.check(lib.tnx_gemm_grouped(code | (var << 8), _vp(dp.data_ptr()), len(p), _vp(ds.data_ptr()),
+                                     R.gemm_tiles(p), None, _stream()), 'gemm')
+        torch.cuda.synchronize()
+        for C, ref, sh in outs:
+            got = C.double().cpu().numpy()
+            assert np.array_equal(got[:, :ref.shape[1]], ref), sh
+            assert np.all(got[:, ref.shape[1]:] == 9.0), sh
+            C.fill_(9.0)
