@@ -422,17 +422,28 @@ __device__ __forceinline__ double row_sum(double v) {
   return v + tnx_row_get<0x121>(v);
 }
 
-// Rotates the columns of W (m x n) until they are orthogonal, V (n x n) along.
-template <typename PW>
+// and over T lanes, a row or the wavefront
+template <int T> __device__ __forceinline__ double lane_sum(double v) {
+  static_assert(T == 16 || T == 64, "a row or a wavefront");
+  if constexpr (T == 64) return tnx_wave_sum(v);
+  else return row_sum(v);
+}
+
+// Rotates the columns of W (m x n) until they are orthogonal, V (n x n) along; T
+// (16 or 64) lanes a pair.  64 where the 16 wavefronts hold all pairs of a round
+// at once (n <= 32): 300 x 20 over 10 decades 676 us with 16 and 416 with 64,
+// 1024 x 7 269 and 93 (230 by four wavefronts on columns in global memory), 280 x
+// 30 534 and 440.
+template <int T, typename PW>
 __device__ __forceinline__ void jacobi_sweeps(PW W, int m, PW V, int n, double eps, int max_sweeps,
                                               int& rotated) {
-  const int l = threadIdx.x & (SVD_T - 1);
+  const int l = threadIdx.x & (T - 1);
   const int np = (n + 1) & ~1;  // players in the round-robin tournament
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     if (threadIdx.x == 0) rotated = 0;
     __syncthreads();
     for (int round = 0; round < np - 1; ++round) {
-      for (int p = threadIdx.x / SVD_T; p < np / 2; p += NQ / SVD_T) {
+      for (int p = threadIdx.x / T; p < np / 2; p += NQ / T) {
         // circle method: player np-1 fixed, others rotate
         int a = (p == 0) ? np - 1 : (round + p) % (np - 1);
         int b = (round + np - 1 - p) % (np - 1);
@@ -441,28 +452,28 @@ __device__ __forceinline__ void jacobi_sweeps(PW W, int m, PW V, int n, double e
         if (a > b) { int t = a; a = b; b = t; }
         const PW wa = W + (int64_t)a * m, wb = W + (int64_t)b * m;
         double al = 0.0, be = 0.0, ga = 0.0;
-        for (int r = l; r < m; r += SVD_T) {
+        for (int r = l; r < m; r += T) {
           const double x = wa[r], y = wb[r];
           al += x * x;
           be += y * y;
           ga += x * y;
         }
-        al = row_sum(al);
-        be = row_sum(be);
-        ga = row_sum(ga);
+        al = lane_sum<T>(al);
+        be = lane_sum<T>(be);
+        ga = lane_sum<T>(ga);
         const double ab = al * be;
         const bool rot = ga != 0.0 && fabs(ga) > eps * (ab > 0.0 ? ab * __builtin_amdgcn_rsq(ab) : 0.0);
         if (rot) {
           const JacobiRot jr = jacobi_rot(al, be, ga, rot, false);
           if (l == 0) rotated = 1;
-          for (int r = l; r < m; r += SVD_T) {
+          for (int r = l; r < m; r += T) {
             double x = wa[r], y = wb[r];
             jacobi_apply(jr, x, y);
             wa[r] = x;
             wb[r] = y;
           }
           const PW va = V + (int64_t)a * n, vb = V + (int64_t)b * n;
-          for (int r = l; r < n; r += SVD_T) {
+          for (int r = l; r < n; r += T) {
             double x = va[r], y = vb[r];
             jacobi_apply(jr, x, y);
             va[r] = x;
@@ -696,7 +707,8 @@ __device__ __forceinline__ void svd_body(const tnx_svd_job& J, int max_sweeps, P
   // rotate while |a.b| > m*eps*|a||b| (columns orthogonal to working accuracy)
   const double eps = 2.220446049250313e-16 * (double)(m > 8 ? m : 8);
   if constexpr (IN_ORDER) jacobi_sweeps_in_order(W, m, V, n, eps, max_sweeps, rotated);
-  else jacobi_sweeps(W, m, V, n, eps, max_sweeps, rotated);
+  else if (n <= 2 * (NQ / 64)) jacobi_sweeps<64>(W, m, V, n, eps, max_sweeps, rotated);
+  else jacobi_sweeps<SVD_T>(W, m, V, n, eps, max_sweeps, rotated);
   sort_columns<false>(W, m, n, sv, order);
   double TNX_GLOBAL* s_out = as_global<double>(J.s);
   double TNX_GLOBAL* u = as_global<double>(J.u);

@@ -1763,3 +1763,33 @@ def test_gemm_ragged_sizes_are_exact(gpu, mode, ta, tb):
             assert np.array_equal(got[:, :ref.shape[1]], ref), sh
             assert np.all(got[:, ref.shape[1]:] == 9.0), sh
             C.fill_(9.0)
+
+
+@pytest.mark.parametrize('m,n', [(257, 1), (257, 2), (300, 20), (500, 31), (400, 32), (400, 33), (3000, 5)])
+def test_svd_jacobi_tall(gpu, m, n):
+    """Tall matrices on the columns, below and above the 32 columns up to which a
+    wavefront takes a pair, in LDS and in global memory, both layouts: bounds of
+    test_svd_jacobi_in_and_out_of_lds."""
+    import torch
+    from tnalg_amd import _lib as L
+    lib = L.load()
+    rng = np.random.RandomState(m + 7 * n)
+    M = (rng.randn(m, n) * np.logspace(0, -12, n)) @ np.linalg.qr(rng.randn(n, n))[0]
+    ref = np.linalg.svd(M, compute_uv=False)
+    for trans in (0, 1):
+        src = _dev(M.T if trans else M)
+        u, s, vt, w = (torch.zeros(k, dtype=torch.float64, device='cuda')
+                       for k in (m * n, n, n * n, m * n + n * n))
+        job = np.array([(src.data_ptr(), u.data_ptr(), s.data_ptr(), vt.data_ptr(), w.data_ptr(),
+                         m, n, m if trans else n, trans, trans, 0)], dtype=L.SVD_JOB)
+        (dj,) = _upload([job])
+        print('svd tall', m, n, 'trans', trans, flush=True)
+        L.check(lib.tnx_svd_jacobi_f64(_vp(dj.data_ptr()), 1, 60, _stream()), 'svd')
+        torch.cuda.synchronize()
+        U = u.cpu().numpy()
+        U = U.reshape(n, m).T if trans else U.reshape(m, n)
+        S, V = s.cpu().numpy(), vt.cpu().numpy().reshape(n, n)
+        assert np.abs(S - ref).max() < 1e-14 * ref[0] * max(1, n)
+        assert np.all(np.diff(S) <= 0)
+        assert np.allclose(U.T @ U, np.eye(n), atol=1e-10)
+        assert np.allclose(U @ V, M, atol=1e-12 * np.abs(M).max())
