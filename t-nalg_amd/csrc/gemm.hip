@@ -94,6 +94,62 @@ template <typename TI, int TT, int MB> struct Operand {
                                                int lim, int k0, int K) {
     typedef TI V __attribute__((ext_vector_type(E), aligned(sizeof(TI))));
     const TI TNX_GLOBAL* base = as_global<const TI>(b);
+    if constexpr (!WIDE && HALF && TT == 64) {
+      // an operand of less than a piece: pieces that reach into its next rows, the
+      // last ones up to the operand's end and then moved; what is not its own k is
+      // zero, other rows' elements belong to outputs that are not stored (in the
+      // 32x32 shape the loads by elements are the faster ones)
+      const int n = KC ? K : lim, rows = KC ? lim : K;
+      const int64_t span = (rows - 1) * ld + n;
+      if (span >= E) {
+        int at[NP], sh[NP];
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const int c = threadIdx.x + 256 * q;
+          const int row = row0 + (KC ? c >> 3 : (c % PR) * E);
+          const int k = k0 + (KC ? (c & 7) * E : c / PR);
+          at[q] = KC ? k : row;
+          const int64_t want = min(KC ? row : k, rows - 1) * ld + (at[q] < n ? at[q] : 0);
+          const int64_t off = min(want, span - E);
+          sh[q] = (int)(want - off);
+          r[q] = __builtin_bit_cast(u4, *(const V TNX_GLOBAL*)(base + off));
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          r[q] = from_element(r[q], sh[q]);
+          if constexpr (KC) {
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const uint32_t lo = at[q] + 2 * x < n ? 0xffffu : 0u, hi = at[q] + 2 * x + 1 < n ? 0xffff0000u : 0u;
+              r[q][x] &= lo | hi;
+            }
+          }
+        }
+        return;
+      }
+    }
+    if constexpr (!WIDE && HALF && TT == 64) {
+      // a matrix of less than a piece: by elements in a loop, as all eight loads
+      // cost every launch of the kernel 3%, in registers and code
+#pragma unroll
+      for (int q = 0; q < NP; ++q) r[q] = u4{0, 0, 0, 0};
+#pragma unroll 2
+      for (int x = 0; x < E; ++x) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const int c = threadIdx.x + 256 * q;
+          const int row = row0 + (KC ? c >> 3 : (c % PR) * E + x);
+          const int k = k0 + (KC ? (c & 7) * E + x : c / PR);
+          const int64_t off = KC ? min(row, lim - 1) * ld + min(k, K - 1)
+                                 : min(k, K - 1) * ld + min(row, lim - 1);
+          const uint32_t e = __builtin_bit_cast(uint16_t, (TI)base[off]);
+          // the elements so far move down, this one comes last
+          r[q] = u4{r[q][0] >> 16 | r[q][1] << 16, r[q][1] >> 16 | r[q][2] << 16,
+                    r[q][2] >> 16 | r[q][3] << 16, r[q][3] >> 16 | e << 16};
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
       const int c = threadIdx.x + 256 * q;
@@ -503,7 +559,7 @@ __global__ __launch_bounds__(256, W) void gemm_grouped_kernel(const tnx_gemm_pro
   s = wide<O, KA, KBc>(P.M, P.N, K)                                                         \
           ? run_stream<MODE, SEQ, TT, PD, KA, KBc, true>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
                                                     wc, As, Bs)                             \
-          : run_stream<MODE, SEQ, TT, PD, KA, KBc, false>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
+          : run_stream<MODE, SEQ, TT, O::HALF ? 1 : PD, KA, KBc, false>(acc, cs, s, s_end, P.M, P.N, row0, col0, wr, \
                                                      wc, As, Bs)
     if (!ta && tb) TNX_STREAM(true, true);
     else if (!ta) TNX_STREAM(true, false);
